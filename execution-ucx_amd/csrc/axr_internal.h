@@ -330,6 +330,9 @@ int launch_notify(uint32_t* flag, uint32_t value, void* stream);
 // segs and wave_seg are device memory.  Copies the records and writes the tile-block index.
 int launch_expand_tables(const Seg* staged, uint32_t n, Seg* segs, uint32_t* wave_seg, uint32_t seg_shift,
                          void* stream);
+// tables[0, bytes) = staged[0, bytes), rounded up to 16 bytes: a table block's pinned half into its
+// device half.
+int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream);
 // dst[0, bytes) = src[0, bytes), both in device memory of the current device, no alignment needed.
 int launch_stream_copy(void* dst, const void* src, size_t bytes, bool nontemporal, void* stream);
 // Device address, on the current device, of the kStaticTableBytes bytes that hold the

@@ -1415,6 +1415,18 @@ __global__ __launch_bounds__(256) void expand_tables_kernel(const Seg* staged, u
   for (uint64_t k = (first + step - 1) >> seg_shift; (k << seg_shift) < last; ++k) wave_seg[k] = i;
 }
 
+// Host-built tables from pinned memory into their device block, 16 bytes per thread.  Bound by one
+// trip over the bus (about 3 us; 106 KB then take 2 us more).  A kernel and not a copy-engine
+// transfer because of where the bytes end up: what the copy engine wrote is in none of the caches,
+// and a bundle whose wavefronts look up a new record every few kilobytes then waits for memory at
+// every one of them, three dependent reads deep (1 GiB of cache blocks in 512 views, 106 KB of
+// tables: gather 451 -> 374 us, scatter 467 -> 380 us, against 333 and 355 us once the tables have
+// been read before).
+__global__ __launch_bounds__(256) void upload_tables_kernel(const u32x4* staged, u32x4* tables, uint32_t nvec) {
+  const uint32_t i = blockIdx.x * kUtilityThreads + threadIdx.x;
+  if (i < nvec) tables[i] = staged[i];
+}
+
 // One contiguous range, 2 KiB per wavefront with the same tile copy as the bundle
 // kernels (two 16-byte loads per lane in flight, an overlapped final vector instead of a
 // byte tail).  The loopback transport moves same-device payloads with it.
@@ -1636,6 +1648,17 @@ int launch_expand_tables(const Seg* staged, uint32_t n, Seg* segs, uint32_t* wav
   hipLaunchKernelGGL(expand_tables_kernel, dim3((n + kUtilityThreads) / kUtilityThreads), dim3(kUtilityThreads), 0,
                      static_cast<hipStream_t>(stream), staged, n, segs, wave_seg, seg_shift);
   return check_hip(hipGetLastError(), "table expansion launch");
+}
+
+int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream) {
+  if (bytes == 0) return AXR_OK;
+  // both blocks are a power of two of at least 4 KiB long: the last vector may be read whole
+  const uint64_t nvec = (static_cast<uint64_t>(bytes) + kVecBytes - 1) / kVecBytes;
+  if (nvec > 0x7fffffffull) return fail(AXR_ERR_UNSUPPORTED, "bundle tables too long for one upload");
+  hipLaunchKernelGGL(upload_tables_kernel, dim3(static_cast<uint32_t>((nvec + kUtilityThreads - 1) / kUtilityThreads)),
+                     dim3(kUtilityThreads), 0, static_cast<hipStream_t>(stream), static_cast<const u32x4*>(staged),
+                     static_cast<u32x4*>(tables), static_cast<uint32_t>(nvec));
+  return check_hip(hipGetLastError(), "table upload launch");
 }
 
 int launch_stream_copy(void* dst, const void* src, size_t bytes, bool nontemporal, void* stream) {

@@ -201,6 +201,7 @@ struct axr_plan {
   bool inline_ready = false;
   uint64_t launches = 0;             // kernel launches since the tables were built
   hipEvent_t upload_event = nullptr;   // from event_acquire
+  bool upload_recorded = false;        // the event lies behind the latest upload
   int upload_event_device = -1;
   hipStream_t upload_stream = nullptr;
   struct BusyStream {
@@ -875,6 +876,30 @@ bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim)
   return true;
 }
 
+// The event behind the upload of the plan's tables, recorded at most once per upload.
+int record_upload(axr_plan* p) {
+  if (p->upload_recorded) return AXR_OK;
+  if (!p->upload_event) {
+    int rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
+    if (rc) return rc;
+  }
+  int rc = check_hip(hipEventRecord(p->upload_event, p->upload_stream), "hipEventRecord");
+  if (!rc) p->upload_recorded = true;
+  return rc;
+}
+
+// Notes that the tables have just been put on their way on `stream`.  The event that a launch on
+// another stream waits for is recorded now, except on the default stream, which can neither be
+// destroyed nor be capturing later: there it is recorded when such a launch comes, so that a plan
+// that stays on its stream pays for no event.
+int note_upload(axr_plan* p, hipStream_t stream) {
+  p->upload_stream = stream;
+  p->upload_recorded = false;
+  p->uploaded = true;
+  remember_stream(p, stream);
+  return stream ? record_upload(p) : AXR_OK;
+}
+
 // Bundles of many contiguous device tensors: one pass over the tensors writes the segment
 // records straight into pinned memory, and a kernel (one thread per segment) brings them to
 // the device and writes the tile-block index, in front of the bundle kernel on the same
@@ -959,15 +984,8 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
   int rc = launch_expand_tables(staged, static_cast<uint32_t>(n), reinterpret_cast<Seg*>(d),
                                 reinterpret_cast<uint32_t*>(d + wave_at), p->cfg.seg_shift, stream);
   if (rc) return rc;
-  if (!p->upload_event) {
-    rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
-    if (rc) return rc;
-  }
-  rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
+  rc = note_upload(p, stream);
   if (rc) return rc;
-  remember_stream(p, stream);
-  p->upload_stream = stream;
-  p->uploaded = true;
   p->device_built = true;
   *done = true;
   return AXR_OK;
@@ -1194,23 +1212,15 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
     } else {
       quiesce(p);   // previous launches may still read the old tables
     }
-    uint8_t* h = static_cast<uint8_t*>(p->block.host);
-    write_tables(p, h);
-    int rc = check_hip(hipMemcpyAsync(p->block.device, h, p->table_bytes, hipMemcpyHostToDevice,
-                                      stream),
-                       "hipMemcpyAsync(plan tables)");
+    write_tables(p, static_cast<uint8_t*>(p->block.host));
+    int rc = launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream);
     if (rc) return rc;
-    if (!p->upload_event) {
-      rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
-      if (rc) return rc;
-    }
-    rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
+    return note_upload(p, stream);
+  }
+  if (stream != p->upload_stream) {
+    int rc = record_upload(p);
     if (rc) return rc;
-    p->upload_stream = stream;
-    p->uploaded = true;
-  } else if (stream != p->upload_stream) {
-    int rc = check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
-    if (rc) return rc;
+    return check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
   }
   return AXR_OK;
 }
@@ -1537,7 +1547,7 @@ int axr_plan_create(const axr_tensor_t* tensors,
 static int plan_free_body(axr_plan_t* plan) {
   if (!plan) return AXR_OK;
   quiesce(plan);
-  if (plan->uploaded && plan->upload_event) (void)hipEventSynchronize(plan->upload_event);
+  if (plan->uploaded && plan->upload_recorded) (void)hipEventSynchronize(plan->upload_event);
   table_block_release(&plan->block);
   event_release(plan->upload_event, plan->upload_event_device);   // fired, or never recorded
   plan->upload_event = nullptr;
@@ -2095,7 +2105,8 @@ static int plan_prepare_body(axr_plan_t* plan, void* stream_) {
   if (plan->ntiles == 0 || plan->resident) return AXR_OK;
   rc = ensure_uploaded(plan, stream);
   if (rc) return rc;
-  rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
+  rc = record_upload(plan);
+  if (!rc) rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
   if (rc) return rc;
   plan->resident = true;
   return AXR_OK;

@@ -111,11 +111,12 @@ class BundlePlan:
         return cls(h.value, receiver=True)
 
     @classmethod
-    def from_header_bound(cls, header: bytes, tensors: Sequence[Any]) -> "BundlePlan":
-        """``from_header(header).bind(tensors)`` in one pass over the header."""
+    def from_header_bound(cls, header: bytes, tensors: Sequence[Any], stream=None) -> "BundlePlan":
+        """``from_header(header).bind(tensors, stream)`` in one pass over the header."""
         lib = _capi.load()
         buf = bytes(header)
-        arr = tensors if isinstance(tensors, TensorArray) else TensorArray.from_objects(tensors)
+        arr = tensors if isinstance(tensors, TensorArray) else TensorArray.from_objects(
+            tensors, stream=_dlpack_stream(stream))
         _refuse_readonly_destinations(arr)
         h = C.c_void_p()
         _capi.check(lib.axr_plan_from_header_bind(buf, len(buf), arr.pointer(), arr.count, C.byref(h)))
@@ -317,12 +318,15 @@ def unpack_bundle(header: bytes, payload: Any, payload_bytes: Optional[int] = No
         ptr, size = int(payload), payload_bytes
     if payload_bytes is not None:
         size = payload_bytes
-    plan = BundlePlan.from_header(header)
     if out is not None:
-        plan.bind(out, stream=stream)
+        try:
+            plan = BundlePlan.from_header_bound(header, out, stream=stream)
+        except Exception:  # noqa: BLE001 - a bad header is reported ahead of a bad destination
+            plan = BundlePlan.from_header(header).bind(out, stream=stream)
         plan.unpack(ptr, size, stream)
         streams.make_visible_to_producers(_stream_handle(stream))
         return plan
+    plan = BundlePlan.from_header(header)
     pieces = plan.split(ptr, size)
     metas = plan.metas()
     owner = payload  # every view keeps the payload block alive

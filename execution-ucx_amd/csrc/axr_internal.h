@@ -104,6 +104,27 @@ constexpr uint32_t transpose_edge(uint32_t element_bytes) {
 constexpr uint32_t transpose_lds_pitch(uint32_t element_bytes) {
   return transpose_edge(element_bytes) * element_bytes + 4u;
 }
+// Skewed blocks (2- to 8-byte elements; written rows that do not start on 64-byte boundaries) stage
+// up to 64 / E - 1 more rows than a block has, rounded up to what one wave-wide access covers.
+constexpr uint32_t kSkewBytes = 64;
+constexpr uint32_t transpose_skew_rows(uint32_t element_bytes) {
+  const uint32_t per_access = kWaveLanes / (transpose_edge(element_bytes) * element_bytes / kVecBytes);
+  return (transpose_edge(element_bytes) + kSkewBytes / element_bytes - 1 + per_access - 1) / per_access * per_access;
+}
+constexpr uint32_t kBlockStrip = 8;
+// Bundles up to this size (what the eight L2s hold) are moved in plain blocks: there the partly
+// written lines are completed in an L2 anyway (bf16, pack + unpack: 8 MB 14.5 plain / 16.2 us
+// skewed, 17 MB 20.8 / 21.0, 34 MB 36.9 / 34.2, 67 MB 69.7 / 63.9, 134 MB 140 / 115).
+constexpr uint64_t kSkewMinPayload = 24u << 20;
+constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4, 5: blocks of that direction are skewed
+// Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
+// 16 bytes of every plane, a wavefront up to kPlaneRounds times that per lane.
+constexpr uint32_t kPlaneRounds = 2;
+constexpr uint32_t kMaxPlanes = 4;
+constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2;   // Dims.lanes_per_run of such a segment
+constexpr uint32_t planes_lds_bytes(uint32_t planes) {   // one vector of padding behind every eight
+  return kPlaneRounds * kWaveLanes * planes * kVecBytes / 8 * 9;
+}
 // When one of the two block dimensions is shorter than a square block's edge the
 // block becomes a rectangle of about this many bytes, its long edge capped.
 constexpr uint32_t kRectBlockBytes = 8192;
@@ -115,7 +136,7 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t mode;
   uint32_t ndim;          // outer (non-run) dimensions after collapsing, <= kMaxOuterDims;
                           // kModeTranspose: batch dimensions (<= kMaxBatchDims)
-  uint32_t tiles_per_run; // kModeRunTiles
+  uint32_t tiles_per_run; // kModeRunTiles; kModeTranspose: blocks per strip (kBlockStrip or 1)
   uint32_t granule;       // kModeElements: bytes moved per lane access (1,2,4,8,16);
                           // kModeRunTiles: 1 + log2(tiles_per_run) when a power of two;
                           // kModeTranspose: element size
@@ -131,14 +152,23 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t tiles_a, tiles_b;
   uint32_t edge_a, edge_b;         // block extent along A and B (elements)
   uint32_t lanes_per_run;          // kModeElements: 0, or the lane slots a ragged run occupies (its
-                                   // 16-byte granules rounded up to a multiple of four)
+                                   // 16-byte granules rounded up to a multiple of four);
+                                   // kModeTranspose: 0, or which side holds the planes of a segment
+                                   // of few planes (kPlanesInPayload, kPlanesInTensor)
   uint32_t nt_allowed;             // kModeElements, kModeTranspose: sides that may keep the launch's
                                    // non-temporal hint when packing (bit 0 tensor, bit 1 payload) and when
                                    // unpacking (bits 2, 3).  Transposed block rows that straddle 128-byte
                                    // lines share them with the neighbouring blocks and are written through
-                                   // the cache; rows shorter than a line are read and written through it
+                                   // the cache; rows shorter than a line are read and written through it.
+                                   // Bits 4, 5: kSkewPack, kSkewUnpack
 };
 static_assert(sizeof(Dims) == 176, "Dims layout");
+
+// Workgroup indices a die takes in a row: a power of two, or one run per die (`whole`).
+constexpr uint32_t kRemapShiftBit = 27, kRemapRunMask = (1u << kRemapShiftBit) - 1u;
+constexpr uint32_t remap_code(uint32_t run, bool whole) {
+  return run | (whole ? 31u : static_cast<uint32_t>(__builtin_ctz(run))) << kRemapShiftBit;
+}
 
 struct KernelArgs {
   const Seg* segs;            // nseg + 1 entries, last is a sentinel with tile_begin == ntiles
@@ -148,7 +178,7 @@ struct KernelArgs {
   uint32_t nseg;
   uint32_t ntiles;
   uint32_t tiles_per_wave;
-  uint32_t xcd_remap;         // 0 or the number of workgroups per die
+  uint32_t xcd_remap;         // 0, or remap_code of the workgroup indices a die takes in a row
   uint32_t seg_shift;         // log2 of the tile-block size of wave_seg
   int64_t tensor_delta = 0;   // added to every tensor-side address of the tables
 };
@@ -194,7 +224,8 @@ struct LaunchConfig {
   uint32_t nontemporal = 3;   // bit 0: tensor-side accesses, bit 1: payload-side accesses
   bool elements = false;   // some segment uses kModeElements or kModeTranspose
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (transposed tiles only)
-  bool xcd_remap = false;  // give each die a contiguous share of the wave index space
+  uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
+                           // multiple of 8 such runs)
 };
 
 // ---------------------------------------------------------------- tunables
@@ -224,6 +255,7 @@ struct Tunables {
   std::atomic<int64_t> gather_run_bytes{1280};
   std::atomic<int64_t> xcd_remap{-1};         // contiguous wave ranges per die: 1 always, 0 never, -1 when
                                   // transposed blocks that share lines with their neighbours dominate
+                                  // (larger bundles then in squares of blocks, see finish_geometry)
   std::atomic<int64_t> transpose{1};          // move transposed views as square blocks through LDS
   std::atomic<int64_t> ragged_runs{1};        // short runs of 16+ bytes that are no multiple of 16 move in
                                   // 16-byte granules (the last one overlapping) instead of narrower ones

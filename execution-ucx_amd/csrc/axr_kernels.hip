@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "axr_internal.h"
 
@@ -493,6 +494,94 @@ __device__ __forceinline__ void transpose_full(gcbytes rd, int64_t rd_pitch, gby
   __builtin_amdgcn_wave_barrier();
 }
 
+// A block whose written rows do not start on 64-byte boundaries (bundles beyond kSkewMinPayload).  Partly written 64-byte pieces are
+// what such a transposition loses its time on, not the reads: 128-byte row pieces at any address
+// read at the aligned rate, written they fall from 5.5 to 3.9 TB/s, and are back at 5.2 once every
+// piece is a whole number of aligned 64-byte units (134 MB in rows of 8198 bytes).  The block is
+// therefore skewed: written row y starts at its first 64-byte boundary behind element x0 and
+// holds T elements from there, so that neighbouring blocks meet on boundaries and only the ends of
+// the whole row are written in part.  For that up to 64 / E - 1 read rows of the next block are
+// staged as well; neighbours along x are neighbouring wavefronts, which find them in their L2.
+// Four 4097 x 4099 bf16 matrices: pack 84 -> 65 us, unpack 78 -> 64, the pair 140 -> 115 (aligned
+// matrices of that size: 89); 4-byte elements 131 -> 108, 8-byte elements 130 -> 107.  What is left
+// is the price of reading 1.5 times the lines and of 12 instead of 16 wavefronts per compute unit.
+//   rd + x * rd_pitch   T elements of read row x (the block's y range)
+//   wr + y * wr_pitch   written row y from its element x = 0 on
+// ext_x >= T; y rows 0 .. T - 1 all exist.
+template <uint32_t E>
+__device__ __forceinline__ void transpose_skewed(gcbytes rd, int64_t rd_pitch, gbytes wr,
+                                                 int64_t wr_pitch, uint32_t x0, uint32_t ext_x,
+                                                 lbytes lds, uint32_t lane, bool nt_wr) {
+  constexpr uint32_t T = transpose_edge(E), PITCH = transpose_lds_pitch(E), EV = kVecBytes / E;
+  constexpr uint32_t NC = T * E / kVecBytes, RPI = kWaveLanes / NC;
+  constexpr uint32_t W = transpose_skew_rows(E), NK = W / RPI;
+  static_assert(W % RPI == 0 && W >= T + kSkewBytes / E - 1, "staged rows");
+  typedef typename unit_of<E>::type U;
+  typedef U __attribute__((aligned(E < 4 ? E : 4))) lds_unit;
+  const uint32_t r = lane / NC, v = lane % NC;
+  // staged rows w0 .. w0 + nrows - 1; at the end of the row the window moves back to end with it,
+  // so that the last, moved back vectors find their elements
+  const uint32_t back = ext_x > W ? ext_x - W : 0u;
+  const uint32_t w0 = x0 < back ? x0 : back;
+  const uint32_t nrows = ext_x - w0 < W ? ext_x - w0 : W;
+  u32x4 q[NK];
+#pragma unroll
+  for (uint32_t k = 0; k < NK; ++k) {
+    const uint32_t row = k * RPI + r;
+    q[k] = load16<false>(rd + static_cast<int64_t>(w0 + (row < nrows ? row : nrows - 1u)) * rd_pitch + v * kVecBytes);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < NK; ++k) {
+    AXR_LDS uint32_t* w = reinterpret_cast<AXR_LDS uint32_t*>(lds + (k * RPI + r) * PITCH + v * kVecBytes);
+    w[0] = q[k].x;
+    w[1] = q[k].y;
+    w[2] = q[k].z;
+    w[3] = q[k].w;
+  }
+  __builtin_amdgcn_wave_barrier();
+  // EV elements of written row y from element x on
+  auto gather = [&](uint32_t x, uint32_t y) {
+    U e[EV];
+#pragma unroll
+    for (uint32_t i = 0; i < EV; ++i)
+      e[i] = *reinterpret_cast<const AXR_LDS lds_unit*>(lds + (x - w0 + i) * PITCH + y * E);
+    u32x4 out;
+    __builtin_memcpy(&out, e, kVecBytes);
+    return out;
+  };
+  auto skew_of = [&](uint32_t y) {   // elements in front of row y's first 64-byte boundary
+    const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uint64_t>(wr)) + y * static_cast<uint32_t>(wr_pitch);
+    return ((0u - at) & (kSkewBytes - 1u)) / E;
+  };
+#pragma unroll
+  for (uint32_t k = 0; k < T / RPI; ++k) {
+    const uint32_t y = k * RPI + r;
+    uint32_t x = x0 + skew_of(y) + v * EV;
+    if (x < ext_x) {
+      if (x + EV > ext_x) x = ext_x - EV;   // overlaps its neighbour with identical data
+      gbytes to = wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E;
+      if (nt_wr) {   // (the empty asm statements keep the arms apart, see transpose_full)
+        asm volatile("");
+        store16<true>(to, gather(x, y));
+        asm volatile("");
+      } else {
+        store16<false>(to, gather(x, y));
+      }
+    }
+  }
+  if (x0 == 0) {   // the elements in front of every row's first boundary, in whole vectors
+    constexpr uint32_t NV = kSkewBytes / kVecBytes, RPH = kWaveLanes / NV;
+    const uint32_t rh = lane / NV, x = (lane % NV) * EV;
+#pragma unroll
+    for (uint32_t k = 0; k < (T + RPH - 1) / RPH; ++k) {
+      const uint32_t y = k * RPH + rh;
+      if (y < T && x < skew_of(y))
+        store16<false>(wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E, gather(x, y));
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Quotient idx / d by multiplication, exact while idx * d < 2^32 (blocks hold at
 // most 2^14 elements with edges up to 2^10).
 __device__ __forceinline__ uint32_t small_div(uint32_t idx, uint32_t d, uint32_t magic) {
@@ -669,6 +758,150 @@ __device__ __forceinline__ void interleaved_to_rows(gcbytes rd, gbytes wr, int64
   __builtin_amdgcn_wave_barrier();
 }
 
+// C planes of 1-, 2- or 4-byte elements <-> the same elements interleaved (image channels, complex
+// pairs), 2 to 4 planes.  A lane owns 16 bytes of every plane: C vectors of the interleaved range,
+// regrouped in registers with byte permutes.  LDS only turns the lane's C neighbouring vectors
+// into wave-wide contiguous accesses.  Every access of the block to memory is in flight at once,
+// C KiB per round and kPlaneRounds rounds.  What it replaces gathered every element from LDS by
+// itself, 16 byte reads per vector, with one or two vectors in flight: 256 images of 224 x 224 x 3
+// bytes 47 -> 32 us for pack + unpack, 4 channels 55 -> 40, 64 such fp32 images 36 -> 32 (plain copy
+// of the bytes: 25.5 us).
+template <uint32_t E>
+__device__ __forceinline__ uint32_t pick_bytes(const uint32_t* d, uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {
+  // byte k of the result is byte sk of d; the indices are constants once the loops are unrolled.
+  // perm(hi, lo, sel): selector values 0-3 take bytes of lo, 4-7 bytes of hi
+  if constexpr (E == 4) return d[s0 / 4];
+  if constexpr (E == 2)
+    return __builtin_amdgcn_perm(d[s2 / 4], d[s0 / 4],
+                                 (s0 & 3u) | (s1 & 3u) << 8 | (4u + (s2 & 3u)) << 16 | (4u + (s3 & 3u)) << 24);
+  const uint32_t lo = __builtin_amdgcn_perm(d[s1 / 4], d[s0 / 4], (s0 & 3u) | (4u + (s1 & 3u)) << 8);
+  const uint32_t hi = __builtin_amdgcn_perm(d[s3 / 4], d[s2 / 4], (s2 & 3u) | (4u + (s3 & 3u)) << 8);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+template <uint32_t E, uint32_t C, bool TO_PLANES>
+__device__ __forceinline__ void regroup_vectors(const u32x4 (&in)[C], u32x4 (&out)[C]) {
+  uint32_t d[4 * C];
+  __builtin_memcpy(d, in, sizeof(d));
+#pragma unroll
+  for (uint32_t k = 0; k < C; ++k) {
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {
+      uint32_t s[4];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t p = w * 4 + j;                      // byte of output vector k
+        const uint32_t g = (k * kVecBytes + p) / E;        // interleaved: element of the range
+        s[j] = TO_PLANES ? (p / E * C + k) * E + p % E : (g % C) * kVecBytes + g / C * E + p % E;
+      }
+      out[k][w] = pick_bytes<E>(d, s[0], s[1], s[2], s[3]);
+    }
+  }
+}
+
+// `groups` lane units (16 bytes of every plane each) from `inter` / plane 0 at `plane` on.
+template <uint32_t E, uint32_t C, bool TO_PLANES>
+__device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t groups,
+                                             lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
+  constexpr uint32_t R = kPlaneRounds;
+  const uint32_t nvec = groups * C;
+  // vector m of the interleaved range in LDS: one vector of padding behind every eight
+  auto slot = [&](uint32_t m) { return lds + m * kVecBytes + (m >> 3) * kVecBytes; };
+  u32x4 x[R][C];
+  auto read_all = [&](auto nt) {
+#pragma unroll
+    for (uint32_t k = 0; k < R; ++k) {
+#pragma unroll
+      for (uint32_t c = 0; c < C; ++c) {
+        if constexpr (TO_PLANES) {
+          const uint32_t m = (k * C + c) * kWaveLanes + lane;
+          x[k][c] = load16<decltype(nt)::value>(inter + (m < nvec ? m : nvec - 1u) * kVecBytes);
+        } else {
+          const uint32_t g = k * kWaveLanes + lane;
+          x[k][c] = load16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch +
+                                                (g < groups ? g : groups - 1u) * kVecBytes);
+        }
+      }
+    }
+  };
+  // (the empty asm statements keep the two arms apart, or the optimizer merges them and drops the hint)
+  if (nt_rd) {
+    asm volatile("");
+    read_all(std::true_type{});
+    asm volatile("");
+  } else {
+    read_all(std::false_type{});
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < R; ++k) {
+#pragma unroll
+    for (uint32_t c = 0; c < C; ++c) asm volatile("" : "+v"(x[k][c])::"memory");
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < R; ++k) {
+    if constexpr (TO_PLANES) {
+#pragma unroll
+      for (uint32_t c = 0; c < C; ++c) *reinterpret_cast<AXR_LDS u32x4*>(slot((k * C + c) * kWaveLanes + lane)) = x[k][c];
+    } else {
+      u32x4 y[C];
+      regroup_vectors<E, C, false>(x[k], y);
+#pragma unroll
+      for (uint32_t c = 0; c < C; ++c) *reinterpret_cast<AXR_LDS u32x4*>(slot((k * kWaveLanes + lane) * C + c)) = y[c];
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  auto write_all = [&](auto nt) {
+#pragma unroll
+    for (uint32_t k = 0; k < R; ++k) {
+      if constexpr (TO_PLANES) {
+        const uint32_t g = k * kWaveLanes + lane;
+        u32x4 in[C], y[C];
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) in[c] = *reinterpret_cast<const AXR_LDS u32x4*>(slot(g * C + c));
+        regroup_vectors<E, C, true>(in, y);
+        if (g < groups) {
+#pragma unroll
+          for (uint32_t c = 0; c < C; ++c)
+            store16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch + g * kVecBytes, y[c]);
+        }
+      } else {
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) {
+          const uint32_t m = (k * C + c) * kWaveLanes + lane;
+          const u32x4 y = *reinterpret_cast<const AXR_LDS u32x4*>(slot(m));
+          if (m < nvec) store16<decltype(nt)::value>(inter + m * kVecBytes, y);
+        }
+      }
+    }
+  };
+  if (nt_wr) {
+    asm volatile("");
+    write_all(std::true_type{});
+    asm volatile("");
+  } else {
+    write_all(std::false_type{});
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <bool TO_PLANES>
+__device__ __forceinline__ void planes_of(uint32_t E, uint32_t C, gbytes inter, gbytes plane, int64_t plane_pitch,
+                                          uint32_t groups, lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
+#define AXR_PLANES(e, c) planes_block<e, c, TO_PLANES>(inter, plane, plane_pitch, groups, lds, lane, nt_rd, nt_wr)
+  switch (E << 4 | C) {
+    case 0x12: AXR_PLANES(1, 2); break;
+    case 0x13: AXR_PLANES(1, 3); break;
+    case 0x14: AXR_PLANES(1, 4); break;
+    case 0x22: AXR_PLANES(2, 2); break;
+    case 0x23: AXR_PLANES(2, 3); break;
+    case 0x24: AXR_PLANES(2, 4); break;
+    case 0x42: AXR_PLANES(4, 2); break;
+    case 0x43: AXR_PLANES(4, 3); break;
+    default: AXR_PLANES(4, 4); break;
+  }
+#undef AXR_PLANES
+}
+
 // Reads nr rows of nc elements (rows rd_pitch bytes apart) and writes nc rows of
 // nr elements (rows wr_pitch bytes apart).
 __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t rd_pitch, gbytes wr,
@@ -718,14 +951,21 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
   const uint32_t es = static_cast<uint32_t>(__builtin_ctz(E));
   const uint32_t T = transpose_edge(E);
   // rows that straddle lines share them with the neighbouring blocks
-  nt_bits &= PACK ? dm->nt_allowed : dm->nt_allowed >> 2;
+  const uint32_t allowed = dm->nt_allowed;
+  nt_bits &= PACK ? allowed : allowed >> 2;
   const uint32_t edge_a = dm->edge_a, edge_b = dm->edge_b;
   const uint32_t ta = dm->tiles_a, tb = dm->tiles_b;
   const uint32_t per_batch = ta * tb;
   uint32_t o = q / per_batch;
   const uint32_t rem = q - o * per_batch;
-  const uint32_t ia = rem / tb;
-  const uint32_t ib = rem - ia * tb;
+  const bool skewed = (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0;
+  // blocks in strips of `strip` along A, walked along B: with 8 of them 64 neighbouring tiles are a
+  // square of 8 x 8 blocks (1: plain rows of blocks)
+  const uint32_t strip = dm->tiles_per_run;
+  const uint32_t is = rem / (strip * tb), in_strip = rem - is * strip * tb;
+  const uint32_t strip_rows = ta - is * strip < strip ? ta - is * strip : strip;
+  const uint32_t ib = in_strip / strip_rows;
+  const uint32_t ia = is * strip + (in_strip - ib * strip_rows);
   int64_t toff = 0;
   uint64_t poff = 0;
   const uint32_t nbatch = dm->ndim;
@@ -741,6 +981,57 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
     }
   }
   uint32_t a0 = ia * edge_a, b0 = ib * edge_b;
+  const int64_t stride_a = dm->stride_a;
+  const uint64_t pstride_b = dm->pstride_b;
+  if (const uint32_t planes = dm->lanes_per_run) {
+    // Few planes <-> interleaved: the short dimension is taken whole; the last block of the long one
+    // is moved back to end at the extent (it moves some elements a second time, with the same values).
+    const bool payload_planes = planes == kPlanesInPayload;   // the long dimension is A, else B
+    const uint32_t ext = payload_planes ? dm->ext_a : dm->ext_b, edge = payload_planes ? edge_a : edge_b;
+    uint32_t n0 = payload_planes ? a0 : b0;
+    n0 = ext - n0 < edge ? ext - edge : n0;
+    const uint32_t C = payload_planes ? edge_b : edge_a;
+    const uint64_t inter_at = static_cast<uint64_t>(n0) * C << es, plane_at = static_cast<uint64_t>(n0) << es;
+    gbytes ten = as_global(seg_ptr) + toff, pp = pay + poff;
+    const bool nt_rd = (nt_bits & (PACK ? 1u : 2u)) != 0, nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
+    const uint32_t groups = edge * E / kVecBytes;
+    if (payload_planes)
+      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(pstride_b), groups, lds, lane, nt_rd, nt_wr);
+    else
+      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, stride_a, groups, lds, lane, nt_rd, nt_wr);
+    return;
+  }
+  if (skewed) {
+    // (both extents hold a whole block; the last block across the rows is moved back)
+    gbytes ten = as_global(seg_ptr) + toff, pp = pay + poff;
+    gbytes rd, wr;
+    int64_t rd_pitch, wr_pitch;
+    uint32_t x0, ext_x;
+    if constexpr (PACK) {
+      if (b0 + T > dm->ext_b) b0 = dm->ext_b - T;
+      rd = ten + (static_cast<uint64_t>(b0) << es);
+      rd_pitch = stride_a;
+      wr = pp + static_cast<uint64_t>(b0) * pstride_b;
+      wr_pitch = static_cast<int64_t>(pstride_b);
+      x0 = a0;
+      ext_x = dm->ext_a;
+    } else {
+      if (a0 + T > dm->ext_a) a0 = dm->ext_a - T;
+      rd = pp + (static_cast<uint64_t>(a0) << es);
+      rd_pitch = static_cast<int64_t>(pstride_b);
+      wr = ten + static_cast<int64_t>(a0) * stride_a;
+      wr_pitch = stride_a;
+      x0 = b0;
+      ext_x = dm->ext_b;
+    }
+    const bool nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
+    switch (E) {
+      case 2: transpose_skewed<2>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds, lane, nt_wr); break;
+      case 4: transpose_skewed<4>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds, lane, nt_wr); break;
+      default: transpose_skewed<8>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds, lane, nt_wr); break;
+    }
+    return;
+  }
   if (edge_a == T && edge_b == T) {
     // Square blocks: the ragged last block of a dimension that holds at least one whole
     // block is moved back so that it ends at the extent.  It overlaps its neighbour and
@@ -753,8 +1044,6 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
   const uint32_t ra = dm->ext_a - a0, rb = dm->ext_b - b0;
   const uint32_t na = ra < edge_a ? ra : edge_a, nb = rb < edge_b ? rb : edge_b;
   const bool square = na == T && nb == T;   // a whole square block: the vector path
-  const int64_t stride_a = dm->stride_a;
-  const uint64_t pstride_b = dm->pstride_b;
   gbytes ten = as_global(seg_ptr) + toff + static_cast<int64_t>(a0) * stride_a +
                (static_cast<uint64_t>(b0) << es);
   gbytes pp = pay + poff + static_cast<uint64_t>(b0) * pstride_b + (static_cast<uint64_t>(a0) << es);
@@ -946,9 +1235,12 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   const uint32_t lane_off = lane * kVecBytes;
   if (a.xcd_remap) {
-    // consecutive workgroup ids land on consecutive dies; hand die d the d-th
-    // contiguous share of the index space so neighbouring tiles share an L2
-    wg = (wg % kXcds) * a.xcd_remap + wg / kXcds;
+    // consecutive workgroup ids land on consecutive dies; hand every die runs of consecutive
+    // workgroup indices, in turn, so that neighbouring tiles share an L2
+    // (no division: runs are a power of two long, or there is one run per die and `shift` is 31)
+    const uint32_t i = wg / kXcds, run = a.xcd_remap & kRemapRunMask, shift = a.xcd_remap >> kRemapShiftBit;
+    const uint32_t round = i >> shift;
+    wg = (round * kXcds + wg % kXcds) * run + (i - (round << shift));
   }
   // wavefronts per workgroup travel in bits 8-15 of the hint argument, which is preloaded into
   // a scalar register: blockDim would be a load from the hidden kernel arguments in front of
@@ -1502,8 +1794,8 @@ int launch_bundle_kernel(bool pack, const KernelArgs& args, const LaunchConfig& 
   // The grid must cover every tile: waves * tiles_per_wave >= ntiles.
   if (cfg.threads == 0 || cfg.threads % kWaveLanes || cfg.threads > kMaxThreadsPerWorkgroup)
     return fail(AXR_ERR_INVALID, "workgroup size must be a multiple of 64 up to 1024");
-  if (args.xcd_remap && (cfg.workgroups % kXcds || args.xcd_remap != cfg.workgroups / kXcds))
-    return fail(AXR_ERR_INVALID, "die remapping needs a grid that is a multiple of 8");
+  if (args.xcd_remap && cfg.workgroups % (kXcds * (args.xcd_remap & kRemapRunMask)))
+    return fail(AXR_ERR_INVALID, "die remapping needs a grid of whole rounds over the dies");
   if (cfg.elements && cfg.threads > kMaxElementThreads)
     return fail(AXR_ERR_INVALID, "bundles with short strided runs need workgroups of at most 256");
   if (static_cast<uint64_t>(cfg.lds_per_wave) * (cfg.threads / kWaveLanes) > 64u * 1024u)

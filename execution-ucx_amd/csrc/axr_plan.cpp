@@ -646,7 +646,7 @@ struct Builder {
     // A transposition: no contiguous inner run beyond one element, but some outer
     // dimension (B) is contiguous in the tensor.  Blocks of A x B go through LDS.
     size_t dim_b = nd;
-    uint32_t edge_a = 0, edge_b = 0;
+    uint32_t edge_a = 0, edge_b = 0, planes = 0;
     if (nd >= 2 && run_bytes <= kVecBytes && (run_bytes & (run_bytes - 1)) == 0 &&
         tunables().transpose != 0) {
       for (size_t d = 0; d + 1 < nd; ++d) {
@@ -664,11 +664,24 @@ struct Builder {
       const uint32_t e = static_cast<uint32_t>(run_bytes);
       const uint64_t t = transpose_edge(e), ea = ext[nd - 1], eb = ext[dim_b];
       const uint64_t elems = kRectBlockBytes / e;
-      if (ea >= t && eb >= t) {
+      const uint64_t ev = kVecBytes / e;
+      // Two to four planes against the same elements interleaved without gaps: whole vectors on
+      // both sides.  The long edge is a whole number of vectors (the last block is moved back).
+      auto plane_edge = [&](uint64_t extent) {
+        return static_cast<uint32_t>(std::min<uint64_t>(kPlaneRounds * kWaveLanes * ev, extent - extent % ev));
+      };
+      if (e <= 4 && eb >= 2 && eb <= kMaxPlanes && ea >= ev && str[nd - 1] == static_cast<int64_t>(eb * e)) {
+        planes = kPlanesInPayload;
+        edge_b = static_cast<uint32_t>(eb);
+        edge_a = plane_edge(ea);
+      } else if (e <= 4 && ea >= 2 && ea <= kMaxPlanes && eb >= ev && dim_b + 2 == nd) {
+        planes = kPlanesInTensor;
+        edge_a = static_cast<uint32_t>(ea);
+        edge_b = plane_edge(eb);
+      } else if (ea >= t && eb >= t) {
         edge_a = edge_b = static_cast<uint32_t>(t);
       } else {
         // the long edge is a whole number of 16-byte vectors where it can be
-        const uint64_t ev = kVecBytes / e;
         auto long_edge = [&](uint64_t extent, uint32_t short_edge) {
           uint64_t edge = std::min<uint64_t>({extent, kRectMaxEdge, elems / short_edge});
           if (edge >= ev) edge -= edge % ev;
@@ -726,8 +739,7 @@ struct Builder {
       // rows of one side plus a dword each, whichever direction needs more
       // (or one pad dword per 128 bytes, for blocks staged as one contiguous range)
       const uint32_t block_bytes = edge_a * edge_b * e;
-      const uint32_t lds = block_bytes + std::max(4u * std::max(edge_a, edge_b), block_bytes / 32u + 16u);
-      p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
+      uint32_t lds = block_bytes + std::max(4u * std::max(edge_a, edge_b), block_bytes / 32u + 16u);
       // A side whose block rows start on 128-byte lines is read or written in whole lines and
       // may stream; a side with another pitch or base shares the first and last line of every
       // block row with the neighbouring blocks, and only a cacheable access lets the second
@@ -736,15 +748,35 @@ struct Builder {
       // times the payload and the pack + unpack rate rises from 3.65 to 3.87 TB/s (with the
       // die-contiguous tile ranges that finish_geometry then selects).
       const uint64_t line = kLineBytes - 1;
-      bool tensor_lines = ((ptr | static_cast<uint64_t>(str[dim_a])) & line) == 0;
-      bool payload_lines = ((off | packed[dim_b]) & line) == 0;
+      // (the interleaved side of a segment of few planes is read and written as one range)
+      bool tensor_lines = ((ptr | (planes == kPlanesInPayload ? 0u : static_cast<uint64_t>(str[dim_a]))) & line) == 0;
+      bool payload_lines = ((off | (planes == kPlanesInTensor ? 0u : packed[dim_b])) & line) == 0;
       for (size_t d = 0; d < nd; ++d) {
         if (d == dim_a || d == dim_b) continue;
         tensor_lines = tensor_lines && (static_cast<uint64_t>(str[d]) & line) == 0;
         payload_lines = payload_lines && (packed[d] & line) == 0;
       }
       dm.nt_allowed = ((tensor_lines ? 1u : 0u) | (payload_lines ? 2u : 0u)) * 5u;   // both directions
-      if (!tensor_lines || !payload_lines) shared_line_tiles += ntile;
+      dm.lanes_per_run = planes;
+      const bool beyond_l2 = p->payload_bytes > kSkewMinPayload;
+      dm.tiles_per_run = beyond_l2 && (!tensor_lines || !payload_lines) ? kBlockStrip : 1u;
+      const bool square = !planes && edge_a == transpose_edge(e) && edge_b == edge_a;
+      if (planes) {
+        lds = planes_lds_bytes(planes == kPlanesInPayload ? edge_b : edge_a);
+      } else if (square && beyond_l2 && e >= 2 && e <= 8 && (dm.ext_a | dm.ext_b) < (1u << 31) &&
+                 (!tensor_lines || !payload_lines)) {
+        // the side that is written gets blocks that start on its own 64-byte boundaries; reads at
+        // any address run at the aligned rate
+        // (whole 64-byte units may stream, which leaves the last-level cache to the payload: pack +
+        // unpack of 134 MB 128 -> 114 us)
+        if (!payload_lines) dm.nt_allowed |= kSkewPack;
+        if (!tensor_lines) dm.nt_allowed |= kSkewUnpack | 4u;
+        shared_line_tiles += ntile;
+        lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
+      } else if (!tensor_lines || !payload_lines) {
+        shared_line_tiles += ntile;
+      }
+      p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
     } else if (run_bytes >= element_mode_limit(run_bytes)) {
       dm.mode = kModeRunTiles;
       const uint64_t tpr = (run_bytes + tile_bytes - 1) / tile_bytes;
@@ -861,13 +893,25 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   const uint64_t per_wg = tpw * waves_per_wg;
   p->cfg.tiles_per_wave = static_cast<uint32_t>(tpw);
   p->cfg.workgroups = static_cast<uint32_t>((p->ntiles + per_wg - 1) / per_wg);
-  // Each die a contiguous share of the tiles: slower for streams of whole lines, but it lets
-  // transposed blocks whose rows straddle lines meet their neighbours in one L2 (automatic
-  // when such blocks are half of the bundle or more).
-  const bool remap = tn.xcd_remap > 0 ||
-                     (tn.xcd_remap < 0 && p->shared_line_tiles != 0 && 2 * p->shared_line_tiles >= p->ntiles);
-  p->cfg.xcd_remap = remap && p->cfg.workgroups >= 4 * kXcds;
-  if (p->cfg.xcd_remap) p->cfg.workgroups = (p->cfg.workgroups + kXcds - 1) / kXcds * kXcds;
+  // Transposed blocks whose rows straddle lines find their neighbours' lines in an L2 when the blocks
+  // around them run on the same die (automatic when such blocks are half of the bundle or more):
+  // every die takes squares of kBlockStrip x kBlockStrip blocks in turn, which for four 4097 x 4099
+  // bf16 matrices brings pack 70 -> 64 us and unpack 64 -> 60.  One contiguous eighth of the tiles
+  // per die, 73 and 73 us there, stays for bundles that fit the L2s (8 x 4 MiB), where the two are
+  // level and for which nothing else is done either, and is what the switch set to 1 gives.
+  uint32_t run = 0;
+  bool whole = false;
+  const bool shared_lines = p->shared_line_tiles != 0 && 2 * p->shared_line_tiles >= p->ntiles;
+  if (tn.xcd_remap > 0 || (tn.xcd_remap < 0 && shared_lines && p->payload_bytes <= kSkewMinPayload)) {
+    whole = true;
+    if (p->cfg.workgroups >= 4 * kXcds) run = (p->cfg.workgroups + kXcds - 1) / kXcds;
+    if (run > kRemapRunMask) run = 0;
+  } else if (tn.xcd_remap < 0 && shared_lines) {
+    run = 1;
+    while (2 * run * per_wg <= kBlockStrip * kBlockStrip) run *= 2;
+  }
+  p->cfg.xcd_remap = run ? remap_code(run, whole) : 0u;
+  if (run) p->cfg.workgroups = (p->cfg.workgroups + kXcds * run - 1) / (kXcds * run) * (kXcds * run);
   p->cfg.tile_rows = rows;
   if (tn.nontemporal < 0) {
     p->cfg.nontemporal = p->payload_bytes > static_cast<uint64_t>(tn.payload_cache_bytes) ? 3u : 1u;
@@ -1385,7 +1429,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   a.nseg = p->segs.empty() ? 0u : static_cast<uint32_t>(p->segs.size() - 1);
   a.ntiles = p->ntiles;
   a.tiles_per_wave = p->cfg.tiles_per_wave;
-  a.xcd_remap = p->cfg.xcd_remap ? p->cfg.workgroups / kXcds : 0;
+  a.xcd_remap = p->cfg.xcd_remap;
   a.seg_shift = p->cfg.seg_shift;
   a.tensor_delta = delta;
   LaunchConfig cfg = p->cfg;
@@ -1872,7 +1916,7 @@ static int pack_noalloc_body(axr_plan_t* p, void* payload, size_t payload_bytes,
   a.nseg = static_cast<uint32_t>(p->segs.size() - 1);
   a.ntiles = p->ntiles;
   a.tiles_per_wave = p->cfg.tiles_per_wave;
-  a.xcd_remap = p->cfg.xcd_remap ? p->cfg.workgroups / kXcds : 0;
+  a.xcd_remap = p->cfg.xcd_remap;
   a.seg_shift = p->cfg.seg_shift;
   auto remember = [&] {
     if (!capturing) remember_stream(p, stream);

@@ -118,12 +118,16 @@ constexpr uint32_t kBlockStrip = 8;
 constexpr uint64_t kSkewMinPayload = 24u << 20;
 constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4, 5: blocks of that direction are skewed
 // Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
-// 16 bytes of every plane, a wavefront up to kPlaneRounds times that per lane.
-constexpr uint32_t kPlaneRounds = 2;
+// 16 bytes of every plane, a wavefront up to plane_rounds times that per lane.  Bytes and 2-byte
+// elements take two rounds; 4-byte elements as many as the 8 KiB rectangle of the other blocks with
+// a short dimension has (1024, 680 and 512 elements of each of 2, 3 and 4 planes).
+constexpr uint32_t plane_rounds(uint32_t element_bytes, uint32_t planes) {
+  return element_bytes < 4 || planes == 4 ? 2u : planes == 3 ? 3u : 4u;
+}
 constexpr uint32_t kMaxPlanes = 4;
 constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2;   // Dims.lanes_per_run of such a segment
-constexpr uint32_t planes_lds_bytes(uint32_t planes) {   // one vector of padding behind every eight
-  return kPlaneRounds * kWaveLanes * planes * kVecBytes / 8 * 9;
+constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes) {   // one vector of padding behind every eight
+  return plane_rounds(element_bytes, planes) * kWaveLanes * planes * kVecBytes / 8 * 9;
 }
 // When one of the two block dimensions is shorter than a square block's edge the
 // block becomes a rectangle of about this many bytes, its long edge capped.

@@ -762,7 +762,7 @@ __device__ __forceinline__ void interleaved_to_rows(gcbytes rd, gbytes wr, int64
 // pairs), 2 to 4 planes.  A lane owns 16 bytes of every plane: C vectors of the interleaved range,
 // regrouped in registers with byte permutes.  LDS only turns the lane's C neighbouring vectors
 // into wave-wide contiguous accesses.  Every access of the block to memory is in flight at once,
-// C KiB per round and kPlaneRounds rounds.  What it replaces gathered every element from LDS by
+// C KiB per round and two to four rounds.  What it replaces gathered every element from LDS by
 // itself, 16 byte reads per vector, with one or two vectors in flight: 256 images of 224 x 224 x 3
 // bytes 47 -> 32 us for pack + unpack, 4 channels 55 -> 40, 64 such fp32 images 36 -> 32 (plain copy
 // of the bytes: 25.5 us).
@@ -803,7 +803,7 @@ __device__ __forceinline__ void regroup_vectors(const u32x4 (&in)[C], u32x4 (&ou
 template <uint32_t E, uint32_t C, bool TO_PLANES>
 __device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t groups,
                                              lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
-  constexpr uint32_t R = kPlaneRounds;
+  constexpr uint32_t R = plane_rounds(E, C);
   const uint32_t nvec = groups * C;
   // vector m of the interleaved range in LDS: one vector of padding behind every eight
   auto slot = [&](uint32_t m) { return lds + m * kVecBytes + (m >> 3) * kVecBytes; };

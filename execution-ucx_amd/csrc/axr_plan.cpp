@@ -665,28 +665,30 @@ struct Builder {
       const uint64_t t = transpose_edge(e), ea = ext[nd - 1], eb = ext[dim_b];
       const uint64_t elems = kRectBlockBytes / e;
       const uint64_t ev = kVecBytes / e;
+      // the long edge of a rectangle is a whole number of 16-byte vectors where it can be
+      auto long_edge = [&](uint64_t extent, uint64_t short_edge) {
+        uint64_t edge = std::min<uint64_t>({extent, kRectMaxEdge, elems / short_edge});
+        if (edge >= ev) edge -= edge % ev;
+        return static_cast<uint32_t>(edge);
+      };
       // Two to four planes against the same elements interleaved without gaps: whole vectors on
       // both sides.  The long edge is a whole number of vectors (the last block is moved back).
-      auto plane_edge = [&](uint64_t extent) {
-        return static_cast<uint32_t>(std::min<uint64_t>(kPlaneRounds * kWaveLanes * ev, extent - extent % ev));
+      auto plane_edge = [&](uint64_t extent, uint64_t count) {
+        if (e == 4) return long_edge(extent, count);
+        return static_cast<uint32_t>(
+            std::min<uint64_t>(plane_rounds(e, static_cast<uint32_t>(count)) * kWaveLanes * ev, extent - extent % ev));
       };
       if (e <= 4 && eb >= 2 && eb <= kMaxPlanes && ea >= ev && str[nd - 1] == static_cast<int64_t>(eb * e)) {
         planes = kPlanesInPayload;
         edge_b = static_cast<uint32_t>(eb);
-        edge_a = plane_edge(ea);
+        edge_a = plane_edge(ea, eb);
       } else if (e <= 4 && ea >= 2 && ea <= kMaxPlanes && eb >= ev && dim_b + 2 == nd) {
         planes = kPlanesInTensor;
         edge_a = static_cast<uint32_t>(ea);
-        edge_b = plane_edge(eb);
+        edge_b = plane_edge(eb, ea);
       } else if (ea >= t && eb >= t) {
         edge_a = edge_b = static_cast<uint32_t>(t);
       } else {
-        // the long edge is a whole number of 16-byte vectors where it can be
-        auto long_edge = [&](uint64_t extent, uint32_t short_edge) {
-          uint64_t edge = std::min<uint64_t>({extent, kRectMaxEdge, elems / short_edge});
-          if (edge >= ev) edge -= edge % ev;
-          return static_cast<uint32_t>(edge);
-        };
         if (ea <= eb) {
           edge_a = static_cast<uint32_t>(std::min(ea, t));
           edge_b = long_edge(eb, edge_a);
@@ -762,7 +764,7 @@ struct Builder {
       dm.tiles_per_run = beyond_l2 && (!tensor_lines || !payload_lines) ? kBlockStrip : 1u;
       const bool square = !planes && edge_a == transpose_edge(e) && edge_b == edge_a;
       if (planes) {
-        lds = planes_lds_bytes(planes == kPlanesInPayload ? edge_b : edge_a);
+        lds = planes_lds_bytes(e, planes == kPlanesInPayload ? edge_b : edge_a);
       } else if (square && beyond_l2 && e >= 2 && e <= 8 && (dm.ext_a | dm.ext_b) < (1u << 31) &&
                  (!tensor_lines || !payload_lines)) {
         // the side that is written gets blocks that start on its own 64-byte boundaries; reads at

@@ -462,6 +462,16 @@ void collapse(const TensorRec& t, const int64_t* shape, const int64_t* strides, 
   }
 }
 
+bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
+  int64_t expect = 1;
+  for (int32_t d = ndim - 1; d >= 0; --d) {
+    if (shape[d] == 1) continue;
+    if (strides[d] != expect) return false;
+    expect *= shape[d];
+  }
+  return true;
+}
+
 // Collapses tensor after tensor.  Views of one geometry come in rows (cache blocks, matrix
 // chunks): a tensor of the same shape, strides and item size as the one asked for before it gets
 // that one's answer (512 five-dimensional cache blocks: 23 -> 9 us for the two passes over them).
@@ -471,12 +481,12 @@ struct Collapser {
   Collapsed c, compact;
 
   const Collapsed& of(const TensorRec& t) {
-    if (!t.has_strides) {   // compact by definition: one run, nothing to collapse
+    const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
+    if (!strides || compact_strides(shape, strides, t.ndim)) {   // one run, nothing to collapse
       compact.nd = 0;
       compact.run_bytes = t.nbytes;
       return compact;
     }
-    const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
     const size_t bytes = static_cast<size_t>(t.ndim) * sizeof(int64_t);
     const bool same = last && last->ndim == t.ndim && (last->bits + 7) / 8 == (t.bits + 7) / 8 &&
                       std::memcmp(p->shape_of(*last), shape, bytes) == 0 &&
@@ -940,16 +950,6 @@ uint32_t rows_for_compact_bundle(const axr_plan* p) {
   return rows;
 }
 
-bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
-  int64_t expect = 1;
-  for (int32_t d = ndim - 1; d >= 0; --d) {
-    if (shape[d] == 1) continue;
-    if (strides[d] != expect) return false;
-    expect *= shape[d];
-  }
-  return true;
-}
-
 // The event behind the upload of the plan's tables, recorded at most once per upload.
 int record_upload(axr_plan* p) {
   if (p->upload_recorded) return AXR_OK;
@@ -1097,9 +1097,10 @@ int build_tables(axr_plan* p) {
     // 5.25 and 5.10 TB/s).
     //
     // A payload that streams is moved in 1 KiB tiles when it consists of compact tensors and
-    // strided views that move as run tiles.
+    // strided views that move as run tiles.  (Only for such a payload is every tensor looked at:
+    // the others are done at the first compact one.)
     uint64_t common_run = 0;
-    bool uniform_runs = !p->tensors.empty(), run_tiles_only = true;
+    bool uniform_runs = !p->tensors.empty(), run_tiles_only = streams_in_small_tiles(p);
     for (const TensorRec& t : p->tensors) {
       if (t.nbytes == 0) continue;
       if (!t.has_strides) {   // a compact tensor: not a bundle of strided views
@@ -1116,7 +1117,7 @@ int build_tables(axr_plan* p) {
         p->payload_bytes <= static_cast<uint64_t>(tn.payload_cache_bytes)) {
       while (rows < kMaxTileRows && rows * kRowBytes < common_run) rows *= 2;
     }
-    if (run_tiles_only && streams_in_small_tiles(p)) rows = 1;
+    if (run_tiles_only) rows = 1;
     while (rows < kMaxTileRows &&
            p->payload_bytes / (static_cast<uint64_t>(rows) * kRowBytes) >
                static_cast<uint64_t>(tn.max_tiles))

@@ -1,14 +1,13 @@
 // Streamed transfer of a large payload in chunks: pack -> loopback send -> unpack,
 // double-buffered over two (or more) lanes, each lane a send slot and a receive slot.
-// Chunk k uses lane k % lanes and runs on stream (k % lanes) % streams.  With one stream
+// Chunk k uses lane k % lanes and runs on stream (k % lanes) % streams, or in line with all
+// others on the first lane's stream and slot (see runs_in_line).  With one stream
 // per lane, stream order alone makes a slot safe to reuse `lanes` chunks later and chunk
 // k + 1's pack overlaps chunk k's wire copy and unpack; with fewer streams than lanes the
-// chunks of one stream run back to back and the extra lanes only let the host queue ahead
-// (all three stages are bound by HBM bandwidth, so on one GPU two stages that run at once
-// contend: one stream with two lanes measured 8 % faster than two streams).  The caller
-// keeps ONE sender plan and ONE receiver plan for all chunks of one geometry and moves them
-// over the data with the per-chunk tensor deltas: nothing is planned, uploaded or allocated
-// per chunk.
+// chunks of one stream run back to back and the extra lanes only let the host queue ahead.
+// The caller keeps ONE sender plan and ONE receiver plan for all chunks of one geometry and
+// moves them over the data with the per-chunk tensor deltas: nothing is planned, uploaded or
+// allocated per chunk.
 //
 // The send goes through the same loopback context calls a caller would make
 // (axr_am_send / axr_am_recv_header / axr_am_recv_buffer_borrow or axr_am_recv_buffer_async),
@@ -57,6 +56,21 @@ int retire(axr_transfer* t, axr_transfer::Lane& lane) {
   if (rc) return rc;
   if (done != 1) return fail(AXR_ERR_HIP, "a chunk's send did not complete");
   return AXR_OK;
+}
+
+// Chunks that run in line: one after the other on the first lane's stream, all through its send
+// slot, which stays in the last-level cache from a chunk's pack to its unpack and on to the next
+// pack.  That holds while the payloads in flight fit the cache or there is only one at a time; two
+// that do not fit evict each other, and what they lose is more than what the overlap of two
+// launches' ramps and tails gives.  Eight chunks of 2- to 4-KiB rows at 1.5 times their length, pack
+// and unpack, two streams / one / one and a single slot: 8 x 67 MB 348 / 376 / 374 us,
+// 8 x 134 MB (two are 256 MiB) 654 / 667 / 668, 8 x 159 MB 914 / 793 / 780, 8 x 201 MB
+// 1237 / 1043 / 969, 8 x 268 MB 1629 / 1309 / 1265; payloads beyond the cache stream and gain
+// little: 8 x 336 MB 1676 / 1646 / 1651, 8 x 537 MB 2681 / 2623 / 2620.  (A plain copy of the
+// bytes of 8 x 268 MB: 1282 us.)
+bool runs_in_line(const axr_transfer* t, uint64_t nbytes) {
+  return t->zero_copy &&
+         (t->streams == 1 || nbytes > static_cast<uint64_t>(tunables().payload_cache_bytes) / t->streams);
 }
 
 void destroy(axr_transfer* t) {
@@ -145,12 +159,16 @@ static int transfer_submit_body(axr_transfer_t* t, axr_plan_t* send_plan, int64_
   if (rc) return rc;
   ++t->submitted;
 
+  // Whose stream and send slot the chunk uses.  A slot is always used on its own lane's stream, so
+  // that stream order alone keeps the chunks that go through it apart.
+  const axr_transfer::Lane& at = runs_in_line(t, nbytes) ? t->lanes[0] : lane;
+
   if (!t->zero_copy && !lane.recv_slot) {
     rc = axr_pool_alloc(t->pool, t->slot_bytes, 256, &lane.recv_slot, nullptr);
     if (rc) return rc;
   }
   uint64_t borrowed_key = 0;
-  void* source = t->zero_copy ? lane.send_slot : lane.recv_slot;
+  void* source = t->zero_copy ? at.send_slot : lane.recv_slot;
   axr_job_t job;
   std::memset(&job, 0, sizeof(job));
   // The payload side keeps the plans' own cache treatment (cacheable up to the size of the
@@ -158,27 +176,27 @@ static int transfer_submit_body(axr_transfer_t* t, axr_plan_t* send_plan, int64_
   // (8.0 ms for 8 GiB against 8.7 ms with everything streaming and 9.5 ms with a cacheable copy).
   job.plan = send_plan;
   job.unpack = 0;
-  job.payload = lane.send_slot;
+  job.payload = at.send_slot;
   job.payload_bytes = nbytes;
   job.tensor_delta = send_delta;
-  rc = axr_submit(&job, 1, lane.stream);
+  rc = axr_submit(&job, 1, at.stream);
   if (rc) return rc;
   auto give_up = [&](int status) {
-    // the pack is on the lane's stream already: let it finish before the slot is reused
-    (void)axr_stream_synchronize(lane.stream);
+    // the pack is on the chunk's stream already: let it finish before the slot is reused
+    (void)axr_stream_synchronize(at.stream);
     return status;
   };
   if (nbytes) {
     axr_am_data_t am;
     std::memset(&am, 0, sizeof(am));
     am.header = axr_buffer_t{const_cast<void*>(header), header_bytes};
-    am.buffer = axr_buffer_t{lane.send_slot, static_cast<size_t>(nbytes)};
+    am.buffer = axr_buffer_t{at.send_slot, static_cast<size_t>(nbytes)};
     am.buffer_type = AXR_MEM_ROCM;
-    am.mem_h = lane.send_mem_h;
-    rc = axr_am_send(t->client, t->conn, &am, lane.stream, &lane.request);
+    am.mem_h = at.send_mem_h;
+    rc = axr_am_send(t->client, t->conn, &am, at.stream, &lane.request);
     if (rc) return give_up(rc);
     // From here on a failure must not leave the send parked or its message queued: the
-    // slot is reused by the chunk after next.
+    // slot is used again by a later chunk.
     axr_am_message_t msg;
     rc = axr_am_recv_header(t->server, &msg);
     if (rc) {
@@ -204,8 +222,8 @@ static int transfer_submit_body(axr_transfer_t* t, axr_plan_t* send_plan, int64_
       void* lent = nullptr;
       size_t lent_bytes = 0;
       rc = axr_am_recv_buffer_borrow(t->server, msg.key, &lent, &lent_bytes, nullptr);
-      if (!rc && (lent != lane.send_slot || lent_bytes != nbytes)) {
-        (void)axr_am_borrow_release(t->server, msg.key, lane.stream);
+      if (!rc && (lent != at.send_slot || lent_bytes != nbytes)) {
+        (void)axr_am_borrow_release(t->server, msg.key, at.stream);
         rc = fail(AXR_ERR_MISMATCH, "the borrowed payload is not the chunk that was sent");
       }
       if (!rc) {
@@ -214,14 +232,14 @@ static int transfer_submit_body(axr_transfer_t* t, axr_plan_t* send_plan, int64_
       }
     } else {
       rc = axr_am_recv_buffer_async(t->server, msg.key, AXR_MEM_ROCM, lane.recv_slot, t->slot_bytes,
-                                    lane.stream);
+                                    at.stream);
     }
     if (rc) {
       (void)axr_am_message_release(t->server, msg.key);
       (void)axr_am_request_cancel(t->client, lane.request);
-      // the lane's stream may already hold this chunk's pack: drain it, so that the slot is
-      // quiet before the next chunk on this lane reuses it
-      (void)axr_stream_synchronize(lane.stream);
+      // the chunk's stream may already hold this chunk's pack: drain it, so that the slot is
+      // quiet before the next chunk reuses it
+      (void)axr_stream_synchronize(at.stream);
       return rc;
     }
     lane.in_flight = true;
@@ -230,18 +248,18 @@ static int transfer_submit_body(axr_transfer_t* t, axr_plan_t* send_plan, int64_
   job.unpack = 1;
   job.payload = source;
   job.tensor_delta = recv_delta;
-  rc = axr_submit(&job, 1, lane.stream);
+  rc = axr_submit(&job, 1, at.stream);
   // the send completes behind the scatter that reads its slot (also when the scatter was refused:
   // the lane must come back to a state in which retire() finds a completed send)
   if (borrowed_key) {
-    const int released = axr_am_borrow_release(t->server, borrowed_key, lane.stream);
+    const int released = axr_am_borrow_release(t->server, borrowed_key, at.stream);
     if (!rc) rc = released;
   }
-  const int recorded = axr_event_record(lane.done, lane.stream);
+  const int recorded = axr_event_record(lane.done, at.stream);
   if (rc || recorded) {
     // whatever was enqueued runs to its end before the error is reported: the lane's event and
     // send request are then settled and the next chunk finds the lane idle
-    (void)axr_stream_synchronize(lane.stream);
+    (void)axr_stream_synchronize(at.stream);
     if (lane.in_flight) {
       int done = 0;
       (void)axr_am_request_test(t->client, lane.request, &done);

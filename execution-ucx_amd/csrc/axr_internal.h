@@ -86,6 +86,14 @@ struct GroupHead {        // 32 bytes
   uint32_t slots;
 };
 static_assert(sizeof(GroupHead) == 32, "GroupHead layout");
+// A group as the host stages it for the device to write its block: its members' records lie side
+// by side in an array of their own.
+struct GroupStage {       // 16 bytes
+  uint64_t off;           // GroupHead.off
+  uint32_t first;         // index of the first member's record
+  uint16_t members, slots;
+};
+static_assert(sizeof(GroupStage) == 16, "GroupStage layout");
 constexpr uint32_t kGroupBlockBytes = sizeof(GroupHead) + kGroupMaxMembers * sizeof(Member);   // 288
 constexpr uint32_t kMemberOffBits = 20;
 constexpr uint32_t group_data_slots(uint32_t nbytes) { return nbytes >= kVecBytes ? (nbytes + kVecBytes - 1) / kVecBytes : 1u; }
@@ -366,6 +374,8 @@ int launch_notify(uint32_t* flag, uint32_t value, void* stream);
 // segs and wave_seg are device memory.  Copies the records and writes the tile-block index.
 int launch_expand_tables(const Seg* staged, uint32_t n, Seg* segs, uint32_t* wave_seg, uint32_t seg_shift,
                          void* stream);
+// members and groups are pinned host memory, blocks device memory: writes the blocks of `n` groups.
+int launch_expand_groups(const Member* members, const GroupStage* groups, uint32_t n, void* blocks, void* stream);
 // tables[0, bytes) = staged[0, bytes), rounded up to 16 bytes: a table block's pinned half into its
 // device half.
 int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream);

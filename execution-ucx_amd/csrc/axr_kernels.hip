@@ -1707,6 +1707,41 @@ __global__ __launch_bounds__(256) void expand_tables_kernel(const Seg* staged, u
   for (uint64_t k = (first + step - 1) >> seg_shift; (k << seg_shift) < last; ++k) wave_seg[k] = i;
 }
 
+// Blocks of a bundle of group tiles.  The host writes 16 bytes per tensor and per group into pinned
+// memory; this kernel, 16 threads per group and one per member, lays them out at the fixed stride
+// the bundle kernel wants and marks the members' first slots.  Bound by the bus, which carries 1.2
+// instead of 3.6 MB for 65,536 tensors of 8 to 512 bytes (85 -> 27 us in front of the first launch).
+__global__ __launch_bounds__(256) void expand_groups_kernel(const Member* members, const GroupStage* groups, uint32_t n,
+                                                            uint8_t* blocks) {
+  const uint32_t i = blockIdx.x * kUtilityThreads + threadIdx.x, g = i / kGroupMaxMembers, k = i % kGroupMaxMembers;
+  if (g >= n) return;   // all sixteen threads of a group
+  const GroupStage group = groups[g];
+  u32x4 rec{0u, 0u, 0u, 0u};   // records past the last member stay zero
+  uint64_t starts[2] = {0, 0};
+  if (k < group.members) {
+    rec = *reinterpret_cast<const u32x4*>(members + group.first + k);
+    const uint32_t begin = rec.w >> 16;
+    starts[0] = begin < 64u ? 1ull << begin : 0ull;
+    starts[1] = begin < 64u ? 0ull : 1ull << (begin & 63u);
+  }
+#pragma unroll
+  for (uint32_t step = 1; step < kGroupMaxMembers; step *= 2) {
+    starts[0] |= __shfl_xor(starts[0], step, kGroupMaxMembers);
+    starts[1] |= __shfl_xor(starts[1], step, kGroupMaxMembers);
+  }
+  u32x4* block = reinterpret_cast<u32x4*>(blocks + static_cast<uint64_t>(g) * kGroupBlockBytes);
+  block[sizeof(GroupHead) / kVecBytes + k] = rec;
+  if (k == 0) {
+    GroupHead head;
+    head.starts[0] = starts[0];
+    head.starts[1] = starts[1];
+    head.off = group.off;
+    head.members = group.members;
+    head.slots = group.slots;
+    *reinterpret_cast<GroupHead*>(block) = head;
+  }
+}
+
 // Host-built tables from pinned memory into their device block, 16 bytes per thread.  Bound by one
 // trip over the bus (about 3 us; 106 KB then take 2 us more).  A kernel and not a copy-engine
 // transfer because of where the bytes end up: what the copy engine wrote is in none of the caches,
@@ -1940,6 +1975,15 @@ int launch_expand_tables(const Seg* staged, uint32_t n, Seg* segs, uint32_t* wav
   hipLaunchKernelGGL(expand_tables_kernel, dim3((n + kUtilityThreads) / kUtilityThreads), dim3(kUtilityThreads), 0,
                      static_cast<hipStream_t>(stream), staged, n, segs, wave_seg, seg_shift);
   return check_hip(hipGetLastError(), "table expansion launch");
+}
+
+int launch_expand_groups(const Member* members, const GroupStage* groups, uint32_t n, void* blocks, void* stream) {
+  if (n == 0) return AXR_OK;
+  if (n > 0x7fffffffu / kGroupMaxMembers) return fail(AXR_ERR_UNSUPPORTED, "too many groups for one launch");
+  const uint32_t threads = n * kGroupMaxMembers;
+  hipLaunchKernelGGL(expand_groups_kernel, dim3((threads + kUtilityThreads - 1) / kUtilityThreads), dim3(kUtilityThreads),
+                     0, static_cast<hipStream_t>(stream), members, groups, n, static_cast<uint8_t*>(blocks));
+  return check_hip(hipGetLastError(), "group expansion launch");
 }
 
 int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream) {

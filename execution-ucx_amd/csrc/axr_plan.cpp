@@ -974,6 +974,88 @@ int note_upload(axr_plan* p, hipStream_t stream) {
   return stream ? record_upload(p) : AXR_OK;
 }
 
+// A table block of at least `bytes`, of which the device reads or writes nothing any more.
+int quiet_block(axr_plan* p, size_t bytes) {
+  if (p->block.host) quiesce(p);   // earlier launches may still read the block
+  if (p->block.host && p->block.bytes < bytes) table_block_release(&p->block);
+  return p->block.host ? AXR_OK : table_block_acquire(bytes, &p->block);
+}
+
+// Bundles of short contiguous device tensors only: one pass over the tensors writes the members'
+// records and the groups they fall into (the division Builder::add_member makes) into pinned
+// memory, and a kernel lays out the group blocks.  No strides to collapse, no blocks and segments
+// to build in host memory and copy.  Launching a fresh plan of 65,536 tensors of 8 to 512 bytes:
+// 693 us on the host and 85 on the device before, 335 and 27 now.  Returns as device_build_tables
+// does.
+int device_build_groups(axr_plan* p, hipStream_t stream, bool* done) {
+  const Tunables& tn = tunables();
+  const size_t n = p->tensors.size();
+  const uint32_t slots_per_group = static_cast<uint32_t>(tn.group_slots);
+  // A group ends because it has all its members, because the next one's slots do not fit (then the
+  // two groups hold more than slots_per_group together), or because the offset is out of its
+  // reach; the last reason is not counted here and ends the attempt if the room runs out.
+  const uint64_t bound = 2 * (p->payload_bytes / kVecBytes + 2 * n) / slots_per_group + n / kGroupMaxMembers + 2;
+  if (bound > (1u << 24)) return AXR_OK;
+  const size_t groups_at = n * sizeof(Member);
+  int rc = quiet_block(p, std::max<size_t>(groups_at + bound * sizeof(GroupStage), bound * kGroupBlockBytes));
+  if (rc) return rc;
+  Member* members = static_cast<Member*>(p->block.host);
+  GroupStage* groups = reinterpret_cast<GroupStage*>(static_cast<uint8_t*>(p->block.host) + groups_at);
+  const uint64_t align_mask = static_cast<uint64_t>(p->align) - 1;
+  bool pinned = false;
+  uint32_t closed = 0;   // groups in front of `group`
+  GroupStage group{};
+  for (size_t i = 0; i < n; ++i) {
+    const TensorRec& t = p->tensors[i];
+    if (t.device_type != kDLROCM && t.device_type != kDLROCMHost) return AXR_OK;
+    if (t.has_strides && !compact_strides(p->shape_of(t), p->strides_of(t), t.ndim)) return AXR_OK;
+    pinned = pinned || t.device_type == kDLROCMHost;
+    const uint64_t end = t.offset + t.nbytes;
+    const uint64_t pad = std::min((end + align_mask) & ~align_mask, p->payload_bytes) - end;
+    if (t.nbytes == 0 || t.nbytes > kGroupMaxMemberBytes || pad >= kMaxAlign) return AXR_OK;
+    const uint32_t need = group_data_slots(static_cast<uint32_t>(t.nbytes)) + group_pad_slots(static_cast<uint32_t>(pad));
+    if (need > slots_per_group / 2) return AXR_OK;
+    if (group.members && (group.members >= kGroupMaxMembers || group.slots + need > slots_per_group ||
+                          t.offset < group.off || t.offset - group.off >= (1ull << kMemberOffBits))) {
+      groups[closed++] = group;
+      group.members = 0;
+    }
+    if (group.members == 0) {
+      if (closed == bound) return AXR_OK;
+      group.off = t.offset;
+      group.first = static_cast<uint32_t>(i);
+      group.slots = 0;
+    }
+    Member m;
+    m.ptr = t.address;
+    m.off_pad = static_cast<uint32_t>(t.offset - group.off) | static_cast<uint32_t>(pad) << kMemberOffBits;
+    m.nbytes = static_cast<uint16_t>(t.nbytes);
+    m.begin = group.slots;
+    members[i] = m;
+    ++group.members;
+    group.slots = static_cast<uint16_t>(group.slots + need);
+  }
+  groups[closed++] = group;
+  p->segs.clear();
+  p->dims.clear();
+  p->wave_seg.clear();
+  p->ntiles = closed;
+  p->cfg.lds_per_wave = 0;
+  p->pinned_host_tensors = pinned;
+  finish_geometry(p, rows_for_compact_bundle(p), closed);
+  p->groups_only = true;
+  p->cfg.seg_shift = kGroupBlocksShift;
+  p->dims_at = p->wave_at = p->members_at = 0;
+  p->table_bytes = static_cast<size_t>(closed) * kGroupBlockBytes;
+  rc = launch_expand_groups(members, groups, closed, p->block.device, stream);
+  if (rc) return rc;
+  rc = note_upload(p, stream);
+  if (rc) return rc;
+  p->device_built = true;
+  *done = true;
+  return AXR_OK;
+}
+
 // Bundles of many contiguous device tensors: one pass over the tensors writes the segment
 // records straight into pinned memory, and a kernel (one thread per segment) brings them to
 // the device and writes the tile-block index, in front of the bundle kernel on the same
@@ -988,10 +1070,12 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
   if (least <= 0 || n < static_cast<uint64_t>(least) || n > (1u << 20) || !p->bound) return AXR_OK;
   if (tn.group_bytes > 0) {
     // a bundle in which a quarter of the tensors are short enough to share wavefronts takes the
-    // general path, which builds group tiles
+    // general path, which builds group tiles next to others, or, when all of them are, the device
+    // builds those
     const uint64_t limit = static_cast<uint64_t>(tn.group_bytes);
     size_t small = 0;
     for (size_t i = 0; i < n; ++i) small += (p->tensors[i].nbytes - 1) < limit ? 1 : 0;   // 1 .. limit
+    if (small == n) return device_build_groups(p, stream, done);
     if (small * 4 >= n) return AXR_OK;
   }
   const uint32_t rows = rows_for_compact_bundle(p);
@@ -1005,16 +1089,8 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
   const size_t blocks_bound = std::max<size_t>(2 * n + 2, static_cast<size_t>(tiles_bound >> 8) + 2);
   const size_t wave_at = align_up((n + 1) * sizeof(Seg), 16);
   const size_t bytes = wave_at + blocks_bound * sizeof(uint32_t);
-  if (p->block.host && p->block.bytes < bytes) {
-    quiesce(p);
-    table_block_release(&p->block);
-  }
-  if (!p->block.host) {
-    int rc = table_block_acquire(bytes, &p->block);
-    if (rc) return rc;
-  } else {
-    quiesce(p);   // earlier launches may still read the block
-  }
+  int rc = quiet_block(p, bytes);
+  if (rc) return rc;
   Seg* staged = static_cast<Seg*>(p->block.host);
   uint64_t tiles = 0;
   bool pinned = false;
@@ -1055,7 +1131,7 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
   p->wave_at = wave_at;
   p->table_bytes = wave_at + ((static_cast<size_t>(p->ntiles) >> p->cfg.seg_shift) + 1) * sizeof(uint32_t);
   uint8_t* d = static_cast<uint8_t*>(p->block.device);
-  int rc = launch_expand_tables(staged, static_cast<uint32_t>(n), reinterpret_cast<Seg*>(d),
+  rc = launch_expand_tables(staged, static_cast<uint32_t>(n), reinterpret_cast<Seg*>(d),
                                 reinterpret_cast<uint32_t*>(d + wave_at), p->cfg.seg_shift, stream);
   if (rc) return rc;
   rc = note_upload(p, stream);

@@ -39,3 +39,55 @@ def test_tables_of_strided_views(pkg, gpu, views, distinct):
         j = i % distinct if distinct > 2 else (i // 7) % 2      # in turn, or in runs of seven
         picked.append(parent[i, :, j % 3, :1 + (j * 37) % 2048] if distinct > 2 else parent[i, :, j, :1400 + 300 * j])
     _round_trip(pkg, gpu, picked, 16, torch)
+
+
+# one group, groups full by members (1 byte each), by slots (512 bytes; alignment gaps as zero slots),
+# both kinds in turn, gaps too long for a group on the way (1024), the last tensor too long for one,
+# an empty tensor among them, and enough for several workgroups of the kernel that lays groups out
+@pytest.mark.parametrize("align", [1, 16, 256, 1024])
+@pytest.mark.parametrize("slots", [128, 64])
+@pytest.mark.parametrize("sizes", [
+    [5], [1] * 16, [1] * 17, [512] * 40, [1, 512] * 50, list(range(1, 513)), [16 + k % 3 for k in range(700)],
+    [8, 500, 33] * 30 + [513], [8, 0, 33] * 30, [1 + 7 * k % 512 for k in range(9001)]], ids=lambda s: f"{len(s)}x{s[-1]}")
+def test_group_blocks_laid_out_by_the_device(pkg, gpu, sizes, slots, align):
+    """Short contiguous tensors, blocks from the device ("device_tables") and from the host: the
+    packed bytes and gaps, the scattered tensors, and the plan after its tables were asked for."""
+    import torch
+    gaps = [(3 * k) % 31 for k in range(len(sizes))]
+    total = sum(sizes) + sum(gaps)
+    arena = torch.randint(0, 256, (total,), dtype=torch.uint8, device=gpu)
+
+    def carve(store):
+        out, at = [], 0
+        for n, gap in zip(sizes, gaps):
+            out.append(store[at + gap:at + gap + n])
+            at += gap + n
+        return out
+
+    views = carve(arena)
+    want_twin = torch.full_like(arena, 0xEE)
+    for o, v in zip(carve(want_twin), views):
+        o.copy_(v)
+    try:
+        pkg.tune(group_slots=slots)
+        for device_tables in (1, 0):
+            pkg.tune(device_tables=device_tables)
+            plan = pkg.BundlePlan.create(views, align=align)
+            n = plan.payload_bytes
+            want = torch.zeros(n, dtype=torch.uint8, device=gpu)
+            for v, off, size in zip(views, *plan.layout()):
+                want[off:off + size] = v
+            for shift in (0, 3):
+                payload = torch.full((n + shift + 64,), 0xCD, dtype=torch.uint8, device=gpu)
+                plan.pack(payload.data_ptr() + shift, n)
+                twin = torch.full_like(arena, 0xEE)
+                recv = pkg.BundlePlan.from_header_bound(plan.header, carve(twin))
+                recv.unpack(payload.data_ptr() + shift, n)
+                assert torch.equal(payload[shift:shift + n], want), (device_tables, shift)
+                assert (payload[:shift] == 0xCD).all() and (payload[shift + n:] == 0xCD).all()
+                assert torch.equal(twin, want_twin), (device_tables, shift)
+                recv.close()
+                assert plan.launch_info()["tiles"] > 0     # host tables from here on
+            plan.close()
+    finally:
+        pkg.tune(group_slots=128, device_tables=512)

@@ -190,6 +190,7 @@ struct axr_plan {
   bool overlapping_dst = false;      // some tensor has a zero stride over an extent > 1
   uint32_t ntiles = 0;
   uint64_t shared_line_tiles = 0;    // tiles of transposed blocks whose rows straddle 128-byte lines
+  uint64_t strip_tiles = 0;          // those of them that lie in strips of kBlockStrip blocks
   LaunchConfig cfg;
   TableBlock block;
   size_t table_bytes = 0;
@@ -369,6 +370,7 @@ void invalidate_tables(axr_plan* p) {
   p->overlapping_dst = false;
   p->ntiles = 0;
   p->shared_line_tiles = 0;
+  p->strip_tiles = 0;
   p->cfg.lds_per_wave = 0;
 }
 
@@ -522,6 +524,7 @@ struct Builder {
   uint64_t head_align;    // 0 or a power of two up to 128
   uint64_t tiles = 0;
   uint64_t shared_line_tiles = 0;   // transposed blocks whose rows straddle 128-byte lines
+  uint64_t strip_tiles = 0;         // those of them that lie in strips of kBlockStrip blocks
   uint64_t group_bytes = 0;         // longest tensor that may share a wavefront (0: none)
   uint32_t slots_per_group = kGroupMaxSlots;
   // the group being collected (when open): the last block of p->group_blocks
@@ -771,8 +774,14 @@ struct Builder {
       dm.nt_allowed = ((tensor_lines ? 1u : 0u) | (payload_lines ? 2u : 0u)) * 5u;   // both directions
       dm.lanes_per_run = planes;
       const bool beyond_l2 = p->payload_bytes > kSkewMinPayload;
-      dm.tiles_per_run = beyond_l2 && (!tensor_lines || !payload_lines) ? kBlockStrip : 1u;
       const bool square = !planes && edge_a == transpose_edge(e) && edge_b == edge_a;
+      // Strips for what finish_geometry hands out in squares.  Blocks of single bytes, 128 x 128 and
+      // not skewed, stay in plain rows: four 4095 x 4097 matrices, pack + unpack, 75.2 us in plain
+      // rows, 77.3 in strips, four 3001 x 2999 43.1 and 45.2; rectangles gain (four of 40 x 150,001
+      // 2-byte elements 50.6 -> 49.7).
+      const bool strips = beyond_l2 && (!tensor_lines || !payload_lines) && !(square && e == 1);
+      dm.tiles_per_run = strips ? kBlockStrip : 1u;
+      if (strips) strip_tiles += ntile;
       if (planes) {
         lds = planes_lds_bytes(e, planes == kPlanesInPayload ? edge_b : edge_a);
       } else if (square && beyond_l2 && e >= 2 && e <= 8 && (dm.ext_a | dm.ext_b) < (1u << 31) &&
@@ -910,11 +919,12 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   // every die takes squares of kBlockStrip x kBlockStrip blocks in turn, which for four 4097 x 4099
   // bf16 matrices brings pack 70 -> 64 us and unpack 64 -> 60.  One contiguous eighth of the tiles
   // per die, 73 and 73 us there, stays for bundles that fit the L2s (8 x 4 MiB), where the two are
-  // level and for which nothing else is done either, and is what the switch set to 1 gives.
+  // level and for which nothing else is done either, and for blocks in plain rows, and is what the
+  // switch set to 1 gives.
   uint32_t run = 0;
   bool whole = false;
   const bool shared_lines = p->shared_line_tiles != 0 && 2 * p->shared_line_tiles >= p->ntiles;
-  if (tn.xcd_remap > 0 || (tn.xcd_remap < 0 && shared_lines && p->payload_bytes <= kSkewMinPayload)) {
+  if (tn.xcd_remap > 0 || (tn.xcd_remap < 0 && shared_lines && 2 * p->strip_tiles < p->ntiles)) {
     whole = true;
     if (p->cfg.workgroups >= 4 * kXcds) run = (p->cfg.workgroups + kXcds - 1) / kXcds;
     if (run > kRemapRunMask) run = 0;
@@ -1271,6 +1281,7 @@ int build_tables(axr_plan* p) {
     p->stage_bytes = std::max<size_t>(p->stage_bytes, static_cast<size_t>(c.end - c.begin));
   p->ntiles = static_cast<uint32_t>(b.tiles);
   p->shared_line_tiles = b.shared_line_tiles;
+  p->strip_tiles = b.strip_tiles;
   Seg sentinel;
   std::memset(&sentinel, 0, sizeof(sentinel));
   sentinel.tile_begin = p->ntiles;

@@ -38,13 +38,13 @@ def round_trip(pkg, gpu, stores, views_of, align, shift=0):
     plan.close()
 
 
-# shapes around the block edge (64, 32, 32 elements) and the staged window, next to a large matrix
+# shapes around the block edge (128, 64, 32, 32 elements; bytes are not skewed) and the staged window, next to a large matrix
 # that takes the bundle beyond the limit; odd rows, odd starts, one side aligned, a gap behind rows
-@pytest.mark.parametrize("item", [2, 4, 8])
+@pytest.mark.parametrize("item", [1, 2, 4, 8])
 @pytest.mark.parametrize("align,lead,shift", [(1, 0, 0), (256, 1, 0), (2, 3, 6)])
 def test_skewed_blocks(pkg, gpu, item, align, lead, shift):
     import torch
-    edge = 64 if item == 2 else 32
+    edge = {1: 128, 2: 64}.get(item, 32)
     shapes = [(2051, (26 << 20) // 2051 // item | 1), (edge, edge), (edge, edge + 1), (edge + 1, edge),
               (2 * edge - 1, edge + 31), (3 * edge + 5, 2 * edge), (4 * edge, edge + 17), (edge - 1, 300), (777, 130)]
     stores = [storage(torch, gpu, r * c, item, lead, i) for i, (r, c) in enumerate(shapes)]

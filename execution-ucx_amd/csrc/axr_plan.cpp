@@ -201,8 +201,7 @@ struct axr_plan {
   std::unique_ptr<InlineTables> inline_tables;   // the tables as a kernel argument (small bundles)
   bool inline_ready = false;
   uint64_t launches = 0;             // kernel launches since the tables were built
-  hipEvent_t upload_event = nullptr;   // from event_acquire
-  bool upload_recorded = false;        // the event lies behind the latest upload
+  hipEvent_t upload_event = nullptr;   // from event_acquire; behind the latest upload once `uploaded` is set
   int upload_event_device = -1;
   hipStream_t upload_stream = nullptr;
   struct BusyStream {
@@ -960,28 +959,21 @@ uint32_t rows_for_compact_bundle(const axr_plan* p) {
   return rows;
 }
 
-// The event behind the upload of the plan's tables, recorded at most once per upload.
-int record_upload(axr_plan* p) {
-  if (p->upload_recorded) return AXR_OK;
+// Notes that the tables have just been put on their way on `stream`.  The event that a launch on
+// another stream waits for is recorded here, right behind the upload, on the default stream as on any
+// other: recorded later it would lie behind whatever the stream was given in between, and a launch
+// elsewhere would wait for work that is not its own.
+int note_upload(axr_plan* p, hipStream_t stream) {
+  remember_stream(p, stream);
   if (!p->upload_event) {
     int rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
     if (rc) return rc;
   }
-  int rc = check_hip(hipEventRecord(p->upload_event, p->upload_stream), "hipEventRecord");
-  if (!rc) p->upload_recorded = true;
-  return rc;
-}
-
-// Notes that the tables have just been put on their way on `stream`.  The event that a launch on
-// another stream waits for is recorded now, except on the default stream, which can neither be
-// destroyed nor be capturing later: there it is recorded when such a launch comes, so that a plan
-// that stays on its stream pays for no event.
-int note_upload(axr_plan* p, hipStream_t stream) {
+  int rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
+  if (rc) return rc;
   p->upload_stream = stream;
-  p->upload_recorded = false;
   p->uploaded = true;
-  remember_stream(p, stream);
-  return stream ? record_upload(p) : AXR_OK;
+  return AXR_OK;
 }
 
 // A table block of at least `bytes`, of which the device reads or writes nothing any more.
@@ -1359,11 +1351,8 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
     if (rc) return rc;
     return note_upload(p, stream);
   }
-  if (stream != p->upload_stream) {
-    int rc = record_upload(p);
-    if (rc) return rc;
+  if (stream != p->upload_stream)
     return check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
-  }
   return AXR_OK;
 }
 
@@ -1689,9 +1678,8 @@ int axr_plan_create(const axr_tensor_t* tensors,
 static int plan_free_body(axr_plan_t* plan) {
   if (!plan) return AXR_OK;
   quiesce(plan);
-  if (plan->uploaded && plan->upload_recorded) (void)hipEventSynchronize(plan->upload_event);
   table_block_release(&plan->block);
-  event_release(plan->upload_event, plan->upload_event_device);   // fired, or never recorded
+  event_release(plan->upload_event, plan->upload_event_device);   // fired: the upload's stream has been drained
   plan->upload_event = nullptr;
   for (HostStage& st : plan->stage) {
     table_block_release(&st.block);
@@ -2247,8 +2235,7 @@ static int plan_prepare_body(axr_plan_t* plan, void* stream_) {
   if (plan->ntiles == 0 || plan->resident) return AXR_OK;
   rc = ensure_uploaded(plan, stream);
   if (rc) return rc;
-  rc = record_upload(plan);
-  if (!rc) rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
+  rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
   if (rc) return rc;
   plan->resident = true;
   return AXR_OK;

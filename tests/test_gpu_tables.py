@@ -91,3 +91,41 @@ def test_group_blocks_laid_out_by_the_device(pkg, gpu, sizes, slots, align):
             plan.close()
     finally:
         pkg.tune(group_slots=128, device_tables=512)
+
+
+# tables from the host (strided views), from compact records, and group blocks: all three go up on
+# the default stream with the plan's first launch
+@pytest.mark.parametrize("kind", ["views", "records", "groups"])
+def test_a_launch_elsewhere_waits_for_the_upload_only(pkg, gpu, kind):
+    """A plan whose tables went up on the default stream, launched on a stream of its own while the
+    default stream is busy with something else: it is done long before that."""
+    import ctypes as C
+
+    import torch
+    lib, capi = pkg._capi.load(), pkg._capi
+    parent = torch.randint(0, 256, (700, 9, 2048), dtype=torch.uint8, device=gpu)
+    if kind == "views":
+        tensors = [parent[i, 1:, :1400 + i % 7] for i in range(200)]
+    else:
+        tensors = [parent[i, 0, :(2000 if kind == "records" else 100) + i % 48] for i in range(700)]
+    plan = pkg.BundlePlan.create(tensors, align=16)
+    n = plan.payload_bytes
+    payload = torch.zeros(n, dtype=torch.uint8, device=gpu)
+    stream = C.c_void_p()
+    capi.check(lib.axr_stream_create(C.byref(stream)))
+    plan.pack(payload.data_ptr(), n)
+    plan.pack(payload.data_ptr(), n)      # (tables that rode in kernel arguments go up now)
+    want = payload.clone()
+    payload.zero_()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(800_000_000)        # 0.4 s or so that the plan has nothing to do with
+    busy = torch.cuda.Event()
+    busy.record()
+    plan.pack(payload.data_ptr(), n, stream.value, order=False)
+    capi.check(lib.axr_stream_synchronize(stream.value))
+    still_busy = not busy.query()
+    torch.cuda.synchronize()
+    assert torch.equal(payload, want)
+    assert still_busy
+    plan.close()
+    capi.check(lib.axr_stream_destroy(stream.value))

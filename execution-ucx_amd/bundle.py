@@ -296,6 +296,22 @@ def pack_bundle(tensors: Sequence[Any], align: int = 256, pool: Optional[DeviceP
     return PackedBundle(plan.header, buf, nbytes, plan)
 
 
+def _bind_header(header: bytes, out: Sequence[Any], stream) -> BundlePlan:
+    """``from_header(header).bind(out, stream)``, in one pass over the header for destinations
+    that can be described without asking anything of them.  Others are asked once, and only for a
+    header that is in order: a producer may give its capsule a single time."""
+    arr = out if isinstance(out, TensorArray) else None
+    if arr is None and isinstance(out, (list, tuple)):
+        arr = TensorArray.from_plain_tensors(out)
+    if arr is None:
+        return BundlePlan.from_header(header).bind(out, stream=stream)
+    try:
+        return BundlePlan.from_header_bound(header, arr, stream=stream)
+    except Exception:
+        BundlePlan.from_header(header).close()    # a bad header is reported ahead of a bad destination
+        raise
+
+
 def unpack_bundle(header: bytes, payload: Any, payload_bytes: Optional[int] = None,
                   out: Optional[Sequence[Any]] = None, stream=None,
                   from_dlpack_fn: Optional[Callable[[Any], Any]] = None):
@@ -319,10 +335,7 @@ def unpack_bundle(header: bytes, payload: Any, payload_bytes: Optional[int] = No
     if payload_bytes is not None:
         size = payload_bytes
     if out is not None:
-        try:
-            plan = BundlePlan.from_header_bound(header, out, stream=stream)
-        except Exception:  # noqa: BLE001 - a bad header is reported ahead of a bad destination
-            plan = BundlePlan.from_header(header).bind(out, stream=stream)
+        plan = _bind_header(header, out, stream)
         plan.unpack(ptr, size, stream)
         streams.make_visible_to_producers(_stream_handle(stream))
         return plan

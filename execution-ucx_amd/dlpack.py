@@ -224,11 +224,7 @@ class TensorArray:
         torch tensors (see ``extract``)."""
         native = _native()
         exporter = _torch_exporter()
-        described = None
-        if exporter:   # a bundle of plain torch tensors is read without one capsule per tensor
-            direct = _native_torch()
-            if direct is not None:
-                described = direct.describe(objs, exporter[2])
+        described = _plain_tensors(objs, exporter)
         if described is None and native is not None:
             try:
                 if stream is None:
@@ -239,6 +235,17 @@ class TensorArray:
                 described = None
         if described is None:   # no helper, or something that is not a DLPack producer
             return cls(extract_many(objs, stream))
+        return cls._described(described, objs)
+
+    @classmethod
+    def from_plain_tensors(cls, objs: Sequence[Any]) -> Optional["TensorArray"]:
+        """The descriptors of torch tensors that can be read without asking any of them for a
+        capsule, so that reading them has no effect a caller could see; None for anything else."""
+        described = _plain_tensors(objs, _torch_exporter())
+        return None if described is None else cls._described(described, objs)
+
+    @classmethod
+    def _described(cls, described: tuple, objs: Sequence[Any]) -> "TensorArray":
         descs, dims, owners = described
         self = cls.__new__(cls)
         n = len(owners)
@@ -259,6 +266,12 @@ class TensorArray:
     @views.setter
     def views(self, value):
         self._views = value
+
+
+def _plain_tensors(objs: Sequence[Any], exporter: tuple) -> Optional[tuple]:
+    """A bundle of plain torch tensors is read without one capsule per tensor."""
+    direct = _native_torch() if exporter else None
+    return None if direct is None else direct.describe(objs, exporter[2])
 
 
 def _torch_exporter() -> tuple:

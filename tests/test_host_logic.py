@@ -504,6 +504,54 @@ def fresh_of(pkg, array, released, tag):
     return pkg.DLPackExport(array.ctypes.data, array.shape, dtype, 1, 0, release=lambda: released.append(tag))
 
 
+def test_unpack_bundle_asks_a_destination_once_and_only_for_a_sound_header(pkg):
+    """Destinations that give their capsule a single time: the error is the caller's own mistake,
+    not that of a second request, and a bad header leaves them unasked."""
+    import torch
+    a, b = np.arange(40, dtype=np.int32), np.arange(6, dtype=np.float32)
+    with pkg.BundlePlan.create([a, b], align=16) as plan:
+        header = plan.header
+    released = []
+    short = np.zeros(39, np.int32)
+    outs = [fresh_of(pkg, short, released, 1), fresh_of(pkg, np.zeros_like(b), released, 2)]
+    with pytest.raises(pkg.MismatchError, match="tensor 0"):
+        pkg.unpack_bundle(header, 0x10000, 1 << 20, out=outs)
+    good = [fresh_of(pkg, np.zeros_like(a), released, 3), fresh_of(pkg, np.zeros_like(b), released, 4)]
+    for bad in (header[:-1], header[:20] + b"\x01" + header[21:], b""):
+        with pytest.raises(pkg.HeaderError):
+            pkg.unpack_bundle(bad, 0x10000, 1 << 20, out=good)
+    pkg.BundlePlan.from_header(header).bind(good).close()      # still to be had
+
+    class Once:
+        def __init__(self, tensor):
+            self.tensor, self.asked = tensor, 0
+
+        def __dlpack__(self, **kwargs):
+            self.asked += 1
+            return self.tensor.__dlpack__()
+
+        def __dlpack_device__(self):
+            return self.tensor.__dlpack_device__()
+
+    once = [Once(torch.zeros(39, dtype=torch.int32)), Once(torch.zeros(6))]
+    with pytest.raises(pkg.MismatchError):
+        pkg.unpack_bundle(header, 0x10000, 1 << 20, out=once)
+    assert [o.asked for o in once] == [1, 1]
+    # plain tensors: the header's fault ahead of theirs, else their own
+    plain = [torch.zeros(39, dtype=torch.int32), torch.zeros(6)]
+    with pytest.raises(pkg.HeaderError):
+        pkg.unpack_bundle(header[:-1], 0x10000, 1 << 20, out=plain)
+    with pytest.raises(pkg.MismatchError, match="tensor 0"):
+        pkg.unpack_bundle(header, 0x10000, 1 << 20, out=plain)
+    with pytest.raises(pkg.MismatchError, match="count"):
+        pkg.unpack_bundle(header, 0x10000, 1 << 20, out=plain[:1])
+    with pytest.raises(pkg.HeaderError):
+        pkg.unpack_bundle(header[:-1], 0x10000, 1 << 20, out=[bytes(4)])
+    frozen = np.frombuffer(bytes(160), dtype=np.int32)
+    with pytest.raises(BufferError):
+        pkg.unpack_bundle(header, 0x10000, 1 << 20, out=[frozen, np.zeros_like(b)])
+
+
 def test_dlpack_export_single_consume(pkg):
     released = []
     src = np.arange(40, dtype=np.int32)

@@ -983,9 +983,9 @@ int quiet_block(axr_plan* p, size_t bytes) {
   return p->block.host ? AXR_OK : table_block_acquire(bytes, &p->block);
 }
 
-// Bundles of short contiguous device tensors only: one pass over the tensors writes the members'
-// records and the groups they fall into (the division Builder::add_member makes) into pinned
-// memory, and a kernel lays out the group blocks.  No strides to collapse, no blocks and segments
+// Bundles of short contiguous device tensors only (device_build_tables has looked at lengths and
+// devices): one pass over the tensors writes the members' records and the groups they fall into (the
+// division Builder::add_member makes) into pinned memory, and a kernel lays out the group blocks.  No strides to collapse, no blocks and segments
 // to build in host memory and copy.  Launching a fresh plan of 65,536 tensors of 8 to 512 bytes:
 // 693 us on the host and 85 on the device before, 335 and 27 now.  Returns as device_build_tables
 // does.
@@ -1009,7 +1009,6 @@ int device_build_groups(axr_plan* p, hipStream_t stream, bool* done) {
   GroupStage group{};
   for (size_t i = 0; i < n; ++i) {
     const TensorRec& t = p->tensors[i];
-    if (t.device_type != kDLROCM && t.device_type != kDLROCMHost) return AXR_OK;
     if (t.has_strides && !compact_strides(p->shape_of(t), p->strides_of(t), t.ndim)) return AXR_OK;
     pinned = pinned || t.device_type == kDLROCMHost;
     const uint64_t end = t.offset + t.nbytes;
@@ -1076,7 +1075,13 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
     // builds those
     const uint64_t limit = static_cast<uint64_t>(tn.group_bytes);
     size_t small = 0;
-    for (size_t i = 0; i < n; ++i) small += (p->tensors[i].nbytes - 1) < limit ? 1 : 0;   // 1 .. limit
+    bool all_device = true;
+    for (size_t i = 0; i < n; ++i) {
+      const TensorRec& t = p->tensors[i];
+      small += (t.nbytes - 1) < limit ? 1 : 0;   // 1 .. limit
+      all_device = all_device && (t.device_type == kDLROCM || t.device_type == kDLROCMHost);
+    }
+    if (!all_device) return AXR_OK;   // before a block is taken: host tensors need no tables on the device
     if (small == n) return device_build_groups(p, stream, done);
     if (small * 4 >= n) return AXR_OK;
   }

@@ -552,6 +552,16 @@ def test_unpack_bundle_asks_a_destination_once_and_only_for_a_sound_header(pkg):
         pkg.unpack_bundle(header, 0x10000, 1 << 20, out=[frozen, np.zeros_like(b)])
 
 
+def test_short_host_tensors_take_no_table_block(pkg):
+    """A bundle of nothing but short host tensors has no table on the device: preparing it
+    allocates nothing there (and so works without one)."""
+    store = np.arange(600 * 64, dtype=np.uint8)
+    with pkg.BundlePlan.create([store[64 * i:64 * i + 1 + i % 60] for i in range(600)], align=1) as plan:
+        plan.prepare()
+        info = plan.launch_info()
+        assert (info["tiles"], info["table_bytes"] > 0, info["host_copies"]) == (0, True, 600)
+
+
 def test_dlpack_export_single_consume(pkg):
     released = []
     src = np.arange(40, dtype=np.int32)

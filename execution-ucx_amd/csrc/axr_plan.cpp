@@ -481,9 +481,10 @@ struct Collapser {
   const TensorRec* last = nullptr;   // `c` is its answer (tensors with strides only)
   Collapsed c, compact;
 
+  // For a tensor with strides (one without is compact: one run, nothing to collapse).
   const Collapsed& of(const TensorRec& t) {
     const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
-    if (!strides || compact_strides(shape, strides, t.ndim)) {   // one run, nothing to collapse
+    if (compact_strides(shape, strides, t.ndim)) {
       compact.nd = 0;
       compact.run_bytes = t.nbytes;
       return compact;
@@ -1188,12 +1189,12 @@ int build_tables(axr_plan* p) {
       if (t.nbytes == 0) continue;
       if (!t.has_strides) {   // a compact tensor: not a bundle of strided views
         uniform_runs = false;
-        continue;
+      } else {
+        const Collapsed& c = collapser.of(t);
+        uniform_runs = uniform_runs && c.nd != 0 && (common_run == 0 || c.run_bytes == common_run);
+        common_run = c.run_bytes;
+        run_tiles_only = run_tiles_only && (c.nd == 0 || c.run_bytes >= static_cast<uint64_t>(tn.gather_run_bytes));
       }
-      const Collapsed& c = collapser.of(t);
-      uniform_runs = uniform_runs && c.nd != 0 && (common_run == 0 || c.run_bytes == common_run);
-      common_run = c.run_bytes;
-      run_tiles_only = run_tiles_only && (c.nd == 0 || c.run_bytes >= static_cast<uint64_t>(tn.gather_run_bytes));
       if (!uniform_runs && !run_tiles_only) break;
     }
     if (uniform_runs && common_run >= 2 * kRowBytes && common_run <= kMaxTileRows * kRowBytes &&
@@ -1224,25 +1225,32 @@ int build_tables(axr_plan* p) {
       for (int32_t d = 0; d < t.ndim; ++d)
         if (strides[d] == 0 && shape[d] > 1) p->overlapping_dst = true;
     }
-    const Collapsed& c = collapser.of(t);
+    const Collapsed* c = nullptr;
+    size_t nd = 0;
+    uint64_t run_bytes = t.nbytes;
+    if (strides) {
+      c = &collapser.of(t);
+      nd = c->nd;
+      run_bytes = c->run_bytes;
+    }
     int rc;
     if (t.device_type == kDLROCMHost) p->pinned_host_tensors = true;
     if (t.device_type == kDLROCM || t.device_type == kDLROCMHost) {
-      if (c.nd == 0 && b.add_member(static_cast<uint32_t>(i), t.address, t.offset, t.nbytes, pad, &rc)) {
+      if (nd == 0 && b.add_member(static_cast<uint32_t>(i), t.address, t.offset, t.nbytes, pad, &rc)) {
         if (rc) return rc;
         continue;
       }
       rc = b.close_group();
       if (rc) return rc;
-      rc = b.add_strided(static_cast<uint32_t>(i), t.address, t.offset, c.extent, c.stride, c.nd,
-                         c.run_bytes);
+      rc = b.add_strided(static_cast<uint32_t>(i), t.address, t.offset, nd ? c->extent : nullptr,
+                         nd ? c->stride : nullptr, nd, run_bytes);
       if (rc) return rc;
       if (pad) p->segs.back().meta |= static_cast<uint32_t>(pad);
     } else if (t.device_type == kDLCPU) {
       rc = b.close_group();
       if (rc) return rc;
-      rc = b.add_host(static_cast<uint32_t>(i), t.address, t.offset, c.extent, c.stride, c.nd,
-                      c.run_bytes);
+      rc = b.add_host(static_cast<uint32_t>(i), t.address, t.offset, nd ? c->extent : nullptr,
+                      nd ? c->stride : nullptr, nd, run_bytes);
       if (rc) return rc;
       if (pad) {
         rc = b.add_seg(static_cast<uint32_t>(i), 0, end, 0, 1, kSegFillOnly);

@@ -101,7 +101,10 @@ constexpr uint32_t group_pad_slots(uint32_t pad) { return pad >= kVecBytes ? (pa
 
 constexpr uint32_t kModeRunTiles = 0;   // every tile is a piece of one contiguous run
 constexpr uint32_t kModeElements = 1;   // tile covers packed bytes; lanes decode granules
-constexpr uint32_t kModeTranspose = 2;  // tile is a square block transposed through LDS
+// kModeTranspose and above: the tile is a block transposed through LDS
+constexpr uint32_t kModeTranspose = 2;  // plain blocks in plain rows
+constexpr uint32_t kModeWalked = 3;     // skewed blocks, or blocks in strips (see block_rule)
+constexpr uint32_t kModePlanes = 4;     // few planes against the same elements interleaved
 
 // Transposed blocks are T x T elements; a block row is 128 bytes (eight 16-byte
 // vectors) for elements up to 4 bytes and 256 bytes for wider ones, so that a
@@ -120,11 +123,51 @@ constexpr uint32_t transpose_skew_rows(uint32_t element_bytes) {
   return (transpose_edge(element_bytes) + kSkewBytes / element_bytes - 1 + per_access - 1) / per_access * per_access;
 }
 constexpr uint32_t kBlockStrip = 8;
-// Bundles up to this size (what the eight L2s hold) are moved in plain blocks: there the partly
-// written lines are completed in an L2 anyway (bf16, pack + unpack: 8 MB 14.5 plain / 16.2 us
-// skewed, 17 MB 20.8 / 21.0, 34 MB 36.9 / 34.2, 67 MB 69.7 / 63.9, 134 MB 140 / 115).
-constexpr uint64_t kSkewMinPayload = 24u << 20;
 constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4, 5: blocks of that direction are skewed
+// How the blocks of a transposition are cut and walked when rows straddle lines: plain or skewed
+// blocks; in plain rows (along B, the dimension that is contiguous in the tensor, then along A, the one
+// that is contiguous in the payload) or in strips of kBlockStrip blocks along A.  Microseconds are pack +
+// unpack in turn, each pass on another of several copies, 1.2 GB in all.
+//  - Bundles up to 32 MiB, what the eight L2s hold, stay plain, partly written lines are completed there
+//    (28 MB, tensor rows on lines, 2-byte elements 29.6 plain / 30.8 skewed, 8-byte ones 27.7 / 29.3;
+//    34 MB of odd rows 41.9 / 40.0).
+//  - Skewed blocks stage up to 1.5 times the elements they write, and twice as many where a row holds
+//    little more than a block: both extents have to reach skew_min_row (70 MB in rows of 101 2-byte
+//    elements 68 plain / 95 skewed, 100 matrices of 428 x 428 4-byte elements 62 / 68; one odd matrix of
+//    70 MB 82 / 67, 4- and 8-byte elements 72 / 62 and 70 / 59).
+//  - Strips bring blocks that share payload lines, neighbours along A, close to each other where B is long
+//    (70 MB of 211 x n 4-byte elements 82 in plain rows / 64, 16-byte ones 77 / 68; from 24 MiB on: 28 MB
+//    40 / 32) and where only the payload's rows straddle lines (34 MB of 8-byte elements 34.0 / 32.8).
+//    Elsewhere plain rows are ahead as long as the last-level cache holds most of a pass (45 MB, payload
+//    rows on lines and odd tensor rows, 39.1 / 40.8; 16-byte elements 3 to 10 % up to 70 MB); beyond that
+//    strips are (one odd matrix of 190 MB 198 / 188, 16-byte elements 188 / 171), save for 16-byte matrices
+//    that are flat (1.02) or have their payload rows on lines (1.03).  128 x 128 blocks of bytes gain
+//    nowhere, blocks shorter than a square one only with 16-byte elements (18 x n, 70 MB 82 / 66).
+constexpr uint64_t kLongMinPayload = 24u << 20, kSkewMinPayload = 32u << 20, kStripMinPayload = 96u << 20;
+constexpr uint32_t skew_min_row(uint32_t element_bytes) {
+  return element_bytes == 4 ? 1024u : element_bytes == 8 ? 128u : 512u;
+}
+struct BlockRule {
+  bool strips = false, skew_pack = false, skew_unpack = false;
+};
+// `square`: blocks of transpose_edge x transpose_edge, otherwise one dimension is shorter than that.
+constexpr BlockRule block_rule(uint32_t element_bytes, uint64_t ext_a, uint64_t ext_b, bool square, uint64_t payload_bytes,
+                               bool tensor_lines, bool payload_lines) {
+  BlockRule rule;
+  if (tensor_lines && payload_lines) return rule;
+  const uint64_t row = skew_min_row(element_bytes);
+  const bool large = ext_a >= row && ext_b >= row && payload_bytes > kSkewMinPayload;
+  const bool long_b = element_bytes > 1 && ext_b >= row && ext_b / 4 >= ext_a && payload_bytes > kLongMinPayload;
+  const bool beyond_cache = payload_bytes > kStripMinPayload;
+  if (element_bytes == 16) {
+    rule.strips = long_b || (square && large && beyond_cache && !payload_lines && ext_b >= ext_a / 2);
+  } else if (square && element_bytes > 1 && (large || long_b)) {
+    rule.strips = long_b || beyond_cache || tensor_lines;
+    rule.skew_pack = !payload_lines && ext_a >= row;
+    rule.skew_unpack = !tensor_lines;
+  }
+  return rule;
+}
 // Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
 // 16 bytes of every plane, a wavefront up to plane_rounds times that per lane.  Bytes and 2-byte
 // elements take two rounds; 4-byte elements as many as the 8 KiB rectangle of the other blocks with
@@ -147,15 +190,15 @@ constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (mea
 struct Dims {             // 176 bytes, one per strided segment
   uint32_t mode;
   uint32_t ndim;          // outer (non-run) dimensions after collapsing, <= kMaxOuterDims;
-                          // kModeTranspose: batch dimensions (<= kMaxBatchDims)
-  uint32_t tiles_per_run; // kModeRunTiles; kModeTranspose: blocks per strip (kBlockStrip or 1)
+                          // transposed: batch dimensions (<= kMaxBatchDims)
+  uint32_t tiles_per_run; // kModeRunTiles; kModeWalked: blocks per strip (kBlockStrip or 1)
   uint32_t granule;       // kModeElements: bytes moved per lane access (1,2,4,8,16);
                           // kModeRunTiles: 1 + log2(tiles_per_run) when a power of two;
-                          // kModeTranspose: element size
+                          // transposed: element size
   uint64_t nbytes;        // bytes of the whole segment
   uint32_t shape[kMaxOuterDims];
   int64_t stride[kMaxOuterDims];   // bytes, outermost first, right-aligned
-  // kModeTranspose: A is the innermost packed dimension (strided in the tensor), B the
+  // transposed: A is the innermost packed dimension (strided in the tensor), B the
   // dimension that is contiguous in the tensor; the rest are batch dimensions.
   uint64_t pstride[kMaxBatchDims]; // packed byte strides of the batch dims (aligned with shape[2..5])
   int64_t stride_a;                // tensor byte stride of A
@@ -165,9 +208,9 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t edge_a, edge_b;         // block extent along A and B (elements)
   uint32_t lanes_per_run;          // kModeElements: 0, or the lane slots a ragged run occupies (its
                                    // 16-byte granules rounded up to a multiple of four);
-                                   // kModeTranspose: 0, or which side holds the planes of a segment
-                                   // of few planes (kPlanesInPayload, kPlanesInTensor)
-  uint32_t nt_allowed;             // kModeElements, kModeTranspose: sides that may keep the launch's
+                                   // kModePlanes: which side holds the planes (kPlanesInPayload,
+                                   // kPlanesInTensor)
+  uint32_t nt_allowed;             // kModeElements, transposed: sides that may keep the launch's
                                    // non-temporal hint when packing (bit 0 tensor, bit 1 payload) and when
                                    // unpacking (bits 2, 3).  Transposed block rows that straddle 128-byte
                                    // lines share them with the neighbouring blocks and are written through
@@ -234,7 +277,7 @@ struct LaunchConfig {
   uint32_t threads = 128;   // per workgroup, a multiple of 64
   uint32_t seg_shift = 0;   // wave_seg has one entry per 2^seg_shift tiles
   uint32_t nontemporal = 3;   // bit 0: tensor-side accesses, bit 1: payload-side accesses
-  bool elements = false;   // some segment uses kModeElements or kModeTranspose
+  bool elements = false;   // some segment uses kModeElements or is transposed
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (transposed tiles only)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
                            // multiple of 8 such runs)

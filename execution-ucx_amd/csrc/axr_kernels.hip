@@ -494,17 +494,18 @@ __device__ __forceinline__ void transpose_full(gcbytes rd, int64_t rd_pitch, gby
   __builtin_amdgcn_wave_barrier();
 }
 
-// A block whose written rows do not start on 64-byte boundaries (bundles beyond kSkewMinPayload).  Partly written 64-byte pieces are
-// what such a transposition loses its time on, not the reads: 128-byte row pieces at any address
-// read at the aligned rate, written they fall from 5.5 to 3.9 TB/s, and are back at 5.2 once every
-// piece is a whole number of aligned 64-byte units (134 MB in rows of 8198 bytes).  The block is
+// A block whose written rows do not start on 64-byte boundaries (where: block_rule).  Partly written
+// 64-byte pieces are what such a transposition loses its time on, not the reads: 128-byte row pieces at
+// any address read at the aligned rate, written they fall from 5.5 to 3.9 TB/s, and are back at 5.2 once
+// every piece is a whole number of aligned 64-byte units (134 MB in rows of 8198 bytes).  The block is
 // therefore skewed: written row y starts at its first 64-byte boundary behind element x0 and
 // holds T elements from there, so that neighbouring blocks meet on boundaries and only the ends of
 // the whole row are written in part.  For that up to 64 / E - 1 read rows of the next block are
 // staged as well; neighbours along x are neighbouring wavefronts, which find them in their L2.
-// Four 4097 x 4099 bf16 matrices: pack 84 -> 65 us, unpack 78 -> 64, the pair 140 -> 115 (aligned
-// matrices of that size: 89); 4-byte elements 131 -> 108, 8-byte elements 130 -> 107.  What is left
-// is the price of reading 1.5 times the lines and of 12 instead of 16 wavefronts per compute unit.
+// Four odd bf16 matrices of 134 MB, pack + unpack in turn over several copies: in strips of plain
+// blocks 148 us, skewed in the pack alone 145, in both 143, and 123 (67 + 60) with the unpack's whole
+// units streamed, which leaves the last-level cache to the payload and the next pack; plain rows of
+// plain blocks 151 (89 + 67).  4-byte elements 141 -> 118, 8-byte ones 134 -> 108.
 //   rd + x * rd_pitch   T elements of read row x (the block's y range)
 //   wr + y * wr_pitch   written row y from its element x = 0 on
 // ext_x >= T; y rows 0 .. T - 1 all exist.
@@ -942,8 +943,10 @@ __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t 
 // Tile q of a transposed segment: batch index (outer dims), then block (ia, ib).
 // Deliberately not inlined: the block routines get a register allocation of
 // their own (inlined into the kernel's segment walk they spilled and cost the
-// other modes registers too), and forty kernel instantiations share two copies.
-template <bool PACK>
+// other modes registers too), and forty kernel instantiations share the copies.
+// One copy per MODE: with the walk in strips and the choice of block routine in
+// the plain one's way, however predictable, 4 KiB blocks took 3 to 8 % longer.
+template <bool PACK, uint32_t MODE>
 __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_table dm, gbytes pay,
                                                uint32_t q, lbytes lds, uint32_t lane,
                                                uint32_t nt_bits) {
@@ -958,14 +961,19 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
   const uint32_t per_batch = ta * tb;
   uint32_t o = q / per_batch;
   const uint32_t rem = q - o * per_batch;
-  const bool skewed = (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0;
-  // blocks in strips of `strip` along A, walked along B: with 8 of them 64 neighbouring tiles are a
-  // square of 8 x 8 blocks (1: plain rows of blocks)
-  const uint32_t strip = dm->tiles_per_run;
-  const uint32_t is = rem / (strip * tb), in_strip = rem - is * strip * tb;
-  const uint32_t strip_rows = ta - is * strip < strip ? ta - is * strip : strip;
-  const uint32_t ib = in_strip / strip_rows;
-  const uint32_t ia = is * strip + (in_strip - ib * strip_rows);
+  uint32_t ia, ib;
+  if constexpr (MODE == kModeWalked) {
+    // blocks in strips of `strip` along A, walked along B: with 8 of them 64 neighbouring tiles are a
+    // square of 8 x 8 blocks (1: plain rows of blocks)
+    const uint32_t strip = dm->tiles_per_run;
+    const uint32_t is = rem / (strip * tb), in_strip = rem - is * strip * tb;
+    const uint32_t strip_rows = ta - is * strip < strip ? ta - is * strip : strip;
+    ib = in_strip / strip_rows;
+    ia = is * strip + (in_strip - ib * strip_rows);
+  } else {
+    ia = rem / tb;
+    ib = rem - ia * tb;
+  }
   int64_t toff = 0;
   uint64_t poff = 0;
   const uint32_t nbatch = dm->ndim;
@@ -981,12 +989,10 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
     }
   }
   uint32_t a0 = ia * edge_a, b0 = ib * edge_b;
-  const int64_t stride_a = dm->stride_a;
-  const uint64_t pstride_b = dm->pstride_b;
-  if (const uint32_t planes = dm->lanes_per_run) {
+  if constexpr (MODE == kModePlanes) {
     // Few planes <-> interleaved: the short dimension is taken whole; the last block of the long one
     // is moved back to end at the extent (it moves some elements a second time, with the same values).
-    const bool payload_planes = planes == kPlanesInPayload;   // the long dimension is A, else B
+    const bool payload_planes = dm->lanes_per_run == kPlanesInPayload;   // the long dimension is A, else B
     const uint32_t ext = payload_planes ? dm->ext_a : dm->ext_b, edge = payload_planes ? edge_a : edge_b;
     uint32_t n0 = payload_planes ? a0 : b0;
     n0 = ext - n0 < edge ? ext - edge : n0;
@@ -996,12 +1002,12 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
     const bool nt_rd = (nt_bits & (PACK ? 1u : 2u)) != 0, nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
     const uint32_t groups = edge * E / kVecBytes;
     if (payload_planes)
-      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(pstride_b), groups, lds, lane, nt_rd, nt_wr);
+      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(dm->pstride_b), groups, lds, lane, nt_rd, nt_wr);
     else
-      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, stride_a, groups, lds, lane, nt_rd, nt_wr);
+      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, dm->stride_a, groups, lds, lane, nt_rd, nt_wr);
     return;
   }
-  if (skewed) {
+  if (MODE == kModeWalked && (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0) {
     // (both extents hold a whole block; the last block across the rows is moved back)
     gbytes ten = as_global(seg_ptr) + toff, pp = pay + poff;
     gbytes rd, wr;
@@ -1010,17 +1016,17 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
     if constexpr (PACK) {
       if (b0 + T > dm->ext_b) b0 = dm->ext_b - T;
       rd = ten + (static_cast<uint64_t>(b0) << es);
-      rd_pitch = stride_a;
-      wr = pp + static_cast<uint64_t>(b0) * pstride_b;
-      wr_pitch = static_cast<int64_t>(pstride_b);
+      rd_pitch = dm->stride_a;
+      wr = pp + static_cast<uint64_t>(b0) * dm->pstride_b;
+      wr_pitch = static_cast<int64_t>(dm->pstride_b);
       x0 = a0;
       ext_x = dm->ext_a;
     } else {
       if (a0 + T > dm->ext_a) a0 = dm->ext_a - T;
       rd = pp + (static_cast<uint64_t>(a0) << es);
-      rd_pitch = static_cast<int64_t>(pstride_b);
-      wr = ten + static_cast<int64_t>(a0) * stride_a;
-      wr_pitch = stride_a;
+      rd_pitch = static_cast<int64_t>(dm->pstride_b);
+      wr = ten + static_cast<int64_t>(a0) * dm->stride_a;
+      wr_pitch = dm->stride_a;
       x0 = b0;
       ext_x = dm->ext_b;
     }
@@ -1044,6 +1050,8 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
   const uint32_t ra = dm->ext_a - a0, rb = dm->ext_b - b0;
   const uint32_t na = ra < edge_a ? ra : edge_a, nb = rb < edge_b ? rb : edge_b;
   const bool square = na == T && nb == T;   // a whole square block: the vector path
+  const int64_t stride_a = dm->stride_a;
+  const uint64_t pstride_b = dm->pstride_b;
   gbytes ten = as_global(seg_ptr) + toff + static_cast<int64_t>(a0) * stride_a +
                (static_cast<uint64_t>(b0) << es);
   gbytes pp = pay + poff + static_cast<uint64_t>(b0) * pstride_b + (static_cast<uint64_t>(a0) << es);
@@ -1327,10 +1335,13 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
           wave_copy<ROWS, NTP, NTT>(p, ten, left, lane, lane_off);
         }
       } else if constexpr (ELEMENTS) {
-        if (dm->mode == kModeTranspose) {
+        const uint32_t mode = dm->mode;
+        if (mode >= kModeTranspose) {
           extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
           lbytes lds = (lbytes)lds_slices + (threadIdx.x >> 6) * lds_per_wave;
-          transpose_tile<PACK>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+          if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+          else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+          else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
         } else {
           element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
         }

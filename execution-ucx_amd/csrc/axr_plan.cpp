@@ -773,29 +773,26 @@ struct Builder {
       }
       dm.nt_allowed = ((tensor_lines ? 1u : 0u) | (payload_lines ? 2u : 0u)) * 5u;   // both directions
       dm.lanes_per_run = planes;
-      const bool beyond_l2 = p->payload_bytes > kSkewMinPayload;
-      const bool square = !planes && edge_a == transpose_edge(e) && edge_b == edge_a;
-      // Strips for what finish_geometry hands out in squares.  Blocks of single bytes, 128 x 128 and
-      // not skewed, stay in plain rows: four 4095 x 4097 matrices, pack + unpack, 75.2 us in plain
-      // rows, 77.3 in strips, four 3001 x 2999 43.1 and 45.2; rectangles gain (four of 40 x 150,001
-      // 2-byte elements 50.6 -> 49.7).
-      const bool strips = beyond_l2 && (!tensor_lines || !payload_lines) && !(square && e == 1);
-      dm.tiles_per_run = strips ? kBlockStrip : 1u;
-      if (strips) strip_tiles += ntile;
+      dm.tiles_per_run = 1;
       if (planes) {
+        dm.mode = kModePlanes;
         lds = planes_lds_bytes(e, planes == kPlanesInPayload ? edge_b : edge_a);
-      } else if (square && beyond_l2 && e >= 2 && e <= 8 && (dm.ext_a | dm.ext_b) < (1u << 31) &&
-                 (!tensor_lines || !payload_lines)) {
-        // the side that is written gets blocks that start on its own 64-byte boundaries; reads at
-        // any address run at the aligned rate
-        // (whole 64-byte units may stream, which leaves the last-level cache to the payload: pack +
-        // unpack of 134 MB 128 -> 114 us)
-        if (!payload_lines) dm.nt_allowed |= kSkewPack;
-        if (!tensor_lines) dm.nt_allowed |= kSkewUnpack | 4u;
-        shared_line_tiles += ntile;
-        lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
       } else if (!tensor_lines || !payload_lines) {
+        const bool square = edge_a == transpose_edge(e) && edge_b == edge_a;
+        BlockRule rule = block_rule(e, dm.ext_a, dm.ext_b, square, p->payload_bytes, tensor_lines, payload_lines);
+        if ((dm.ext_a | dm.ext_b) >= (1u << 31)) rule.skew_pack = rule.skew_unpack = false;
         shared_line_tiles += ntile;
+        if (rule.strips || rule.skew_pack || rule.skew_unpack) dm.mode = kModeWalked;
+        if (rule.strips) {
+          dm.tiles_per_run = kBlockStrip;
+          strip_tiles += ntile;
+        }
+        // The side that is written gets blocks that start on its own 64-byte boundaries.  Whole 64-byte
+        // units may stream: streamed into the tensors they leave the last-level cache to the payload and
+        // the next pass (134 MB of 2-byte elements, pack + unpack 143 -> 123 us).
+        if (rule.skew_pack) dm.nt_allowed |= kSkewPack;
+        if (rule.skew_unpack) dm.nt_allowed |= kSkewUnpack | 4u;
+        if (rule.skew_pack || rule.skew_unpack) lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
       }
       p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
     } else if (run_bytes >= element_mode_limit(run_bytes)) {
@@ -898,7 +895,7 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   for (const Dims& dm : p->dims) {
     p->cfg.elements = p->cfg.elements || dm.mode != kModeRunTiles;
     ragged_rows = ragged_rows || (dm.mode == kModeElements && dm.lanes_per_run != 0);
-    blocks = blocks || dm.mode == kModeTranspose;
+    blocks = blocks || dm.mode >= kModeTranspose;
   }
   if (p->cfg.elements) p->cfg.threads = std::min(p->cfg.threads, kMaxElementThreads);
   // Short rows that are no multiple of 16 bytes (lane slots left idle behind each run) run 2.5-5 %
@@ -916,11 +913,9 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   p->cfg.workgroups = static_cast<uint32_t>((p->ntiles + per_wg - 1) / per_wg);
   // Transposed blocks whose rows straddle lines find their neighbours' lines in an L2 when the blocks
   // around them run on the same die (automatic when such blocks are half of the bundle or more):
-  // every die takes squares of kBlockStrip x kBlockStrip blocks in turn, which for four 4097 x 4099
-  // bf16 matrices brings pack 70 -> 64 us and unpack 64 -> 60.  One contiguous eighth of the tiles
-  // per die, 73 and 73 us there, stays for bundles that fit the L2s (8 x 4 MiB), where the two are
-  // level and for which nothing else is done either, and for blocks in plain rows, and is what the
-  // switch set to 1 gives.
+  // every die takes squares of kBlockStrip x kBlockStrip blocks in turn where most of the blocks lie in
+  // strips, else one contiguous eighth of the tiles, which keeps plain rows of blocks together (the two
+  // are compared at block_rule) and is what the switch set to 1 gives.
   uint32_t run = 0;
   bool whole = false;
   const bool shared_lines = p->shared_line_tiles != 0 && 2 * p->shared_line_tiles >= p->ntiles;
@@ -2328,7 +2323,7 @@ static int plan_segments_body(axr_plan_t* plan, axr_segment_info_t* out, size_t 
         o.shape[d] = dm.shape[kMaxOuterDims - dm.ndim + d];
         o.stride_bytes[d] = dm.stride[kMaxOuterDims - dm.ndim + d];
       }
-      if (dm.mode == kModeTranspose) {
+      if (dm.mode >= kModeTranspose) {
         // all dims in packed (C) order: the batch dims with B, the dim that is
         // contiguous in the tensor, at its place among them, then A
         struct Dim { uint32_t extent; int64_t stride; uint64_t packed; };

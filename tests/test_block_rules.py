@@ -1,0 +1,78 @@
+"""Which transposed views are moved in skewed blocks and in strips of blocks: the planner's rule
+(csrc/axr_internal.h), compiled on its own and asked over element sizes, shapes and bundle sizes."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include <cstdio>
+#include "axr_internal.h"
+using namespace axr;
+int main() {
+  unsigned e, square, tensor_lines, payload_lines;
+  unsigned long long a, b, payload;
+  while (std::scanf("%u %llu %llu %u %llu %u %u", &e, &a, &b, &square, &payload, &tensor_lines, &payload_lines) == 7) {
+    const BlockRule r = block_rule(e, a, b, square, payload, tensor_lines, payload_lines);
+    std::printf("%d%d%d\n", r.strips, r.skew_pack, r.skew_unpack);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rule")
+    src, exe = str(folder / "rule.cpp"), str(folder / "rule")
+    with open(src, "w") as f:
+        f.write(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src, "-o", exe], check=True, timeout=120)
+
+    def ask(cases):
+        """[(element bytes, A, B, MiB, tensor rows on lines, payload rows on lines)] -> [(strips, pack, unpack)]"""
+        edge = {1: 128, 2: 64, 4: 32, 8: 32, 16: 16}
+        lines = "".join(f"{e} {a} {b} {int(a >= edge[e] and b >= edge[e])} {int(mib * (1 << 20))} {t} {p}\n"
+                        for e, a, b, mib, t, p in cases)
+        out = subprocess.run([exe], input=lines, capture_output=True, text=True, check=True, timeout=60).stdout.split()
+        assert len(out) == len(cases)
+        return [tuple(c == "1" for c in o) for o in out]
+    return ask
+
+
+def test_small_bundles_and_whole_lines_stay_plain(rule):
+    cases = [(e, 2001, 2003, mib, t, p) for e in (1, 2, 4, 8, 16)
+             for mib, t, p in ((8, 0, 0), (32, 0, 0), (32, 1, 0), (200, 1, 1))]
+    assert set(rule(cases)) == {(False, False, False)}
+
+
+def test_short_rows_are_not_skewed(rule):
+    """Rows of little more than a block, where staging the neighbour's elements costs up to 40 %."""
+    for mib in (33, 70, 190):
+        cases = [(e, 300001, b, mib, 0, 0) for e, short in ((2, (65, 101, 211, 511)), (4, (33, 41, 101, 211, 1023)),
+                                                             (8, (33, 41, 101, 127))) for b in short]
+        cases += [(e, n, n, mib, 0, 0) for e, n in ((2, 422), (4, 298), (4, 705), (8, 119))]     # batches of small matrices
+        assert set(rule(cases)) == {(False, False, False)}
+
+
+def test_large_matrices_are_skewed_on_the_side_that_straddles_lines(rule):
+    for e in (2, 4, 8):
+        for mib in (34, 134):
+            both, tensor_odd, payload_odd = rule([(e, 2001, 2003, mib, 0, 0), (e, 2048, 2003, mib, 0, 1),
+                                                  (e, 2001, 2048, mib, 1, 0)])
+            assert both[1:] == (True, True) and tensor_odd[1:] == (False, True) and payload_odd[1:] == (True, False)
+            assert both[0] == tensor_odd[0] == (mib > 96) and payload_odd[0]
+    assert {r[1:] for r in rule([(e, 2001, 2003, 134, 0, 0) for e in (1, 16)])} == {(False, False)}
+
+
+def test_strips_where_b_is_long_or_the_cache_is_left(rule):
+    """Long B: strips from 24 MiB on; else 16-byte elements, and flat ones at no size."""
+    assert all(r[0] for r in rule([(e, 211, 4001, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (25, 70, 190)]))
+    assert not any(r[0] for r in rule([(e, 211, 4001, 24, 0, 0) for e in (2, 4, 8, 16)]))
+    assert not any(r[0] for r in rule([(16, 1459, 1461, 70, 0, 0), (16, 30001, 801, 190, 0, 0), (16, 1456, 1461, 190, 0, 1),
+                                       (1, 211, 90001, 190, 0, 0)]))
+    assert rule([(16, 1459, 1461, 190, 0, 0)])[0][0]
+    # one dimension shorter than a square block
+    assert [r[0] for r in rule([(e, 12, 90001, 70, 0, 0) for e in (1, 2, 4, 8, 16)])] == [False] * 4 + [True]

@@ -5,13 +5,14 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-DTYPES = {1: "uint8", 2: "int16", 4: "int32", 8: "int64"}
+DTYPES = {1: "uint8", 2: "int16", 4: "int32", 8: "int64", 16: "complex128"}
 
 
 def storage(torch, gpu, n, item, lead, seed):
     g = torch.Generator(device=gpu)
     g.manual_seed(seed)
-    raw = torch.randint(0, 256, ((n + lead) * item,), dtype=torch.uint8, device=gpu, generator=g)
+    # (bytes below 120: no NaN among the complex numbers)
+    raw = torch.randint(0, 256 if item < 16 else 120, ((n + lead) * item,), dtype=torch.uint8, device=gpu, generator=g)
     return raw.view(getattr(torch, DTYPES[item]))
 
 
@@ -54,6 +55,80 @@ def test_skewed_blocks(pkg, gpu, item, align, lead, shift):
         return full[:-1] + [full[-1][:123]]        # the last one leaves a gap behind every row
 
     round_trip(pkg, gpu, stores, views, align, shift)
+
+
+# Shapes at the edges of the rule that takes blocks to the skewed routine and to strips (rows of
+# `least` elements; B four times as long as A; one dimension just above a block), with batch
+# dimensions, next to a matrix that takes the bundle beyond 32 or 96 MiB; several tiles per wavefront,
+# streaming on both sides, either die mapping
+@pytest.mark.parametrize("item", [2, 4, 8, 16])
+@pytest.mark.parametrize("mib", [33, 97])
+@pytest.mark.parametrize("tunables", [{}, {"nontemporal": 3, "max_waves": 3001}, {"nontemporal": 0, "threads": 64},
+                                      {"xcd_remap": 1}, {"xcd_remap": 0, "max_waves": 500}], ids=str)
+@pytest.mark.parametrize("align,lead", [(1, 1), (256, 0)])
+def test_blocks_at_the_edges_of_their_rule(pkg, gpu, item, mib, tunables, align, lead):
+    import torch
+    edge, least = {2: (64, 512), 4: (32, 1024), 8: (32, 128), 16: (16, 512)}[item]
+    shapes = [(least, least), (least + 1, least + edge - 1), (least + edge + 31, least + 1), (least - 1, 4 * least),
+              (edge, max(4 * edge, least)), (edge + 3, max(4 * edge + 12, least) + 1), (edge + 3, 4 * edge + 11),
+              (4 * least + 3, least), (2, 3, least + 5, least + edge // 2 + 1), (5, edge + 9, max(4 * edge + 36, least) + 3)]
+    if align == 256:     # rows on lines on one side or the other
+        lines = 128 // min(item, 128)
+        shapes += [(least + 1, (least // lines + 2) * lines), ((least // lines + 2) * lines, least + 1)]
+    have = sum(torch.Size(s).numel() for s in shapes) * item
+    rows = 2051
+    shapes.append((rows, max(((mib << 20) - have) // rows // item, 1) | 1))
+    stores = [storage(torch, gpu, torch.Size(s).numel(), item, lead, i) for i, s in enumerate(shapes)]
+
+    def views(ss):
+        return [s[lead:lead + torch.Size(shape).numel()].view(shape).transpose(-1, -2) for s, shape in zip(ss, shapes)]
+
+    try:
+        pkg.tune(**tunables)
+        round_trip(pkg, gpu, stores, views, align, 0 if align > 1 else 3)
+    finally:
+        pkg.tune(nontemporal=-1, max_waves=1 << 20, threads=0, xcd_remap=-1)
+
+
+@pytest.mark.parametrize("item", [2, 4, 8])
+@pytest.mark.parametrize("remap", [-1, 0])
+def test_skewed_blocks_in_submitted_jobs_at_another_address(pkg, gpu, item, remap):
+    """Joint and single launches of plans moved by a tensor delta that changes how rows lie to
+    64-byte boundaries."""
+    import torch
+    lib, capi = pkg._capi.load(), pkg._capi
+    r, c = 2051, (34 << 20) // 2051 // item | 1
+    there, back = 5, 9          # elements from where the plans were made
+    src, dst = (torch.randint(0, 120, (r * c + 16,), dtype=torch.uint8, device=gpu).to(getattr(torch, DTYPES[item])) for _ in "ab")
+    want_dst = dst.clone()
+    flat = [torch.randint(0, 256, (100001,), dtype=torch.uint8, device=gpu) for _ in range(2)]
+
+    def view(s, at):
+        return s[at:at + r * c].view(r, c).t()
+
+    try:
+        pkg.tune(xcd_remap=remap)
+        send, other = pkg.BundlePlan.create([view(src, 0)], align=1), pkg.BundlePlan.create([flat[0]], align=1)
+        recv = pkg.BundlePlan.from_header_bound(send.header, [view(dst, 0)])
+        n = send.payload_bytes
+        payload, small = torch.zeros(n + 3, dtype=torch.uint8, device=gpu), torch.zeros(100001, dtype=torch.uint8, device=gpu)
+        jobs = (capi.Job * 2)()
+        jobs[0] = capi.Job(send._h, 0, payload.data_ptr() + 3, n, there * item)
+        jobs[1] = capi.Job(other._h, 0, small.data_ptr(), small.numel(), 0)
+        capi.check(lib.axr_submit(jobs, 2, None))
+        torch.cuda.synchronize()
+        assert torch.equal(payload[3:], view(src, there).contiguous().reshape(-1).view(torch.uint8))
+        assert torch.equal(small, flat[0])
+        jobs[0] = capi.Job(other._h, 0, small.data_ptr(), small.numel(), 0)
+        jobs[1] = capi.Job(recv._h, 1, payload.data_ptr() + 3, n, back * item)
+        capi.check(lib.axr_submit(jobs, 2, None))
+        torch.cuda.synchronize()
+        view(want_dst, back).copy_(view(src, there))
+        assert torch.equal(dst, want_dst)
+    finally:
+        pkg.tune(xcd_remap=-1)
+    for p in (send, other, recv):
+        p.close()
 
 
 # the long dimension below one vector, one vector, ragged, a whole block, one element more, several

@@ -168,6 +168,11 @@ constexpr BlockRule block_rule(uint32_t element_bytes, uint64_t ext_a, uint64_t 
   }
   return rule;
 }
+// When one of the two block dimensions is shorter than a square block's edge the
+// block becomes a rectangle of about this many bytes, its long edge capped.
+constexpr uint32_t kRectBlockBytes = 8192;
+constexpr uint32_t kRectMaxEdge = 1024;
+constexpr uint32_t kMinBlockBytes = 1024;   // smaller blocks than this are left to element mode
 // Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
 // 16 bytes of every plane, a wavefront up to plane_rounds times that per lane.  Bytes and 2-byte
 // elements take two rounds; 4-byte elements as many as the 8 KiB rectangle of the other blocks with
@@ -180,10 +185,21 @@ constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2;   // Dims.lanes_pe
 constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes) {   // one vector of padding behind every eight
   return plane_rounds(element_bytes, planes) * kWaveLanes * planes * kVecBytes / 8 * 9;
 }
-// When one of the two block dimensions is shorter than a square block's edge the
-// block becomes a rectangle of about this many bytes, its long edge capped.
-constexpr uint32_t kRectBlockBytes = 8192;
-constexpr uint32_t kRectMaxEdge = 1024;
+// Whether planes of `extent` elements are moved like this.  Whole vectors of 4-byte elements that one
+// access per lane holds are not: rectangles take no second round for them (38 MB in three planes of 200
+// elements 44 us for pack + unpack, 50 in rounds).
+constexpr bool in_planes(uint32_t element_bytes, uint64_t extent) {
+  return element_bytes <= 4 && extent * element_bytes >= kVecBytes &&
+         !(element_bytes == 4 && extent <= kWaveLanes * kVecBytes / 4 && extent % 4 == 0);
+}
+// Elements of every plane that a block takes of `extent` of them: whole vectors, as many as fit; the
+// block behind the last whole one takes what is left.
+constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t extent) {
+  const uint32_t vec = kVecBytes / element_bytes, square = kRectBlockBytes / 4 / planes;
+  const uint32_t block = element_bytes < 4 ? plane_rounds(element_bytes, planes) * kWaveLanes * vec
+                                           : (square < kRectMaxEdge ? square : kRectMaxEdge) / vec * vec;
+  return extent < block ? static_cast<uint32_t>((extent + vec - 1) / vec * vec) : block;
+}
 constexpr uint32_t kMaxBatchDims = 4;
 constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (measured: 8 KiB beats 2, 4 and 16)
 

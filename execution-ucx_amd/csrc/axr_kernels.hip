@@ -800,12 +800,21 @@ __device__ __forceinline__ void regroup_vectors(const u32x4 (&in)[C], u32x4 (&ou
   }
 }
 
-// `groups` lane units (16 bytes of every plane each) from `inter` / plane 0 at `plane` on.
+// `count` >= 16 / E elements of every plane from `inter` / plane 0 at `plane` on, in units of 16 bytes of
+// every plane.  The last unit is moved back to end with them (it moves some elements a second time, with
+// the same values), so that a ragged end costs a unit and not another block.
 template <uint32_t E, uint32_t C, bool TO_PLANES>
-__device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t groups,
+__device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t count,
                                              lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
   constexpr uint32_t R = plane_rounds(E, C);
-  const uint32_t nvec = groups * C;
+  const uint32_t groups = (count * E + kVecBytes - 1) / kVecBytes, nvec = groups * C;
+  const uint32_t back = groups * kVecBytes - count * E;   // bytes of a plane
+  // where unit g lies in a plane, and vector m in the interleaved range (past the last: the last)
+  auto plane_at = [&](uint32_t g) { return g < groups - 1u ? g * kVecBytes : (groups - 1u) * kVecBytes - back; };
+  auto inter_at = [&](uint32_t m) {
+    const uint32_t v = m < nvec ? m : nvec - 1u;
+    return v * kVecBytes - (v < nvec - C ? 0u : back * C);
+  };
   // vector m of the interleaved range in LDS: one vector of padding behind every eight
   auto slot = [&](uint32_t m) { return lds + m * kVecBytes + (m >> 3) * kVecBytes; };
   u32x4 x[R][C];
@@ -814,14 +823,10 @@ __device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t
     for (uint32_t k = 0; k < R; ++k) {
 #pragma unroll
       for (uint32_t c = 0; c < C; ++c) {
-        if constexpr (TO_PLANES) {
-          const uint32_t m = (k * C + c) * kWaveLanes + lane;
-          x[k][c] = load16<decltype(nt)::value>(inter + (m < nvec ? m : nvec - 1u) * kVecBytes);
-        } else {
-          const uint32_t g = k * kWaveLanes + lane;
-          x[k][c] = load16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch +
-                                                (g < groups ? g : groups - 1u) * kVecBytes);
-        }
+        if constexpr (TO_PLANES)
+          x[k][c] = load16<decltype(nt)::value>(inter + inter_at((k * C + c) * kWaveLanes + lane));
+        else
+          x[k][c] = load16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch + plane_at(k * kWaveLanes + lane));
       }
     }
   };
@@ -863,14 +868,14 @@ __device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t
         if (g < groups) {
 #pragma unroll
           for (uint32_t c = 0; c < C; ++c)
-            store16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch + g * kVecBytes, y[c]);
+            store16<decltype(nt)::value>(plane + static_cast<int64_t>(c) * plane_pitch + plane_at(g), y[c]);
         }
       } else {
 #pragma unroll
         for (uint32_t c = 0; c < C; ++c) {
           const uint32_t m = (k * C + c) * kWaveLanes + lane;
           const u32x4 y = *reinterpret_cast<const AXR_LDS u32x4*>(slot(m));
-          if (m < nvec) store16<decltype(nt)::value>(inter + m * kVecBytes, y);
+          if (m < nvec) store16<decltype(nt)::value>(inter + inter_at(m), y);
         }
       }
     }
@@ -887,8 +892,8 @@ __device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t
 
 template <bool TO_PLANES>
 __device__ __forceinline__ void planes_of(uint32_t E, uint32_t C, gbytes inter, gbytes plane, int64_t plane_pitch,
-                                          uint32_t groups, lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
-#define AXR_PLANES(e, c) planes_block<e, c, TO_PLANES>(inter, plane, plane_pitch, groups, lds, lane, nt_rd, nt_wr)
+                                          uint32_t count, lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
+#define AXR_PLANES(e, c) planes_block<e, c, TO_PLANES>(inter, plane, plane_pitch, count, lds, lane, nt_rd, nt_wr)
   switch (E << 4 | C) {
     case 0x12: AXR_PLANES(1, 2); break;
     case 0x13: AXR_PLANES(1, 3); break;
@@ -990,21 +995,22 @@ __device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_
   }
   uint32_t a0 = ia * edge_a, b0 = ib * edge_b;
   if constexpr (MODE == kModePlanes) {
-    // Few planes <-> interleaved: the short dimension is taken whole; the last block of the long one
-    // is moved back to end at the extent (it moves some elements a second time, with the same values).
+    // Few planes <-> interleaved: the short dimension is taken whole.  What is left of the long one
+    // may be less than a vector: the block is then moved back to hold one.
     const bool payload_planes = dm->lanes_per_run == kPlanesInPayload;   // the long dimension is A, else B
     const uint32_t ext = payload_planes ? dm->ext_a : dm->ext_b, edge = payload_planes ? edge_a : edge_b;
+    const uint32_t least = kVecBytes / E;
     uint32_t n0 = payload_planes ? a0 : b0;
-    n0 = ext - n0 < edge ? ext - edge : n0;
+    n0 = ext - n0 < least ? ext - least : n0;
+    const uint32_t count = ext - n0 < edge ? ext - n0 : edge;
     const uint32_t C = payload_planes ? edge_b : edge_a;
     const uint64_t inter_at = static_cast<uint64_t>(n0) * C << es, plane_at = static_cast<uint64_t>(n0) << es;
     gbytes ten = as_global(seg_ptr) + toff, pp = pay + poff;
     const bool nt_rd = (nt_bits & (PACK ? 1u : 2u)) != 0, nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
-    const uint32_t groups = edge * E / kVecBytes;
     if (payload_planes)
-      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(dm->pstride_b), groups, lds, lane, nt_rd, nt_wr);
+      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(dm->pstride_b), count, lds, lane, nt_rd, nt_wr);
     else
-      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, dm->stride_a, groups, lds, lane, nt_rd, nt_wr);
+      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, dm->stride_a, count, lds, lane, nt_rd, nt_wr);
     return;
   }
   if (MODE == kModeWalked && (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0) {

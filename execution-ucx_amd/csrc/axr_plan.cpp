@@ -684,21 +684,14 @@ struct Builder {
         if (edge >= ev) edge -= edge % ev;
         return static_cast<uint32_t>(edge);
       };
-      // Two to four planes against the same elements interleaved without gaps: whole vectors on
-      // both sides.  The long edge is a whole number of vectors (the last block is moved back).
-      auto plane_edge = [&](uint64_t extent, uint64_t count) {
-        if (e == 4) return long_edge(extent, count);
-        return static_cast<uint32_t>(
-            std::min<uint64_t>(plane_rounds(e, static_cast<uint32_t>(count)) * kWaveLanes * ev, extent - extent % ev));
-      };
-      if (e <= 4 && eb >= 2 && eb <= kMaxPlanes && ea >= ev && str[nd - 1] == static_cast<int64_t>(eb * e)) {
+      if (eb >= 2 && eb <= kMaxPlanes && in_planes(e, ea) && str[nd - 1] == static_cast<int64_t>(eb * e)) {
         planes = kPlanesInPayload;
         edge_b = static_cast<uint32_t>(eb);
-        edge_a = plane_edge(ea, eb);
-      } else if (e <= 4 && ea >= 2 && ea <= kMaxPlanes && eb >= ev && dim_b + 2 == nd) {
+        edge_a = plane_edge(e, static_cast<uint32_t>(eb), ea);
+      } else if (ea >= 2 && ea <= kMaxPlanes && in_planes(e, eb) && dim_b + 2 == nd) {
         planes = kPlanesInTensor;
         edge_a = static_cast<uint32_t>(ea);
-        edge_b = plane_edge(eb, ea);
+        edge_b = plane_edge(e, static_cast<uint32_t>(ea), eb);
       } else if (ea >= t && eb >= t) {
         edge_a = edge_b = static_cast<uint32_t>(t);
       } else {
@@ -710,7 +703,7 @@ struct Builder {
           edge_a = long_edge(ea, edge_b);
         }
       }
-      if (static_cast<uint64_t>(edge_a) * edge_b * e < 1024) dim_b = nd;
+      if (static_cast<uint64_t>(edge_a) * edge_b * e < kMinBlockBytes) dim_b = nd;
     }
     if (dim_b < nd) {
       const uint32_t e = static_cast<uint32_t>(run_bytes);

@@ -76,3 +76,29 @@ def test_strips_where_b_is_long_or_the_cache_is_left(rule):
     assert rule([(16, 1459, 1461, 190, 0, 0)])[0][0]
     # one dimension shorter than a square block
     assert [r[0] for r in rule([(e, 12, 90001, 70, 0, 0) for e in (1, 2, 4, 8, 16)])] == [False] * 4 + [True]
+
+
+def test_plane_blocks_do_not_overlap(tmp_path):
+    """Every element of a plane belongs to one block, but for the last block's end, which may reach
+    less than a vector beyond the extent (and is moved back by that much)."""
+    source = r"""
+#include "axr_internal.h"
+using namespace axr;
+constexpr bool covered(uint32_t e, uint32_t planes) {
+  for (uint64_t extent = kVecBytes / e; extent < 6000; ++extent) {
+    const uint64_t edge = plane_edge(e, planes, extent), blocks = (extent + edge - 1) / edge;
+    if (edge % (kVecBytes / e) != 0 || edge * e > plane_rounds(e, planes) * kRowBytes) return false;
+    if (blocks == 1 && edge - extent >= kVecBytes / e) return false;
+  }
+  return true;
+}
+static_assert(covered(1, 2) && covered(1, 3) && covered(1, 4), "bytes");
+static_assert(covered(2, 2) && covered(2, 3) && covered(2, 4), "2-byte elements");
+static_assert(covered(4, 2) && covered(4, 3) && covered(4, 4), "4-byte elements");
+static_assert(in_planes(1, 16) && !in_planes(1, 15) && in_planes(4, 201) && !in_planes(4, 200) && !in_planes(8, 4096), "range");
+"""
+    src = str(tmp_path / "planes.cpp")
+    with open(src, "w") as f:
+        f.write(source)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=100000000", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)

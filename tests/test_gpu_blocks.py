@@ -149,3 +149,32 @@ def test_planes_and_interleaved(pkg, gpu, item, planes, long):
     for make in (views, planar):
         for align, shift in ((1, 0), (256, 3)):
             round_trip(pkg, gpu, stores, make, align, shift)
+
+
+# ends that are no whole vector: one vector and a bit, just below and above a block (2048, 1024 and
+# 1024 / 680 / 512 elements), less than a vector behind the last whole block; several tiles per
+# wavefront and streaming on both sides
+@pytest.mark.parametrize("item", [1, 2, 4])
+@pytest.mark.parametrize("planes", [2, 3, 4])
+@pytest.mark.parametrize("long", [17, 90, 345, 511, 513, 679, 681, 1023, 1025, 1361, 2047, 2051, 3000, 4097])
+@pytest.mark.parametrize("tunables", [{}, {"nontemporal": 3, "max_waves": 37}], ids=["plain", "streams"])
+def test_ragged_planes(pkg, gpu, item, planes, long, tunables):
+    import torch
+    stores = [storage(torch, gpu, 40 * long * planes, item, lead, lead) for lead in (0, 1)]
+
+    def inter(ss):
+        return [s[k:].view(40, long, planes).permute(0, 2, 1) for k, s in enumerate(ss)]
+
+    def planar(ss):
+        return [s[k:].view(40, planes, long).permute(0, 2, 1) for k, s in enumerate(ss)]
+
+    def apart(ss):       # a gap behind every plane
+        return [s[k:].view(20, planes, 2 * long)[:, :, :long].permute(0, 2, 1) for k, s in enumerate(ss)]
+
+    try:
+        pkg.tune(**tunables)
+        for make in (inter, planar, apart):
+            round_trip(pkg, gpu, stores, make, 1, 3)
+            round_trip(pkg, gpu, stores, make, 256, 0)
+    finally:
+        pkg.tune(nontemporal=-1, max_waves=1 << 20)

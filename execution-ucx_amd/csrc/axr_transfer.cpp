@@ -1,7 +1,7 @@
 // Streamed transfer of a large payload in chunks: pack -> loopback send -> unpack,
 // double-buffered over two (or more) lanes, each lane a send slot and a receive slot.
-// Chunk k uses lane k % lanes and runs on stream (k % lanes) % streams, or in line with all
-// others on the first lane's stream and slot (see runs_in_line).  With one stream
+// Chunk k uses lane k % lanes and runs on stream (k % lanes) % streams, or in line with its
+// neighbours on the first lane's stream and slot (see runs_in_line).  With one stream
 // per lane, stream order alone makes a slot safe to reuse `lanes` chunks later and chunk
 // k + 1's pack overlaps chunk k's wire copy and unpack; with fewer streams than lanes the
 // chunks of one stream run back to back and the extra lanes only let the host queue ahead.
@@ -58,19 +58,17 @@ int retire(axr_transfer* t, axr_transfer::Lane& lane) {
   return AXR_OK;
 }
 
-// Chunks that run in line: one after the other on the first lane's stream, all through its send
-// slot, which stays in the last-level cache from a chunk's pack to its unpack and on to the next
-// pack.  That holds while the payloads in flight fit the cache or there is only one at a time; two
-// that do not fit evict each other, and what they lose is more than what the overlap of two
-// launches' ramps and tails gives.  Eight chunks of 2- to 4-KiB rows at 1.5 times their length, pack
-// and unpack, two streams / one / one and a single slot: 8 x 67 MB 348 / 376 / 374 us,
-// 8 x 134 MB (two are 256 MiB) 654 / 667 / 668, 8 x 159 MB 914 / 793 / 780, 8 x 201 MB
-// 1237 / 1043 / 969, 8 x 268 MB 1629 / 1309 / 1265; payloads beyond the cache stream and gain
-// little: 8 x 336 MB 1676 / 1646 / 1651, 8 x 537 MB 2681 / 2623 / 2620.  (A plain copy of the
-// bytes of 8 x 268 MB: 1282 us.)
+// Borrowed chunks that run in line: one after the other on the first lane's stream, all through its
+// send slot, which stays in the last-level cache from a chunk's pack to its unpack and on to the next
+// pack.  Where the payloads of all streams fit the cache, the overlap of two launches' ramps and tails
+// is worth more; where one alone does not, nothing is kept there either way.  In between they evict
+// each other.  Eight chunks of 2- to 4-KiB rows at 1.5 times their length through kept plans, from the
+// first submission to the end of the wait, two streams / in line: 8 x 67 MB 377 / 431 us, 8 x 134 MB (two
+// are 256 MiB) 681 / 729, 8 x 159 MB 920 / 842, 8 x 201 MB 1243 / 1037, 8 x 268 MB 1645 / 1340; 8 x 336 MB
+// 1690 / 1719, 8 x 537 MB 2684 / 2695.  (A plain copy of the bytes of 8 x 268 MB: 1282 us.)
 bool runs_in_line(const axr_transfer* t, uint64_t nbytes) {
-  return t->zero_copy &&
-         (t->streams == 1 || nbytes > static_cast<uint64_t>(tunables().payload_cache_bytes) / t->streams);
+  const uint64_t cache = static_cast<uint64_t>(tunables().payload_cache_bytes);
+  return t->zero_copy && (t->streams == 1 || (nbytes > cache / t->streams && nbytes <= cache));
 }
 
 void destroy(axr_transfer* t) {

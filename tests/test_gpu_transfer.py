@@ -6,9 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lanes,streams", [(1, 1), (2, 1), (2, 2), (3, 2)])
-@pytest.mark.parametrize("cache", ["fits", "one byte short"])
+@pytest.mark.parametrize("cache", ["fits", "one byte short", "beyond"])
 def test_chunks_in_line(pkg, gpu, lanes, streams, cache):
-    """Two geometries in turn; `streams` payloads of the larger one just fit the cache, or do not."""
+    """Two geometries in turn; `streams` payloads of the larger one just fit the cache, or do not, or
+    not even one does."""
     import torch
     big, small = (4, 257, 300), (3, 5, 300)          # views, rows, columns
     tune = pkg._capi.load().axr_tune_set
@@ -25,7 +26,8 @@ def test_chunks_in_line(pkg, gpu, lanes, streams, cache):
     want = torch.zeros_like(src)
     torch.cuda.synchronize()
     try:
-        assert tune(b"payload_cache_bytes", streams * largest - (cache != "fits")) == 0
+        limit = largest - 1 if cache == "beyond" else streams * largest - (cache != "fits")
+        assert tune(b"payload_cache_bytes", limit) == 0
         for k in range(12):
             views, rows, cols = (big, small)[k % 5 == 3]
             send, recv = pairs[k % 5 == 3]

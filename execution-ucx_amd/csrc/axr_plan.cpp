@@ -490,7 +490,7 @@ struct Collapser {
       return compact;
     }
     const size_t bytes = static_cast<size_t>(t.ndim) * sizeof(int64_t);
-    const bool same = last && last->ndim == t.ndim && (last->bits + 7) / 8 == (t.bits + 7) / 8 &&
+    const bool same = last && last->nbytes == t.nbytes && last->ndim == t.ndim && (last->bits + 7) / 8 == (t.bits + 7) / 8 &&
                       std::memcmp(p->shape_of(*last), shape, bytes) == 0 &&
                       std::memcmp(p->strides_of(*last), strides, bytes) == 0;
     if (!same) collapse(t, shape, strides, (static_cast<uint64_t>(t.bits) + 7) / 8, &c);
@@ -828,7 +828,9 @@ struct Builder {
     // Views of one geometry that follow each other (the blocks of a cache, the chunks of a matrix)
     // share one record: the wavefronts find it in the scalar cache instead of fetching a new one
     // from memory at every view, and there is less to write and to bring to the device.
-    if (p->dims.empty() || std::memcmp(&p->dims.back(), &dm, sizeof(dm)) != 0) p->dims.push_back(dm);
+    // (lengths first: views that all differ pay for one comparison)
+    if (p->dims.empty() || p->dims.back().nbytes != nbytes || std::memcmp(&p->dims.back(), &dm, sizeof(dm)) != 0)
+      p->dims.push_back(dm);
     return add_seg(tensor, ptr, off, run_bytes, ntile, static_cast<uint32_t>(p->dims.size()));
   }
 

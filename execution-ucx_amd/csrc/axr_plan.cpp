@@ -976,14 +976,31 @@ int quiet_block(axr_plan* p, size_t bytes) {
 
 // Bundles of short contiguous device tensors only (device_build_tables has looked at lengths and
 // devices): one pass over the tensors writes the members' records and the groups they fall into (the
-// division Builder::add_member makes) into pinned memory, and a kernel lays out the group blocks.  No strides to collapse, no blocks and segments
-// to build in host memory and copy.  Launching a fresh plan of 65,536 tensors of 8 to 512 bytes:
-// 693 us on the host and 85 on the device before, 335 and 27 now.  Returns as device_build_tables
-// does.
+// division Builder::add_member makes, except that a group of one stays a group) into pinned memory, and
+// a kernel lays out the group blocks.  No strides to collapse, no blocks and segments to build in host
+// memory and copy.  Launching a fresh plan of 65,536 tensors of 8 to 512 bytes: 693 us on the host and
+// 85 on the device before, 335 and 27 now.  Returns as device_build_tables does.
 int device_build_groups(axr_plan* p, hipStream_t stream, bool* done) {
   const Tunables& tn = tunables();
   const size_t n = p->tensors.size();
   const uint32_t slots_per_group = static_cast<uint32_t>(tn.group_slots);
+  const uint64_t align_mask = static_cast<uint64_t>(p->align) - 1;
+  // the gap behind tensor `t`, and the lane slots the two take of a group (more than half: no member)
+  auto pad_of = [&](const TensorRec& t) {
+    const uint64_t end = t.offset + t.nbytes;
+    return std::min((end + align_mask) & ~align_mask, p->payload_bytes) - end;
+  };
+  auto slots_of = [&](const TensorRec& t) {
+    return group_data_slots(static_cast<uint32_t>(t.nbytes)) + group_pad_slots(static_cast<uint32_t>(pad_of(t)));
+  };
+  // Alignments that can leave a gap too long for a group are looked at before a block is taken: the
+  // room below counts every gap, and for gaps that no group would hold it is many times what the
+  // general path needs (65,536 tensors of 8 bytes at 4096: 128 MiB in each half of the block against 4).
+  const uint32_t longest = static_cast<uint32_t>(tn.group_bytes);
+  if (group_data_slots(longest) + group_pad_slots(p->align - 1) > slots_per_group / 2) {
+    for (const TensorRec& t : p->tensors)
+      if (slots_of(t) > slots_per_group / 2) return AXR_OK;
+  }
   // A group ends because it has all its members, because the next one's slots do not fit (then the
   // two groups hold more than slots_per_group together), or because the offset is out of its
   // reach; the last reason is not counted here and ends the attempt if the room runs out.
@@ -994,7 +1011,6 @@ int device_build_groups(axr_plan* p, hipStream_t stream, bool* done) {
   if (rc) return rc;
   Member* members = static_cast<Member*>(p->block.host);
   GroupStage* groups = reinterpret_cast<GroupStage*>(static_cast<uint8_t*>(p->block.host) + groups_at);
-  const uint64_t align_mask = static_cast<uint64_t>(p->align) - 1;
   bool pinned = false;
   uint32_t closed = 0;   // groups in front of `group`
   GroupStage group{};
@@ -1002,10 +1018,9 @@ int device_build_groups(axr_plan* p, hipStream_t stream, bool* done) {
     const TensorRec& t = p->tensors[i];
     if (t.has_strides && !compact_strides(p->shape_of(t), p->strides_of(t), t.ndim)) return AXR_OK;
     pinned = pinned || t.device_type == kDLROCMHost;
-    const uint64_t end = t.offset + t.nbytes;
-    const uint64_t pad = std::min((end + align_mask) & ~align_mask, p->payload_bytes) - end;
+    const uint64_t pad = pad_of(t);
     if (t.nbytes == 0 || t.nbytes > kGroupMaxMemberBytes || pad >= kMaxAlign) return AXR_OK;
-    const uint32_t need = group_data_slots(static_cast<uint32_t>(t.nbytes)) + group_pad_slots(static_cast<uint32_t>(pad));
+    const uint32_t need = slots_of(t);
     if (need > slots_per_group / 2) return AXR_OK;
     if (group.members && (group.members >= kGroupMaxMembers || group.slots + need > slots_per_group ||
                           t.offset < group.off || t.offset - group.off >= (1ull << kMemberOffBits))) {

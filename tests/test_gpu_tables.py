@@ -129,3 +129,27 @@ def test_a_launch_elsewhere_waits_for_the_upload_only(pkg, gpu, kind):
     assert still_busy
     plan.close()
     capi.check(lib.axr_stream_destroy(stream.value))
+
+
+def test_gaps_too_long_for_groups_take_no_room_for_them(pkg, gpu):
+    """Short tensors whose alignment gaps fit no group: the table block stays at what the general path
+    needs (a record of 32 bytes and an index entry each), it is not sized for groups of gaps."""
+    import torch
+    n = 60000
+    arena = torch.randint(0, 256, (16 * n,), dtype=torch.uint8, device=gpu)
+    views = [arena[16 * i:16 * i + 8] for i in range(n)]
+    plan = pkg.BundlePlan.create(views, align=4096)
+    payload = torch.full((plan.payload_bytes,), 0xCD, dtype=torch.uint8, device=gpu)
+    first = pkg.BundlePlan.create(views[:1], align=4096)    # whatever a first launch takes
+    first.pack(payload.data_ptr(), first.payload_bytes)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    plan.pack(payload.data_ptr(), plan.payload_bytes)
+    torch.cuda.synchronize()
+    taken = before - torch.cuda.mem_get_info()[0]
+    # 40 bytes per tensor, in a block of a power of two, in pages of 2 MiB
+    assert taken <= 2 * 40 * n + (4 << 20), taken
+    want = torch.zeros_like(payload)
+    want.as_strided((n, 8), (4096, 1)).copy_(arena.view(n, 16)[:, :8])
+    assert torch.equal(payload, want)
+    plan.close()

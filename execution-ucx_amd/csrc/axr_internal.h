@@ -168,6 +168,24 @@ constexpr BlockRule block_rule(uint32_t element_bytes, uint64_t ext_a, uint64_t 
   }
   return rule;
 }
+// Streamed chunks that the receiver borrows: in turn on their lanes' streams, or in line on one stream
+// and slot.  Where the payloads of all streams fit the last-level cache, the overlap of two launches'
+// ramps and tails is worth more than a slot that stays there, and where one alone does not, nothing stays
+// either way.  In between the slots evict each other, but not before they exceed the cache by more than
+// a launch that is just ending has left behind, and sooner where more lanes than streams take turns.
+// Twelve chunks through kept plans, from the first submission to the end of the wait, in turn / in line in us
+// (rows of 4 KiB; rows of 1 KiB and 64 KiB agree within 5 MB):
+//   2 lanes, 2 streams: 136 MB 1005 / 1102, 153 MB 1187 / 1212, 158 MB 1263 / 1248, 175 MB 1509 / 1358
+//   3, 3:               94 MB 722 / 825, 105 MB 853 / 899, 110 MB 931 / 928, 116 MB 1023 / 971
+//   4, 4:               84 MB 729 / 760, 94 MB 810 / 829, 100 MB 886 / 867;  6, 6: 84 MB 744 / 764, 94 MB 855 / 837
+//   4, 2:               136 MB 1048 / 1103, 142 MB 1106 / 1145, 148 MB 1259 / 1187;  6, 3: 94 MB 803 / 833, 105 MB 940 / 903
+// 8 x 268 MB on two streams 1645 / 1340 (a plain copy of the bytes: 1282), 8 x 336 MB 1690 / 1719, 8 x 537 MB
+// 2684 / 2695.
+constexpr bool chunks_in_line(uint64_t nbytes, size_t lanes, size_t streams, uint64_t cache) {
+  if (streams <= 1) return true;
+  const uint64_t spare = lanes > streams ? cache / 24 : cache / 12;
+  return nbytes <= cache && nbytes > cache / streams + spare && nbytes > cache / 20 * 7;
+}
 // When one of the two block dimensions is shorter than a square block's edge the
 // block becomes a rectangle of about this many bytes, its long edge capped.
 constexpr uint32_t kRectBlockBytes = 8192;

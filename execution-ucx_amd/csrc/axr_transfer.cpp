@@ -60,15 +60,10 @@ int retire(axr_transfer* t, axr_transfer::Lane& lane) {
 
 // Borrowed chunks that run in line: one after the other on the first lane's stream, all through its
 // send slot, which stays in the last-level cache from a chunk's pack to its unpack and on to the next
-// pack.  Where the payloads of all streams fit the cache, the overlap of two launches' ramps and tails
-// is worth more; where one alone does not, nothing is kept there either way.  In between they evict
-// each other.  Eight chunks of 2- to 4-KiB rows at 1.5 times their length through kept plans, from the
-// first submission to the end of the wait, two streams / in line: 8 x 67 MB 377 / 431 us, 8 x 134 MB (two
-// are 256 MiB) 681 / 729, 8 x 159 MB 920 / 842, 8 x 201 MB 1243 / 1037, 8 x 268 MB 1645 / 1340; 8 x 336 MB
-// 1690 / 1719, 8 x 537 MB 2684 / 2695.  (A plain copy of the bytes of 8 x 268 MB: 1282 us.)
+// pack (sizes: chunks_in_line).
 bool runs_in_line(const axr_transfer* t, uint64_t nbytes) {
-  const uint64_t cache = static_cast<uint64_t>(tunables().payload_cache_bytes);
-  return t->zero_copy && (t->streams == 1 || (nbytes > cache / t->streams && nbytes <= cache));
+  return t->zero_copy && chunks_in_line(nbytes, t->lanes.size(), t->streams,
+                                        static_cast<uint64_t>(tunables().payload_cache_bytes));
 }
 
 void destroy(axr_transfer* t) {

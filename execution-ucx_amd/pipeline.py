@@ -4,8 +4,9 @@ pack -> loopback send -> unpack on two HIP streams of one GPU.
 The work is done by the library's ``axr_transfer_*`` object (C ABI): chunk k runs
 entirely on lane k % lanes (a stream with a send slot and a receive slot), so stream
 order makes a slot safe to reuse two chunks later and chunk k + 1's pack overlaps chunk
-k's wire copy and unpack.  Zero-copy chunks of which one fits the last-level cache but not
-one per stream run one after the other on the first lane's stream and slot instead.  Chunks
+k's wire copy and unpack.  Zero-copy chunks of which one fits the last-level cache while
+one per stream clearly exceeds it run one after the other on the first lane's stream and
+slot instead.  Chunks
 of one geometry share ONE sender plan and ONE receiver plan; each chunk only names how far
 its tensors lie from the ones the plans were bound to.  Nothing blocks the host until
 ``finish`` (beyond waiting for the chunk that last used a lane).

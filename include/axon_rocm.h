@@ -643,11 +643,12 @@ AXR_API int axr_am_context_create_ucx(const char* name, axr_am_context_t** ctx);
  * chunks run back to back on one stream and the other lanes only let the host queue
  * ahead.  Borrowed chunks (the default, see axr_transfer_set_zero_copy) do so whatever
  * `streams` says, and through the first lane's send slot, if one of them fits the
- * last-level cache ("payload_cache_bytes") but `streams` of them do not (the other
- * lanes' slots stay allocated for chunks of other sizes).  The transport is a
- * loopback context pair inside the object: every chunk with a payload is a rendezvous
- * whose fetch is either a borrow of the send slot (the default) or a stream-ordered
- * device copy from the send slot to a receive slot (axr_transfer_set_zero_copy).
+ * last-level cache ("payload_cache_bytes") while `streams` of them exceed it, by a sixth
+ * for two streams and by more for more (the other lanes' slots stay allocated for chunks
+ * of other sizes).  The transport is a loopback context pair inside the object: every
+ * chunk with a payload is a rendezvous whose fetch is either a borrow of the send slot
+ * (the default) or a stream-ordered device copy from the send slot to a receive slot
+ * (axr_transfer_set_zero_copy).
  *
  * The caller keeps ONE sender plan and ONE receiver plan (axr_plan_from_header of
  * the sender's header, bound to the destination tensors) for all chunks of one

@@ -1,5 +1,5 @@
-"""Which transposed views are moved in skewed blocks and in strips of blocks: the planner's rule
-(csrc/axr_internal.h), compiled on its own and asked over element sizes, shapes and bundle sizes."""
+"""Which transposed views are moved in skewed blocks and in strips of blocks, and which streamed chunks
+run in line: the rules of csrc/axr_internal.h, compiled on their own."""
 import os
 import subprocess
 
@@ -101,4 +101,19 @@ static_assert(in_planes(1, 16) && !in_planes(1, 15) && in_planes(4, 201) && !in_
     with open(src, "w") as f:
         f.write(source)
     subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=100000000", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
+
+
+def test_chunks_in_line(tmp_path):
+    """On the side that was measured to be faster, for sizes where the two differ by more than 4 %."""
+    turn = [(2, 2, 136), (2, 2, 148), (3, 3, 94), (3, 3, 105), (4, 4, 68), (4, 4, 84), (4, 2, 136), (6, 3, 84), (2, 2, 269),
+            (2, 2, 537), (3, 3, 336), (8, 8, 16)]
+    line = [(2, 2, 164), (2, 2, 175), (2, 2, 268), (3, 3, 116), (4, 4, 105), (6, 6, 105), (4, 2, 148), (6, 3, 110), (2, 1, 16),
+            (8, 1, 600), (1, 1, 16)]
+    checks = "".join(f"static_assert({no}chunks_in_line({mb}000000ull, {lanes}, {streams}, 256ull << 20), \"{lanes} {streams} {mb}\");\n"
+                     for cases, no in ((turn, "!"), (line, "")) for lanes, streams, mb in cases)
+    src = str(tmp_path / "line.cpp")
+    with open(src, "w") as f:
+        f.write('#include "axr_internal.h"\nusing namespace axr;\n' + checks)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)

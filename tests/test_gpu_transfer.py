@@ -6,10 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lanes,streams", [(1, 1), (2, 1), (2, 2), (3, 2)])
-@pytest.mark.parametrize("cache", ["fits", "one byte short", "beyond"])
+@pytest.mark.parametrize("cache", ["fits", "one byte short", "holds one", "beyond"])
 def test_chunks_in_line(pkg, gpu, lanes, streams, cache):
     """Two geometries in turn; `streams` payloads of the larger one just fit the cache, or do not, or
-    not even one does."""
+    one and no more does (in line), or not even one does."""
     import torch
     big, small = (4, 257, 300), (3, 5, 300)          # views, rows, columns
     tune = pkg._capi.load().axr_tune_set
@@ -26,7 +26,8 @@ def test_chunks_in_line(pkg, gpu, lanes, streams, cache):
     want = torch.zeros_like(src)
     torch.cuda.synchronize()
     try:
-        limit = largest - 1 if cache == "beyond" else streams * largest - (cache != "fits")
+        limit = {"fits": streams * largest, "one byte short": streams * largest - 1, "holds one": largest,
+                 "beyond": largest - 1}[cache]
         assert tune(b"payload_cache_bytes", limit) == 0
         for k in range(12):
             views, rows, cols = (big, small)[k % 5 == 3]

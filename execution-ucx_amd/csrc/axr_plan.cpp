@@ -1351,6 +1351,13 @@ void write_tables(const axr_plan* p, uint8_t* h) {
   if (!p->group_blocks.empty()) std::memcpy(h + p->members_at, p->group_blocks.data(), p->group_blocks.size());
 }
 
+// Host-built tables of up to this many bytes are brought up by a kernel, whose writes stay near the compute
+// dies (see upload_tables_kernel); longer ones by the copy engine, which has the faster way over the bus
+// (first launch after 256 KiB of tables 23 us by kernel / 27 by copy, 1 MiB 52 / 52, 1.5 MiB 65 / 61, 4 MiB
+// 124 / 108; a fresh bundle of 500 views, 104 KB, 54 / 61 us, of 5,000 views, 1 MB, 265 / 264, of 32,000
+// short tensors and a long one, 2.6 MB, 672 / 656).
+constexpr size_t kKernelUploadBytes = 1u << 20;
+
 int ensure_uploaded(axr_plan* p, hipStream_t stream) {
   if (p->ntiles == 0) return AXR_OK;
   if (!p->uploaded) {
@@ -1365,7 +1372,10 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
       quiesce(p);   // previous launches may still read the old tables
     }
     write_tables(p, static_cast<uint8_t*>(p->block.host));
-    int rc = launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream);
+    int rc = p->table_bytes <= kKernelUploadBytes
+                 ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
+                 : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
+                             "hipMemcpyAsync(plan tables)");
     if (rc) return rc;
     return note_upload(p, stream);
   }

@@ -463,7 +463,7 @@ void collapse(const TensorRec& t, const int64_t* shape, const int64_t* strides, 
   }
 }
 
-bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
+__attribute__((noinline)) bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
   int64_t expect = 1;
   for (int32_t d = ndim - 1; d >= 0; --d) {
     if (shape[d] == 1) continue;
@@ -473,25 +473,31 @@ bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim)
   return true;
 }
 
+// Whether a tensor with strides is compact: one run, nothing to collapse.  (Its outermost stride gives
+// most others away; out of line the loop costs compact tensors of several dimensions 4 ns less.)
+bool is_compact(const axr_plan* p, const TensorRec& t) {
+  const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
+  const uint64_t item = (static_cast<uint64_t>(t.bits) + 7) / 8;
+  if (t.ndim > 0 && shape[0] != 1 && static_cast<uint64_t>(strides[0]) * static_cast<uint64_t>(shape[0]) * item != t.nbytes)
+    return false;
+  return compact_strides(shape, strides, t.ndim);
+}
+
 // Collapses tensor after tensor.  Views of one geometry come in rows (cache blocks, matrix
 // chunks): a tensor of the same shape, strides and item size as the one asked for before it gets
-// that one's answer (512 five-dimensional cache blocks: 23 -> 9 us for the two passes over them).
+// that one's answer (512 five-dimensional cache blocks: 23 -> 9 us for the two passes over them;
+// two dimensions are collapsed in the time that the comparison takes).
 struct Collapser {
   const axr_plan* p;
-  const TensorRec* last = nullptr;   // `c` is its answer (tensors with strides only)
-  Collapsed c, compact;
+  const TensorRec* last = nullptr;   // `c` is its answer
+  Collapsed c;
 
-  // For a tensor with strides (one without is compact: one run, nothing to collapse).
+  // For a tensor that is not compact.
   const Collapsed& of(const TensorRec& t) {
     const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
-    if (compact_strides(shape, strides, t.ndim)) {
-      compact.nd = 0;
-      compact.run_bytes = t.nbytes;
-      return compact;
-    }
     const size_t bytes = static_cast<size_t>(t.ndim) * sizeof(int64_t);
-    const bool same = last && last->nbytes == t.nbytes && last->ndim == t.ndim && (last->bits + 7) / 8 == (t.bits + 7) / 8 &&
-                      std::memcmp(p->shape_of(*last), shape, bytes) == 0 &&
+    const bool same = t.ndim > 2 && last && last->nbytes == t.nbytes && last->ndim == t.ndim &&
+                      (last->bits + 7) / 8 == (t.bits + 7) / 8 && std::memcmp(p->shape_of(*last), shape, bytes) == 0 &&
                       std::memcmp(p->strides_of(*last), strides, bytes) == 0;
     if (!same) collapse(t, shape, strides, (static_cast<uint64_t>(t.bits) + 7) / 8, &c);
     last = &t;
@@ -1192,8 +1198,8 @@ int build_tables(axr_plan* p) {
     bool uniform_runs = !p->tensors.empty(), run_tiles_only = streams_in_small_tiles(p);
     for (const TensorRec& t : p->tensors) {
       if (t.nbytes == 0) continue;
-      if (!t.has_strides) {   // a compact tensor: not a bundle of strided views
-        uniform_runs = false;
+      if (!t.has_strides || is_compact(p, t)) {
+        uniform_runs = false;   // a compact tensor: not a bundle of strided views
       } else {
         const Collapsed& c = collapser.of(t);
         uniform_runs = uniform_runs && c.nd != 0 && (common_run == 0 || c.run_bytes == common_run);
@@ -1233,7 +1239,7 @@ int build_tables(axr_plan* p) {
     const Collapsed* c = nullptr;
     size_t nd = 0;
     uint64_t run_bytes = t.nbytes;
-    if (strides) {
+    if (strides && !is_compact(p, t)) {
       c = &collapser.of(t);
       nd = c->nd;
       run_bytes = c->run_bytes;

@@ -463,7 +463,7 @@ void collapse(const TensorRec& t, const int64_t* shape, const int64_t* strides, 
   }
 }
 
-__attribute__((noinline)) bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
+bool compact_strides(const int64_t* shape, const int64_t* strides, int32_t ndim) {
   int64_t expect = 1;
   for (int32_t d = ndim - 1; d >= 0; --d) {
     if (shape[d] == 1) continue;
@@ -473,37 +473,22 @@ __attribute__((noinline)) bool compact_strides(const int64_t* shape, const int64
   return true;
 }
 
-// Whether a tensor with strides is compact: one run, nothing to collapse.  (Its outermost stride gives
-// most others away; out of line the loop costs compact tensors of several dimensions 4 ns less.)
+uint64_t item_bytes(const TensorRec& t) { return (static_cast<uint64_t>(t.bits) + 7) / 8; }
+
+// Whether a tensor with strides is compact: one run, nothing to collapse.  Its outermost stride gives
+// most others away.  (Out of line the loop costs compact tensors of several dimensions 4 ns less where
+// tables are built on the host.  An answer kept for the next tensor of the same geometry was slower than
+// collapsing that one, too: 20,000 views 395 against 355 us.)
+__attribute__((noinline)) bool compact_strides_called(const int64_t* shape, const int64_t* strides, int32_t ndim) {
+  return compact_strides(shape, strides, ndim);
+}
 bool is_compact(const axr_plan* p, const TensorRec& t) {
   const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
-  const uint64_t item = (static_cast<uint64_t>(t.bits) + 7) / 8;
-  if (t.ndim > 0 && shape[0] != 1 && static_cast<uint64_t>(strides[0]) * static_cast<uint64_t>(shape[0]) * item != t.nbytes)
+  if (t.ndim > 0 && shape[0] != 1 &&
+      static_cast<uint64_t>(strides[0]) * static_cast<uint64_t>(shape[0]) * item_bytes(t) != t.nbytes)
     return false;
-  return compact_strides(shape, strides, t.ndim);
+  return compact_strides_called(shape, strides, t.ndim);
 }
-
-// Collapses tensor after tensor.  Views of one geometry come in rows (cache blocks, matrix
-// chunks): a tensor of the same shape, strides and item size as the one asked for before it gets
-// that one's answer (512 five-dimensional cache blocks: 23 -> 9 us for the two passes over them;
-// two dimensions are collapsed in the time that the comparison takes).
-struct Collapser {
-  const axr_plan* p;
-  const TensorRec* last = nullptr;   // `c` is its answer
-  Collapsed c;
-
-  // For a tensor that is not compact.
-  const Collapsed& of(const TensorRec& t) {
-    const int64_t *shape = p->shape_of(t), *strides = p->strides_of(t);
-    const size_t bytes = static_cast<size_t>(t.ndim) * sizeof(int64_t);
-    const bool same = t.ndim > 2 && last && last->nbytes == t.nbytes && last->ndim == t.ndim &&
-                      (last->bits + 7) / 8 == (t.bits + 7) / 8 && std::memcmp(p->shape_of(*last), shape, bytes) == 0 &&
-                      std::memcmp(p->strides_of(*last), strides, bytes) == 0;
-    if (!same) collapse(t, shape, strides, (static_cast<uint64_t>(t.bits) + 7) / 8, &c);
-    last = &t;
-    return c;
-  }
-};
 
 // Largest power of two up to 16 that divides the run length.
 uint32_t granule_of(uint64_t run_bytes) {
@@ -1178,7 +1163,6 @@ int build_tables(axr_plan* p) {
   if (p->device_built) quiesce(p);   // the host tables replace the device-built ones at the next launch
   invalidate_tables(p);
   const Tunables& tn = tunables();
-  Collapser collapser{p};
   uint32_t rows = static_cast<uint32_t>(tn.tile_rows);
   if (rows == 0) {
     rows = 2;
@@ -1201,7 +1185,8 @@ int build_tables(axr_plan* p) {
       if (!t.has_strides || is_compact(p, t)) {
         uniform_runs = false;   // a compact tensor: not a bundle of strided views
       } else {
-        const Collapsed& c = collapser.of(t);
+        Collapsed c;
+        collapse(t, p->shape_of(t), p->strides_of(t), item_bytes(t), &c);
         uniform_runs = uniform_runs && c.nd != 0 && (common_run == 0 || c.run_bytes == common_run);
         common_run = c.run_bytes;
         run_tiles_only = run_tiles_only && (c.nd == 0 || c.run_bytes >= static_cast<uint64_t>(tn.gather_run_bytes));
@@ -1236,13 +1221,13 @@ int build_tables(axr_plan* p) {
       for (int32_t d = 0; d < t.ndim; ++d)
         if (strides[d] == 0 && shape[d] > 1) p->overlapping_dst = true;
     }
-    const Collapsed* c = nullptr;
+    Collapsed c;
     size_t nd = 0;
     uint64_t run_bytes = t.nbytes;
     if (strides && !is_compact(p, t)) {
-      c = &collapser.of(t);
-      nd = c->nd;
-      run_bytes = c->run_bytes;
+      collapse(t, shape, strides, item_bytes(t), &c);
+      nd = c.nd;
+      run_bytes = c.run_bytes;
     }
     int rc;
     if (t.device_type == kDLROCMHost) p->pinned_host_tensors = true;
@@ -1253,15 +1238,13 @@ int build_tables(axr_plan* p) {
       }
       rc = b.close_group();
       if (rc) return rc;
-      rc = b.add_strided(static_cast<uint32_t>(i), t.address, t.offset, nd ? c->extent : nullptr,
-                         nd ? c->stride : nullptr, nd, run_bytes);
+      rc = b.add_strided(static_cast<uint32_t>(i), t.address, t.offset, c.extent, c.stride, nd, run_bytes);
       if (rc) return rc;
       if (pad) p->segs.back().meta |= static_cast<uint32_t>(pad);
     } else if (t.device_type == kDLCPU) {
       rc = b.close_group();
       if (rc) return rc;
-      rc = b.add_host(static_cast<uint32_t>(i), t.address, t.offset, nd ? c->extent : nullptr,
-                      nd ? c->stride : nullptr, nd, run_bytes);
+      rc = b.add_host(static_cast<uint32_t>(i), t.address, t.offset, c.extent, c.stride, nd, run_bytes);
       if (rc) return rc;
       if (pad) {
         rc = b.add_seg(static_cast<uint32_t>(i), 0, end, 0, 1, kSegFillOnly);

@@ -128,22 +128,25 @@ constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4
 // blocks; in plain rows (along B, the dimension that is contiguous in the tensor, then along A, the one
 // that is contiguous in the payload) or in strips of kBlockStrip blocks along A.  Microseconds are pack +
 // unpack in turn, each pass on another of several copies, 1.2 GB in all.
-//  - Bundles up to 32 MiB, what the eight L2s hold, stay plain, partly written lines are completed there
-//    (28 MB, tensor rows on lines, 2-byte elements 29.6 plain / 30.8 skewed, 8-byte ones 27.7 / 29.3;
-//    34 MB of odd rows 41.9 / 40.0).
+//  - Bundles up to 28 MiB (8-byte elements 26), most of what the eight L2s hold, stay plain, partly written
+//    lines are completed there (7379 x 989 2-byte elements, twice, 29.2 MB, 26.3 plain / 28.4 skewed; 29.7 MB
+//    30.9 / 29.1, 34 MB of odd rows 41.9 / 40.0; 8-byte elements 26.4 MB 23.5 / 24.1, 28.3 MB 30.2 / 25.8; 400
+//    shapes: means 1.01 of plain at 26 MB, 0.94 at 28, 0.91 from 30 MB on).
 //  - Skewed blocks stage up to 1.5 times the elements they write, and twice as many where a row holds
 //    little more than a block: both extents have to reach skew_min_row (70 MB in rows of 101 2-byte
 //    elements 68 plain / 95 skewed, 100 matrices of 428 x 428 4-byte elements 62 / 68; one odd matrix of
 //    70 MB 82 / 67, 4- and 8-byte elements 72 / 62 and 70 / 59).
 //  - Strips bring blocks that share payload lines, neighbours along A, close to each other where B is long
-//    (70 MB of 211 x n 4-byte elements 82 in plain rows / 64, 16-byte ones 77 / 68; from 24 MiB on: 28 MB
-//    40 / 32) and where only the payload's rows straddle lines (34 MB of 8-byte elements 34.0 / 32.8).
+//    (70 MB of 211 x n 4-byte elements 82 in plain rows / 64, 16-byte ones 77 / 68; very long ones from
+//    24 MiB on: 72 x 16001 2-byte elements, 25.3 MB, 33.5 / 29.6, but 72 x 2003, 26.0 MB, 26.0 / 30.4, and
+//    30.9 MB 36.6 / 34.9) and where only the payload's rows straddle lines (34 MB of 8-byte elements 34.0 / 32.8).
 //    Elsewhere plain rows are ahead as long as the last-level cache holds most of a pass (45 MB, payload
 //    rows on lines and odd tensor rows, 39.1 / 40.8; 16-byte elements 3 to 10 % up to 70 MB); beyond that
 //    strips are (one odd matrix of 190 MB 198 / 188, 16-byte elements 188 / 171), save for 16-byte matrices
 //    that are flat (1.02) or have their payload rows on lines (1.03).  128 x 128 blocks of bytes gain
 //    nowhere, blocks shorter than a square one only with 16-byte elements (18 x n, 70 MB 82 / 66).
-constexpr uint64_t kLongMinPayload = 24u << 20, kSkewMinPayload = 32u << 20, kStripMinPayload = 96u << 20;
+constexpr uint64_t kLongMinPayload = 24u << 20, kStripMinPayload = 96u << 20, kLongRow = 6000;
+constexpr uint64_t skew_min_payload(uint32_t element_bytes) { return (element_bytes == 8 ? 26u : 28u) << 20; }
 constexpr uint32_t skew_min_row(uint32_t element_bytes) {
   return element_bytes == 4 ? 1024u : element_bytes == 8 ? 128u : 512u;
 }
@@ -156,8 +159,9 @@ constexpr BlockRule block_rule(uint32_t element_bytes, uint64_t ext_a, uint64_t 
   BlockRule rule;
   if (tensor_lines && payload_lines) return rule;
   const uint64_t row = skew_min_row(element_bytes);
-  const bool large = ext_a >= row && ext_b >= row && payload_bytes > kSkewMinPayload;
-  const bool long_b = element_bytes > 1 && ext_b >= row && ext_b / 4 >= ext_a && payload_bytes > kLongMinPayload;
+  const bool large = ext_a >= row && ext_b >= row && payload_bytes > skew_min_payload(element_bytes);
+  const bool long_b = element_bytes > 1 && ext_b >= row && ext_b / 4 >= ext_a &&
+                      payload_bytes > (ext_b >= kLongRow ? kLongMinPayload : skew_min_payload(element_bytes));
   const bool beyond_cache = payload_bytes > kStripMinPayload;
   if (element_bytes == 16) {
     rule.strips = long_b || (square && large && beyond_cache && !payload_lines && ext_b >= ext_a / 2);

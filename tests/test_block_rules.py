@@ -44,7 +44,7 @@ def rule(tmp_path_factory):
 
 def test_small_bundles_and_whole_lines_stay_plain(rule):
     cases = [(e, 2001, 2003, mib, t, p) for e in (1, 2, 4, 8, 16)
-             for mib, t, p in ((8, 0, 0), (32, 0, 0), (32, 1, 0), (200, 1, 1))]
+             for mib, t, p in ((8, 0, 0), (26, 0, 0), (28 - 2 * (e == 8), 1, 0), (200, 1, 1))]
     assert set(rule(cases)) == {(False, False, False)}
 
 
@@ -59,7 +59,7 @@ def test_short_rows_are_not_skewed(rule):
 
 def test_large_matrices_are_skewed_on_the_side_that_straddles_lines(rule):
     for e in (2, 4, 8):
-        for mib in (34, 134):
+        for mib in (29 - 2 * (e == 8), 34, 134):
             both, tensor_odd, payload_odd = rule([(e, 2001, 2003, mib, 0, 0), (e, 2048, 2003, mib, 0, 1),
                                                   (e, 2001, 2048, mib, 1, 0)])
             assert both[1:] == (True, True) and tensor_odd[1:] == (False, True) and payload_odd[1:] == (True, False)
@@ -68,9 +68,11 @@ def test_large_matrices_are_skewed_on_the_side_that_straddles_lines(rule):
 
 
 def test_strips_where_b_is_long_or_the_cache_is_left(rule):
-    """Long B: strips from 24 MiB on; else 16-byte elements, and flat ones at no size."""
-    assert all(r[0] for r in rule([(e, 211, 4001, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (25, 70, 190)]))
-    assert not any(r[0] for r in rule([(e, 211, 4001, 24, 0, 0) for e in (2, 4, 8, 16)]))
+    """Long B: strips from 28 MiB on (8-byte elements 26), very long ones from 24; else 16-byte elements, and flat ones at no
+    size."""
+    assert all(r[0] for r in rule([(e, 211, 4001, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (29, 70, 190)]))
+    assert all(r[0] for r in rule([(e, 211, 6007, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (25, 70, 190)]))
+    assert not any(r[0] for r in rule([(e, 211, b, mib, 0, 0) for e in (2, 4, 8, 16) for b, mib in ((4001, 26), (6007, 24))]))
     assert not any(r[0] for r in rule([(16, 1459, 1461, 70, 0, 0), (16, 30001, 801, 190, 0, 0), (16, 1456, 1461, 190, 0, 1),
                                        (1, 211, 90001, 190, 0, 0)]))
     assert rule([(16, 1459, 1461, 190, 0, 0)])[0][0]

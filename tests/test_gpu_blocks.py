@@ -1,4 +1,4 @@
-"""Transposed views at the edges of their blocks: skewed blocks (bundles beyond 24 MiB whose written
+"""Transposed views at the edges of their blocks: skewed blocks (bundles beyond 28 MiB whose written
 rows do not start on 64-byte boundaries) and few planes against interleaved elements.  Packed bytes
 against torch's compact copies, views scattered back into zeroed twins, nothing written beside them."""
 import pytest
@@ -46,7 +46,7 @@ def round_trip(pkg, gpu, stores, views_of, align, shift=0):
 def test_skewed_blocks(pkg, gpu, item, align, lead, shift):
     import torch
     edge = {1: 128, 2: 64}.get(item, 32)
-    shapes = [(2051, (26 << 20) // 2051 // item | 1), (edge, edge), (edge, edge + 1), (edge + 1, edge),
+    shapes = [(2051, (34 << 20) // 2051 // item | 1), (edge, edge), (edge, edge + 1), (edge + 1, edge),
               (2 * edge - 1, edge + 31), (3 * edge + 5, 2 * edge), (4 * edge, edge + 17), (edge - 1, 300), (777, 130)]
     stores = [storage(torch, gpu, r * c, item, lead, i) for i, (r, c) in enumerate(shapes)]
 

@@ -139,13 +139,16 @@ constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4
 //  - Strips bring blocks that share payload lines, neighbours along A, close to each other where B is long
 //    (70 MB of 211 x n 4-byte elements 82 in plain rows / 64, 16-byte ones 77 / 68; very long ones from
 //    24 MiB on: 72 x 16001 2-byte elements, 25.3 MB, 33.5 / 29.6, but 72 x 2003, 26.0 MB, 26.0 / 30.4, and
-//    30.9 MB 36.6 / 34.9) and where only the payload's rows straddle lines (34 MB of 8-byte elements 34.0 / 32.8).
+//    30.9 MB 36.6 / 34.9; beyond 192 MiB not where A is short and B not very long: 72 x 2003 2- and 4-byte
+//    elements are 9 % behind plain rows at 240 MB, level and 8 % ahead at 130 MB) and where only the
+//    payload's rows straddle lines (34 MB of 8-byte elements 34.0 / 32.8).
 //    Elsewhere plain rows are ahead as long as the last-level cache holds most of a pass (45 MB, payload
 //    rows on lines and odd tensor rows, 39.1 / 40.8; 16-byte elements 3 to 10 % up to 70 MB); beyond that
 //    strips are (one odd matrix of 190 MB 198 / 188, 16-byte elements 188 / 171), save for 16-byte matrices
 //    that are flat (1.02) or have their payload rows on lines (1.03).  128 x 128 blocks of bytes gain
 //    nowhere, blocks shorter than a square one only with 16-byte elements (18 x n, 70 MB 82 / 66).
-constexpr uint64_t kLongMinPayload = 24u << 20, kStripMinPayload = 96u << 20, kLongRow = 6000;
+constexpr uint64_t kLongMinPayload = 24u << 20, kStripMinPayload = 96u << 20, kThinMaxPayload = 192u << 20;
+constexpr uint64_t kLongRow = 6000, kThinRows = 128;
 constexpr uint64_t skew_min_payload(uint32_t element_bytes) { return (element_bytes == 8 ? 26u : 28u) << 20; }
 constexpr uint32_t skew_min_row(uint32_t element_bytes) {
   return element_bytes == 4 ? 1024u : element_bytes == 8 ? 128u : 512u;
@@ -160,7 +163,8 @@ constexpr BlockRule block_rule(uint32_t element_bytes, uint64_t ext_a, uint64_t 
   if (tensor_lines && payload_lines) return rule;
   const uint64_t row = skew_min_row(element_bytes);
   const bool large = ext_a >= row && ext_b >= row && payload_bytes > skew_min_payload(element_bytes);
-  const bool long_b = element_bytes > 1 && ext_b >= row && ext_b / 4 >= ext_a &&
+  const bool thin = ext_a < kThinRows && ext_b < kLongRow && payload_bytes > kThinMaxPayload;
+  const bool long_b = element_bytes > 1 && ext_b >= row && ext_b / 4 >= ext_a && !thin &&
                       payload_bytes > (ext_b >= kLongRow ? kLongMinPayload : skew_min_payload(element_bytes));
   const bool beyond_cache = payload_bytes > kStripMinPayload;
   if (element_bytes == 16) {

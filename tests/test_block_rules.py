@@ -73,6 +73,9 @@ def test_strips_where_b_is_long_or_the_cache_is_left(rule):
     assert all(r[0] for r in rule([(e, 211, 4001, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (29, 70, 190)]))
     assert all(r[0] for r in rule([(e, 211, 6007, mib, 0, 0) for e in (2, 4, 8, 16) for mib in (25, 70, 190)]))
     assert not any(r[0] for r in rule([(e, 211, b, mib, 0, 0) for e in (2, 4, 8, 16) for b, mib in ((4001, 26), (6007, 24))]))
+    # a short A beyond 192 MiB: only with a very long B
+    assert [r for e in (2, 4, 8) for r in rule([(e, 72, 4001, 193, 0, 0)])] == [(False, False, False)] * 3
+    assert all(r[0] for r in rule([(e, a, b, mib, 0, 0) for e in (2, 4, 8) for a, b, mib in ((72, 6007, 230), (72, 4001, 192), (150, 4001, 230))]))
     assert not any(r[0] for r in rule([(16, 1459, 1461, 70, 0, 0), (16, 30001, 801, 190, 0, 0), (16, 1456, 1461, 190, 0, 1),
                                        (1, 211, 90001, 190, 0, 0)]))
     assert rule([(16, 1459, 1461, 190, 0, 0)])[0][0]

@@ -105,6 +105,9 @@ constexpr uint32_t kModeElements = 1;   // tile covers packed bytes; lanes decod
 constexpr uint32_t kModeTranspose = 2;  // plain blocks in plain rows
 constexpr uint32_t kModeWalked = 3;     // skewed blocks, or blocks in strips (see block_rule)
 constexpr uint32_t kModePlanes = 4;     // few planes against the same elements interleaved
+// Kernels are built for the segments a bundle has: runs and groups of short tensors only, views of one
+// mode above kModeRunTiles only (the kind is that mode), or anything.
+constexpr uint32_t kKindRuns = 0, kKindAny = 5;
 
 // Transposed blocks are T x T elements; a block row is 128 bytes (eight 16-byte
 // vectors) for elements up to 4 bytes and 256 bytes for wider ones, so that a
@@ -320,6 +323,7 @@ struct LaunchConfig {
   uint32_t seg_shift = 0;   // wave_seg has one entry per 2^seg_shift tiles
   uint32_t nontemporal = 3;   // bit 0: tensor-side accesses, bit 1: payload-side accesses
   bool elements = false;   // some segment uses kModeElements or is transposed
+  uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (transposed tiles only)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
                            // multiple of 8 such runs)

@@ -71,6 +71,19 @@ __device__ __forceinline__ gbytes as_global(uint64_t address) {
   return reinterpret_cast<gbytes>(address);
 }
 
+// A function that is not inlined gets its arguments in vector registers, whether or not they are the
+// same in every lane.  These say that they are: tables are then read by scalar loads, branches are
+// scalar branches instead of lane masks, and addresses have a scalar base.
+__device__ __forceinline__ uint64_t uniform(uint64_t v) {
+  return static_cast<uint64_t>(uniform(static_cast<uint32_t>(v))) |
+         static_cast<uint64_t>(uniform(static_cast<uint32_t>(v >> 32))) << 32;
+}
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+  if constexpr (sizeof(T*) == 8) return reinterpret_cast<T*>(uniform(reinterpret_cast<uint64_t>(p)));
+  else return reinterpret_cast<T*>(uniform(reinterpret_cast<uint32_t>(p)));
+}
+
 // Wave-cooperative copy of one tile.  src, dst and the length are
 // wave-uniform, lane_off is lane * 16.  A full tile is ROWS loads then ROWS
 // stores per lane.
@@ -375,6 +388,8 @@ __device__ __forceinline__ void element_tile(uint64_t seg_ptr, uint64_t run_byte
 #define AXR_LDS __attribute__((address_space(3)))
 typedef AXR_LDS uint8_t* lbytes;
 
+// ---------------------------------------------------------------- rows
+//
 template <uint32_t E> struct unit_of;
 template <> struct unit_of<1> { typedef uint8_t type; };
 template <> struct unit_of<2> { typedef uint16_t type; };
@@ -952,7 +967,7 @@ __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t 
 // One copy per MODE: with the walk in strips and the choice of block routine in
 // the plain one's way, however predictable, 4 KiB blocks took 3 to 8 % longer.
 template <bool PACK, uint32_t MODE>
-__device__ __attribute__((noinline)) void transpose_tile(uint64_t seg_ptr, dims_table dm, gbytes pay,
+__device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, gbytes pay,
                                                uint32_t q, lbytes lds, uint32_t lane,
                                                uint32_t nt_bits) {
   const uint32_t E = dm->granule;
@@ -1093,13 +1108,9 @@ __device__ __attribute__((noinline)) void group_tile(const AXR_CONST GroupHead* 
   typedef uint16_t __attribute__((aligned(1))) loose16;
   constexpr uint32_t R = kGroupMaxSlots / kWaveLanes;
   static_assert(R == 2, "two masks per group head");
-  {
-    // the block's address is the same in every lane: say so, and the head arrives by scalar load
-    const uint64_t a = reinterpret_cast<uint64_t>(head);
-    head = reinterpret_cast<const AXR_CONST GroupHead*>(
-        static_cast<uint64_t>(uniform(static_cast<uint32_t>(a))) |
-        static_cast<uint64_t>(uniform(static_cast<uint32_t>(a >> 32))) << 32);
-  }
+  head = uniform(head);
+  payload = uniform(payload);
+  delta = uniform(delta);
   // Lane l holds member l % 16's record (only lanes 0..15 are ever asked for theirs).  Every lane
   // loads, so that no branch stands between this load and the loads of the head: a load under a
   // lane mask is waited for inside its branch, which put two memory round trips in a row here.
@@ -1236,18 +1247,39 @@ __device__ __attribute__((noinline)) void group_tile(const AXR_CONST GroupHead* 
   }
 }
 
+// A tile copy whose hints are known at run time only (bit 0 tensor side, bit 1 payload side).
+template <bool PACK, uint32_t ROWS, bool NTT, bool NTP>
+__device__ __forceinline__ void copy_tile(gbytes tensor, gbytes payload, uint64_t left, uint32_t lane, uint32_t lane_off) {
+  if constexpr (PACK) wave_copy<ROWS, NTT, NTP>(tensor, payload, left, lane, lane_off);
+  else wave_copy<ROWS, NTP, NTT>(payload, tensor, left, lane, lane_off);
+}
+template <bool PACK, uint32_t ROWS>
+__device__ __forceinline__ void copy_tile_hinted(gbytes tensor, gbytes payload, uint64_t left, uint32_t lane,
+                                                 uint32_t lane_off, uint32_t nt_bits) {
+  // (the empty asm statements keep the arms apart, or the optimizer merges them and drops the hints)
+  switch (nt_bits & 3u) {
+    case 0: copy_tile<PACK, ROWS, false, false>(tensor, payload, left, lane, lane_off); break;
+    case 1: asm volatile(""); copy_tile<PACK, ROWS, true, false>(tensor, payload, left, lane, lane_off); asm volatile(""); break;
+    case 2: asm volatile(" "); copy_tile<PACK, ROWS, false, true>(tensor, payload, left, lane, lane_off); asm volatile(" "); break;
+    default: asm volatile("  "); copy_tile<PACK, ROWS, true, true>(tensor, payload, left, lane, lane_off); asm volatile("  "); break;
+  }
+}
+
 // The whole pack or unpack of a bundle: every wavefront finds the segment of its
 // first tile through the tile-block index and walks forward from there.  `wg` is the
 // workgroup's index within this bundle's share of the grid; `a.tensor_delta` is added to
 // every tensor-side address (one plan serves tensors of the same geometry elsewhere).
-template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, bool ELEMENTS>
+// KIND: what segments the bundle may have.  kKindRuns: runs and groups of short tensors, with the hints
+// NTT and NTP; kKindAny: every mode, hints from `nt_bits`; otherwise the one mode that all of them have.
+template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, uint32_t KIND>
 __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
                                             const AXR_CONST uint32_t* wave_seg, gbytes payload,
                                             const KernelArgs& a, uint32_t wg, uint32_t lds_per_wave,
                                             uint32_t nt_bits) {
+  constexpr bool runs = KIND == kKindRuns || KIND == kKindAny;   // runs, groups and fills may occur
   constexpr uint32_t kTile = ROWS * kRowBytes;
-  const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
-  const uint32_t lane_off = lane * kVecBytes;
+  uint32_t lane = threadIdx.x & (kWaveLanes - 1);
+  uint32_t lane_off = lane * kVecBytes;
   if (a.xcd_remap) {
     // consecutive workgroup ids land on consecutive dies; hand every die runs of consecutive
     // workgroup indices, in turn, so that neighbouring tiles share an L2
@@ -1267,7 +1299,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   const uint32_t t_end =
       (a.ntiles - t > a.tiles_per_wave) ? t + a.tiles_per_wave : a.ntiles;
   const uint64_t delta = static_cast<uint64_t>(a.tensor_delta);
-  if (a.seg_shift == kGroupBlocksShift) {
+  if (runs && a.seg_shift == kGroupBlocksShift) {
     // a bundle of group tiles only: tile t's block lies at a fixed stride behind `dims`
     const AXR_CONST uint8_t* blocks = reinterpret_cast<const AXR_CONST uint8_t*>(dims);
     for (; t < t_end; ++t)
@@ -1295,12 +1327,15 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
       seg_end = segs[s + 1].tile_begin;
       continue;
     }
+    // What a tile works out from its lane and its tables is worked out per tile: kept over the loop, which
+    // few wavefronts go round twice, the many routines' constants take over a hundred more registers.
+    if constexpr (KIND != kKindRuns) asm volatile("" : "+v"(lane), "+v"(lane_off), "+s"(nt_bits), "+s"(dims));
     const uint32_t q = t - seg_begin;
     const uint32_t pad = seg_meta & kSegPadMask;
     const uint32_t dsel = seg_meta >> kSegDimsShift;
     const bool last = (t + 1 == seg_end);
     gbytes pay = payload + seg_off;
-    if (dsel == 0) {
+    if (runs && dsel == 0) {
       // One contiguous run.  Its first `head` bytes (fewer than 128) are peeled off and
       // moved by tile 0 on top of its own range, so that every tile starts on a 128-byte
       // line of the side that is written.
@@ -1309,24 +1344,27 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
       const uint64_t boff = head + static_cast<uint64_t>(q) * kTile;
       const uint64_t left = run > boff ? run - boff : 0;
       gbytes ten = as_global(seg_ptr);
-      if constexpr (PACK) {
-        if (head && q == 0) wave_copy_partial<1, NTT, NTP>(ten, pay, head, lane, lane_off);
-        wave_copy<ROWS, NTT, NTP>(ten + boff, pay + boff, left, lane, lane_off);
-        if (last && pad) wave_zero(pay + run, pad, lane);
-      } else {
-        if (head && q == 0) wave_copy_partial<1, NTP, NTT>(pay, ten, head, lane, lane_off);
-        wave_copy<ROWS, NTP, NTT>(pay + boff, ten + boff, left, lane, lane_off);
+      if (head && q == 0) {
+        if constexpr (KIND == kKindAny) wave_copy_partial<1, false, false>(PACK ? ten : pay, PACK ? pay : ten, head, lane, lane_off);
+        else if constexpr (PACK) wave_copy_partial<1, NTT, NTP>(ten, pay, head, lane, lane_off);
+        else wave_copy_partial<1, NTP, NTT>(pay, ten, head, lane, lane_off);
       }
-    } else if (dsel == kSegFillOnly) {
+      if constexpr (KIND == kKindAny) copy_tile_hinted<PACK, ROWS>(ten + boff, pay + boff, left, lane, lane_off, nt_bits);
+      else copy_tile<PACK, ROWS, NTT, NTP>(ten + boff, pay + boff, left, lane, lane_off);
+      if constexpr (PACK) {
+        if (last && pad) wave_zero(pay + run, pad, lane);
+      }
+    } else if (runs && dsel == kSegFillOnly) {
       if constexpr (PACK) wave_zero(pay, pad, lane);
-    } else if (dsel == kSegGroup) {
+    } else if (runs && dsel == kSegGroup) {
       // seg_ptr is an offset into the table block here, not a tensor address
       const AXR_CONST GroupHead* head = reinterpret_cast<const AXR_CONST GroupHead*>(
           reinterpret_cast<const AXR_CONST uint8_t*>(segs) + (seg_ptr - delta));
       group_tile<PACK>(head, payload, delta, lane);
     } else {
       dims_table dm = dims + (dsel - 1);
-      if (dm->mode == kModeRunTiles) {
+      const uint32_t mode = runs ? dm->mode : KIND;
+      if (runs && mode == kModeRunTiles) {
         const uint32_t tpr = dm->tiles_per_run;
         const uint32_t tpr_log2 = dm->granule;   // run-tile mode: 1 + log2(tpr) when a power of two
         const uint32_t run = tpr_log2 ? q >> (tpr_log2 - 1) : q / tpr;
@@ -1335,22 +1373,15 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         const uint64_t left = seg_run - boff;
         gbytes ten = as_global(seg_ptr) + run_offset(dm, run) + boff;
         gbytes p = pay + static_cast<uint64_t>(run) * seg_run + boff;
-        if constexpr (PACK) {
-          wave_copy<ROWS, NTT, NTP>(ten, p, left, lane, lane_off);
-        } else {
-          wave_copy<ROWS, NTP, NTT>(p, ten, left, lane, lane_off);
-        }
-      } else if constexpr (ELEMENTS) {
-        const uint32_t mode = dm->mode;
-        if (mode >= kModeTranspose) {
-          extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
-          lbytes lds = (lbytes)lds_slices + (threadIdx.x >> 6) * lds_per_wave;
-          if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
-          else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
-          else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
-        } else {
-          element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
-        }
+        if constexpr (KIND == kKindAny) copy_tile_hinted<PACK, ROWS>(ten, p, left, lane, lane_off, nt_bits);
+        else copy_tile<PACK, ROWS, NTT, NTP>(ten, p, left, lane, lane_off);
+      } else if constexpr (KIND != kKindRuns) {
+        extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
+        lbytes lds = (lbytes)lds_slices + uniform(threadIdx.x >> 6) * lds_per_wave;
+        if (mode == kModeElements) element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
+        else if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+        else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+        else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
       }
       if constexpr (PACK) {
         if (last && pad) wave_zero(pay + dm->nbytes, pad, lane);
@@ -1361,19 +1392,19 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
 }
 
 // Tables in device memory (uploaded once per plan).
-// At least four waves per SIMD (at most 128 VGPRs): the streaming instantiations
-// use far fewer, and the general ones sit just around that limit, where one
-// register too many would cost a quarter of the occupancy.
-template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, bool ELEMENTS>
-__global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? kMaxElementThreads : kMaxThreadsPerWorkgroup) void bundle_kernel(
-    const Seg* segs_arg, const Dims* dims_arg, const uint32_t* wave_seg_arg, uint8_t* payload_arg,
-    uint32_t ntiles, uint32_t tiles_per_wave, uint32_t xcd_remap, uint32_t geometry, int64_t tensor_delta) {
-  // Scalar arguments (not one struct) so that the compiler can preload them into SGPRs at
-  // dispatch instead of fetching the kernarg segment first.  Fourteen dwords are preloaded,
-  // which is why the LDS bytes per wavefront (bits 0-16), the hints with the wavefronts per
-  // workgroup (bits 17-23, the argument bundle_body takes) and the tile-block shift (bits
-  // 24-31) share one of them: the address delta then fits in as well, and no wavefront waits
-  // for a kernel-argument load before it can form its first tensor address.
+// Scalar arguments (not one struct) so that the compiler can preload them into SGPRs at
+// dispatch instead of fetching the kernarg segment first.  Fourteen dwords are preloaded,
+// which is why the LDS bytes per wavefront (bits 0-16), the hints with the wavefronts per
+// workgroup (bits 17-23, the argument bundle_body takes) and the tile-block shift (bits
+// 24-31) share one of them: the address delta then fits in as well, and no wavefront waits
+// for a kernel-argument load before it can form its first tensor address.
+#define AXR_BUNDLE_PARAMETERS                                                                       \
+  const Seg *segs_arg, const Dims *dims_arg, const uint32_t *wave_seg_arg, uint8_t *payload_arg, uint32_t ntiles, \
+      uint32_t tiles_per_wave, uint32_t xcd_remap, uint32_t geometry, int64_t tensor_delta
+#define AXR_BUNDLE_ARGUMENTS \
+  segs_arg, dims_arg, wave_seg_arg, payload_arg, ntiles, tiles_per_wave, xcd_remap, geometry, tensor_delta
+template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, uint32_t KIND>
+__device__ __forceinline__ void bundle_from_arguments(AXR_BUNDLE_PARAMETERS) {
   const uint32_t lds_per_wave = geometry & 0x1ffffu;
   const uint32_t nt_bits = (geometry >> 17 & 3u) | (geometry >> 19 & 0x1fu) << 8;
   KernelArgs a;
@@ -1382,12 +1413,36 @@ __global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? 
   a.xcd_remap = xcd_remap;
   a.seg_shift = geometry >> 24;
   a.tensor_delta = tensor_delta;
-  bundle_body<PACK, ROWS, NTT, NTP, ELEMENTS>(
+  bundle_body<PACK, ROWS, NTT, NTP, KIND>(
       reinterpret_cast<seg_table>(reinterpret_cast<uintptr_t>(segs_arg)),
       reinterpret_cast<dims_table>(reinterpret_cast<uintptr_t>(dims_arg)),
       reinterpret_cast<const AXR_CONST uint32_t*>(reinterpret_cast<uintptr_t>(wave_seg_arg)),
       reinterpret_cast<gbytes>(reinterpret_cast<uintptr_t>(payload_arg)), a, blockIdx.x, lds_per_wave,
       nt_bits);
+}
+
+// Bundles of runs and of groups of short tensors.
+template <bool PACK, uint32_t ROWS, bool NTT, bool NTP>
+__global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(kMaxThreadsPerWorkgroup) void bundle_kernel(
+    AXR_BUNDLE_PARAMETERS) {
+  bundle_from_arguments<PACK, ROWS, NTT, NTP, kKindRuns>(AXR_BUNDLE_ARGUMENTS);
+}
+
+// Bundles with views whose tiles are more than copies of runs: all of one mode, or kKindAny.  What such a
+// tile waits for is memory, so a compute unit should hold many of them, and how many it holds is a matter of
+// registers: built together as functions that are called, the routines took 120 (16 wavefronts on a compute
+// unit) and read their tables through vector loads; a kernel for each of them takes 43 to 87 and reads them by
+// scalar loads.  256 uint8 images of 224 x 224 x 3, pack + unpack, 32.3 -> 30.1 us, four odd transposed bf16
+// matrices 112.7 -> 108.5, 2^18 rows of 256 bytes 50.4 -> 48.5.  Wavefronts per SIMD that the registers are
+// held to: LDS allows 4 to 5 for blocks, and 23 on a compute unit for planes; plain blocks are
+// 1 % faster with the registers of 4 than with those of 7, kKindAny would spill at 6.
+constexpr uint32_t waves_of_kind(uint32_t kind, uint32_t rows) {
+  return kind == kModeElements ? 8 : kind == kModePlanes ? 6 : kind == kKindAny && rows <= 8 ? 5 : 4;
+}
+template <bool PACK, uint32_t ROWS, uint32_t KIND>
+__global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, ROWS), KIND == kModeTranspose ? 4 : 8)))
+__launch_bounds__(kMaxElementThreads) void views_kernel(AXR_BUNDLE_PARAMETERS) {
+  bundle_from_arguments<PACK, ROWS, false, false, KIND>(AXR_BUNDLE_ARGUMENTS);
 }
 
 // Several bundles in ONE launch: the grid is cut into consecutive workgroup ranges, one per
@@ -1413,8 +1468,9 @@ __device__ __forceinline__ uint32_t at_or_beyond(uint32_t wg, uint32_t begin) {
 // them; the rest of its job's descriptor (payload address, address delta, strided-view table) is
 // read from the table meanwhile.  Launches of more jobs, or of jobs whose wavefronts take several
 // tiles, read the descriptor first (first workgroups of jobs that do not exist are kNoJobBegin).
-template <uint32_t ROWS, bool NTT, bool NTP, bool ELEMENTS>
-__global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? kMaxElementThreads : kMaxThreadsPerWorkgroup) void bundle_jobs_kernel(
+template <uint32_t ROWS, bool NTT, bool NTP, uint32_t KIND>
+__global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, ROWS))))
+__launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThreads) void bundle_jobs_kernel(
     uint32_t head, uint32_t nt_bits, uint32_t b1, uint32_t ntiles0, uint64_t index0, uint64_t segs0,
     uint64_t index1, uint64_t segs1, uint32_t ntiles1, uint32_t lds_per_wave, JobTable jobs_arg) {
   (void)jobs_arg;
@@ -1474,9 +1530,9 @@ __global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? 
   gbytes payload = reinterpret_cast<gbytes>(d->payload);
   const uint32_t local = in_turn ? wg >> 1 : wg - begin;
   if (unpack) {   // workgroup-uniform
-    bundle_body<false, ROWS, NTT, NTP, ELEMENTS>(segs, dims, wave_seg, payload, a, local, lds_per_wave, nt_bits);
+    bundle_body<false, ROWS, NTT, NTP, KIND>(segs, dims, wave_seg, payload, a, local, lds_per_wave, nt_bits);
   } else {
-    bundle_body<true, ROWS, NTT, NTP, ELEMENTS>(segs, dims, wave_seg, payload, a, local, lds_per_wave, nt_bits);
+    bundle_body<true, ROWS, NTT, NTP, KIND>(segs, dims, wave_seg, payload, a, local, lds_per_wave, nt_bits);
   }
 }
 
@@ -1494,8 +1550,9 @@ struct InlineScalars {   // mirrors the argument list of bundle_kernel_inline
 constexpr uint32_t kInlineTablesOffset = __builtin_offsetof(InlineScalars, tables);
 static_assert(kInlineTablesOffset == 48 && alignof(InlineTables) == 16, "kernarg layout");
 
-template <bool PACK, bool ELEMENTS>
-__global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? kMaxElementThreads : kMaxThreadsPerWorkgroup) void bundle_kernel_inline(
+template <bool PACK, uint32_t KIND>
+__global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, 2))))
+__launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThreads) void bundle_kernel_inline(
     uint8_t* payload_arg, uint32_t ntiles, uint32_t tiles_per_wave, uint32_t xcd_remap,
     uint32_t seg_shift, uint32_t lds_per_wave, uint32_t nt_bits, uint32_t dims_at, uint32_t wave_at,
     InlineTables tables) {
@@ -1510,7 +1567,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(ELEMENTS ? 
   a.seg_shift = seg_shift;
   a.tensor_delta = 0;
   // tensor side streaming, payload side cacheable: what small bundles use
-  bundle_body<PACK, 2, true, false, ELEMENTS>(
+  bundle_body<PACK, 2, true, false, KIND>(
       reinterpret_cast<seg_table>(base + kInlineTablesHead),
       reinterpret_cast<dims_table>(base + kInlineTablesHead + dims_at),
       reinterpret_cast<const AXR_CONST uint32_t*>(base + kInlineTablesHead + wave_at),
@@ -1802,19 +1859,30 @@ int launch_rows(const KernelArgs& args, const LaunchConfig& cfg, hipStream_t str
   const uint32_t geometry = cfg.lds_per_wave | (cfg.nontemporal & 3u) << 17 |
                             (cfg.threads / kWaveLanes) << 19 | args.seg_shift << 24;
 #define AXR_ARGS args.segs, args.dims, args.wave_seg, args.payload, args.ntiles, args.tiles_per_wave, args.xcd_remap, geometry, args.tensor_delta
-#define AXR_LAUNCH(NTT, NTP, EL) \
-  hipLaunchKernelGGL((bundle_kernel<PACK, ROWS, NTT, NTP, EL>), grid, block, lds_bytes, stream, AXR_ARGS)
-  // cfg.elements: strided tensors with short runs or transpositions are present
-  switch ((cfg.elements ? 4u : 0u) | (cfg.nontemporal & 3u)) {   // bit 0: tensor side, bit 1: payload side
-    case 0: AXR_LAUNCH(false, false, false); break;
-    case 1: AXR_LAUNCH(true, false, false); break;
-    case 2: AXR_LAUNCH(false, true, false); break;
-    case 3: AXR_LAUNCH(true, true, false); break;
-    case 4: AXR_LAUNCH(false, false, true); break;
-    case 5: AXR_LAUNCH(true, false, true); break;
-    case 6: AXR_LAUNCH(false, true, true); break;
-    default: AXR_LAUNCH(true, true, true); break;
+#define AXR_VIEWS(KIND) hipLaunchKernelGGL((views_kernel<PACK, ROWS, KIND>), grid, block, lds_bytes, stream, AXR_ARGS)
+#define AXR_LAUNCH(NTT, NTP) \
+  hipLaunchKernelGGL((bundle_kernel<PACK, ROWS, NTT, NTP>), grid, block, lds_bytes, stream, AXR_ARGS)
+  if (cfg.elements) {   // short runs or transpositions are present
+    if constexpr (ROWS == 2) {
+      switch (cfg.kind) {
+        case kModeElements: AXR_VIEWS(kModeElements); break;
+        case kModeTranspose: AXR_VIEWS(kModeTranspose); break;
+        case kModeWalked: AXR_VIEWS(kModeWalked); break;
+        case kModePlanes: AXR_VIEWS(kModePlanes); break;
+        default: AXR_VIEWS(kKindAny); break;
+      }
+    } else {
+      AXR_VIEWS(kKindAny);
+    }
+  } else {
+    switch (cfg.nontemporal & 3u) {   // bit 0: tensor side, bit 1: payload side
+      case 0: AXR_LAUNCH(false, false); break;
+      case 1: AXR_LAUNCH(true, false); break;
+      case 2: AXR_LAUNCH(false, true); break;
+      default: AXR_LAUNCH(true, true); break;
+    }
   }
+#undef AXR_VIEWS
 #undef AXR_LAUNCH
 #undef AXR_ARGS
   return check_hip(hipGetLastError(), "bundle kernel launch");
@@ -1889,28 +1957,28 @@ int launch_bundle_jobs(const JobTable& jobs, const LaunchConfig& cfg, void* stre
                         (jobs.job[0].unpack ? 0x200u : 0u) | (jobs.count > 1 && jobs.job[1].unpack ? 0x400u : 0u) |
                         (one_tile_each ? 0x800u : 0u) |
                         (jobs.job[0].seg_shift & 0xffu) << 16 | (jobs.count > 1 ? jobs.job[1].seg_shift & 0xffu : 0u) << 24;
-#define AXR_JOBS(ROWS, NTT, NTP, EL) \
-  hipLaunchKernelGGL((bundle_jobs_kernel<ROWS, NTT, NTP, EL>), grid, block, lds_bytes, s, head, jobs.nt_bits,   \
+#define AXR_JOBS(ROWS, NTT, NTP, KIND) \
+  hipLaunchKernelGGL((bundle_jobs_kernel<ROWS, NTT, NTP, KIND>), grid, block, lds_bytes, s, head, jobs.nt_bits, \
                      jobs.begins[1], jobs.job[0].ntiles, jobs.job[0].wave_seg, jobs.job[0].segs,               \
                      jobs.job[1].wave_seg, jobs.job[1].segs, jobs.job[1].ntiles, jobs.lds_per_wave, jobs)
-#define AXR_JOBS_NT(ROWS, EL)                                    \
-  switch (cfg.nontemporal & 3u) {                                \
-    case 0: AXR_JOBS(ROWS, false, false, EL); break;             \
-    case 1: AXR_JOBS(ROWS, true, false, EL); break;              \
-    case 2: AXR_JOBS(ROWS, false, true, EL); break;              \
-    default: AXR_JOBS(ROWS, true, true, EL); break;              \
+#define AXR_JOBS_NT(ROWS)                                               \
+  switch (cfg.nontemporal & 3u) {                                       \
+    case 0: AXR_JOBS(ROWS, false, false, kKindRuns); break;             \
+    case 1: AXR_JOBS(ROWS, true, false, kKindRuns); break;              \
+    case 2: AXR_JOBS(ROWS, false, true, kKindRuns); break;              \
+    default: AXR_JOBS(ROWS, true, true, kKindRuns); break;              \
   }
   if (cfg.elements) {
-    // bundles with short strided runs or transpositions: the default tile only
+    // bundles with short strided runs or transpositions: the default tile only, hints at run time
     if (cfg.tile_rows != 2) return fail(AXR_ERR_INVALID, "element-mode jobs need 2 KiB tiles");
-    AXR_JOBS_NT(2, true)
+    AXR_JOBS(2, true, true, kKindAny);
   } else {
     switch (cfg.tile_rows) {
-      case 1: AXR_JOBS_NT(1, false) break;
-      case 2: AXR_JOBS_NT(2, false) break;
-      case 4: AXR_JOBS_NT(4, false) break;
-      case 8: AXR_JOBS_NT(8, false) break;
-      case 16: AXR_JOBS_NT(16, false) break;
+      case 1: AXR_JOBS_NT(1) break;
+      case 2: AXR_JOBS_NT(2) break;
+      case 4: AXR_JOBS_NT(4) break;
+      case 8: AXR_JOBS_NT(8) break;
+      case 16: AXR_JOBS_NT(16) break;
       default: return fail(AXR_ERR_INVALID, "tile_rows must be 1, 2, 4, 8 or 16");
     }
   }
@@ -1939,14 +2007,14 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
   const dim3 grid(cfg.workgroups), block(cfg.threads);
   const uint32_t lds_bytes = cfg.elements ? cfg.lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define AXR_INLINE_LAUNCH(PACK, EL)                                                              \
-  hipLaunchKernelGGL((bundle_kernel_inline<PACK, EL>), grid, block, lds_bytes, s, args.payload,   \
+#define AXR_INLINE_LAUNCH(PACK, KIND)                                                             \
+  hipLaunchKernelGGL((bundle_kernel_inline<PACK, KIND>), grid, block, lds_bytes, s, args.payload,  \
                      args.ntiles, args.tiles_per_wave, args.xcd_remap, args.seg_shift,            \
                      cfg.lds_per_wave, hint_argument(cfg), dims_at, wave_at, tables)
-  if (pack) {
-    if (cfg.elements) AXR_INLINE_LAUNCH(true, true); else AXR_INLINE_LAUNCH(true, false);
+  if (!cfg.elements) {
+    if (pack) AXR_INLINE_LAUNCH(true, kKindRuns); else AXR_INLINE_LAUNCH(false, kKindRuns);
   } else {
-    if (cfg.elements) AXR_INLINE_LAUNCH(false, true); else AXR_INLINE_LAUNCH(false, false);
+    if (pack) AXR_INLINE_LAUNCH(true, kKindAny); else AXR_INLINE_LAUNCH(false, kKindAny);
   }
 #undef AXR_INLINE_LAUNCH
   return check_hip(hipGetLastError(), "bundle kernel launch (inline tables)");

@@ -883,6 +883,17 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
     ragged_rows = ragged_rows || (dm.mode == kModeElements && dm.lanes_per_run != 0);
     blocks = blocks || dm.mode >= kModeTranspose;
   }
+  p->cfg.kind = kKindAny;
+  if (p->cfg.elements && rows == 2) {   // the kernels of a single mode are built for the default tile
+    const uint32_t mode = p->dims[0].mode;
+    bool one = mode != kModeRunTiles;
+    for (const Dims& dm : p->dims) one = one && dm.mode == mode;
+    for (size_t i = 0; i < nseg && one; ++i) {
+      const uint32_t dsel = p->segs[i].meta >> kSegDimsShift;
+      one = dsel != 0 && dsel != kSegFillOnly && dsel != kSegGroup;
+    }
+    if (one) p->cfg.kind = mode;
+  }
   if (p->cfg.elements) p->cfg.threads = std::min(p->cfg.threads, kMaxElementThreads);
   // Short rows that are no multiple of 16 bytes (lane slots left idle behind each run) run 2.5-5 %
   // faster in workgroups of one wavefront (rows of 250 B: 4.97 -> 5.22 TB/s, of 100 B: 3.06 ->
@@ -2188,6 +2199,7 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: the jobs' grids exceed one launch");
       wg += p->cfg.workgroups;
       cfg.elements = cfg.elements || p->cfg.elements;
+      if (p->cfg.kind != cfg.kind) cfg.kind = kKindAny;   // (also the kind of a plan without such views)
       cfg.lds_per_wave = std::max(cfg.lds_per_wave, p->cfg.lds_per_wave);
     }
     table.count = static_cast<uint32_t>(end - i);

@@ -101,13 +101,15 @@ constexpr uint32_t group_pad_slots(uint32_t pad) { return pad >= kVecBytes ? (pa
 
 constexpr uint32_t kModeRunTiles = 0;   // every tile is a piece of one contiguous run
 constexpr uint32_t kModeElements = 1;   // tile covers packed bytes; lanes decode granules
+// kModeRows and above: the tile goes through LDS
+constexpr uint32_t kModeRows = 2;       // tile covers whole runs, cut on each side's own 64-byte boundaries
 // kModeTranspose and above: the tile is a block transposed through LDS
-constexpr uint32_t kModeTranspose = 2;  // plain blocks in plain rows
-constexpr uint32_t kModeWalked = 3;     // skewed blocks, or blocks in strips (see block_rule)
-constexpr uint32_t kModePlanes = 4;     // few planes against the same elements interleaved
+constexpr uint32_t kModeTranspose = 3;  // plain blocks in plain rows
+constexpr uint32_t kModeWalked = 4;     // skewed blocks, or blocks in strips (see block_rule)
+constexpr uint32_t kModePlanes = 5;     // few planes against the same elements interleaved
 // Kernels are built for the segments a bundle has: runs and groups of short tensors only, views of one
 // mode above kModeRunTiles only (the kind is that mode), or anything.
-constexpr uint32_t kKindRuns = 0, kKindAny = 5;
+constexpr uint32_t kKindRuns = 0, kKindAny = 6;
 
 // Transposed blocks are T x T elements; a block row is 128 bytes (eight 16-byte
 // vectors) for elements up to 4 bytes and 256 bytes for wider ones, so that a
@@ -231,12 +233,30 @@ constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t 
 }
 constexpr uint32_t kMaxBatchDims = 4;
 constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (measured: 8 KiB beats 2, 4 and 16)
+// kModeRows: the 16-byte slots a row may need, in whole 64-byte units, when its first byte lies up to
+// `start` bytes behind one; the slots a lane moves (see rows_moves for the sizes); LDS for the rows of a tile.
+constexpr uint32_t kUnitBytes = 64;
+constexpr uint32_t kMaxRowSlots = 4;
+constexpr uint64_t kMaxRowBytes = kMaxRowSlots * kRowBytes / 2 - kUnitBytes;   // two rows to a tile at least
+constexpr uint32_t row_slots(uint64_t run_bytes, uint32_t start) {
+  return static_cast<uint32_t>((start + run_bytes + kUnitBytes - 1) / kUnitBytes * (kUnitBytes / kVecBytes));
+}
+// `mixed`: next to tensors that are moved otherwise.  The kernel for those holds fewer wavefronts, and larger
+// tiles make up for it (2^18 rows of 128 bytes at 131 34.9 us for pack + unpack before, 39.0 with two slots per
+// lane, 33.9 with four; of 666 at 1554 159 / 164 / 142).
+constexpr uint32_t row_slots_per_lane(uint32_t slots, bool mixed) {
+  return mixed || slots <= 4 || 2 * slots > 3 * kWaveLanes ? kMaxRowSlots : 2 * slots <= 2 * kWaveLanes ? 2u : 3u;
+}
+constexpr uint32_t rows_lds_bytes(uint32_t rows, uint64_t run_bytes) {
+  return static_cast<uint32_t>(rows * run_bytes) + kUnitBytes;
+}
 
 struct Dims {             // 176 bytes, one per strided segment
   uint32_t mode;
   uint32_t ndim;          // outer (non-run) dimensions after collapsing, <= kMaxOuterDims;
                           // transposed: batch dimensions (<= kMaxBatchDims)
-  uint32_t tiles_per_run; // kModeRunTiles; kModeWalked: blocks per strip (kBlockStrip or 1)
+  uint32_t tiles_per_run; // kModeRunTiles; kModeRows: runs per tile; kModeWalked: blocks per strip
+                          // (kBlockStrip or 1)
   uint32_t granule;       // kModeElements: bytes moved per lane access (1,2,4,8,16);
                           // kModeRunTiles: 1 + log2(tiles_per_run) when a power of two;
                           // transposed: element size
@@ -251,8 +271,8 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t ext_a, ext_b;
   uint32_t tiles_a, tiles_b;
   uint32_t edge_a, edge_b;         // block extent along A and B (elements)
-  uint32_t lanes_per_run;          // kModeElements: 0, or the lane slots a ragged run occupies (its
-                                   // 16-byte granules rounded up to a multiple of four);
+  uint32_t lanes_per_run;          // kModeRows: the lane slots a run occupies (pstride[0] holds the
+                                   // number of runs, edge_a the slots per lane);
                                    // kModePlanes: which side holds the planes (kPlanesInPayload,
                                    // kPlanesInTensor)
   uint32_t nt_allowed;             // kModeElements, transposed: sides that may keep the launch's
@@ -350,16 +370,15 @@ struct Tunables {
   // last-level cache when the consumer (unpack, or the transport's copy) reads it.
   std::atomic<int64_t> nontemporal{-1};
   std::atomic<int64_t> payload_cache_bytes{256ll << 20};
-  // Strided runs shorter than this use element mode when they are 16 bytes or
-  // longer (16-byte granules, exact or ragged), anything else up to a fifth of it
-  // (measured crossovers).
+  // Strided runs shorter than this are not moved as run tiles when they are 16 bytes or
+  // longer, anything else up to a fifth of it (measured crossovers).
   std::atomic<int64_t> gather_run_bytes{1280};
   std::atomic<int64_t> xcd_remap{-1};         // contiguous wave ranges per die: 1 always, 0 never, -1 when
                                   // transposed blocks that share lines with their neighbours dominate
                                   // (larger bundles then in squares of blocks, see finish_geometry)
   std::atomic<int64_t> transpose{1};          // move transposed views as square blocks through LDS
-  std::atomic<int64_t> ragged_runs{1};        // short runs of 16+ bytes that are no multiple of 16 move in
-                                  // 16-byte granules (the last one overlapping) instead of narrower ones
+  std::atomic<int64_t> ragged_runs{1};        // short runs of 16+ bytes move in whole rows (kModeRows) instead
+                                  // of in granules of a power of two that divides them
   // Contiguous segments longer than a tile start their tiles on a multiple of this many
   // bytes of the written side (0: tiles start at the segment's first byte).  Measured on the
   // 4096-tensor bundle: 16 lifts the tight layout by 2 % (every 16-byte store aligned) and

@@ -180,11 +180,73 @@ __device__ __forceinline__ int64_t run_offset(dims_table dm, uint32_t run) {
   return off;
 }
 
+// Where the runs of a view begin relative to its run `first`: the coordinates of that run, decoded once
+// per tile, and the distance of later runs from it.
+struct RunWalk {
+  dims_table dm;
+  uint32_t nd, idx0[kMaxOuterDims];
+  int64_t base;          // byte offset of run `first`
+
+  __device__ __forceinline__ RunWalk(dims_table table, uint32_t first) : dm(table), nd(table->ndim), base(0) {
+    uint32_t r = first;
+#pragma unroll
+    for (int d = static_cast<int>(kMaxOuterDims) - 1; d >= 0; --d) {
+      idx0[d] = 0;
+      if (static_cast<uint32_t>(d) + nd >= kMaxOuterDims) {
+        const uint32_t extent = dm->shape[d];
+        const uint32_t next = r / extent;
+        idx0[d] = r - next * extent;
+        base += static_cast<int64_t>(idx0[d]) * dm->stride[d];
+        r = next;
+      }
+    }
+  }
+
+  // Byte offset of run first + carry from run `first` (carry < 2^14).
+  __device__ __forceinline__ int64_t offset(uint32_t carry) const {
+    const int64_t stride_last = dm->stride[kMaxOuterDims - 1];
+    if (nd == 1)   // one strided dimension (rows of a matrix): the run index is the only coordinate
+      return static_cast<int64_t>(carry) * stride_last;
+    if (nd == 2) {
+      // two strided dimensions (every k-th element of the rows of a matrix, a slice of a
+      // 3-d tensor): one quotient, no carry beyond the outer one, nothing to vote on.
+      // v < extent + 2^14, so the multiply-high quotient is exact for extents below 2^15.
+      const uint32_t extent_last = dm->shape[kMaxOuterDims - 1];
+      const uint32_t magic_last = 0xffffffffu / extent_last + 1u;
+      uint32_t v = idx0[kMaxOuterDims - 1] + carry;
+      uint32_t c = extent_last < 32768u ? __umulhi(v, magic_last) : v / extent_last;
+      c = extent_last == 1 ? v : c;
+      v -= c * extent_last;
+      return static_cast<int64_t>(static_cast<int32_t>(v - idx0[kMaxOuterDims - 1])) * stride_last +
+             static_cast<int64_t>(c) * dm->stride[kMaxOuterDims - 2];
+    }
+    int64_t toff = 0;
+#pragma unroll
+    for (int d = static_cast<int>(kMaxOuterDims) - 1; d >= 0; --d) {
+      if (static_cast<uint32_t>(d) + nd >= kMaxOuterDims) {
+        if (__builtin_amdgcn_ballot_w64(carry != 0) == 0) break;   // wave-uniform
+        const uint32_t extent = dm->shape[d];
+        uint32_t v = idx0[d] + carry;
+        uint32_t c = 0;
+        if (__builtin_amdgcn_ballot_w64(v >= extent) != 0) {
+          // v < extent + 2^14: for extents below 2^15 the multiply-high quotient is
+          // exact (v * extent < 2^32)
+          c = extent < 32768u ? __umulhi(v, 0xffffffffu / extent + 1u) : v / extent;
+          c = extent == 1 ? v : c;
+          v -= c * extent;
+        }
+        toff += static_cast<int64_t>(static_cast<int32_t>(v - idx0[d])) * dm->stride[d];
+        carry = c;
+      }
+    }
+    return toff;
+  }
+};
+
 // Moves the ng granules (type T) of one element-mode tile, U per lane at a
 // time: addresses first, then all loads, then all stores, so a lane keeps U
 // accesses in flight instead of a load-wait-store chain per granule.
-// decode(e, &packed) gives granule e's tensor-side offset from tbase and its
-// payload offset from pbase.
+// decode(e) gives granule e's tensor-side offset from tbase; its payload offset is e * sizeof(T).
 template <bool PACK, typename T, uint32_t U, typename DECODE>
 __device__ __forceinline__ void element_moves(gbytes tbase, gbytes pbase, uint32_t ng,
                                               uint32_t lane, uint32_t nt_bits, DECODE decode) {
@@ -200,11 +262,9 @@ __device__ __forceinline__ void element_moves(gbytes tbase, gbytes pbase, uint32
     for (uint32_t u = 0; u < U; ++u) {
       const uint32_t e = e0 + u * kWaveLanes;
       const uint32_t ec = e < ng ? e : ng - 1u;   // slots past the end repeat the last slot's load
-      uint64_t packed;
-      bool live;                                  // false for a slot that pads a run to whole quads
-      tp[u] = tbase + decode(ec, &packed, &live);
-      pp[u] = pbase + packed;
-      moves[u] = live && e < ng;
+      tp[u] = tbase + decode(ec);
+      pp[u] = pbase + ec * static_cast<uint32_t>(sizeof(T));
+      moves[u] = e < ng;
     }
     if (nt_rd) {
       asm volatile("");
@@ -253,33 +313,11 @@ __device__ __forceinline__ void element_tile(uint64_t seg_ptr, uint64_t run_byte
   constexpr uint32_t kTile = ROWS * kRowBytes < kMinElementTileBytes ? kMinElementTileBytes : ROWS * kRowBytes;
   const uint32_t g = dm->granule;
   const uint32_t gs = static_cast<uint32_t>(__builtin_ctz(g));
-  // Runs of 16 bytes or more that are no whole number of 64-byte quads (ragged runs):
-  // a run is ceil(run / 16) granules of 16 bytes, its last granule covers the run's
-  // final 16 bytes (overlapping the one before it with identical data when the length
-  // is no multiple of 16), and the run occupies `lanes_per_run` lane slots, the granule
-  // count rounded up to a multiple of four: the memory pipeline takes a wave's
-  // 16-byte accesses four lanes at a time, and a group of four that lies in one run
-  // is one 64-byte request where a group that straddles two runs is two.  Slots past a
-  // run's last granule move nothing.  Tiles then count slots, not packed bytes.
-  const uint32_t lpr = dm->lanes_per_run;
-  const bool ragged = lpr != 0;
-  const uint32_t run32 = static_cast<uint32_t>(run_bytes);
-  const uint32_t granules = ragged ? (run32 + 15u) >> 4 : static_cast<uint32_t>(run_bytes >> gs);
-  const uint32_t gpr = ragged ? lpr : granules;   // slots per run
-  const uint32_t nd = dm->ndim;
-  const uint64_t b0 = static_cast<uint64_t>(q) * kTile;   // exact runs: packed byte of the tile
-  uint64_t e0;
-  uint32_t ng;
-  if (ragged) {
-    e0 = static_cast<uint64_t>(q) * (kTile / kVecBytes);
-    const uint64_t left = dm->pstride[0] - e0;            // slots of the whole segment
-    ng = left < kTile / kVecBytes ? static_cast<uint32_t>(left) : kTile / kVecBytes;
-  } else {
-    const uint64_t left = dm->nbytes - b0;
-    const uint32_t n = left < kTile ? static_cast<uint32_t>(left) : kTile;
-    e0 = b0 >> gs;
-    ng = n >> gs;
-  }
+  const uint32_t gpr = static_cast<uint32_t>(run_bytes >> gs);   // granules per run
+  const uint64_t b0 = static_cast<uint64_t>(q) * kTile;          // packed byte of the tile
+  const uint64_t left = dm->nbytes - b0;
+  const uint32_t ng = (left < kTile ? static_cast<uint32_t>(left) : kTile) >> gs;
+  const uint64_t e0 = b0 >> gs;
   uint32_t run0, w0;
   if ((e0 >> 32) == 0) {
     const uint32_t e32 = static_cast<uint32_t>(e0);
@@ -289,79 +327,17 @@ __device__ __forceinline__ void element_tile(uint64_t seg_ptr, uint64_t run_byte
     run0 = static_cast<uint32_t>(e0 / gpr);
     w0 = static_cast<uint32_t>(e0 - static_cast<uint64_t>(run0) * gpr);
   }
-  uint32_t idx0[kMaxOuterDims];
-  int64_t base = 0;
-  {
-    uint32_t r = run0;
-#pragma unroll
-    for (int d = static_cast<int>(kMaxOuterDims) - 1; d >= 0; --d) {
-      idx0[d] = 0;
-      if (static_cast<uint32_t>(d) + nd >= kMaxOuterDims) {
-        const uint32_t extent = dm->shape[d];
-        const uint32_t next = r / extent;
-        idx0[d] = r - next * extent;
-        base += static_cast<int64_t>(idx0[d]) * dm->stride[d];
-        r = next;
-      }
-    }
-  }
+  const RunWalk walk(dm, run0);
   const uint32_t gpr_magic = 0xffffffffu / gpr + 1u;
-  const int64_t stride_last = dm->stride[kMaxOuterDims - 1];
-  const int64_t stride_prev = dm->stride[kMaxOuterDims - 2];
-  const uint32_t extent_last = dm->shape[kMaxOuterDims - 1];
-  const uint32_t magic_last = 0xffffffffu / extent_last + 1u;
-  gbytes tbase = as_global(seg_ptr) + base;
-  gbytes pbase = ragged ? pay + static_cast<uint64_t>(run0) * run32 : pay + b0;
-  // tensor-side byte offset (relative to the tile's first run) of granule e of the
-  // tile, and its payload offset (relative to pbase)
-  auto decode = [&](uint32_t e, uint64_t* packed, bool* live) -> int64_t {
+  gbytes tbase = as_global(seg_ptr) + walk.base;
+  gbytes pbase = pay + b0;
+  // tensor-side byte offset (relative to the tile's first run) of granule e of the tile
+  auto decode = [&](uint32_t e) -> int64_t {
     uint32_t w = w0 + e;
     // w < gpr + tile / g: for gpr <= 2^15, w * gpr < 2^32 and the multiply-high quotient is exact
-    uint32_t carry = gpr == 1 ? w : (gpr <= 32768u ? __umulhi(w, gpr_magic) : w / gpr);
+    const uint32_t carry = gpr == 1 ? w : (gpr <= 32768u ? __umulhi(w, gpr_magic) : w / gpr);
     w -= carry * gpr;
-    uint32_t in_run = w << gs;
-    if (ragged) {
-      *live = w < granules;
-      in_run = w + 1u >= granules ? run32 - kVecBytes : in_run;
-      *packed = static_cast<uint64_t>(carry) * run32 + in_run;
-    } else {
-      *live = true;
-      *packed = static_cast<uint64_t>(e) << gs;
-    }
-    int64_t toff = static_cast<int64_t>(in_run);
-    if (nd == 1) {   // one strided dimension (rows of a matrix): the run index is the only coordinate
-      return toff + static_cast<int64_t>(carry) * stride_last;
-    }
-    if (nd == 2) {
-      // two strided dimensions (every k-th element of the rows of a matrix, a slice of a
-      // 3-d tensor): one quotient, no carry beyond the outer one, nothing to vote on.
-      // v < extent + 2^14, so the multiply-high quotient is exact for extents below 2^15.
-      uint32_t v = idx0[kMaxOuterDims - 1] + carry;
-      uint32_t c = extent_last < 32768u ? __umulhi(v, magic_last) : v / extent_last;
-      c = extent_last == 1 ? v : c;
-      v -= c * extent_last;
-      return toff + static_cast<int64_t>(static_cast<int32_t>(v - idx0[kMaxOuterDims - 1])) * stride_last +
-             static_cast<int64_t>(c) * stride_prev;
-    }
-#pragma unroll
-    for (int d = static_cast<int>(kMaxOuterDims) - 1; d >= 0; --d) {
-      if (static_cast<uint32_t>(d) + nd >= kMaxOuterDims) {
-        if (__builtin_amdgcn_ballot_w64(carry != 0) == 0) break;   // wave-uniform
-        const uint32_t extent = dm->shape[d];
-        uint32_t v = idx0[d] + carry;
-        uint32_t c = 0;
-        if (__builtin_amdgcn_ballot_w64(v >= extent) != 0) {
-          // v < extent + 2^14: for extents below 2^15 the multiply-high quotient is
-          // exact (v * extent < 2^32)
-          c = extent < 32768u ? __umulhi(v, 0xffffffffu / extent + 1u) : v / extent;
-          c = extent == 1 ? v : c;
-          v -= c * extent;
-        }
-        toff += static_cast<int64_t>(static_cast<int32_t>(v - idx0[d])) * dm->stride[d];
-        carry = c;
-      }
-    }
-    return toff;
+    return static_cast<int64_t>(w << gs) + walk.offset(carry);
   };
   // Accesses per lane and round: four in flight.
   switch (g) {
@@ -390,6 +366,161 @@ typedef AXR_LDS uint8_t* lbytes;
 
 // ---------------------------------------------------------------- rows
 //
+// Short runs of 16 bytes or more: rows of a slice, of any length, from any start.  The memory pipeline
+// takes a wave's 16-byte accesses four lanes at a time; four lanes in one aligned 64-byte unit are one
+// request, anything else is two, and units written in two parts cost most of all.  No assignment of
+// 16-byte pieces to lanes suits both sides, so a wavefront parks whole rows in LDS as they lie in the
+// payload and cuts each side on its own boundaries: every row into 16-byte slots of its own 64-byte
+// units, the payload range likewise.  The first and the last piece of a row and of the range move inside
+// and overlap their neighbour with identical bytes, so nothing outside is read or written.  A row occupies
+// S = lanes_per_run slots, enough for the worst start its strides allow; a start that an address delta
+// has made worse than that is not aligned (a = 0), which only costs requests.
+// U is how many slots a lane moves, all in flight together.  Two (about 2 KiB) are best as long as two
+// rows fit: with 3, 4 and 8 slots 2^18 rows of 250 bytes at 333 take 59, 63 and 64 us for pack + unpack
+// instead of 58, of 666 at 1554 141, 144 and 146 instead of 135; where two slots hold one row of a kilobyte
+// only they take 264 instead of 171.
+// Against 16-byte pieces moved without LDS, 8 KiB per wavefront, pack + unpack in turn, 2^18 rows, before /
+// now: 100 bytes at 256 40 / 34 us, 102 at 258 53 / 49, 128 at 256 29 / 26, 250 at 333 68 / 58, 256 at 512
+// 50 / 46, 256 at 515 73 / 65, 512 at 1024 89 / 82, 666 at 1554 156 / 138, 1001 at 1301 184 / 181, 1024 at 2048
+// 165 / 155; 2^20 rows of 250 at 1024 203 / 195, of 36 at 64 57 / 54.  What is left of the odd ones is
+// units whose other bytes are not the view's: each is read and merged by the memory.
+template <bool PACK, uint32_t U>
+__device__ __forceinline__ void rows_moves(uint64_t seg_ptr, uint32_t run, dims_table dm, gbytes pay,
+                                           uint32_t q, lbytes lds, uint32_t lane, uint32_t nt_bits) {
+  typedef AXR_LDS u32x4_loose* lvec;   // (LDS accesses of any alignment, like the global ones)
+  typedef const AXR_LDS u32x4_loose* lcvec;
+  constexpr uint32_t V = U + 1;        // 16-byte pieces of the payload range per lane: (63 + 16 * 64 U) / 16 at most
+  nt_bits &= PACK ? dm->nt_allowed : dm->nt_allowed >> 2;
+  const bool nt_rd = (nt_bits & (PACK ? 1u : 2u)) != 0, nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
+  const uint32_t per_tile = dm->tiles_per_run, S = dm->lanes_per_run;
+  const uint32_t row0 = q * per_tile, left = static_cast<uint32_t>(dm->pstride[0]) - row0;
+  const uint32_t rows = left < per_tile ? left : per_tile;
+  const uint32_t slots = rows * S;
+  const RunWalk walk(dm, row0);
+  gbytes tbase = as_global(seg_ptr) + walk.base;
+  gbytes pbase = pay + static_cast<uint64_t>(row0) * run;
+  // The image in LDS holds the payload range from its first 64-byte unit on: bytes [skew, end).
+  const uint32_t skew = static_cast<uint32_t>(reinterpret_cast<uint64_t>(pbase)) & (kUnitBytes - 1u);
+  const uint32_t end = skew + rows * run, pieces = (end + kVecBytes - 1u) / kVecBytes;
+  gbytes image = pbase - skew;
+  const uint32_t magic = 0xffffffffu / S + 1u;
+  auto piece = [&](uint32_t j) {       // where piece j lies in the image
+    const uint32_t o = j * kVecBytes < skew ? skew : j * kVecBytes;
+    return o + kVecBytes <= end ? o : end - kVecBytes;
+  };
+  auto piece_counts = [&](uint32_t j) { return j < pieces && (j + 1u) * kVecBytes > skew; };
+  // slot e: its address in the tensor and its place in the image; false when it moves nothing
+  auto slot = [&](uint32_t e, gbytes* at, uint32_t* in_image) {
+    const uint32_t ec = e < slots ? e : slots - 1u;
+    const uint32_t row = __umulhi(ec, magic), w = ec - row * S;   // ec < 2^9: exact
+    gbytes t = tbase + walk.offset(row);
+    uint32_t a = static_cast<uint32_t>(reinterpret_cast<uint64_t>(t)) & (kUnitBytes - 1u);
+    a = a + run <= S * kVecBytes ? a : 0u;
+    const int32_t o = static_cast<int32_t>(w * kVecBytes - a), last = static_cast<int32_t>(run - kVecBytes);
+    const int32_t inside = o < 0 ? 0 : (o > last ? last : o);
+    *at = t + inside;
+    *in_image = skew + row * run + static_cast<uint32_t>(inside);
+    return e < slots && o > -static_cast<int32_t>(kVecBytes) && o < static_cast<int32_t>(run);
+  };
+  // (hints: one wave-uniform branch around each batch, the arms kept apart by the empty asm statements)
+  if constexpr (PACK) {
+    gbytes at[U];
+    uint32_t to[U];
+    bool moves[U];
+    u32x4 x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) moves[u] = slot(lane + u * kWaveLanes, &at[u], &to[u]);
+    if (nt_rd) {
+      asm volatile("");
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) x[u] = load16<true>(at[u]);
+      asm volatile("");
+    } else {
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) x[u] = load16<false>(at[u]);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) asm volatile("" : "+v"(x[u])::"memory");
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      if (moves[u]) *reinterpret_cast<lvec>(lds + to[u]) = x[u];
+    }
+    __builtin_amdgcn_wave_barrier();
+    u32x4 y[V];
+    uint32_t p[V];
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) {
+      p[k] = piece(lane + k * kWaveLanes);
+      y[k] = *reinterpret_cast<lcvec>(lds + p[k]);
+    }
+    if (nt_wr) {
+      asm volatile("");
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) {
+        if (piece_counts(lane + k * kWaveLanes)) store16<true>(image + p[k], y[k]);
+      }
+      asm volatile("");
+    } else {
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) {
+        if (piece_counts(lane + k * kWaveLanes)) store16<false>(image + p[k], y[k]);
+      }
+    }
+  } else {
+    u32x4 y[V];
+    uint32_t p[V];
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) p[k] = piece(lane + k * kWaveLanes);
+    if (nt_rd) {
+      asm volatile("");
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) y[k] = load16<true>(image + p[k]);
+      asm volatile("");
+    } else {
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) y[k] = load16<false>(image + p[k]);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) asm volatile("" : "+v"(y[k])::"memory");
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) *reinterpret_cast<lvec>(lds + p[k]) = y[k];
+    __builtin_amdgcn_wave_barrier();
+    gbytes at[U];
+    bool moves[U];
+    u32x4 x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      uint32_t from;
+      moves[u] = slot(lane + u * kWaveLanes, &at[u], &from);
+      x[u] = *reinterpret_cast<lcvec>(lds + from);
+    }
+    if (nt_wr) {
+      asm volatile("");
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        if (moves[u]) store16<true>(at[u], x[u]);
+      }
+      asm volatile("");
+    } else {
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        if (moves[u]) store16<false>(at[u], x[u]);
+      }
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <bool PACK>
+__device__ __forceinline__ void rows_tile(uint64_t seg_ptr, uint32_t run, dims_table dm, gbytes pay, uint32_t q,
+                                          lbytes lds, uint32_t lane, uint32_t nt_bits) {
+  switch (dm->edge_a) {   // slots per lane
+    case 2: rows_moves<PACK, 2>(seg_ptr, run, dm, pay, q, lds, lane, nt_bits); break;
+    case 3: rows_moves<PACK, 3>(seg_ptr, run, dm, pay, q, lds, lane, nt_bits); break;
+    default: rows_moves<PACK, kMaxRowSlots>(seg_ptr, run, dm, pay, q, lds, lane, nt_bits); break;
+  }
+}
+
 template <uint32_t E> struct unit_of;
 template <> struct unit_of<1> { typedef uint8_t type; };
 template <> struct unit_of<2> { typedef uint16_t type; };
@@ -1379,6 +1510,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
         lbytes lds = (lbytes)lds_slices + uniform(threadIdx.x >> 6) * lds_per_wave;
         if (mode == kModeElements) element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
+        else if (mode == kModeRows) rows_tile<PACK>(seg_ptr, static_cast<uint32_t>(seg_run), dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
         else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
@@ -1431,13 +1563,13 @@ __global__ __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(kMaxThreads
 // Bundles with views whose tiles are more than copies of runs: all of one mode, or kKindAny.  What such a
 // tile waits for is memory, so a compute unit should hold many of them, and how many it holds is a matter of
 // registers: built together as functions that are called, the routines took 120 (16 wavefronts on a compute
-// unit) and read their tables through vector loads; a kernel for each of them takes 43 to 87 and reads them by
+// unit) and read their tables through vector loads; a kernel for each of them takes 41 to 87 and reads them by
 // scalar loads.  256 uint8 images of 224 x 224 x 3, pack + unpack, 32.3 -> 30.1 us, four odd transposed bf16
 // matrices 112.7 -> 108.5, 2^18 rows of 256 bytes 50.4 -> 48.5.  Wavefronts per SIMD that the registers are
-// held to: LDS allows 4 to 5 for blocks, and 23 on a compute unit for planes; plain blocks are
+// held to: LDS allows 4 to 5 for blocks and 23 to 46 on a compute unit for rows and planes; plain blocks are
 // 1 % faster with the registers of 4 than with those of 7, kKindAny would spill at 6.
 constexpr uint32_t waves_of_kind(uint32_t kind, uint32_t rows) {
-  return kind == kModeElements ? 8 : kind == kModePlanes ? 6 : kind == kKindAny && rows <= 8 ? 5 : 4;
+  return kind == kModeElements || kind == kModeRows ? 8 : kind == kModePlanes ? 6 : kind == kKindAny && rows <= 8 ? 5 : 4;
 }
 template <bool PACK, uint32_t ROWS, uint32_t KIND>
 __global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, ROWS), KIND == kModeTranspose ? 4 : 8)))
@@ -1866,6 +1998,7 @@ int launch_rows(const KernelArgs& args, const LaunchConfig& cfg, hipStream_t str
     if constexpr (ROWS == 2) {
       switch (cfg.kind) {
         case kModeElements: AXR_VIEWS(kModeElements); break;
+        case kModeRows: AXR_VIEWS(kModeRows); break;
         case kModeTranspose: AXR_VIEWS(kModeTranspose); break;
         case kModeWalked: AXR_VIEWS(kModeWalked); break;
         case kModePlanes: AXR_VIEWS(kModePlanes); break;
@@ -1971,7 +2104,7 @@ int launch_bundle_jobs(const JobTable& jobs, const LaunchConfig& cfg, void* stre
   if (cfg.elements) {
     // bundles with short strided runs or transpositions: the default tile only, hints at run time
     if (cfg.tile_rows != 2) return fail(AXR_ERR_INVALID, "element-mode jobs need 2 KiB tiles");
-    AXR_JOBS(2, true, true, kKindAny);
+    if (cfg.kind == kModeRows) AXR_JOBS(2, true, true, kModeRows); else AXR_JOBS(2, true, true, kKindAny);
   } else {
     switch (cfg.tile_rows) {
       case 1: AXR_JOBS_NT(1) break;
@@ -2013,6 +2146,8 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
                      cfg.lds_per_wave, hint_argument(cfg), dims_at, wave_at, tables)
   if (!cfg.elements) {
     if (pack) AXR_INLINE_LAUNCH(true, kKindRuns); else AXR_INLINE_LAUNCH(false, kKindRuns);
+  } else if (cfg.kind == kModeRows) {
+    if (pack) AXR_INLINE_LAUNCH(true, kModeRows); else AXR_INLINE_LAUNCH(false, kModeRows);
   } else {
     if (pack) AXR_INLINE_LAUNCH(true, kKindAny); else AXR_INLINE_LAUNCH(false, kKindAny);
   }

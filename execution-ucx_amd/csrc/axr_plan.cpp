@@ -497,14 +497,13 @@ uint32_t granule_of(uint64_t run_bytes) {
   return g;
 }
 
-// Runs shorter than this move in element mode.  With 16-byte granules (exact or ragged)
-// element mode is ahead of run tiles up to runs of about 1 KiB and level with them from
-// 1280 bytes on; narrower granules move fewer bytes per access and lose to the
+// Runs shorter than this do not move as run tiles.  In whole rows they are ahead of run tiles up to 1280
+// bytes and longer ones are left to those; narrower granules move fewer bytes per access and lose to the
 // (length-agnostic) run-tile copy much earlier.
 uint64_t element_mode_limit(uint64_t run_bytes) {
   const uint64_t limit = static_cast<uint64_t>(tunables().gather_run_bytes);
   if (granule_of(run_bytes) == 16) return limit;
-  if (run_bytes >= kVecBytes && tunables().ragged_runs != 0) return limit;
+  if (run_bytes >= kVecBytes && tunables().ragged_runs != 0) return std::min<uint64_t>(limit, kMaxRowBytes + 1);
   return (limit + 4) / 5;
 }
 
@@ -516,6 +515,7 @@ struct Builder {
   uint64_t tiles = 0;
   uint64_t shared_line_tiles = 0;   // transposed blocks whose rows straddle 128-byte lines
   uint64_t strip_tiles = 0;         // those of them that lie in strips of kBlockStrip blocks
+  bool mixed = false;               // some tensor, of those seen so far, is not moved in whole short rows
   uint64_t group_bytes = 0;         // longest tensor that may share a wavefront (0: none)
   uint32_t slots_per_group = kGroupMaxSlots;
   // the group being collected (when open): the last block of p->group_blocks
@@ -592,6 +592,7 @@ struct Builder {
 
   int add_seg(uint32_t tensor, uint64_t ptr, uint64_t off, uint64_t run_bytes, uint64_t ntile,
               uint32_t dsel) {
+    mixed = mixed || dsel == 0 || dsel >= kSegGroup || p->dims[dsel - 1].mode != kModeRows;
     if (tiles + ntile > 0xffffffffull) return fail(AXR_ERR_UNSUPPORTED, "bundle has too many tiles");
     Seg s;
     s.ptr = ptr;
@@ -797,20 +798,24 @@ struct Builder {
       // Rows shorter than a line use every line they touch only in part: such lines are
       // cheaper read and written through the cache than streamed (100-byte rows: +5 to 7 %).
       dm.nt_allowed = (run_bytes >= kLineBytes ? 3u : 2u) * 5u;   // the same in both directions
-      const uint64_t element_tile = std::max<uint32_t>(tile_bytes, kMinElementTileBytes);
-      const uint64_t granules_per_run = (run_bytes + kVecBytes - 1) / kVecBytes;
-      if (run_bytes >= kVecBytes && tunables().ragged_runs != 0 &&
-          (dm.granule != kVecBytes || (granules_per_run & 3) != 0)) {
-        // ragged runs: ceil(run / 16) granules of 16 bytes per run, the last one covering
-        // the run's final 16 bytes, in a whole number of four-lane groups; tiles count
-        // lane slots
+      // how far behind the start of a 64-byte unit a run may begin: the strides move it in multiples of `step`
+      uint64_t step = kUnitBytes;
+      for (size_t d = 0; d < nd; ++d) step |= static_cast<uint64_t>(str[d]);
+      step &= 0 - step;
+      const uint32_t start = static_cast<uint32_t>((ptr & (step - 1)) + kUnitBytes - step);
+      // (rows of less than a unit are left where they straddle two: slots for both would be half empty)
+      const uint32_t slots = row_slots(run_bytes, run_bytes < kUnitBytes ? 0 : start);
+      if (run_bytes >= kVecBytes && run_bytes <= kMaxRowBytes && tunables().ragged_runs != 0) {
+        dm.mode = kModeRows;
         dm.granule = kVecBytes;
-        dm.lanes_per_run = static_cast<uint32_t>((granules_per_run + 3) & ~3ull);
-        const uint64_t slots = runs * dm.lanes_per_run;
-        dm.pstride[0] = slots;
-        const uint64_t per_tile = element_tile / kVecBytes;
-        ntile = (slots + per_tile - 1) / per_tile;
+        dm.lanes_per_run = slots;
+        dm.edge_a = row_slots_per_lane(slots, mixed);
+        dm.tiles_per_run = dm.edge_a * kWaveLanes / slots;
+        dm.pstride[0] = runs;
+        ntile = (runs + dm.tiles_per_run - 1) / dm.tiles_per_run;
+        p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (rows_lds_bytes(dm.tiles_per_run, run_bytes) + 15u) & ~15u);
       } else {
+        const uint64_t element_tile = std::max<uint32_t>(tile_bytes, kMinElementTileBytes);
         ntile = (nbytes + element_tile - 1) / element_tile;
       }
     }
@@ -871,18 +876,16 @@ bool streams_in_small_tiles(const axr_plan* p) {
 // few large tensors gets a tiny index, a bundle of many small ones an entry per few tiles).
 void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct = false) {
   const Tunables& tn = tunables();
-  uint64_t tpw = (p->ntiles + static_cast<uint64_t>(tn.max_waves) - 1) /
-                 static_cast<uint64_t>(tn.max_waves);
+  // (tiles of short rows are a quarter of the others' length, and their wavefronts as much shorter)
+  bool short_rows = false;
+  for (const Dims& dm : p->dims) short_rows = short_rows || dm.mode == kModeRows;
+  const uint64_t max_waves = static_cast<uint64_t>(tn.max_waves) * (short_rows ? 4 : 1);
+  uint64_t tpw = (p->ntiles + max_waves - 1) / max_waves;
   if (tpw == 0) tpw = 1;
   p->cfg.threads = tn.threads ? static_cast<uint32_t>(tn.threads)
                               : (rows == 1 && tn.tile_rows == 0 ? kWaveLanes : (p->ntiles < 65536 ? 256u : 128u));
   p->cfg.elements = false;
-  bool ragged_rows = false, blocks = false;
-  for (const Dims& dm : p->dims) {
-    p->cfg.elements = p->cfg.elements || dm.mode != kModeRunTiles;
-    ragged_rows = ragged_rows || (dm.mode == kModeElements && dm.lanes_per_run != 0);
-    blocks = blocks || dm.mode >= kModeTranspose;
-  }
+  for (const Dims& dm : p->dims) p->cfg.elements = p->cfg.elements || dm.mode != kModeRunTiles;
   p->cfg.kind = kKindAny;
   if (p->cfg.elements && rows == 2) {   // the kernels of a single mode are built for the default tile
     const uint32_t mode = p->dims[0].mode;
@@ -895,10 +898,6 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
     if (one) p->cfg.kind = mode;
   }
   if (p->cfg.elements) p->cfg.threads = std::min(p->cfg.threads, kMaxElementThreads);
-  // Short rows that are no multiple of 16 bytes (lane slots left idle behind each run) run 2.5-5 %
-  // faster in workgroups of one wavefront (rows of 250 B: 4.97 -> 5.22 TB/s, of 100 B: 3.06 ->
-  // 3.14); rows of whole granules and transposed blocks are fastest at 256 threads.
-  if (tn.threads == 0 && ragged_rows && !blocks) p->cfg.threads = kWaveLanes;
   if (p->cfg.lds_per_wave) {
     // transposed blocks: every wave of a workgroup owns a slice of at most 64 KiB of LDS
     const uint32_t fit = (64u * 1024u / p->cfg.lds_per_wave) * kWaveLanes;
@@ -1175,6 +1174,7 @@ int build_tables(axr_plan* p) {
   invalidate_tables(p);
   const Tunables& tn = tunables();
   uint32_t rows = static_cast<uint32_t>(tn.tile_rows);
+  bool compact = false;   // some tensor is compact, of those that are looked at here
   if (rows == 0) {
     rows = 2;
     // A bundle made only of strided views with one short run length (pitched
@@ -1195,6 +1195,7 @@ int build_tables(axr_plan* p) {
       if (t.nbytes == 0) continue;
       if (!t.has_strides || is_compact(p, t)) {
         uniform_runs = false;   // a compact tensor: not a bundle of strided views
+        compact = true;
       } else {
         Collapsed c;
         collapse(t, p->shape_of(t), p->strides_of(t), item_bytes(t), &c);
@@ -1218,6 +1219,7 @@ int build_tables(axr_plan* p) {
             static_cast<uint64_t>(tn.head_align)};
   b.group_bytes = static_cast<uint64_t>(tn.group_bytes);
   b.slots_per_group = static_cast<uint32_t>(tn.group_slots);
+  b.mixed = compact;
   p->segs.reserve(p->tensors.size() + 1);
   p->seg_tensor.reserve(p->tensors.size());
 
@@ -2335,11 +2337,12 @@ static int plan_segments_body(axr_plan_t* plan, axr_segment_info_t* out, size_t 
       o.mode = 3;
     } else {
       const Dims& dm = plan->dims[dsel - 1];
-      o.mode = dm.mode == kModeRunTiles ? 1 : (dm.mode == kModeElements ? 2 : 5);
+      o.mode = dm.mode == kModeRunTiles ? 1 : (dm.mode == kModeElements || dm.mode == kModeRows ? 2 : 5);
       o.nbytes = dm.nbytes;
       o.ndim = dm.ndim;
       o.granule = dm.granule;
-      o.lanes_per_run = dm.mode == kModeElements ? dm.lanes_per_run : 0;
+      // (the slots of a run whose start lies on a 64-byte boundary, where it leaves some of them unused)
+      o.lanes_per_run = dm.mode == kModeRows && s.run_bytes % kUnitBytes != 0 ? row_slots(s.run_bytes, 0) : 0;
       for (uint32_t d = 0; d < dm.ndim; ++d) {
         o.shape[d] = dm.shape[kMaxOuterDims - dm.ndim + d];
         o.stride_bytes[d] = dm.stride[kMaxOuterDims - dm.ndim + d];

@@ -409,9 +409,9 @@ typedef struct axr_segment_info {
                              moves on top of its own range, so that the tiles
                              start on a 128-byte line of the written side      */
   uint32_t lanes_per_run; /* mode 2 with 16-byte granules: lane slots a run occupies
-                             (its granules, the last one covering the run's final 16
-                             bytes, rounded up to a multiple of four); 0: the tiles
-                             count packed bytes                                  */
+                             when it starts on a 64-byte boundary (its granules, the
+                             last one covering the run's final 16 bytes, rounded up to
+                             a multiple of four); 0 where it leaves none unused      */
   uint32_t shape[6];
   int64_t stride_bytes[6];
 } axr_segment_info_t;
@@ -427,15 +427,15 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * last-level cache; 1 for payloads of compact tensors and long strided runs between
  * payload_cache_bytes and max_tiles KiB, which stream to and from memory), "max_tiles",
  * "max_waves", "threads" (workgroup size; 0 = automatic: 256 below 65,536 tiles, 128 above, 64
- * with the automatic 1 KiB tiles and for short strided rows that are no multiple of 16
- * bytes), "nontemporal" (-1 auto, or bit 0
+ * with the automatic 1 KiB tiles), "nontemporal" (-1 auto, or bit 0
  * tensor side / bit 1 payload side), "payload_cache_bytes", "gather_run_bytes",
  * "xcd_remap" (each accelerator die walks one contiguous share of the tiles: 1 always,
  * 0 never, -1 (default) for bundles made mostly of transposed views whose rows do not
  * start on 128-byte lines, where neighbouring blocks then meet in one L2),
  * "transpose" (1: transposed views move as square blocks through
- * LDS; 0: element by element), "ragged_runs" (1: short strided runs whose
- * length is no multiple of 16 bytes still move in 16-byte granules),
+ * LDS; 0: element by element), "ragged_runs" (1: short strided runs of 16
+ * bytes and more move in whole rows, in 16-byte pieces whatever their length; 0: in
+ * pieces of the largest power of two that divides them),
  * "head_align" (contiguous tensors longer than a tile start their tiles on a
  * multiple of this many bytes of the written side - the payload for a plan made
  * by axr_plan_create, the tensor for one made by axr_plan_from_header; a power

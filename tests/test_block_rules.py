@@ -122,3 +122,34 @@ def test_chunks_in_line(tmp_path):
         f.write('#include "axr_internal.h"\nusing namespace axr;\n' + checks)
     subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
+
+
+def test_row_slots(tmp_path):
+    """Rows of every length from every start: the slots of its 64-byte units cover a row, a tile holds two rows
+    at least and no more than its lanes and its LDS, and the payload pieces of a tile fit theirs."""
+    source = r"""
+#include "axr_internal.h"
+using namespace axr;
+constexpr bool fits(uint64_t run, uint32_t start, bool mixed) {
+  const uint32_t slots = row_slots(run, start), lanes = row_slots_per_lane(slots, mixed) * kWaveLanes, rows = lanes / slots;
+  if (slots % 4 != 0 || slots * kVecBytes < start + run || rows < 2 || rows * slots > lanes) return false;
+  if ((kUnitBytes - 1 + rows * run + kVecBytes - 1) / kVecBytes > lanes + kWaveLanes) return false;
+  return kUnitBytes - 1 + rows * run <= rows_lds_bytes(static_cast<uint32_t>(rows), run) && rows_lds_bytes(rows, run) <= 16384;
+}
+constexpr bool all(uint32_t start, bool mixed) {
+  for (uint64_t run = kVecBytes; run <= kMaxRowBytes; ++run)
+    if (!fits(run, start, mixed)) return false;
+  return true;
+}
+constexpr bool every_start(bool mixed) {
+  for (uint32_t start = 0; start < kUnitBytes; ++start)
+    if (!all(start, mixed)) return false;
+  return true;
+}
+static_assert(every_start(false) && every_start(true), "rows");
+"""
+    src = str(tmp_path / "rows.cpp")
+    with open(src, "w") as f:
+        f.write(source)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=200000000", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)

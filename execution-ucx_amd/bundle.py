@@ -17,7 +17,7 @@ from dataclasses import dataclass
 from typing import Any, Callable, List, NamedTuple, Optional, Sequence, Tuple
 
 from . import _capi, streams
-from .dlpack import DLPackExport, TensorArray, TensorView
+from .dlpack import DLPackExport, TensorArray, TensorView, plain_plan
 from .memory import DevicePool, PoolBuffer
 
 
@@ -86,6 +86,7 @@ class BundlePlan:
         self._h = handle
         self._keep = keepalive
         self._receiver = receiver      # made from a header: its tensors are written by unpack
+        self._header = None            # the header where the plan reads it in place
 
     # ---- construction
     @classmethod
@@ -95,6 +96,9 @@ class BundlePlan:
         ``stream``: the stream the plan will be packed on, when it is known already; producers
         other than torch tensors are then told through ``__dlpack__(stream=...)``."""
         lib = _capi.load()
+        made = plain_plan(lib, tensors, align)
+        if made is not None:
+            return cls(made[0], keepalive=made[1])
         # descriptors may be prepared once and reused per call
         arr = tensors if isinstance(tensors, TensorArray) else TensorArray.from_objects(
             tensors, stream=_dlpack_stream(stream))
@@ -232,6 +236,7 @@ class BundlePlan:
             _capi.check(self._lib.axr_plan_free(self._h))
             self._h = None
             self._keep = None
+            self._header = None
 
     def __enter__(self):
         return self
@@ -301,6 +306,12 @@ def _bind_header(header: bytes, out: Sequence[Any], stream) -> BundlePlan:
     that can be described without asking anything of them.  Others are asked once, and only for a
     header that is in order: a producer may give its capsule a single time."""
     arr = out if isinstance(out, TensorArray) else None
+    buf = bytes(header)
+    made = plain_plan(_capi.load(), out, header=buf)
+    if made is not None:
+        plan = BundlePlan(made[0], keepalive=made[1], receiver=True)
+        plan._header = buf
+        return plan
     if arr is None and isinstance(out, (list, tuple)):
         arr = TensorArray.from_plain_tensors(out)
     if arr is None:

@@ -26,6 +26,7 @@
 #include <new>
 
 #include "axr_internal.h"
+#include "axr_source.h"
 
 using namespace axr;
 
@@ -64,6 +65,11 @@ class RawVec {
   void resize(size_t m) {   // new elements hold whatever the memory held
     reserve(m);
     n_ = m;
+  }
+  T* extend(size_t more) {   // room for `more` elements behind the others, doubled when it runs out
+    if (more > cap_ - n_) reserve(std::max(n_ + more, 2 * cap_));
+    n_ += more;
+    return ptr_ + (n_ - more);
   }
   void assign(const T* first, const T* last) {
     resize(static_cast<size_t>(last - first));
@@ -164,11 +170,13 @@ inline int nbytes_rule(int32_t ndim, const int64_t* shape, uint8_t bits, uint64_
 struct axr_plan {
   uint32_t align = 1;
   RawVec<TensorRec> tensors;
-  std::vector<int64_t> dims64;       // shapes and strides of all tensors
+  RawVec<int64_t> dims64;       // shapes and strides of all tensors
   RawVec<TensorRec> staged_tensors;  // axr_plan_bind fills these and swaps on success
-  std::vector<int64_t> staged_dims64;
+  RawVec<int64_t> staged_dims64;
   uint64_t payload_bytes = 0, data_bytes = 0;
   RawVec<uint8_t> header;
+  const uint8_t* borrowed_header = nullptr;   // the header where the plan keeps none of its own (axr_plan_bind_from)
+  size_t borrowed_header_bytes = 0;
   bool bound = false;
   bool receiver = false;             // made by axr_plan_from_header: tiles are anchored on the tensor side
 
@@ -255,7 +263,7 @@ void plan_delete(axr_plan* p) {
     return v.capacity() * sizeof(v[0]);
   };
   RawVec<TensorRec> tensors, tensors2;
-  std::vector<int64_t> dims64, dims64_2;
+  RawVec<int64_t> dims64, dims64_2;
   RawVec<uint8_t> header;
   std::vector<Seg> segs;
   std::vector<Dims> dims;
@@ -1583,7 +1591,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   return AXR_OK;
 }
 
-int store_tensor(std::vector<int64_t>& dims64, const axr_tensor_t& in, TensorRec* rec) {
+int store_tensor(RawVec<int64_t>& dims64, const axr_tensor_t& in, TensorRec* rec) {
   rec->device_type = in.device_type;
   rec->device_id = in.device_id;
   rec->ndim = in.ndim;
@@ -1596,16 +1604,19 @@ int store_tensor(std::vector<int64_t>& dims64, const axr_tensor_t& in, TensorRec
   rec->strides_at = 0;
   rec->has_strides = in.strides != nullptr && in.ndim > 0;
   if (in.ndim == 1) {
-    dims64.push_back(in.shape[0]);
+    int64_t* d = dims64.extend(rec->has_strides ? 2 : 1);
+    d[0] = in.shape[0];
     if (rec->has_strides) {
       rec->strides_at = rec->shape_at + 1;
-      dims64.push_back(in.strides[0]);
+      d[1] = in.strides[0];
     }
-  } else {
-    dims64.insert(dims64.end(), in.shape, in.shape + in.ndim);
+  } else if (in.ndim) {
+    const size_t nd = static_cast<size_t>(in.ndim);
+    int64_t* d = dims64.extend(rec->has_strides ? 2 * nd : nd);
+    std::memcpy(d, in.shape, 8 * nd);
     if (rec->has_strides) {
-      rec->strides_at = static_cast<uint32_t>(dims64.size());
-      dims64.insert(dims64.end(), in.strides, in.strides + in.ndim);
+      rec->strides_at = rec->shape_at + static_cast<uint32_t>(nd);
+      std::memcpy(d + nd, in.strides, 8 * nd);
     }
   }
   if (rec->nbytes != 0 && in.data == nullptr)
@@ -1613,6 +1624,34 @@ int store_tensor(std::vector<int64_t>& dims64, const axr_tensor_t& in, TensorRec
   rec->address = reinterpret_cast<uint64_t>(in.data) + in.byte_offset;
   return AXR_OK;
 }
+
+// The tensors of a plan under construction, one after the other: an array, or a source that describes
+// them in small lots.
+struct ArraySource {
+  const axr_tensor_t* tensors;
+  bool given() const { return tensors != nullptr; }
+  int get(size_t i, const axr_tensor_t** t) {
+    *t = &tensors[i];
+    return AXR_OK;
+  }
+};
+struct PulledSource {
+  static constexpr size_t kLot = 64;
+  axr_tensor_source* source;
+  size_t held = 0;       // tensors described so far
+  axr_tensor_t lot[kLot];
+  explicit PulledSource(axr_tensor_source* s) : source(s) {}
+  bool given() const { return true; }
+  int get(size_t i, const axr_tensor_t** t) {
+    if (i == held) {
+      const size_t n = std::min(kLot, source->count - held);
+      if (source->describe(source, held, n, lot)) return fail(AXR_ERR_UNSUPPORTED, "tensors that cannot be described here");
+      held += n;
+    }
+    *t = &lot[i % kLot];
+    return AXR_OK;
+  }
+};
 
 }  // namespace
 
@@ -1626,13 +1665,9 @@ int axr_tensor_nbytes(const axr_tensor_t* t, uint64_t* nbytes) {
   return guarded([&] { return tensor_nbytes_body(t, nbytes); });
 }
 
-static int plan_create_body(const axr_tensor_t* tensors, size_t n, uint32_t align, uint32_t flags,
-                            axr_plan_t** plan) {
-  if (!plan) return fail(AXR_ERR_INVALID, "axr_plan_create: null result");
-  *plan = nullptr;
-  if (n && !tensors) return fail(AXR_ERR_INVALID, "axr_plan_create: null tensor array");
-  if (n > 0xffffffffull) return fail(AXR_ERR_INVALID, "axr_plan_create: too many tensors");
-  if (flags != 0) return fail(AXR_ERR_INVALID, "axr_plan_create: flags are reserved and must be 0");
+extern "C++" {
+template <typename Source>
+static int plan_create_body(Source&& source, size_t n, uint32_t align, axr_plan_t** plan) {
   int rc = check_align(align);
   if (rc) return rc;
   PlanInProgress guard(plan_new());
@@ -1650,10 +1685,11 @@ static int plan_create_body(const axr_tensor_t* tensors, size_t n, uint32_t alig
   const uint64_t mask = static_cast<uint64_t>(align) - 1;
   for (size_t i = 0; i < n; ++i) {
     TensorRec& t = p->tensors[i];
-    rc = store_tensor(p->dims64, tensors[i], &t);
-    if (rc) {
-      return rc;
-    }
+    const axr_tensor_t* in = nullptr;
+    rc = source.get(i, &in);
+    if (rc) return rc;
+    rc = store_tensor(p->dims64, *in, &t);
+    if (rc) return rc;
     {
       // room for this record and every fixed part still to come
       const size_t at = static_cast<size_t>(w - h.data());
@@ -1682,10 +1718,10 @@ static int plan_create_body(const axr_tensor_t* tensors, size_t n, uint32_t alig
     std::memcpy(w, &rec, kTensorHeader);
     w += kTensorHeader;
     if (t.ndim == 1) {   // the common case without a call
-      std::memcpy(w, tensors[i].shape, 8);
+      std::memcpy(w, in->shape, 8);
       w += 8;
     } else if (t.ndim) {
-      std::memcpy(w, tensors[i].shape, 8 * static_cast<size_t>(t.ndim));
+      std::memcpy(w, in->shape, 8 * static_cast<size_t>(t.ndim));
       w += 8 * static_cast<size_t>(t.ndim);
     }
   }
@@ -1697,12 +1733,27 @@ static int plan_create_body(const axr_tensor_t* tensors, size_t n, uint32_t alig
   *plan = guard.release();
   return AXR_OK;
 }
+}  // extern "C++"
 int axr_plan_create(const axr_tensor_t* tensors,
                     size_t n,
                     uint32_t align,
                     uint32_t flags,
                     axr_plan_t** plan) {
-  return guarded([&] { return plan_create_body(tensors, n, align, flags, plan); });
+  return guarded([&] {
+    if (!plan) return fail(AXR_ERR_INVALID, "axr_plan_create: null result");
+    *plan = nullptr;
+    if (n && !tensors) return fail(AXR_ERR_INVALID, "axr_plan_create: null tensor array");
+    if (n > 0xffffffffull) return fail(AXR_ERR_INVALID, "axr_plan_create: too many tensors");
+    if (flags != 0) return fail(AXR_ERR_INVALID, "axr_plan_create: flags are reserved and must be 0");
+    return plan_create_body(ArraySource{tensors}, n, align, plan);
+  });
+}
+int axr_plan_create_from(axr_tensor_source* tensors, uint32_t align, axr_plan_t** plan) {
+  return guarded([&] {
+    *plan = nullptr;
+    if (tensors->count > 0xffffffffull) return fail(AXR_ERR_INVALID, "axr_plan_create: too many tensors");
+    return plan_create_body(PulledSource(tensors), tensors->count, align, plan);
+  });
 }
 
 static int plan_free_body(axr_plan_t* plan) {
@@ -1783,18 +1834,20 @@ int axr_plan_tensor_meta(const axr_plan_t* plan, size_t i, axr_tensor_t* meta) {
 
 static int plan_header_body(const axr_plan_t* plan, const void** header, size_t* length) {
   if (!plan || !header || !length) return fail(AXR_ERR_INVALID, "axr_plan_header: null argument");
-  *header = plan->header.data();
-  *length = plan->header.size();
+  *header = plan->borrowed_header ? plan->borrowed_header : plan->header.data();
+  *length = plan->borrowed_header ? plan->borrowed_header_bytes : plan->header.size();
   return AXR_OK;
 }
 int axr_plan_header(const axr_plan_t* plan, const void** header, size_t* length) {
   return guarded([&] { return plan_header_body(plan, header, length); });
 }
 
-// `bound` (may be null): the receiver's tensors, attached in the same pass (axr_plan_from_header
-// followed by axr_plan_bind, without a second walk over the records).
-static int plan_from_header_body(const void* header, size_t length, const axr_tensor_t* bound,
-                                 size_t nbound, bool binding, axr_plan_t** plan) {
+// `source`: the receiver's tensors where `binding` is set, attached in the same pass (axr_plan_from_header
+// followed by axr_plan_bind, without a second walk over the records).  `borrow`: the header stays the caller's.
+extern "C++" {
+template <typename Source>
+static int plan_from_header_body(const void* header, size_t length, Source&& source, size_t nbound, bool binding,
+                                 bool borrow, axr_plan_t** plan) {
   if (!plan) return fail(AXR_ERR_INVALID, "axr_plan_from_header: null result");
   *plan = nullptr;
   if (!header) return fail(AXR_ERR_INVALID, "axr_plan_from_header: null header");
@@ -1811,7 +1864,7 @@ static int plan_from_header_body(const void* header, size_t length, const axr_te
     return fail(AXR_ERR_HEADER, "bundle header truncated");
   if (binding) {
     if (nbound != n) return fail(AXR_ERR_MISMATCH, "axr_plan_from_header_bind: tensor count differs from the header");
-    if (n && !bound) return fail(AXR_ERR_INVALID, "axr_plan_from_header_bind: null tensor array");
+    if (n && !source.given()) return fail(AXR_ERR_INVALID, "axr_plan_from_header_bind: null tensor array");
   }
   PlanInProgress guard(plan_new());
   axr_plan* p = guard.p;
@@ -1852,7 +1905,7 @@ static int plan_from_header_body(const void* header, size_t length, const axr_te
       t.has_strides = false;
       t.shape_at = static_cast<uint32_t>(p->dims64.size());
       if (t.ndim == 1) {
-        p->dims64.push_back(get<int64_t>(h + at));
+        *p->dims64.extend(1) = get<int64_t>(h + at);
       } else if (t.ndim) {
         p->dims64.resize(t.shape_at + static_cast<size_t>(t.ndim));
         std::memcpy(p->dims64.data() + t.shape_at, h + at, 8 * static_cast<size_t>(t.ndim));
@@ -1873,10 +1926,11 @@ static int plan_from_header_body(const void* header, size_t length, const axr_te
     }
     if (binding) {
       const uint32_t sent_item = (static_cast<uint32_t>(t.bits) + 7) / 8;
-      int rc = store_tensor(p->dims64, bound[i], &t);   // size rule, null checks; replaces the record
-      if (rc) {
-        return rc;
-      }
+      const axr_tensor_t* in = nullptr;
+      int rc = source.get(i, &in);
+      if (rc) return rc;
+      rc = store_tensor(p->dims64, *in, &t);   // size rule, null checks; replaces the record
+      if (rc) return rc;
       if (t.nbytes != nb || (nb != 0 && (static_cast<uint32_t>(t.bits) + 7) / 8 != sent_item)) {
         return fail(AXR_ERR_MISMATCH, "axr_plan_from_header_bind: tensor " + std::to_string(i) +
                                           " does not match the header's size or element width");
@@ -1901,18 +1955,27 @@ static int plan_from_header_body(const void* header, size_t length, const axr_te
   }
   p->payload_bytes = end;
   p->data_bytes = data;
-  p->header.assign(h, h + length);
+  if (borrow) {
+    p->borrowed_header = h;
+    p->borrowed_header_bytes = length;
+  } else {
+    p->header.assign(h, h + length);
+  }
   p->bound = binding;
   p->receiver = true;
   *plan = guard.release();
   return AXR_OK;
 }
+}  // extern "C++"
 int axr_plan_from_header(const void* header, size_t length, axr_plan_t** plan) {
-  return guarded([&] { return plan_from_header_body(header, length, nullptr, 0, false, plan); });
+  return guarded([&] { return plan_from_header_body(header, length, ArraySource{nullptr}, 0, false, false, plan); });
 }
 int axr_plan_from_header_bind(const void* header, size_t length, const axr_tensor_t* tensors, size_t n,
                               axr_plan_t** plan) {
-  return guarded([&] { return plan_from_header_body(header, length, tensors, n, true, plan); });
+  return guarded([&] { return plan_from_header_body(header, length, ArraySource{tensors}, n, true, false, plan); });
+}
+int axr_plan_bind_from(const void* header, size_t length, axr_tensor_source* tensors, axr_plan_t** plan) {
+  return guarded([&] { return plan_from_header_body(header, length, PulledSource(tensors), tensors->count, true, true, plan); });
 }
 
 static int plan_bind_body(axr_plan_t* plan, const axr_tensor_t* tensors, size_t n) {
@@ -1923,7 +1986,7 @@ static int plan_bind_body(axr_plan_t* plan, const axr_tensor_t* tensors, size_t 
   // Everything is validated and staged first (in vectors the plan keeps for this): a
   // failure leaves the plan as it was.
   RawVec<TensorRec>& recs = plan->staged_tensors;
-  std::vector<int64_t>& dims64 = plan->staged_dims64;
+  RawVec<int64_t>& dims64 = plan->staged_dims64;
   recs.resize(n);
   dims64.clear();
   dims64.reserve(plan->dims64.size() * 2);

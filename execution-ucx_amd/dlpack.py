@@ -274,6 +274,31 @@ def _plain_tensors(objs: Sequence[Any], exporter: tuple) -> Optional[tuple]:
     return None if direct is None else direct.describe(objs, exporter[2])
 
 
+_PLAN_MAKERS: dict = {}    # library -> addresses of axr_plan_create_from and axr_plan_bind_from
+
+
+def plain_plan(lib, objs: Any, align: int = 0, header: Optional[bytes] = None) -> Optional[tuple]:
+    """A plan made straight from a list or tuple of torch tensors that can be read without asking any
+    of them for a capsule: ``(handle, owners)``.  Without a header the sender's, with one the receiver's,
+    which reads ``header`` in place for as long as it lives.  None for anything else and for what the
+    planner refuses; asking again one step at a time then gives the answer or the error."""
+    if type(objs) is not list and type(objs) is not tuple:
+        return None
+    exporter = _torch_exporter()
+    direct = _native_torch() if exporter else None
+    if direct is None:
+        return None
+    makers = _PLAN_MAKERS.get(lib)
+    if makers is None:
+        makers = _PLAN_MAKERS[lib] = tuple(C.cast(getattr(lib, name), C.c_void_p).value
+                                           for name in ("axr_plan_create_from", "axr_plan_bind_from"))
+    if header is not None:
+        return direct.plan_bind(header, objs, exporter[2], makers[1])
+    if type(align) is not int or not 0 < align <= 4096:
+        return None
+    return direct.plan_create(objs, exporter[2], align, makers[0])
+
+
 def _torch_exporter() -> tuple:
     """``(torch.Tensor, to_dlpack, device)`` for the C helper, or ``()``.
 

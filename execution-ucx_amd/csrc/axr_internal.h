@@ -413,7 +413,8 @@ struct Tunables {
   // that arrived did not match the receiver's plan (and counts down to 0 = off).
   std::atomic<int64_t> transfer_fail_after_send{0};
   std::atomic<int64_t> inline_tables{16384};  // bundles of up to this many tiles whose tables fit the kernel
-                                  // arguments are launched without a table upload; 0: never
+                                  // arguments are launched without a table upload (larger ones
+                                  // outside of captures, see large_inline); 0: never
 };
 Tunables& tunables();
 
@@ -467,8 +468,8 @@ int guarded(Body&& body) noexcept {
 
 int launch_bundle_kernel(bool pack, const KernelArgs& args, const LaunchConfig& cfg,
                          void* stream);
-// Same launch with the tables inside the kernel arguments (default geometry only:
-// 2 KiB tiles, tensor side streaming, payload side cacheable, no die remapping).
+// Same launch with the tables inside the kernel arguments (two geometries only: 2 KiB tiles, tensor side
+// streaming, payload side cacheable; runs in tiles of 1 KiB, both sides streaming; no die remapping).
 int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchConfig& cfg,
                                 const InlineTables& tables, uint32_t dims_at, uint32_t wave_at,
                                 void* stream);

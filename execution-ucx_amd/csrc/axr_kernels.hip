@@ -1682,7 +1682,7 @@ struct InlineScalars {   // mirrors the argument list of bundle_kernel_inline
 constexpr uint32_t kInlineTablesOffset = __builtin_offsetof(InlineScalars, tables);
 static_assert(kInlineTablesOffset == 48 && alignof(InlineTables) == 16, "kernarg layout");
 
-template <bool PACK, uint32_t KIND>
+template <bool PACK, uint32_t KIND, uint32_t ROWS, bool NTP>
 __global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, 2))))
 __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThreads) void bundle_kernel_inline(
     uint8_t* payload_arg, uint32_t ntiles, uint32_t tiles_per_wave, uint32_t xcd_remap,
@@ -1698,8 +1698,8 @@ __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThrea
   a.xcd_remap = xcd_remap;
   a.seg_shift = seg_shift;
   a.tensor_delta = 0;
-  // tensor side streaming, payload side cacheable: what small bundles use
-  bundle_body<PACK, 2, true, false, KIND>(
+  // tensor side streaming; the payload side cacheable in 2 KiB tiles, streaming in tiles of 1 KiB
+  bundle_body<PACK, ROWS, true, NTP, KIND>(
       reinterpret_cast<seg_table>(base + kInlineTablesHead),
       reinterpret_cast<dims_table>(base + kInlineTablesHead + dims_at),
       reinterpret_cast<const AXR_CONST uint32_t*>(base + kInlineTablesHead + wave_at),
@@ -2124,8 +2124,9 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
                                 const InlineTables& tables, uint32_t dims_at, uint32_t wave_at,
                                 void* stream) {
   if (args.ntiles == 0 || cfg.workgroups == 0) return AXR_OK;
-  if (cfg.tile_rows != 2 || (cfg.nontemporal & 3u) != 1u || args.xcd_remap)
-    return fail(AXR_ERR_INVALID, "inline tables go with the default launch geometry only");
+  const bool streaming = cfg.tile_rows == 1 && (cfg.nontemporal & 3u) == 3u && !cfg.elements;
+  if ((!streaming && (cfg.tile_rows != 2 || (cfg.nontemporal & 3u) != 1u)) || args.xcd_remap)
+    return fail(AXR_ERR_INVALID, "inline tables go with two launch geometries only");
   if (cfg.threads == 0 || cfg.threads % kWaveLanes ||
       cfg.threads > (cfg.elements ? kMaxElementThreads : kMaxThreadsPerWorkgroup))
     return fail(AXR_ERR_INVALID, "workgroup size does not fit the kernel");
@@ -2140,16 +2141,18 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
   const dim3 grid(cfg.workgroups), block(cfg.threads);
   const uint32_t lds_bytes = cfg.elements ? cfg.lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define AXR_INLINE_LAUNCH(PACK, KIND)                                                             \
-  hipLaunchKernelGGL((bundle_kernel_inline<PACK, KIND>), grid, block, lds_bytes, s, args.payload,  \
+#define AXR_INLINE_LAUNCH(PACK, KIND, ROWS, NTP)                                                  \
+  hipLaunchKernelGGL((bundle_kernel_inline<PACK, KIND, ROWS, NTP>), grid, block, lds_bytes, s, args.payload,  \
                      args.ntiles, args.tiles_per_wave, args.xcd_remap, args.seg_shift,            \
                      cfg.lds_per_wave, hint_argument(cfg), dims_at, wave_at, tables)
-  if (!cfg.elements) {
-    if (pack) AXR_INLINE_LAUNCH(true, kKindRuns); else AXR_INLINE_LAUNCH(false, kKindRuns);
+  if (streaming) {
+    if (pack) AXR_INLINE_LAUNCH(true, kKindRuns, 1, true); else AXR_INLINE_LAUNCH(false, kKindRuns, 1, true);
+  } else if (!cfg.elements) {
+    if (pack) AXR_INLINE_LAUNCH(true, kKindRuns, 2, false); else AXR_INLINE_LAUNCH(false, kKindRuns, 2, false);
   } else if (cfg.kind == kModeRows) {
-    if (pack) AXR_INLINE_LAUNCH(true, kModeRows); else AXR_INLINE_LAUNCH(false, kModeRows);
+    if (pack) AXR_INLINE_LAUNCH(true, kModeRows, 2, false); else AXR_INLINE_LAUNCH(false, kModeRows, 2, false);
   } else {
-    if (pack) AXR_INLINE_LAUNCH(true, kKindAny); else AXR_INLINE_LAUNCH(false, kKindAny);
+    if (pack) AXR_INLINE_LAUNCH(true, kKindAny, 2, false); else AXR_INLINE_LAUNCH(false, kKindAny, 2, false);
   }
 #undef AXR_INLINE_LAUNCH
   return check_hip(hipGetLastError(), "bundle kernel launch (inline tables)");

@@ -1163,6 +1163,21 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
   return AXR_OK;
 }
 
+// Bundles of few large tensors, in 2 KiB tiles or streaming in tiles of 1 KiB, may carry their tables in the
+// arguments of their first launch as small bundles do, where nothing is captured.  An upload is a launch,
+// an event behind it and a wait for both in front of the bundle kernel: the nine bf16 weights of a layer,
+// fresh, pack + unpack, 284 us uploaded / 273 in the arguments at 405 MB, 223 / 213 at 306 MB, 94 / 82.5 at
+// 101 MB.  (Views keep their tables on the device: a bundle of theirs this large is better off with the
+// kernel for their mode, see waves_of_kind.)
+constexpr size_t kInlineWalk = 4;
+bool large_inline(const axr_plan* p) {
+  const int64_t limit = tunables().inline_tables;
+  const uint32_t hints = p->cfg.nontemporal & 3u;
+  return limit > 0 && p->ntiles > static_cast<uint64_t>(limit) && !p->cfg.elements && !p->cfg.xcd_remap &&
+         p->cfg.seg_shift < kGroupBlocksShift &&
+         ((p->cfg.tile_rows == 1 && hints == 3u) || (p->cfg.tile_rows == 2 && hints == 1u));
+}
+
 // Tables for a launch on `stream`: what is there already, else built by the device when the
 // bundle qualifies and the stream is not capturing, else built on the host.
 int ensure_tables(axr_plan* p, hipStream_t stream, bool capturing) {
@@ -1316,6 +1331,22 @@ int build_tables(axr_plan* p) {
   // records and the index
   p->groups_only = nseg != 0 && p->group_blocks.size() == nseg * kGroupBlockBytes;
   if (p->groups_only) p->cfg.seg_shift = kGroupBlocksShift;
+
+  // A large bundle takes wider blocks where its tables then fit the kernel arguments and no block holds
+  // more than kInlineWalk segments besides the one that it begins in (a long tensor among many short ones
+  // keeps its narrow blocks: a wavefront walks the segments one by one).
+  if (large_inline(p)) {
+    uint32_t wide = p->cfg.seg_shift;
+    auto bytes_at = [&](uint32_t s) {
+      return align_up(align_up(p->segs.size() * sizeof(Seg), 16) + p->dims.size() * sizeof(Dims), 16) +
+             align_up(((static_cast<size_t>(p->ntiles) >> s) + 1) * sizeof(uint32_t), 16) + p->group_blocks.size();
+    };
+    while (wide < 31 && bytes_at(wide) + kInlineTablesHead > kInlineTableBytes && (p->ntiles >> wide) != 0) ++wide;
+    bool near = bytes_at(wide) + kInlineTablesHead <= kInlineTableBytes;
+    for (size_t i = kInlineWalk; i < nseg && near; ++i)
+      near = p->segs[i - kInlineWalk].tile_begin >> wide != p->segs[i].tile_begin >> wide;
+    if (near) p->cfg.seg_shift = wide;
+  }
 
   // Tile-block index: entry k = segment that holds tile k << seg_shift.  Blocks
   // are sized to about one segment each (a power of two, at most 256 tiles), so
@@ -1481,9 +1512,11 @@ int move_host_tensors(axr_plan* p, bool pack, uint8_t* payload, hipStream_t stre
 }
 
 // Small bundles with the default launch geometry can carry their tables inside the
-// kernel arguments (3.5 KiB at most) instead of a device block.
-bool tables_fit_kernel_arguments(const axr_plan* p) {
+// kernel arguments (3.5 KiB at most) instead of a device block.  `small_only`: not the large
+// ones, which need axr_plan_prepare before they are captured and the static area without allocation.
+bool tables_fit_kernel_arguments(const axr_plan* p, bool small_only = true) {
   const int64_t limit = tunables().inline_tables;
+  if (!small_only && p->tables_built && p->table_bytes + kInlineTablesHead <= kInlineTableBytes && large_inline(p)) return true;
   return limit > 0 && p->tables_built && p->ntiles <= static_cast<uint64_t>(limit) &&
          p->table_bytes + kInlineTablesHead <= kInlineTableBytes && p->cfg.tile_rows == 2 &&
          (p->cfg.nontemporal & 3u) == 1u && !p->cfg.xcd_remap;
@@ -1552,7 +1585,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   LaunchConfig cfg = p->cfg;
   cfg.nontemporal = effective_nontemporal(p, job_flags);
   if (delta == 0 && cfg.nontemporal == (p->cfg.nontemporal & 3u) &&
-      (capturing ? !p->resident : p->launches == 0 && !p->uploaded) && tables_fit_kernel_arguments(p)) {
+      (capturing ? !p->resident : p->launches == 0 && !p->uploaded) && tables_fit_kernel_arguments(p, capturing)) {
     // Small bundle, first launch: the tables ride in the kernel arguments.  The launch
     // owns its copy, so a capturing stream may record it.  A plan that is launched again
     // is being reused: from the second launch on it pays one upload and then the shorter

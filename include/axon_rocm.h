@@ -379,8 +379,8 @@ typedef struct axr_launch_info {
   uint32_t host_copies;    /* contiguous pieces of kDLCPU tensors              */
   uint32_t host_chunks;    /* device copies that move them (pinned staging)    */
   uint32_t inline_tables;  /* 1: the next launch carries the tables inside the
-                              kernel arguments (small bundle, first launch:
-                              no upload, no device block)                      */
+                              kernel arguments, captured or not (small bundle,
+                              first launch: no upload, no device block)        */
   uint32_t reserved;
 } axr_launch_info_t;
 AXR_API int axr_plan_launch_info(axr_plan_t* plan, axr_launch_info_t* info);
@@ -472,7 +472,8 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * "inline_tables" (the first launch of a bundle of at most this many tiles
  * whose tables fit into 3.5 KiB carries the tables inside the kernel arguments:
  * no table block and no upload; a plan that is launched again uploads its
- * tables then; 0 switches that off; read at every
+ * tables then; compact tensors and long strided runs do so beyond it as well
+ * unless they are captured; 0 switches all that off; read at every
  * axr_pack / axr_unpack).  Unknown key -> AXR_ERR_INVALID. */
 AXR_API int axr_tune_set(const char* key, int64_t value);
 AXR_API int axr_tune_get(const char* key, int64_t* value);

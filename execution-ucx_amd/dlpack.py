@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import ctypes as C
 import itertools
+import sys
 from dataclasses import dataclass
 from typing import Any, Callable, List, Optional, Sequence, Tuple
 
@@ -132,7 +133,6 @@ class NotDLPackError(TypeError, RuntimeError):
 
 
 def _is_framework_tensor(obj: Any) -> bool:
-    import sys
     torch = sys.modules.get("torch")
     return torch is not None and isinstance(obj, torch.Tensor)
 
@@ -270,8 +270,18 @@ class TensorArray:
 
 def _plain_tensors(objs: Sequence[Any], exporter: tuple) -> Optional[tuple]:
     """A bundle of plain torch tensors is read without one capsule per tensor."""
+    if type(objs) is list and not _plain_start(objs):
+        return None
     direct = _native_torch() if exporter else None
     return None if direct is None else direct.describe(objs, exporter[2])
+
+
+def _plain_start(objs: Any) -> bool:
+    """Whether asking for plain tensors is worth the attempt: not for a list of another library's arrays."""
+    torch = sys.modules.get("torch")
+    if torch is None:
+        return False
+    return not objs or type(objs[0]) is torch.Tensor or type(objs[0]) is torch.nn.Parameter
 
 
 _PLAN_MAKERS: dict = {}    # library -> addresses of axr_plan_create_from and axr_plan_bind_from
@@ -282,7 +292,7 @@ def plain_plan(lib, objs: Any, align: int = 0, header: Optional[bytes] = None) -
     of them for a capsule: ``(handle, owners)``.  Without a header the sender's, with one the receiver's,
     which reads ``header`` in place for as long as it lives.  None for anything else and for what the
     planner refuses; asking again one step at a time then gives the answer or the error."""
-    if type(objs) is not list and type(objs) is not tuple:
+    if (type(objs) is not list and type(objs) is not tuple) or not _plain_start(objs):
         return None
     exporter = _torch_exporter()
     direct = _native_torch() if exporter else None
@@ -310,7 +320,6 @@ def _torch_exporter() -> tuple:
     default stream, which is checked here once per bundle.  Anywhere else every
     tensor goes through ``__dlpack__()``.
     """
-    import sys
     torch = sys.modules.get("torch")
     if torch is None:
         return ()

@@ -511,8 +511,11 @@ void table_block_release(TableBlock* block);
 // Events without timing for the current device, recycled: creating one costs more than a
 // microsecond, and every fresh plan that uploads tables needs one.  An event goes back
 // only once it has fired (or was never recorded).
-int event_acquire(void** event, int* device);
-void event_release(void* event, int device);
+// device_scope: an event that makes what kernels wrote to device memory visible to kernels of other
+// streams, and nothing to the host or of the copy engine's.  The kernel behind it starts 2 us
+// sooner (48 cache blocks of 32 runs, fresh, pack + unpack, 44.5 -> 40.8 us).
+int event_acquire(bool device_scope, void** event, int* device);
+void event_release(bool device_scope, void* event, int device);
 
 }  // namespace axr
 

@@ -211,6 +211,7 @@ struct axr_plan {
   uint64_t launches = 0;             // kernel launches since the tables were built
   hipEvent_t upload_event = nullptr;   // from event_acquire; behind the latest upload once `uploaded` is set
   int upload_event_device = -1;
+  bool upload_event_by_kernel = false;   // a device-scope event: a kernel wrote the tables
   hipStream_t upload_stream = nullptr;
   struct BusyStream {
     hipStream_t stream;
@@ -963,11 +964,16 @@ uint32_t rows_for_compact_bundle(const axr_plan* p) {
 // another stream waits for is recorded here, right behind the upload, on the default stream as on any
 // other: recorded later it would lie behind whatever the stream was given in between, and a launch
 // elsewhere would wait for work that is not its own.
-int note_upload(axr_plan* p, hipStream_t stream) {
+int note_upload(axr_plan* p, hipStream_t stream, bool by_kernel = true) {
   remember_stream(p, stream);
+  if (p->upload_event && p->upload_event_by_kernel != by_kernel) {   // (an earlier upload's, drained before its block was reused)
+    event_release(p->upload_event_by_kernel, p->upload_event, p->upload_event_device);
+    p->upload_event = nullptr;
+  }
   if (!p->upload_event) {
-    int rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
+    int rc = event_acquire(by_kernel, reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
     if (rc) return rc;
+    p->upload_event_by_kernel = by_kernel;
   }
   int rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
   if (rc) return rc;
@@ -1413,12 +1419,13 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
       quiesce(p);   // previous launches may still read the old tables
     }
     write_tables(p, static_cast<uint8_t*>(p->block.host));
-    int rc = p->table_bytes <= kKernelUploadBytes
+    const bool by_kernel = p->table_bytes <= kKernelUploadBytes;
+    int rc = by_kernel
                  ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
                  : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
                              "hipMemcpyAsync(plan tables)");
     if (rc) return rc;
-    return note_upload(p, stream);
+    return note_upload(p, stream, by_kernel);
   }
   if (stream != p->upload_stream)
     return check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
@@ -1793,7 +1800,7 @@ static int plan_free_body(axr_plan_t* plan) {
   if (!plan) return AXR_OK;
   quiesce(plan);
   table_block_release(&plan->block);
-  event_release(plan->upload_event, plan->upload_event_device);   // fired: the upload's stream has been drained
+  event_release(plan->upload_event_by_kernel, plan->upload_event, plan->upload_event_device);   // fired: the upload's stream has been drained
   plan->upload_event = nullptr;
   for (HostStage& st : plan->stage) {
     table_block_release(&st.block);

@@ -1,0 +1,60 @@
+"""Plans whose tables went up on one stream, launched on others that have to wait for them."""
+import ctypes as C
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+
+# views and records go up by a kernel, groups are laid out by one, long tables go up by the copy engine
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["views", "records", "groups", "long"])
+def test_streams_find_the_tables_of_another_stream(pkg, gpu, kind):
+    """Fresh plans over and over in recycled table blocks, so that tables read too early or out of a
+    cache would be those of the plan before; the same plan is then bound anew."""
+    lib, capi = pkg._capi.load(), pkg._capi
+    streams = []
+    for _ in range(3):
+        s = C.c_void_p()
+        capi.check(lib.axr_stream_create(C.byref(s)))
+        streams.append(s.value)
+    parent = torch.randint(0, 256, (700, 9, 2048), dtype=torch.uint8, device=gpu)
+    flat = parent.view(-1)
+
+    def tensors(k):
+        if kind == "views":
+            return [parent[i, 1:, :1400 + (i + k) % 7] for i in range(200)]
+        if kind == "records":
+            return [parent[i, 0, :2000 + (i + k) % 48] for i in range(700)]
+        if kind == "groups":
+            return [parent[i, 0, :100 + (i + k) % 48] for i in range(700)]
+        return [flat[40 * i:40 * i + 21 + (i + k) % 17] for i in range(20000)] + [parent[:3, ::2, :1500 + k]]
+
+    def want(ts, plan):
+        out = torch.zeros(plan.payload_bytes, dtype=torch.uint8, device=gpu)
+        for t, at, n in zip(ts, *plan.layout()):
+            out[at:at + n] = t.reshape(-1)
+        return out
+
+    for k in range(6 if kind != "long" else 2):
+        ts = tensors(k)
+        with pkg.BundlePlan.create(ts, align=16) as plan:
+            expect = want(ts, plan)
+            outs = [torch.zeros_like(expect) for _ in range(4)]
+            torch.cuda.synchronize()
+            for out, s in zip(outs, [None] + streams):
+                plan.pack(out.data_ptr(), out.numel(), s, order=False)
+            torch.cuda.synchronize()
+            assert all(torch.equal(out, expect) for out in outs)
+            if kind == "long":
+                continue
+            plan.bind([t.clone() for t in ts])    # tables anew, uploaded on another stream
+            for out in outs:
+                out.zero_()
+            torch.cuda.synchronize()
+            for out, s in zip(outs, streams + [None]):
+                plan.pack(out.data_ptr(), out.numel(), s, order=False)
+            torch.cuda.synchronize()
+            assert all(torch.equal(out, expect) for out in outs)
+    for s in streams:
+        capi.check(lib.axr_stream_destroy(s))

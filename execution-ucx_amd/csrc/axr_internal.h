@@ -345,6 +345,8 @@ struct LaunchConfig {
   bool elements = false;   // some segment uses kModeElements or is transposed
   uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (transposed tiles only)
+  uint32_t cached_tail = 0;    // MiB at the end of a streaming payload that a pack leaves in the cache (runs in
+                           // 1 KiB tiles only; see finish_geometry)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
                            // multiple of 8 such runs)
 };

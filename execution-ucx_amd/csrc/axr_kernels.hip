@@ -1408,6 +1408,9 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
                                             const KernelArgs& a, uint32_t wg, uint32_t lds_per_wave,
                                             uint32_t nt_bits) {
   constexpr bool runs = KIND == kKindRuns || KIND == kKindAny;   // runs, groups and fills may occur
+  // Where a payload that streams is packed in tiles of 1 KiB, `lds_per_wave` says how many MiB at its end are
+  // written with ordinary stores all the same (LaunchConfig::cached_tail; runs need no LDS).
+  constexpr bool tail_stays = PACK && KIND == kKindRuns && ROWS == 1 && NTT && NTP;
   constexpr uint32_t kTile = ROWS * kRowBytes;
   uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   uint32_t lane_off = lane * kVecBytes;
@@ -1430,6 +1433,22 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   const uint32_t t_end =
       (a.ntiles - t > a.tiles_per_wave) ? t + a.tiles_per_wave : a.ntiles;
   const uint64_t delta = static_cast<uint64_t>(a.tensor_delta);
+  // a whole tile or what is left of a run, at `ten` in the tensor and at `pay` in the payload
+  auto copy = [&](gbytes ten, gbytes pay, uint64_t left) {
+    if constexpr (KIND == kKindAny) {
+      copy_tile_hinted<PACK, ROWS>(ten, pay, left, lane, lane_off, nt_bits);
+    } else if constexpr (tail_stays) {
+      if (a.ntiles - t <= lds_per_wave << 10) {   // (asm: as in copy_tile_hinted)
+        asm volatile("");
+        copy_tile<PACK, ROWS, NTT, false>(ten, pay, left, lane, lane_off);
+        asm volatile("");
+      } else {
+        copy_tile<PACK, ROWS, NTT, true>(ten, pay, left, lane, lane_off);
+      }
+    } else {
+      copy_tile<PACK, ROWS, NTT, NTP>(ten, pay, left, lane, lane_off);
+    }
+  };
   if (runs && a.seg_shift == kGroupBlocksShift) {
     // a bundle of group tiles only: tile t's block lies at a fixed stride behind `dims`
     const AXR_CONST uint8_t* blocks = reinterpret_cast<const AXR_CONST uint8_t*>(dims);
@@ -1480,8 +1499,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         else if constexpr (PACK) wave_copy_partial<1, NTT, NTP>(ten, pay, head, lane, lane_off);
         else wave_copy_partial<1, NTP, NTT>(pay, ten, head, lane, lane_off);
       }
-      if constexpr (KIND == kKindAny) copy_tile_hinted<PACK, ROWS>(ten + boff, pay + boff, left, lane, lane_off, nt_bits);
-      else copy_tile<PACK, ROWS, NTT, NTP>(ten + boff, pay + boff, left, lane, lane_off);
+      copy(ten + boff, pay + boff, left);
       if constexpr (PACK) {
         if (last && pad) wave_zero(pay + run, pad, lane);
       }
@@ -1504,8 +1522,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         const uint64_t left = seg_run - boff;
         gbytes ten = as_global(seg_ptr) + run_offset(dm, run) + boff;
         gbytes p = pay + static_cast<uint64_t>(run) * seg_run + boff;
-        if constexpr (KIND == kKindAny) copy_tile_hinted<PACK, ROWS>(ten, p, left, lane, lane_off, nt_bits);
-        else copy_tile<PACK, ROWS, NTT, NTP>(ten, p, left, lane, lane_off);
+        copy(ten, p, left);
       } else if constexpr (KIND != kKindRuns) {
         extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
         lbytes lds = (lbytes)lds_slices + uniform(threadIdx.x >> 6) * lds_per_wave;
@@ -1985,10 +2002,11 @@ template <bool PACK, uint32_t ROWS>
 int launch_rows(const KernelArgs& args, const LaunchConfig& cfg, hipStream_t stream) {
   const dim3 grid(cfg.workgroups), block(cfg.threads);
   const uint32_t lds_bytes = cfg.elements ? cfg.lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
-  if (cfg.lds_per_wave > 0x1ffffu || args.seg_shift > 0xffu || cfg.threads / kWaveLanes > 0x1fu)
+  const uint32_t low = cfg.elements ? cfg.lds_per_wave : cfg.cached_tail;
+  if (low > 0x1ffffu || args.seg_shift > 0xffu || cfg.threads / kWaveLanes > 0x1fu)
     return fail(AXR_ERR_INVALID, "launch geometry does not fit the kernel's geometry argument");
-  // LDS bytes per wavefront | hints << 17 | wavefronts per workgroup << 19 | tile-block shift << 24
-  const uint32_t geometry = cfg.lds_per_wave | (cfg.nontemporal & 3u) << 17 |
+  // LDS bytes per wavefront, or MiB of cached tail | hints << 17 | wavefronts per workgroup << 19 | tile-block shift << 24
+  const uint32_t geometry = low | (cfg.nontemporal & 3u) << 17 |
                             (cfg.threads / kWaveLanes) << 19 | args.seg_shift << 24;
 #define AXR_ARGS args.segs, args.dims, args.wave_seg, args.payload, args.ntiles, args.tiles_per_wave, args.xcd_remap, geometry, args.tensor_delta
 #define AXR_VIEWS(KIND) hipLaunchKernelGGL((views_kernel<PACK, ROWS, KIND>), grid, block, lds_bytes, stream, AXR_ARGS)
@@ -2144,7 +2162,7 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
 #define AXR_INLINE_LAUNCH(PACK, KIND, ROWS, NTP)                                                  \
   hipLaunchKernelGGL((bundle_kernel_inline<PACK, KIND, ROWS, NTP>), grid, block, lds_bytes, s, args.payload,  \
                      args.ntiles, args.tiles_per_wave, args.xcd_remap, args.seg_shift,            \
-                     cfg.lds_per_wave, hint_argument(cfg), dims_at, wave_at, tables)
+                     cfg.elements ? cfg.lds_per_wave : cfg.cached_tail, hint_argument(cfg), dims_at, wave_at, tables)
   if (streaming) {
     if (pack) AXR_INLINE_LAUNCH(true, kKindRuns, 1, true); else AXR_INLINE_LAUNCH(false, kKindRuns, 1, true);
   } else if (!cfg.elements) {

@@ -940,6 +940,19 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   } else {
     p->cfg.nontemporal = static_cast<uint32_t>(tn.nontemporal) & 3u;
   }
+  // The last-level cache has room for a part of a payload that streams: the sender writes the end of it with
+  // ordinary stores, and whoever reads the payload next finds that part there (an unpack reads it streaming
+  // like the rest, which leaves it in place until it is read: with ordinary loads it was evicted first, 249
+  // instead of 238 us below).  7/8 of the cache: from about 15/16 on, depending on what else is in use, the end
+  // evicts its own beginning.  Pack + unpack of the nine bf16 weights of a layer, three bundles in turn, all
+  // streaming / 160 / 192 / 224 / 240 / 250 MiB kept: 405 MB 248.5 / 242 / 240 / 237 / 236 / 235 us, one bundle
+  // over and over 247.5 / 242.5 / 240.6 / 237.7 / 236.5 / 246; 419 MB of cache blocks 268 / 264 / 262 / 259 / 258 /
+  // 279; 1 GiB of compact tensors 649 / - / 639 / 638 / 636 / -.  A pack whose payload nobody reads takes 129
+  // instead of 125 us at 405 MB: it writes back what an earlier one left.
+  p->cfg.cached_tail = 0;
+  if (rows == 1 && !p->cfg.elements && p->cfg.nontemporal == 3u && tn.nontemporal < 0)
+    p->cfg.cached_tail = static_cast<uint32_t>(
+        std::min<uint64_t>(static_cast<uint64_t>(tn.payload_cache_bytes) / 8 * 7, p->payload_bytes) >> 20);
   uint32_t shift = 0;
   while (shift < 8 && (static_cast<uint64_t>(nseg) << (shift + 1)) <= p->ntiles) ++shift;
   // as many tiles as segments (none without a tile): tile t is segment t, no index to consult
@@ -1591,6 +1604,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   a.tensor_delta = delta;
   LaunchConfig cfg = p->cfg;
   cfg.nontemporal = effective_nontemporal(p, job_flags);
+  if (job_flags & AXR_JOB_PAYLOAD_STREAMING) cfg.cached_tail = 0;   // asked for: all of it streams
   if (delta == 0 && cfg.nontemporal == (p->cfg.nontemporal & 3u) &&
       (capturing ? !p->resident : p->launches == 0 && !p->uploaded) && tables_fit_kernel_arguments(p, capturing)) {
     // Small bundle, first launch: the tables ride in the kernel arguments.  The launch
@@ -1599,7 +1613,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
     // argument list (a 3.5 KiB argument costs 0.4 us per launch, the upload 4 us on the
     // host and 4 us on the device, once).
     if (!p->inline_ready) fill_inline_tables(p);
-    rc = launch_bundle_kernel_inline(pack, a, p->cfg, *p->inline_tables,
+    rc = launch_bundle_kernel_inline(pack, a, cfg, *p->inline_tables,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
     if (rc) return rc;

@@ -428,7 +428,9 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * payload_cache_bytes and max_tiles KiB, which stream to and from memory), "max_tiles",
  * "max_waves", "threads" (workgroup size; 0 = automatic: 256 below 65,536 tiles, 128 above, 64
  * with the automatic 1 KiB tiles), "nontemporal" (-1 auto, or bit 0
- * tensor side / bit 1 payload side), "payload_cache_bytes", "gather_run_bytes",
+ * tensor side / bit 1 payload side), "payload_cache_bytes" (of a larger payload that moves
+ * in 1 KiB tiles the last 7/8 of as many bytes stay cacheable when it is packed),
+ * "gather_run_bytes",
  * "xcd_remap" (each accelerator die walks one contiguous share of the tiles: 1 always,
  * 0 never, -1 (default) for bundles made mostly of transposed views whose rows do not
  * start on 128-byte lines, where neighbouring blocks then meet in one L2),

@@ -391,8 +391,10 @@ struct Tunables {
   std::atomic<int64_t> loopback_copy_kernel{1};
   // Bundles of at least this many tensors, all of them contiguous device tensors, get their
   // tables in one pass over the tensors into pinned memory plus a kernel that brings them to
-  // the device and writes the tile-block index (0: the general host path always).
-  std::atomic<int64_t> device_tables{512};
+  // the device and writes the tile-block index (0: the general host path always).  Fresh bundles of 256 B
+  // to 64 KiB, pack + unpack, host / device tables: 256 tensors 49.1 / 49.7 us, 300 51.8 / 51.5, 360 55.9 / 53.9,
+  // 420 59.7 / 56.4; of 600 to 4000 bytes 300 49.2 / 51.4, 480 60.8 / 58.9.
+  std::atomic<int64_t> device_tables{320};
   // axr_stream_synchronize may first poll, for up to this many microseconds, a word of pinned
   // memory that a one-wave kernel enqueued behind the stream's work writes, before it falls
   // back to the runtime's wait (0, the default: the runtime's wait only).  See the header.
@@ -416,7 +418,8 @@ struct Tunables {
   std::atomic<int64_t> transfer_fail_after_send{0};
   std::atomic<int64_t> inline_tables{16384};  // bundles of up to this many tiles whose tables fit the kernel
                                   // arguments are launched without a table upload (larger ones
-                                  // outside of captures, see large_inline); 0: never
+                                  // outside of captures, see large_inline), and read theirs in pinned
+                                  // memory (see first_launch_reads_host_block); 0: never
 };
 Tunables& tunables();
 

@@ -204,6 +204,7 @@ struct axr_plan {
   size_t table_bytes = 0;
   size_t dims_at = 0, wave_at = 0, members_at = 0;
   bool uploaded = false;
+  bool tables_in_host_block = false;   // block.host holds the tables (a first launch has read them there)
   bool resident = false;             // upload known to be complete (axr_plan_prepare)
   size_t stage_bytes = 0;            // longest host chunk: size of the staging blocks
   std::unique_ptr<InlineTables> inline_tables;   // the tables as a kernel argument (small bundles)
@@ -361,6 +362,7 @@ void invalidate_tables(axr_plan* p) {
   p->tables_built = false;
   p->device_built = false;
   p->uploaded = false;
+  p->tables_in_host_block = false;
   p->resident = false;
   p->inline_ready = false;
   p->launches = 0;
@@ -1116,7 +1118,11 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
       all_device = all_device && (t.device_type == kDLROCM || t.device_type == kDLROCMHost);
     }
     if (!all_device) return AXR_OK;   // before a block is taken: host tensors need no tables on the device
-    if (small == n) return device_build_groups(p, stream, done);
+    if (small == n) {
+      // only from 1.6 times as many on: fresh, pack + unpack, groups from the host, read there / from the device,
+      // 330 tensors of 8 to 512 bytes 47.8 / 55.2 us, 500 57.0 / 62.7, 700 (more than 32 KiB) 76 / 72
+      return n * 5 >= static_cast<uint64_t>(least) * 8 ? device_build_groups(p, stream, done) : AXR_OK;
+    }
     if (small * 4 >= n) return AXR_OK;
   }
   const uint32_t rows = rows_for_compact_bundle(p);
@@ -1418,25 +1424,47 @@ void write_tables(const axr_plan* p, uint8_t* h) {
 // short tensors and a long one, 2.6 MB, 672 / 656).
 constexpr size_t kKernelUploadBytes = 1u << 20;
 
+// Puts the host-built tables into the pinned half of the plan's table block.
+int write_host_block(axr_plan* p) {
+  if (p->tables_in_host_block) return AXR_OK;
+  if (p->block.host && (p->block.bytes < p->table_bytes)) {
+    quiesce(p);
+    table_block_release(&p->block);
+  }
+  if (!p->block.host) {
+    int rc = table_block_acquire(p->table_bytes, &p->block);
+    if (rc) return rc;
+  } else {
+    quiesce(p);   // previous launches may still read the old tables
+  }
+  write_tables(p, static_cast<uint8_t*>(p->block.host));
+  p->tables_in_host_block = true;
+  return AXR_OK;
+}
+
+// Whether a plan's first launch reads its host-built tables where the host has written them.  Every wavefront
+// then waits for the bus instead of for a cache, but the upload, the event behind it and the wait for both
+// go, about 5 us of a fresh bundle's round trip, pack + unpack, uploaded / read in place: 128 tensors of 256 B to
+// 64 KiB 47.0 / 42.1 us, 200 49.9 / 45.6, 300 56.2 / 51.7, 300 of 64 KiB 54.7 / 51.3, 256 cache blocks of 16 runs
+// 62.9 / 58.5.  Not where a wavefront reads a view's own record as well (140 views that all differ, 64 rows of 300
+// bytes each, 53.3 / 55.9; 100 rows of 2000 bytes 69.2 / 80.4), and with many wavefronts the reads add up (512
+// blocks of 64 runs, 1 GiB, 745 / 860).  A plan that is launched again is being reused and uploads then.
+constexpr size_t kHostTableBytes = 32u << 10;
+bool first_launch_reads_host_block(const axr_plan* p) {
+  const int64_t limit = tunables().inline_tables;
+  return p->launches == 0 && !p->uploaded && p->tables_built && p->table_bytes <= kHostTableBytes &&
+         limit > 0 && p->ntiles <= static_cast<uint64_t>(limit) && !p->cfg.elements && p->dims.size() <= 1;
+}
+
 int ensure_uploaded(axr_plan* p, hipStream_t stream) {
   if (p->ntiles == 0) return AXR_OK;
   if (!p->uploaded) {
-    if (p->block.host && (p->block.bytes < p->table_bytes)) {
-      quiesce(p);
-      table_block_release(&p->block);
-    }
-    if (!p->block.host) {
-      int rc = table_block_acquire(p->table_bytes, &p->block);
-      if (rc) return rc;
-    } else {
-      quiesce(p);   // previous launches may still read the old tables
-    }
-    write_tables(p, static_cast<uint8_t*>(p->block.host));
+    int rc = write_host_block(p);
+    if (rc) return rc;
     const bool by_kernel = p->table_bytes <= kKernelUploadBytes;
-    int rc = by_kernel
-                 ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
-                 : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
-                             "hipMemcpyAsync(plan tables)");
+    rc = by_kernel ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
+                   : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
+                               "hipMemcpyAsync(plan tables)");
     if (rc) return rc;
     return note_upload(p, stream, by_kernel);
   }
@@ -1627,11 +1655,15 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   }
   if (capturing && !p->resident)
     return fail(AXR_ERR_INVALID, "call axr_plan_prepare before capturing this plan in a graph");
-  if (!p->resident) {
-    rc = ensure_uploaded(p, stream);
-    if (rc) return rc;
+  uint8_t* d;
+  if (!capturing && !p->resident && first_launch_reads_host_block(p)) {
+    rc = write_host_block(p);
+    d = static_cast<uint8_t*>(p->block.host);
+  } else {
+    if (!p->resident) rc = ensure_uploaded(p, stream);
+    d = static_cast<uint8_t*>(p->block.device);
   }
-  uint8_t* d = static_cast<uint8_t*>(p->block.device);
+  if (rc) return rc;
   a.segs = reinterpret_cast<const Seg*>(d);
   a.dims = reinterpret_cast<const Dims*>(d + dims_arg_at(p));
   a.wave_seg = reinterpret_cast<const uint32_t*>(d + p->wave_at);

@@ -457,8 +457,8 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * "device_tables" (a bundle of at least this many tensors, all contiguous device
  * tensors, takes a short path to its device tables: one pass over the tensors into
  * pinned memory and a kernel that brings the records to the device and writes the
- * tile-block index, instead of the general host build plus an upload; default 512,
- * 0: never),
+ * tile-block index, instead of the general host build plus an upload; default 320,
+ * 1.6 times as many where all are short; 0: never),
  * "loopback_copy_kernel" (1, default: the loopback context moves a device payload
  * to device memory with the library's copy kernel; 0: with hipMemcpyAsync),
  * "group_bytes" (contiguous device tensors of at most this many bytes that follow each
@@ -475,8 +475,9 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * whose tables fit into 3.5 KiB carries the tables inside the kernel arguments:
  * no table block and no upload; a plan that is launched again uploads its
  * tables then; compact tensors and long strided runs do so beyond it as well
- * unless they are captured; 0 switches all that off; read at every
- * axr_pack / axr_unpack).  Unknown key -> AXR_ERR_INVALID. */
+ * unless they are captured, and where tables of up to 32 KiB without a view's own
+ * records do not fit, the first launch reads them in pinned memory; 0 switches
+ * all that off; read at every axr_pack / axr_unpack).  Unknown key -> AXR_ERR_INVALID. */
 AXR_API int axr_tune_set(const char* key, int64_t value);
 AXR_API int axr_tune_get(const char* key, int64_t* value);
 

@@ -233,19 +233,59 @@ constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t 
 }
 constexpr uint32_t kMaxBatchDims = 4;
 constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (measured: 8 KiB beats 2, 4 and 16)
-// kModeRows: the 16-byte slots a row may need, in whole 64-byte units, when its first byte lies up to
-// `start` bytes behind one; the slots a lane moves (see rows_moves for the sizes); LDS for the rows of a tile.
+// kModeRows: the 16-byte slots a row needs, in whole 64-byte units, when its first byte lies up to
+// `start` bytes behind one; the slots a lane moves; LDS for the rows of a tile.
 constexpr uint32_t kUnitBytes = 64;
 constexpr uint32_t kMaxRowSlots = 4;
 constexpr uint64_t kMaxRowBytes = kMaxRowSlots * kRowBytes / 2 - kUnitBytes;   // two rows to a tile at least
 constexpr uint32_t row_slots(uint64_t run_bytes, uint32_t start) {
   return static_cast<uint32_t>((start + run_bytes + kUnitBytes - 1) / kUnitBytes * (kUnitBytes / kVecBytes));
 }
+// Two, or three where that leaves a tenth less of a wavefront's slots without a row; four only for rows of
+// which three would hold one.  (Three pieces: 36 bytes at 37, 32 MiB, two 20.8, three 19.3 us for two packs.)
 // `mixed`: next to tensors that are moved otherwise.  The kernel for those holds fewer wavefronts, and larger
-// tiles make up for it (2^18 rows of 128 bytes at 131 34.9 us for pack + unpack before, 39.0 with two slots per
-// lane, 33.9 with four; of 666 at 1554 159 / 164 / 142).
+// tiles make up for it (2^18 rows of 128 bytes at 131 39.0 us for pack + unpack with two slots per lane, 33.9
+// with four; of 666 at 1554 164 / 142).
 constexpr uint32_t row_slots_per_lane(uint32_t slots, bool mixed) {
-  return mixed || slots <= 4 || 2 * slots > 3 * kWaveLanes ? kMaxRowSlots : 2 * slots <= 2 * kWaveLanes ? 2u : 3u;
+  const uint32_t two = 2 * kWaveLanes / slots, three = 3 * kWaveLanes / slots;   // rows to a tile
+  return mixed || three < 2 ? kMaxRowSlots : slots == 3 || 20 * three > 33 * two ? 3u : 2u;
+}
+// The slots of rows that lie `pitch` bytes apart and start up to `start` bytes behind a unit.
+// Slots for the worst start cut every row on its units, but a row of one to two units then takes three of them,
+// and what the lanes without a piece cost is more than the requests that are saved.  So they are taken where
+// they cost no row of a tile, and for two to seven units where the bundle has left the caches: by receivers,
+// which write the rows, from 24 MiB on, by senders of whole units, three or more, as well (such rows have no slot
+// to spare for another start: 256 at 292, 32 MiB, pack + unpack in turn 0.93, two packs in a launch 1.1), by the others
+// where the payload streams.  Slots for the worst start against
+// slots for a start on a unit, time of pack / unpack alone: 72 bytes at 73, 32 MiB 1.41 / 1.28; 200 at 201,
+// 12 MiB 1.16 / 1.15, 100 MiB 1.18 / 0.83, 200 MiB 1.25 / 0.73; 130 at 131, 200 MiB 1.37 / 0.72; 500 at 501, 100 MiB
+// 1.30 / 1.08; 144 at 168, 400 MiB 1.01 / 0.99 and 0.78 in one launch.
+// Rows of up to 48 bytes whose neighbour lies in the same unit, or in the next one of a bundle that the caches
+// hold, take as many slots as they have pieces (16 bytes at 24 0.6 times the time of whole units for pack and
+// 0.7 for unpack up to 100 MiB; 32 at 128 1.03 times).
+// Where a quarter of the slots of a row or more stay empty, more slots per lane make up for it: three, and for
+// rows of 65 to 80 bytes, five pieces of eight, four as long as the caches help (130 at 131, 200 MiB, pack alone: two
+// slots 1.43 times the time of three; 72 at 73, 32 MiB, two packs in a launch: two 26.5 us, three 21.8, four 20.1; 72 at
+// 128, 300 MiB 6 % slower with four than with two).
+constexpr uint64_t kRowUnitsPayload = 24ull << 20, kRowCachedPayload = 64ull << 20, kRowFilledPayload = 128ull << 20;
+struct RowRule {
+  uint32_t slots, per_lane;
+};
+constexpr RowRule row_rule(uint64_t run_bytes, uint64_t pitch, uint32_t start, bool receiver, uint64_t payload_bytes, bool streams) {
+  const uint32_t pieces = static_cast<uint32_t>((run_bytes + kVecBytes - 1) / kVecBytes);
+  if (pieces <= 3 && pitch < (payload_bytes < kRowCachedPayload ? 2 : 1) * kUnitBytes) {
+    const uint32_t slots = pieces < 2 ? 2u : pieces;
+    return {slots, row_slots_per_lane(slots, false)};
+  }
+  const uint32_t whole = row_slots(run_bytes, 0), worst = row_slots(run_bytes, start);
+  if (run_bytes >= 2 * kUnitBytes && run_bytes < 7 * kUnitBytes &&
+      (streams || (payload_bytes >= kRowUnitsPayload && (receiver || (run_bytes > 2 * kUnitBytes && run_bytes % kUnitBytes == 0)))))
+    return {worst, 2u};
+  uint32_t per_lane = row_slots_per_lane(whole, false);
+  if (whole >= 8 && pieces * 4 <= whole * 3)
+    per_lane = pieces != 5 ? 3u : payload_bytes < kRowFilledPayload ? kMaxRowSlots : 2u;
+  const uint32_t lanes = per_lane * kWaveLanes;
+  return {lanes / worst == lanes / whole ? worst : whole, per_lane};
 }
 constexpr uint32_t rows_lds_bytes(uint32_t rows, uint64_t run_bytes) {
   return static_cast<uint32_t>(rows * run_bytes) + kUnitBytes;

@@ -373,12 +373,9 @@ typedef AXR_LDS uint8_t* lbytes;
 // payload and cuts each side on its own boundaries: every row into 16-byte slots of its own 64-byte
 // units, the payload range likewise.  The first and the last piece of a row and of the range move inside
 // and overlap their neighbour with identical bytes, so nothing outside is read or written.  A row occupies
-// S = lanes_per_run slots, enough for the worst start its strides allow; a start that an address delta
-// has made worse than that is not aligned (a = 0), which only costs requests.
-// U is how many slots a lane moves, all in flight together.  Two (about 2 KiB) are best as long as two
-// rows fit: with 3, 4 and 8 slots 2^18 rows of 250 bytes at 333 take 59, 63 and 64 us for pack + unpack
-// instead of 58, of 666 at 1554 141, 144 and 146 instead of 135; where two slots hold one row of a kilobyte
-// only they take 264 instead of 171.
+// S = lanes_per_run slots (see row_rule): where they do not reach from the start of its first unit to its end,
+// it is cut from its own first byte on (a = 0), which only costs requests.
+// U is how many slots a lane moves, all in flight together.
 // Against 16-byte pieces moved without LDS, 8 KiB per wavefront, pack + unpack in turn, 2^18 rows, before /
 // now: 100 bytes at 256 40 / 34 us, 102 at 258 53 / 49, 128 at 256 29 / 26, 250 at 333 68 / 58, 256 at 512
 // 50 / 46, 256 at 515 73 / 65, 512 at 1024 89 / 82, 666 at 1554 156 / 138, 1001 at 1301 184 / 181, 1024 at 2048

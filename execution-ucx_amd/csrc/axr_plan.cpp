@@ -814,14 +814,15 @@ struct Builder {
       for (size_t d = 0; d < nd; ++d) step |= static_cast<uint64_t>(str[d]);
       step &= 0 - step;
       const uint32_t start = static_cast<uint32_t>((ptr & (step - 1)) + kUnitBytes - step);
-      // (rows of less than a unit are left where they straddle two: slots for both would be half empty)
-      const uint32_t slots = row_slots(run_bytes, run_bytes < kUnitBytes ? 0 : start);
       if (run_bytes >= kVecBytes && run_bytes <= kMaxRowBytes && tunables().ragged_runs != 0) {
         dm.mode = kModeRows;
         dm.granule = kVecBytes;
-        dm.lanes_per_run = slots;
-        dm.edge_a = row_slots_per_lane(slots, mixed);
-        dm.tiles_per_run = dm.edge_a * kWaveLanes / slots;
+        const int64_t pitch = str[nd - 1];
+        const RowRule rule = row_rule(run_bytes, static_cast<uint64_t>(pitch < 0 ? -pitch : pitch), start, p->receiver, p->payload_bytes,
+                                      p->payload_bytes > static_cast<uint64_t>(tunables().payload_cache_bytes));
+        dm.lanes_per_run = rule.slots;
+        dm.edge_a = mixed ? row_slots_per_lane(rule.slots, true) : rule.per_lane;
+        dm.tiles_per_run = dm.edge_a * kWaveLanes / rule.slots;
         dm.pstride[0] = runs;
         ntile = (runs + dm.tiles_per_run - 1) / dm.tiles_per_run;
         p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (rows_lds_bytes(dm.tiles_per_run, run_bytes) + 15u) & ~15u);

@@ -153,3 +153,50 @@ static_assert(every_start(false) && every_start(true), "rows");
         f.write(source)
     subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=200000000", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
+
+
+def test_row_rule(tmp_path):
+    """The slots a row gets cover it, a tile holds two rows at least and no more than its lanes and its LDS, and the
+    payload pieces of a tile fit theirs, for every length, every start, both sides and payloads of every class."""
+    source = r"""
+#include "axr_internal.h"
+using namespace axr;
+constexpr bool fits(uint64_t run, uint64_t pitch, uint32_t start, bool receiver, uint64_t payload, bool streams) {
+  const RowRule r = row_rule(run, pitch, start, receiver, payload, streams);
+  const uint32_t lanes = r.per_lane * kWaveLanes, rows = lanes / r.slots;
+  if (r.per_lane < 2 || r.per_lane > kMaxRowSlots || r.slots < 2 || r.slots * kVecBytes < run || rows < 2) return false;
+  if ((kUnitBytes - 1 + rows * run + kVecBytes - 1) / kVecBytes > lanes + kWaveLanes) return false;
+  return kUnitBytes - 1 + rows * run <= rows_lds_bytes(rows, run) && rows_lds_bytes(rows, run) <= 16384;
+}
+constexpr bool all() {
+  for (uint64_t run = kVecBytes; run <= kMaxRowBytes; ++run)
+    for (uint64_t pitch : {run, run + 1, run + 64, uint64_t(0), uint64_t(1) << 40})
+      for (uint32_t start : {0u, 1u, 16u, 48u, 63u})
+        for (uint64_t payload : {uint64_t(1), kRowUnitsPayload, kRowCachedPayload, kRowFilledPayload, uint64_t(1) << 38})
+          for (int receiver = 0; receiver < 2; ++receiver)
+            if (!fits(run, pitch, start, receiver != 0, payload, false) || !fits(run, pitch, start, receiver != 0, payload, true)) return false;
+  return true;
+}
+static_assert(all(), "rows");
+constexpr bool is(RowRule r, uint32_t slots, uint32_t per_lane) { return r.slots == slots && r.per_lane == per_lane; }
+constexpr uint64_t M = 1 << 20;
+// rows of one to two units: slots for a start on a unit whatever the start is
+static_assert(is(row_rule(72, 73, 63, false, 32 * M, false), 8, 4) && is(row_rule(72, 73, 63, false, 200 * M, false), 8, 2));
+static_assert(is(row_rule(100, 101, 63, true, 100 * M, false), 8, 2) && is(row_rule(100, 128, 0, false, 100 * M, false), 8, 2));
+static_assert(is(row_rule(64, 65, 63, true, 32 * M, false), 4, 2) && is(row_rule(130, 131, 63, false, 32 * M, false), 12, 3));
+// longer ones: slots for the worst start on the side that is written and where the payload streams
+static_assert(is(row_rule(200, 201, 63, false, 100 * M, false), 16, 2) && is(row_rule(200, 201, 63, true, 100 * M, false), 20, 2));
+static_assert(is(row_rule(200, 201, 63, true, 12 * M, false), 16, 2) && is(row_rule(200, 201, 63, false, 300 * M, true), 20, 2));
+static_assert(is(row_rule(256, 292, 60, false, 32 * M, false), 20, 2) && is(row_rule(128, 129, 63, false, 32 * M, false), 8, 2));
+// where they cost no row of a tile
+static_assert(is(row_rule(666, 667, 63, false, 32 * M, false), 48, 3) && is(row_rule(600, 601, 63, false, 32 * M, false), 40, 2));
+// very short rows next to each other
+static_assert(is(row_rule(16, 24, 56, false, 8 * M, false), 2, 2) && is(row_rule(36, 37, 63, true, 200 * M, false), 3, 3));
+static_assert(is(row_rule(32, 64, 0, false, 12 * M, false), 2, 2) && is(row_rule(32, 64, 0, false, 100 * M, false), 4, 2) &&
+              is(row_rule(32, 128, 0, false, 12 * M, false), 4, 2));
+"""
+    src = str(tmp_path / "rule.cpp")
+    with open(src, "w") as f:
+        f.write(source)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=400000000", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=240)

@@ -96,3 +96,11 @@ def test_long_rows_up_to_the_limit(pkg, gpu):
             round_trip(pkg, gpu, 100 * 2100 + 1, lambda s: [s[1:100 * 2100 + 1].view(100, 2100)[:, :length]], 1, 0)
     finally:
         pkg.tune(gather_run_bytes=1280)
+
+
+@pytest.mark.parametrize("length,pitch,mib", [(130, 131, 25), (200, 232, 25), (256, 292, 25), (72, 73, 2), (72, 73, 130), (24, 64, 66),
+                                              (40, 41, 66), (384, 385, 257)])
+def test_rows_of_larger_bundles(pkg, gpu, length, pitch, mib):
+    """Payloads around the sizes from which rows are given other slots, on one side or on both."""
+    rows = mib * (1 << 20) // length + 1
+    round_trip(pkg, gpu, rows * pitch, lambda s: [s[:rows * pitch].view(rows, pitch)[:, :length]], 256, 0)

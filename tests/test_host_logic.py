@@ -307,6 +307,14 @@ def test_short_runs_use_element_mode(pkg):
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 260], strides=[4000, 1]), ragged_runs=0)[0][0]["mode"] == 1
 
 
+def test_rows_share_a_tile_whatever_their_start(pkg):
+    """Rows of one to two 64-byte units take two units of slots also where they start anywhere in one: tiles of 32
+    rows of 72 bytes at 73, of 16 rows of 100 bytes at 101 and at 128, of 32 of 64 bytes at 65."""
+    for length, pitch, rows in ((72, 73, 32), (100, 101, 16), (100, 128, 16), (64, 65, 32)):
+        segs, _ = seg_of(pkg, tv(pkg, 0x10000, [9999, length], strides=[pitch, 1]))
+        assert (segs[0]["mode"], segs[0]["tiles"]) == (2, -(-9999 // rows)), (length, pitch)
+
+
 def test_transposed_views_use_square_blocks(pkg):
     # fp16 [300, 200] transposed: B (contiguous in the tensor) = 300, A (packed inner) = 200
     segs, info = seg_of(pkg, tv(pkg, 0x10000, [300, 200], strides=[1, 300], dtype=(4, 16, 1)))

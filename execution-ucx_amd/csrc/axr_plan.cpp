@@ -526,7 +526,7 @@ struct Builder {
   uint64_t tiles = 0;
   uint64_t shared_line_tiles = 0;   // transposed blocks whose rows straddle 128-byte lines
   uint64_t strip_tiles = 0;         // those of them that lie in strips of kBlockStrip blocks
-  bool mixed = false;               // some tensor, of those seen so far, is not moved in whole short rows
+  bool rows = false, others = false;   // tensors moved in whole short rows, and any other way
   uint64_t group_bytes = 0;         // longest tensor that may share a wavefront (0: none)
   uint32_t slots_per_group = kGroupMaxSlots;
   // the group being collected (when open): the last block of p->group_blocks
@@ -603,7 +603,7 @@ struct Builder {
 
   int add_seg(uint32_t tensor, uint64_t ptr, uint64_t off, uint64_t run_bytes, uint64_t ntile,
               uint32_t dsel) {
-    mixed = mixed || dsel == 0 || dsel >= kSegGroup || p->dims[dsel - 1].mode != kModeRows;
+    (dsel != 0 && dsel < kSegGroup && p->dims[dsel - 1].mode == kModeRows ? rows : others) = true;
     if (tiles + ntile > 0xffffffffull) return fail(AXR_ERR_UNSUPPORTED, "bundle has too many tiles");
     Seg s;
     s.ptr = ptr;
@@ -821,8 +821,8 @@ struct Builder {
         const RowRule rule = row_rule(run_bytes, static_cast<uint64_t>(pitch < 0 ? -pitch : pitch), start, p->receiver, p->payload_bytes,
                                       p->payload_bytes > static_cast<uint64_t>(tunables().payload_cache_bytes));
         dm.lanes_per_run = rule.slots;
-        dm.edge_a = mixed ? row_slots_per_lane(rule.slots, true) : rule.per_lane;
-        dm.tiles_per_run = dm.edge_a * kWaveLanes / rule.slots;
+        dm.edge_a = rule.per_lane;
+        dm.tiles_per_run = rule.per_lane * kWaveLanes / rule.slots;
         dm.pstride[0] = runs;
         ntile = (runs + dm.tiles_per_run - 1) / dm.tiles_per_run;
         p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (rows_lds_bytes(dm.tiles_per_run, run_bytes) + 15u) & ~15u);
@@ -840,6 +840,31 @@ struct Builder {
     if (p->dims.empty() || p->dims.back().nbytes != nbytes || std::memcmp(&p->dims.back(), &dm, sizeof(dm)) != 0)
       p->dims.push_back(dm);
     return add_seg(tensor, ptr, off, run_bytes, ntile, static_cast<uint32_t>(p->dims.size()));
+  }
+
+  // Short rows next to other tensors are moved by the kernel for any mode and take its larger tiles.  Known once
+  // every tensor has been seen, or the order of the tensors would decide.
+  void settle_rows() {
+    if (!rows || !others) return;
+    for (Dims& dm : p->dims) {
+      if (dm.mode != kModeRows) continue;
+      dm.edge_a = row_slots_per_lane(dm.lanes_per_run, true);
+      dm.tiles_per_run = dm.edge_a * kWaveLanes / dm.lanes_per_run;
+    }
+    const uint64_t end = tiles;
+    tiles = 0;
+    for (size_t i = 0; i < p->segs.size(); ++i) {
+      Seg& sg = p->segs[i];
+      uint64_t ntile = (i + 1 < p->segs.size() ? p->segs[i + 1].tile_begin : end) - sg.tile_begin;
+      const uint32_t dsel = sg.meta >> kSegDimsShift;
+      if (dsel != 0 && dsel < kSegGroup && p->dims[dsel - 1].mode == kModeRows) {
+        const Dims& dm = p->dims[dsel - 1];
+        ntile = (dm.pstride[0] + dm.tiles_per_run - 1) / dm.tiles_per_run;
+        p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (rows_lds_bytes(dm.tiles_per_run, sg.run_bytes) + 15u) & ~15u);
+      }
+      sg.tile_begin = static_cast<uint32_t>(tiles);
+      tiles += ntile;
+    }
   }
 
   // Host (kDLCPU) tensors move with one async copy per contiguous run.
@@ -1223,7 +1248,6 @@ int build_tables(axr_plan* p) {
   invalidate_tables(p);
   const Tunables& tn = tunables();
   uint32_t rows = static_cast<uint32_t>(tn.tile_rows);
-  bool compact = false;   // some tensor is compact, of those that are looked at here
   if (rows == 0) {
     rows = 2;
     // A bundle made only of strided views with one short run length (pitched
@@ -1244,7 +1268,6 @@ int build_tables(axr_plan* p) {
       if (t.nbytes == 0) continue;
       if (!t.has_strides || is_compact(p, t)) {
         uniform_runs = false;   // a compact tensor: not a bundle of strided views
-        compact = true;
       } else {
         Collapsed c;
         collapse(t, p->shape_of(t), p->strides_of(t), item_bytes(t), &c);
@@ -1268,7 +1291,6 @@ int build_tables(axr_plan* p) {
             static_cast<uint64_t>(tn.head_align)};
   b.group_bytes = static_cast<uint64_t>(tn.group_bytes);
   b.slots_per_group = static_cast<uint32_t>(tn.group_slots);
-  b.mixed = compact;
   p->segs.reserve(p->tensors.size() + 1);
   p->seg_tensor.reserve(p->tensors.size());
 
@@ -1322,6 +1344,7 @@ int build_tables(axr_plan* p) {
     int rc = b.close_group();
     if (rc) return rc;
   }
+  b.settle_rows();
   // Group neighbouring host pieces (in payload order, at most an alignment gap
   // apart) into chunks that fit one staging block.
   for (uint32_t i = 0; i < p->host_copies.size(); ++i) {

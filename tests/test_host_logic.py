@@ -3,6 +3,7 @@ the header declares, the planner agrees with the oracle, the header codec
 matches the golden fixtures, the segment table is what the design says, and
 every path that would need a device fails loudly instead of falling back."""
 import ctypes as C
+import itertools
 import json
 import os
 import re
@@ -313,6 +314,35 @@ def test_rows_share_a_tile_whatever_their_start(pkg):
     for length, pitch, rows in ((72, 73, 32), (100, 101, 16), (100, 128, 16), (64, 65, 32)):
         segs, _ = seg_of(pkg, tv(pkg, 0x10000, [9999, length], strides=[pitch, 1]))
         assert (segs[0]["mode"], segs[0]["tiles"]) == (2, -(-9999 // rows)), (length, pitch)
+
+
+def test_rows_are_tiled_alike_in_every_order_of_the_tensors(pkg):
+    """Short rows next to other tensors take the tiles of the kernel for any mode (four slots per lane) wherever
+    in the bundle they lie, and rows alone, of one length or of two, the smaller ones."""
+    a = tv(pkg, 0x10000, [9999, 128], strides=[131, 1])
+    b = tv(pkg, 0x200000, [5000, 100], strides=[117, 1])
+    compact, blocks = tv(pkg, 0x400000, [100000]), tv(pkg, 0x500000, [300, 200], strides=[1, 300])
+    empty, host = tv(pkg, 0x600000, [0, 7]), tv(pkg, 0x700000, [100], device_type=1)
+
+    def tiles(tensors, align=1):
+        with pkg.BundlePlan.create(tensors, align=align) as plan:
+            rows = [s for s in plan.segments() if s["mode"] == 2]
+            segs = [s for s in plan.segments() if s["mode"] not in (4, 6)]
+            assert sum(s["tiles"] for s in segs) == plan.launch_info()["tiles"]
+            return {s["run_bytes"]: s["tiles"] for s in rows}
+
+    alone = {128: -(-9999 // 16), 100: -(-5000 // 16)}
+    among = {128: -(-9999 // 32), 100: -(-5000 // 32)}
+    for order in itertools.permutations([a, b, compact]):
+        assert tiles(list(order)) == among
+    for order in itertools.permutations([a, b, blocks]):
+        assert tiles(list(order)) == among
+    for order in itertools.permutations([a, b, empty]):
+        assert tiles(list(order)) == alone
+    for order in itertools.permutations([a, b, host]):     # nothing of the host tensor is the kernel's,
+        assert tiles(list(order)) == alone
+        assert tiles(list(order), align=256) == (alone if order[-1] is host else among)      # but the gap behind it is
+    assert tiles([a]) == {128: alone[128]} and tiles([a, compact]) == tiles([compact, a]) == {128: among[128]}
 
 
 def test_transposed_views_use_square_blocks(pkg):

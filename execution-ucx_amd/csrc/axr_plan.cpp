@@ -913,18 +913,11 @@ bool streams_in_small_tiles(const axr_plan* p) {
 // few large tensors gets a tiny index, a bundle of many small ones an entry per few tiles).
 void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct = false) {
   const Tunables& tn = tunables();
-  // (tiles of short rows are a quarter of the others' length, and their wavefronts as much shorter)
-  bool short_rows = false;
-  for (const Dims& dm : p->dims) short_rows = short_rows || dm.mode == kModeRows;
-  const uint64_t max_waves = static_cast<uint64_t>(tn.max_waves) * (short_rows ? 4 : 1);
-  uint64_t tpw = (p->ntiles + max_waves - 1) / max_waves;
-  if (tpw == 0) tpw = 1;
-  p->cfg.threads = tn.threads ? static_cast<uint32_t>(tn.threads)
-                              : (rows == 1 && tn.tile_rows == 0 ? kWaveLanes : (p->ntiles < 65536 ? 256u : 128u));
   p->cfg.elements = false;
   for (const Dims& dm : p->dims) p->cfg.elements = p->cfg.elements || dm.mode != kModeRunTiles;
   p->cfg.kind = kKindAny;
-  if (p->cfg.elements && rows == 2) {   // the kernels of a single mode are built for the default tile
+  bool rows_alone = false;
+  if (p->cfg.elements) {
     const uint32_t mode = p->dims[0].mode;
     bool one = mode != kModeRunTiles;
     for (const Dims& dm : p->dims) one = one && dm.mode == mode;
@@ -932,8 +925,16 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
       const uint32_t dsel = p->segs[i].meta >> kSegDimsShift;
       one = dsel != 0 && dsel != kSegFillOnly && dsel != kSegGroup;
     }
-    if (one) p->cfg.kind = mode;
+    if (one && rows == 2) p->cfg.kind = mode;   // the kernels of a single mode are built for the default tile
+    rows_alone = one && mode == kModeRows;
   }
+  // (tiles of short rows alone are a quarter of the others' length, and their wavefronts as much shorter: 2^23 rows of
+  // 300 bytes, pack + unpack, with as many wavefronts as of others 2215 us, with four times as many 2050)
+  const uint64_t max_waves = static_cast<uint64_t>(tn.max_waves) * (rows_alone ? 4 : 1);
+  uint64_t tpw = (p->ntiles + max_waves - 1) / max_waves;
+  if (tpw == 0) tpw = 1;
+  p->cfg.threads = tn.threads ? static_cast<uint32_t>(tn.threads)
+                              : (rows == 1 && tn.tile_rows == 0 ? kWaveLanes : (p->ntiles < 65536 ? 256u : 128u));
   if (p->cfg.elements) p->cfg.threads = std::min(p->cfg.threads, kMaxElementThreads);
   if (p->cfg.lds_per_wave) {
     // transposed blocks: every wave of a workgroup owns a slice of at most 64 KiB of LDS

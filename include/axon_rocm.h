@@ -426,7 +426,8 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * to 16 KiB for bundles of strided views of one run length whose payload stays in the
  * last-level cache; 1 for payloads of compact tensors and long strided runs between
  * payload_cache_bytes and max_tiles KiB, which stream to and from memory), "max_tiles",
- * "max_waves", "threads" (workgroup size; 0 = automatic: 256 below 65,536 tiles, 128 above, 64
+ * "max_waves" (wavefronts of a launch; four times as many for views of short rows alone, whose
+ * tiles are a quarter as long), "threads" (workgroup size; 0 = automatic: 256 below 65,536 tiles, 128 above, 64
  * with the automatic 1 KiB tiles), "nontemporal" (-1 auto, or bit 0
  * tensor side / bit 1 payload side), "payload_cache_bytes" (of a larger payload that moves
  * in 1 KiB tiles the last 7/8 of as many bytes stay cacheable when it is packed),

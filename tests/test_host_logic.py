@@ -345,6 +345,27 @@ def test_rows_are_tiled_alike_in_every_order_of_the_tensors(pkg):
     assert tiles([a]) == {128: alone[128]} and tiles([a, compact]) == tiles([compact, a]) == {128: among[128]}
 
 
+def test_wavefronts_of_a_launch(pkg):
+    """max_waves holds for every bundle but views of short rows alone, which may have four times as many."""
+    rows = tv(pkg, 0x10000, [60000, 128], strides=[131, 1])
+    compact = [tv(pkg, 0x1000000 + i * 100000, [90000]) for i in range(40)]
+    old = C.c_int64()
+    pkg._capi.check(pkg._capi.load().axr_tune_get(b"max_waves", C.byref(old)))
+
+    def waves(tensors):
+        with pkg.BundlePlan.create(tensors) as plan:
+            info = plan.launch_info()
+            assert info["tiles"] > 1000
+            return info["workgroups"] * info["threads_per_workgroup"] // 64
+
+    pkg.tune(max_waves=100)
+    try:
+        assert waves(compact) <= 100 and waves([rows] + compact) <= 100 and waves(compact + [rows]) <= 100
+        assert 300 < waves([rows]) <= 400
+    finally:
+        pkg.tune(max_waves=old.value)
+
+
 def test_transposed_views_use_square_blocks(pkg):
     # fp16 [300, 200] transposed: B (contiguous in the tensor) = 300, A (packed inner) = 200
     segs, info = seg_of(pkg, tv(pkg, 0x10000, [300, 200], strides=[1, 300], dtype=(4, 16, 1)))

@@ -2318,6 +2318,7 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     const axr_plan *x = jx.plan, *y = jy.plan;
     return x->cfg.tile_rows == y->cfg.tile_rows && x->cfg.threads == y->cfg.threads &&
            effective_nontemporal(x, jx.flags) == effective_nontemporal(y, jy.flags) &&
+           kinds_share_launch(x->cfg.kind, x->ntiles, y->cfg.kind, y->ntiles) &&
            (!(x->cfg.elements || y->cfg.elements) || (x->cfg.tile_rows == 2 && x->cfg.threads <= kMaxElementThreads));
   };
   size_t i = 0;

@@ -200,3 +200,19 @@ static_assert(is(row_rule(32, 64, 0, false, 12 * M, false), 2, 2) && is(row_rule
         f.write(source)
     subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=400000000", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=240)
+
+
+def test_rows_that_share_a_launch(tmp_path):
+    """Many tiles of short rows share a launch with each other and not with bundles of other kinds; few do."""
+    source = r"""
+#include "axr_internal.h"
+using namespace axr;
+static_assert(kinds_share_launch(kModeRows, 1u << 20, kModeRows, 3) && kinds_share_launch(kModeRows, 2048, kKindAny, 1u << 20));
+static_assert(!kinds_share_launch(kModeRows, 2049, kKindAny, 3) && !kinds_share_launch(kModeTranspose, 3, kModeRows, 2049));
+static_assert(kinds_share_launch(kModeTranspose, 1u << 20, kKindAny, 1u << 20));
+"""
+    src = str(tmp_path / "share.cpp")
+    with open(src, "w") as f:
+        f.write(source)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)

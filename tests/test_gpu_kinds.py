@@ -19,6 +19,7 @@ def storage(gpu, nbytes, seed):
 FAMILIES = {
     "whole_rows": (90 * 512, lambda s: [s.view(90, 512)[:, :128], s.view(90, 512)[:, 256:448]]),
     "odd_rows": (91 * 259, lambda s: [s.view(91, 259)[:, 1:101], s.view(91, 259)[5:, 102:259]]),
+    "many_rows": (40000 * 131, lambda s: [s.view(40000, 131)[:, :100]]),
     "narrow_rows": (1 << 15, lambda s: [s.view(4096, 8)[:, :6]]),
     "blocks": (300 * 196, lambda s: [s.view(300, 196).t(), s.view(300, 196)[1:, 3:190].t()]),
     "odd_blocks": (2051 * 17001 * 2, lambda s: [s.view(torch.int16).view(2051, 17001).t()]),
@@ -27,9 +28,9 @@ FAMILIES = {
     "long_rows": (40 * 5000, lambda s: [s.view(40, 5000)[:, :3001]]),
     "short": (64 * 1000, lambda s: [s[i * 1000 + 7:i * 1000 + 7 + 9 * i + 1] for i in range(50)]),
 }
-BUNDLES = [[name] for name in FAMILIES if name != "short"] + [
+BUNDLES = [[name] for name in FAMILIES if name not in ("short", "many_rows")] + [
     ["short"], ["odd_rows", "runs"], ["planes", "short"], ["blocks", "whole_rows"], ["narrow_rows", "odd_rows", "long_rows"],
-    [name for name in FAMILIES if name != "odd_blocks"]]
+    [name for name in FAMILIES if name not in ("odd_blocks", "many_rows")]]
 
 
 def tunables_now(pkg, names):
@@ -120,3 +121,20 @@ def test_kinds_in_one_launch(pkg, gpu, left, right, threads, nontemporal):
         b.close()
     finally:
         pkg.tune(**old)
+
+
+@pytest.mark.parametrize("others", [["runs"], ["blocks"], ["short", "odd_rows"]], ids="+".join)
+def test_many_rows_submitted_with_others(pkg, gpu, others):
+    """More tiles of short rows than share a launch with another kind: every job's bytes, whichever launch it is in."""
+    capi = pkg._capi
+    bundles = [Moved(pkg, gpu, [n], 64, 9 + i) for i, n in enumerate(["many_rows"] + others + ["many_rows"])]
+    assert sum(s["tiles"] for s in bundles[0].send.segments()) > 2048
+    for unpack in (0, 1):
+        jobs = (capi.Job * len(bundles))()
+        for j, m in zip(jobs, bundles):
+            j.plan, j.unpack = (m.recv if unpack else m.send)._h, unpack
+            j.payload, j.payload_bytes = m.payload.data_ptr(), m.n
+        capi.check(capi.load().axr_submit(jobs, len(bundles), C.c_void_p()))
+    for m in bundles:
+        m.check()
+        m.close()

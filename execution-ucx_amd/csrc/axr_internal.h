@@ -563,9 +563,9 @@ void table_block_release(TableBlock* block);
 // Events without timing for the current device, recycled: creating one costs more than a
 // microsecond, and every fresh plan that uploads tables needs one.  An event goes back
 // only once it has fired (or was never recorded).
-// device_scope: an event that makes what kernels wrote to device memory visible to kernels of other
-// streams, and nothing to the host or of the copy engine's.  The kernel behind it starts 2 us
-// sooner (48 cache blocks of 32 runs, fresh, pack + unpack, 44.5 -> 40.8 us).
+// device_scope: an event whose record releases what kernels wrote to the device, for streams of the same device
+// that wait for it (hipEventReleaseToDevice), and not to the host or other devices.  The kernel behind it starts
+// 2 us sooner (48 cache blocks of 32 runs, fresh, pack + unpack, 44.5 -> 40.8 us).  The host waits for no such event.
 int event_acquire(bool device_scope, void** event, int* device);
 void event_release(bool device_scope, void* event, int device);
 

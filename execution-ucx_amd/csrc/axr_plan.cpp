@@ -2441,7 +2441,9 @@ static int plan_prepare_body(axr_plan_t* plan, void* stream_) {
   if (plan->ntiles == 0 || plan->resident) return AXR_OK;
   rc = ensure_uploaded(plan, stream);
   if (rc) return rc;
-  rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
+  // The upload or a wait for it is on `stream` now.  Later launches read the tables on any stream without
+  // waiting for anything, so the host waits for the stream itself and not for an event of device scope.
+  rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize(plan tables)");
   if (rc) return rc;
   plan->resident = true;
   return AXR_OK;

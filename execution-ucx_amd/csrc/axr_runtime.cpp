@@ -120,7 +120,7 @@ int event_acquire(bool device_scope, void** event, int* device) {
     }
   }
   hipEvent_t e = nullptr;
-  rc = check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming | (device_scope ? hipEventDisableSystemFence : 0u)), "hipEventCreate");
+  rc = check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming | (device_scope ? hipEventReleaseToDevice : 0u)), "hipEventCreate");
   if (rc) return rc;
   *event = e;
   *device = dev;

@@ -58,3 +58,51 @@ def test_streams_find_the_tables_of_another_stream(pkg, gpu, kind):
             assert all(torch.equal(out, expect) for out in outs)
     for s in streams:
         capi.check(lib.axr_stream_destroy(s))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["views", "records", "groups"])
+def test_prepared_plans_on_streams_that_wait_for_nothing(pkg, gpu, kind):
+    """axr_plan_prepare on one stream, launches on three others with no event between them, over and over in
+    recycled table blocks; then with the tables rebuilt for other tensors, prepared on a stream that had not
+    launched the plan before."""
+    lib, capi = pkg._capi.load(), pkg._capi
+    streams = []
+    for _ in range(3):
+        s = C.c_void_p()
+        capi.check(lib.axr_stream_create(C.byref(s)))
+        streams.append(s.value)
+    parent = torch.randint(0, 256, (700, 9, 2048), dtype=torch.uint8, device=gpu)
+
+    def tensors(k):
+        if kind == "views":
+            return [parent[i, 1:, :1400 + (i + k) % 7] for i in range(200)]
+        return [parent[i, 0, :(2000 if kind == "records" else 100) + (i + k) % 48] for i in range(700)]
+
+    for k in range(8):
+        ts = tensors(k)
+        with pkg.BundlePlan.create(ts, align=16) as plan:
+            expect = torch.zeros(plan.payload_bytes, dtype=torch.uint8, device=gpu)
+            for t, at, n in zip(ts, *plan.layout()):
+                expect[at:at + n] = t.reshape(-1)
+            outs = [torch.zeros_like(expect) for _ in range(3)]
+            for first in (0, 1):
+                torch.cuda.synchronize()
+                plan.prepare(streams[(k + first) % 3])
+                for j, out in enumerate(outs):
+                    plan.pack(out.data_ptr(), out.numel(), streams[(k + first + 1 + j) % 3], order=False)
+                torch.cuda.synchronize()
+                assert all(torch.equal(out, expect) for out in outs)
+                plan.bind([t.clone() for t in ts])
+                for out in outs:
+                    out.zero_()
+            # uploaded by a launch, prepared on another stream, launched on the third one
+            torch.cuda.synchronize()
+            for j in range(2):
+                plan.pack(outs[j].data_ptr(), outs[j].numel(), streams[0], order=False)
+            plan.prepare(streams[1])
+            plan.pack(outs[2].data_ptr(), outs[2].numel(), streams[2], order=False)
+            torch.cuda.synchronize()
+            assert all(torch.equal(out, expect) for out in outs)
+    for s in streams:
+        capi.check(lib.axr_stream_destroy(s))

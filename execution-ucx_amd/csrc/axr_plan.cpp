@@ -2518,8 +2518,7 @@ static int plan_segments_body(axr_plan_t* plan, axr_segment_info_t* out, size_t 
       o.nbytes = dm.nbytes;
       o.ndim = dm.ndim;
       o.granule = dm.granule;
-      // (the slots of a run whose start lies on a 64-byte boundary, where it leaves some of them unused)
-      o.lanes_per_run = dm.mode == kModeRows && s.run_bytes % kUnitBytes != 0 ? row_slots(s.run_bytes, 0) : 0;
+      o.lanes_per_run = dm.mode == kModeRows ? dm.lanes_per_run : 0;
       for (uint32_t d = 0; d < dm.ndim; ++d) {
         o.shape[d] = dm.shape[kMaxOuterDims - dm.ndim + d];
         o.stride_bytes[d] = dm.stride[kMaxOuterDims - dm.ndim + d];

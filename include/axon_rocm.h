@@ -408,10 +408,10 @@ typedef struct axr_segment_info {
   uint32_t head;          /* mode 0: leading bytes (< 128) that the first tile
                              moves on top of its own range, so that the tiles
                              start on a 128-byte line of the written side      */
-  uint32_t lanes_per_run; /* mode 2 with 16-byte granules: lane slots a run occupies
-                             when it starts on a 64-byte boundary (its granules, the
-                             last one covering the run's final 16 bytes, rounded up to
-                             a multiple of four); 0 where it leaves none unused      */
+  uint32_t lanes_per_run; /* mode 2, whole runs of 16 bytes and more: the 16-byte lane
+                             slots a run occupies in its tile (at least as many as it
+                             has granules, the last one covering its final 16 bytes);
+                             0: the tiles count packed bytes                     */
   uint32_t shape[6];
   int64_t stride_bytes[6];
 } axr_segment_info_t;

@@ -301,8 +301,9 @@ def test_short_runs_use_element_mode(pkg):
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 1280], strides=[4000, 1]))[0][0]["mode"] == 1
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 1279], strides=[4000, 1]))[0][0]["mode"] == 2
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 1281], strides=[4000, 1]))[0][0]["mode"] == 1
-    # runs of a whole number of 64-byte groups keep counting packed bytes; others pad to four lanes
-    assert seg_of(pkg, tv(pkg, 0x10000, [5, 128], strides=[4000, 1]))[0][0]["lanes_per_run"] == 0
+    # whole runs take whole 64-byte units of slots; pieces of packed bytes have none
+    assert seg_of(pkg, tv(pkg, 0x10000, [5, 128], strides=[4000, 1]))[0][0]["lanes_per_run"] == 8
+    assert seg_of(pkg, tv(pkg, 0x10000, [5, 100], strides=[4000, 1]), ragged_runs=0)[0][0]["lanes_per_run"] == 0
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 112], strides=[4000, 1]))[0][0]["lanes_per_run"] == 8
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 100], strides=[4000, 1]))[0][0]["lanes_per_run"] == 8
     assert seg_of(pkg, tv(pkg, 0x10000, [5, 260], strides=[4000, 1]), ragged_runs=0)[0][0]["mode"] == 1
@@ -314,6 +315,22 @@ def test_rows_share_a_tile_whatever_their_start(pkg):
     for length, pitch, rows in ((72, 73, 32), (100, 101, 16), (100, 128, 16), (64, 65, 32)):
         segs, _ = seg_of(pkg, tv(pkg, 0x10000, [9999, length], strides=[pitch, 1]))
         assert (segs[0]["mode"], segs[0]["tiles"]) == (2, -(-9999 // rows)), (length, pitch)
+
+
+@pytest.mark.parametrize("length,pitch,rows,sent,received", [
+    (72, 73, 1000, (8, 32), (8, 32)), (72, 73, 2 << 20, (8, 16), (8, 16)), (130, 131, 1000, (12, 16), (12, 16)),
+    (130, 131, 200000, (12, 16), (16, 8)), (256, 292, 100000, (20, 6), (20, 6)), (200, 201, 2 << 20, (20, 6), (20, 6)),
+    (666, 667, 1000, (48, 4), (48, 4)), (666, 704, 1000, (44, 4), (44, 4)), (16, 24, 1000, (2, 64), (2, 64)),
+    (40, 41, 1000, (3, 64), (3, 64)), (32, 128, 1000, (4, 32), (4, 32)), (1279, 1281, 1000, (84, 2), (84, 2))])
+def test_reported_slots_are_those_of_the_tiles(pkg, length, pitch, rows, sent, received):
+    """lanes_per_run of rows on both sides, and the tiles that follow from the rows that many slots leave in one."""
+    views = [tv(pkg, base, [rows, length], strides=[pitch, 1]) for base in (0x10000, 0x7f0000000000)]
+    with pkg.BundlePlan.create(views[:1], align=256) as send, \
+            pkg.BundlePlan.from_header_bound(send.header, views[1:]) as recv:
+        for plan, (slots, per_tile) in ((send, sent), (recv, received)):
+            (s,) = plan.segments()
+            assert (s["mode"], s["granule"], s["lanes_per_run"]) == (2, 16, slots)
+            assert s["tiles"] == plan.launch_info()["tiles"] == -(-rows // per_tile)
 
 
 def test_rows_are_tiled_alike_in_every_order_of_the_tensors(pkg):

@@ -1861,7 +1861,9 @@ int axr_plan_create(const axr_tensor_t* tensors,
 }
 int axr_plan_create_from(axr_tensor_source* tensors, uint32_t align, axr_plan_t** plan) {
   return guarded([&] {
+    if (!plan) return fail(AXR_ERR_INVALID, "axr_plan_create_from: null result");
     *plan = nullptr;
+    if (!tensors || (tensors->count && !tensors->describe)) return fail(AXR_ERR_INVALID, "axr_plan_create_from: null tensor source");
     if (tensors->count > 0xffffffffull) return fail(AXR_ERR_INVALID, "axr_plan_create: too many tensors");
     return plan_create_body(PulledSource(tensors), tensors->count, align, plan);
   });
@@ -2086,7 +2088,12 @@ int axr_plan_from_header_bind(const void* header, size_t length, const axr_tenso
   return guarded([&] { return plan_from_header_body(header, length, ArraySource{tensors}, n, true, false, plan); });
 }
 int axr_plan_bind_from(const void* header, size_t length, axr_tensor_source* tensors, axr_plan_t** plan) {
-  return guarded([&] { return plan_from_header_body(header, length, PulledSource(tensors), tensors->count, true, true, plan); });
+  return guarded([&] {
+    if (!plan) return fail(AXR_ERR_INVALID, "axr_plan_bind_from: null result");
+    *plan = nullptr;
+    if (!tensors || (tensors->count && !tensors->describe)) return fail(AXR_ERR_INVALID, "axr_plan_bind_from: null tensor source");
+    return plan_from_header_body(header, length, PulledSource(tensors), tensors->count, true, true, plan);
+  });
 }
 
 static int plan_bind_body(axr_plan_t* plan, const axr_tensor_t* tensors, size_t n) {

@@ -83,3 +83,27 @@ def test_what_is_refused_is_refused_as_before(pkg):
         bundle._bind_header(b"x" * len(header), [good], None)
     with pytest.raises(Exception, match="truncated|trailing|bad tensor record"):
         bundle._bind_header(header[:-8], [good, torch.zeros(7)], None)
+
+
+def test_null_sources_are_refused(pkg):
+    """What the siblings that take an array refuse: no result, no source, a source that cannot describe."""
+    import ctypes as C
+    lib = pkg._capi.load()
+
+    class Source(C.Structure):
+        _fields_ = [("count", C.c_size_t), ("describe", C.c_void_p)]
+
+    create, bind = lib.axr_plan_create_from, lib.axr_plan_bind_from
+    create.argtypes, create.restype = [C.c_void_p, C.c_uint32, C.c_void_p], C.c_int
+    bind.argtypes, bind.restype = [C.c_void_p, C.c_size_t, C.c_void_p, C.c_void_p], C.c_int
+    with pkg.BundlePlan.create([torch.zeros(3)], align=1) as plan:
+        header = plan.header
+    h, mute, none = C.c_void_p(), Source(1, None), Source(0, None)
+    invalid = -1
+    assert create(C.byref(none), 1, None) == invalid and bind(header, len(header), C.byref(none), None) == invalid
+    for source in (None, C.byref(mute)):
+        assert create(source, 1, C.byref(h)) == invalid and not h.value
+        assert bind(header, len(header), source, C.byref(h)) == invalid and not h.value
+    assert bind(None, 0, C.byref(none), C.byref(h)) == invalid
+    assert create(C.byref(none), 1, C.byref(h)) == 0 and h.value      # no tensors: nothing to describe
+    pkg._capi.check(lib.axr_plan_free(h))

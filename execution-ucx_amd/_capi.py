@@ -139,7 +139,7 @@ class LaunchInfo(C.Structure):
         ("host_copies", C.c_uint32),
         ("host_chunks", C.c_uint32),
         ("inline_tables", C.c_uint32),
-        ("reserved", C.c_uint32),
+        ("last_launch", C.c_uint32),
     ]
 
 

@@ -182,7 +182,7 @@ class BundlePlan:
     def launch_info(self) -> dict:
         info = _capi.LaunchInfo()
         _capi.check(self._lib.axr_plan_launch_info(self._h, C.byref(info)))
-        return {f: getattr(info, f) for f, _ in info._fields_ if f != "reserved"}
+        return {f: getattr(info, f) for f, _ in info._fields_}
 
     def segments(self) -> List[dict]:
         n = C.c_size_t()

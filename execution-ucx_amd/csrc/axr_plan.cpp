@@ -210,6 +210,7 @@ struct axr_plan {
   std::unique_ptr<InlineTables> inline_tables;   // the tables as a kernel argument (small bundles)
   bool inline_ready = false;
   uint64_t launches = 0;             // kernel launches since the tables were built
+  uint32_t last_launch = 0;          // axr_launch_info_t::last_launch
   hipEvent_t upload_event = nullptr;   // from event_acquire; behind the latest upload once `uploaded` is set
   int upload_event_device = -1;
   bool upload_event_by_kernel = false;   // a device-scope event: a kernel wrote the tables
@@ -1604,6 +1605,17 @@ void fill_inline_tables(axr_plan* p) {
   p->inline_ready = true;
 }
 
+// The plan has been launched: where its tables were and what moved it (see axr_launch_info_t::last_launch).
+enum class Tables : uint32_t { kArguments = 1, kPinned, kUploaded, kDeviceBuilt };
+void note_launch(axr_plan* p, Tables tables, const LaunchConfig& cfg, bool pack) {
+  ++p->launches;
+  uint32_t kind = cfg.elements ? cfg.kind : kKindRuns;
+  if (tables == Tables::kArguments && kind != kKindRuns && kind != kModeRows) kind = kKindAny;   // see launch_bundle_kernel_inline
+  const bool tail = pack && !cfg.elements && cfg.tile_rows == 1 && (cfg.nontemporal & 3u) == 3u;
+  p->last_launch = static_cast<uint32_t>(tables) | kind << 4 | (tail ? cfg.cached_tail << 8 : 0u);
+}
+Tables device_tables_of(const axr_plan* p) { return p->device_built ? Tables::kDeviceBuilt : Tables::kUploaded; }
+
 // The cache hint bits a job runs with: the plan's own, or with the payload side forced.
 uint32_t effective_nontemporal(const axr_plan* p, uint32_t job_flags) {
   uint32_t nt = p->cfg.nontemporal & 3u;
@@ -1670,7 +1682,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
     if (rc) return rc;
-    ++p->launches;
+    note_launch(p, Tables::kArguments, cfg, pack);
     if (!pack && p->pinned_host_tensors) stream_note_host_writes(stream);
     // The launch needs nothing of the plan any more, but callers rely on axr_plan_free and
     // axr_plan_bind returning only when the plan's launches are done (they release the
@@ -1681,7 +1693,9 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   if (capturing && !p->resident)
     return fail(AXR_ERR_INVALID, "call axr_plan_prepare before capturing this plan in a graph");
   uint8_t* d;
+  Tables tables = device_tables_of(p);
   if (!capturing && !p->resident && first_launch_reads_host_block(p)) {
+    tables = Tables::kPinned;
     rc = write_host_block(p);
     d = static_cast<uint8_t*>(p->block.host);
   } else {
@@ -1694,7 +1708,7 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
   a.wave_seg = reinterpret_cast<const uint32_t*>(d + p->wave_at);
   rc = launch_bundle_kernel(pack, a, cfg, stream);
   if (rc) return rc;
-  ++p->launches;
+  note_launch(p, tables, cfg, pack);
   if (!pack && p->pinned_host_tensors) stream_note_host_writes(stream);
   // a capturing stream cannot be drained later; the caller keeps the plan alive
   // for as long as the graph can run
@@ -2216,7 +2230,7 @@ static int pack_noalloc_body(axr_plan_t* p, void* payload, size_t payload_bytes,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
     if (rc) return rc;
-    ++p->launches;
+    note_launch(p, Tables::kArguments, p->cfg, true);
     remember();
     return AXR_OK;
   }
@@ -2265,7 +2279,7 @@ static int pack_noalloc_body(axr_plan_t* p, void* payload, size_t payload_bytes,
     a.dims = reinterpret_cast<const Dims*>(d + dims_arg_at(p));
     a.wave_seg = reinterpret_cast<const uint32_t*>(d + p->wave_at);
     rc = launch_bundle_kernel(true, a, p->cfg, stream);
-    if (!rc) ++p->launches;
+    if (!rc) note_launch(p, Tables::kUploaded, p->cfg, true);
   }
   if (enqueued) {
     remember();
@@ -2404,11 +2418,12 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       if (cfg.threads > fit)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs with transposed views of different block sizes");
     }
+    if (cfg.kind != kModeRows) cfg.kind = kKindAny;   // the kernels there are for several jobs
     int rc = launch_bundle_jobs(table, cfg, stream);
     if (rc) return rc;
     for (size_t k = i; k < end; ++k) {
       axr_plan* p = jobs[k].plan;
-      ++p->launches;
+      note_launch(p, device_tables_of(p), cfg, false);   // (joint launches have no cached tail)
       if (jobs[k].unpack && p->pinned_host_tensors) stream_note_host_writes(stream);
       if (!capturing) remember_stream(p, stream);
     }
@@ -2436,7 +2451,7 @@ static int plan_launch_info_body(axr_plan_t* plan, axr_launch_info_t* info) {
                                 tables_fit_kernel_arguments(plan)
                             ? 1u
                             : 0u;
-  info->reserved = 0;
+  info->last_launch = plan->last_launch;
   return AXR_OK;
 }
 static int plan_prepare_body(axr_plan_t* plan, void* stream_) {

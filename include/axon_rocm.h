@@ -381,7 +381,16 @@ typedef struct axr_launch_info {
   uint32_t inline_tables;  /* 1: the next launch carries the tables inside the
                               kernel arguments, captured or not (small bundle,
                               first launch: no upload, no device block)        */
-  uint32_t reserved;
+  uint32_t last_launch;    /* how the plan was launched last, 0 before its first
+                              launch.  Bits 0-3: its tables were in 1 the kernel
+                              arguments, 2 pinned host memory, 3 device memory,
+                              laid out by the host, 4 device memory, laid out by a
+                              kernel.  Bits 4-7: the kernel, 0 for runs and groups
+                              only, for views of one kind 1 packed bytes, 2 rows,
+                              3 blocks, 4 blocks that are skewed or in strips,
+                              5 planes, and 6 for any.  Bits 8-31: MiB at the end of
+                              the payload that were packed with ordinary stores
+                              while the rest streamed                          */
 } axr_launch_info_t;
 AXR_API int axr_plan_launch_info(axr_plan_t* plan, axr_launch_info_t* info);
 

@@ -37,9 +37,11 @@ def test_first_and_later_launches_move_the_same_bytes(pkg, gpu, name, align, str
         want = torch.zeros(send.payload_bytes, dtype=torch.uint8, device=gpu)
         for t, at in zip(src, send.layout()[0]):
             want[at:at + t.numel()] = t
-        for _ in range(2):      # from the kernel arguments where they fit, then uploaded
+        for launch in range(2):      # from the kernel arguments where they fit, then uploaded
             payload = torch.full_like(want, 0x5a)
             send.pack(payload.data_ptr(), payload.numel())
+            in_arguments = launch == 0 and name not in ("crowd", "too_many")
+            assert send.launch_info()["last_launch"] & 15 == (1 if in_arguments else 3)
             assert torch.equal(payload, want)
             for t in dst:
                 t.zero_()

@@ -107,3 +107,22 @@ def test_null_sources_are_refused(pkg):
     assert bind(None, 0, C.byref(none), C.byref(h)) == invalid
     assert create(C.byref(none), 1, C.byref(h)) == 0 and h.value      # no tensors: nothing to describe
     pkg._capi.check(lib.axr_plan_free(h))
+
+
+def test_lists_with_other_arrays_are_not_tried(pkg, monkeypatch):
+    """An array in front, in the middle or at the end of tensors: no attempt that reads the tensors for nothing."""
+    from execution_ucx_amd import dlpack
+
+    class Native:
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} was asked")
+
+    good, other = torch.zeros(3), np.zeros(3, np.float32)
+    monkeypatch.setattr(dlpack, "_native_torch", lambda: Native())
+    for at in (0, 4, 8):
+        objs = [good] * 9
+        objs[at] = other
+        assert dlpack.plain_plan(pkg._capi.load(), objs, 1) is None
+        assert dlpack.plain_plan(pkg._capi.load(), tuple(objs), header=b"") is None
+    with pytest.raises(AssertionError, match="plan_create"):
+        dlpack.plain_plan(pkg._capi.load(), [good] * 9, 1)

@@ -242,10 +242,10 @@ constexpr uint32_t row_slots(uint64_t run_bytes, uint32_t start) {
   return static_cast<uint32_t>((start + run_bytes + kUnitBytes - 1) / kUnitBytes * (kUnitBytes / kVecBytes));
 }
 // Two, or three where that leaves a tenth less of a wavefront's slots without a row; four only for rows of
-// which three would hold one.  (Three pieces: 36 bytes at 37, 32 MiB, two 20.8, three 19.3 us for two packs.)
+// which three would hold one.  (Three pieces: 36 bytes at 37, 32 MiB, two 22.8, three 19.8 us for two packs.)
 // `mixed`: next to tensors that are moved otherwise.  The kernel for those holds fewer wavefronts, and larger
-// tiles make up for it (2^18 rows of 128 bytes at 131 39.0 us for pack + unpack with two slots per lane, 33.9
-// with four; of 666 at 1554 164 / 142).
+// tiles make up for it (2^18 rows of 128 bytes at 131, pack + unpack, next to 1 MiB of compact tensor 35.3 us with two
+// slots per lane, 32.8 with three, 32.5 with four; next to a transposed matrix 47.1 / 39.7 / 36.9).
 constexpr uint32_t row_slots_per_lane(uint32_t slots, bool mixed) {
   const uint32_t two = 2 * kWaveLanes / slots, three = 3 * kWaveLanes / slots;   // rows to a tile
   return mixed || three < 2 ? kMaxRowSlots : slots == 3 || 20 * three > 33 * two ? 3u : 2u;
@@ -255,10 +255,10 @@ constexpr uint32_t row_slots_per_lane(uint32_t slots, bool mixed) {
 // and what the lanes without a piece cost is more than the requests that are saved.  So they are taken where
 // they cost no row of a tile, and for two to seven units where the bundle has left the caches: by receivers,
 // which write the rows, from 24 MiB on, by senders of whole units, three or more, as well (such rows have no slot
-// to spare for another start: 256 at 292, 32 MiB, pack + unpack in turn 0.93, two packs in a launch 1.1), by the others
-// where the payload streams.  Slots for the worst start against
-// slots for a start on a unit, time of pack / unpack alone: 72 bytes at 73, 32 MiB 1.41 / 1.28; 200 at 201,
-// 12 MiB 1.16 / 1.15, 100 MiB 1.18 / 0.83, 200 MiB 1.25 / 0.73; 130 at 131, 200 MiB 1.37 / 0.72; 500 at 501, 100 MiB
+// to spare for another start: 256 at 292, 32 MiB, pack + unpack in turn 28.4 -> 26.7 us, two packs in a launch
+// 22.6 -> 23.9), by the others where the payload streams.  Slots for the worst start against slots for a start on a
+// unit, time of pack / unpack alone: 72 bytes at 73, 32 MiB 20.0 / 19.6 us against 13.1 / 15.0; 200 at 201, 12 MiB
+// 1.16 / 1.15 times, 100 MiB 1.18 / 0.83, 200 MiB 1.25 / 0.73; 130 at 131, 200 MiB 1.37 / 0.72; 500 at 501, 100 MiB
 // 1.30 / 1.08; 144 at 168, 400 MiB 1.01 / 0.99 and 0.78 in one launch.
 // Rows of up to 48 bytes whose neighbour lies in the same unit, or in the next one of a bundle that the caches
 // hold, take as many slots as they have pieces (16 bytes at 24 0.6 times the time of whole units for pack and
@@ -266,7 +266,7 @@ constexpr uint32_t row_slots_per_lane(uint32_t slots, bool mixed) {
 // Where a quarter of the slots of a row or more stay empty, more slots per lane make up for it: three, and for
 // rows of 65 to 80 bytes, five pieces of eight, four as long as the caches help (130 at 131, 200 MiB, pack alone: two
 // slots 1.43 times the time of three; 72 at 73, 32 MiB, two packs in a launch: two 26.5 us, three 21.8, four 20.1; 72 at
-// 128, 300 MiB 6 % slower with four than with two).
+// 128, 300 MiB 8 % slower with four than with two).
 constexpr uint64_t kRowUnitsPayload = 24ull << 20, kRowCachedPayload = 64ull << 20, kRowFilledPayload = 128ull << 20;
 struct RowRule {
   uint32_t slots, per_lane;
@@ -389,9 +389,9 @@ struct LaunchConfig {
   uint32_t threads = 128;   // per workgroup, a multiple of 64
   uint32_t seg_shift = 0;   // wave_seg has one entry per 2^seg_shift tiles
   uint32_t nontemporal = 3;   // bit 0: tensor-side accesses, bit 1: payload-side accesses
-  bool elements = false;   // some segment uses kModeElements or is transposed
+  bool elements = false;   // some segment's mode is above kModeRunTiles
   uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
-  uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (transposed tiles only)
+  uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (kModeRows and above)
   uint32_t cached_tail = 0;    // MiB at the end of a streaming payload that a pack leaves in the cache (runs in
                            // 1 KiB tiles only; see finish_geometry)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a

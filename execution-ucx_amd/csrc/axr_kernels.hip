@@ -10,8 +10,9 @@
 // keeps ROWS KiB in flight and every access is a fully coalesced 1 KiB row.
 //
 // Strided views with long runs use the same tile copy per run.  Views with
-// short runs (element mode) and transpositions (square or rectangular blocks
-// staged through LDS) live in separate instantiations of the kernel, so that
+// short runs (rows staged through LDS, runs under 16 bytes piece by piece) and
+// transpositions (blocks and planes staged through LDS) have kernels of their own,
+// one for each of them and one for bundles of several (views_kernel), so that
 // bundles without them run the small streaming kernels.
 #include <hip/hip_runtime.h>
 
@@ -299,7 +300,7 @@ __device__ __forceinline__ void element_moves(gbytes tbase, gbytes pbase, uint32
 
 // Element mode: the tile covers kTile packed bytes of a strided segment whose
 // contiguous runs are short; each lane decodes the tensor address of its own
-// granules.  Only kernels instantiated with ELEMENTS carry this code, so the
+// granules.  Only kernels of the kinds kModeElements and kKindAny carry this code, so the
 // streaming kernels keep a small register footprint.  The planner keeps every
 // extent and the run count below 2^31, so the per-granule arithmetic is 32-bit;
 // the tile's first run is decoded once (wave-uniform) and each lane only
@@ -377,10 +378,13 @@ typedef AXR_LDS uint8_t* lbytes;
 // it is cut from its own first byte on (a = 0), which only costs requests.
 // U is how many slots a lane moves, all in flight together.
 // Against 16-byte pieces moved without LDS, 8 KiB per wavefront, pack + unpack in turn, 2^18 rows, before /
-// now: 100 bytes at 256 40 / 34 us, 102 at 258 53 / 49, 128 at 256 29 / 26, 250 at 333 68 / 58, 256 at 512
-// 50 / 46, 256 at 515 73 / 65, 512 at 1024 89 / 82, 666 at 1554 156 / 138, 1001 at 1301 184 / 181, 1024 at 2048
-// 165 / 155; 2^20 rows of 250 at 1024 203 / 195, of 36 at 64 57 / 54.  What is left of the odd ones is
-// units whose other bytes are not the view's: each is read and merged by the memory.
+// now: 72 bytes at 73 19.7 / 18.7 us, 100 at 256 23.0 / 21.6, 102 at 258 28.8 / 26.2, 128 at 256 26.2 / 22.9, 250 at 333
+// 62.5 / 52.4, 256 at 512 44.1 / 38.7, 256 at 515 66.8 / 60.7, 512 at 1024 75.1 / 68.6, 666 at 704 98.4 / 92.9, 666 at 1554
+// 125.8 / 113.3, 1001 at 1301 159.1 / 142.5, 1024 at 2048 134.7 / 129.3; 2^20 rows of 24 at 25 29.8 / 21.3, of 36 at 64
+// 39.6 / 36.8, of 250 at 1024 171.8 / 164.2.  What is left of the odd ones is units that the view has in part: a pack
+// reads them whole (FETCH_SIZE 1.28 times the payload for 100 bytes at 256), an unpack writes their 32-byte sectors
+// in part (WRITE_SIZE 1.28 times) and reads nothing for it.  Unpacks of 16 to 24 bytes at 24 to 28 are 3 to 8 % behind
+// the pieces from 200 MB on.
 template <bool PACK, uint32_t U>
 __device__ __forceinline__ void rows_moves(uint64_t seg_ptr, uint32_t run, dims_table dm, gbytes pay,
                                            uint32_t q, lbytes lds, uint32_t lane, uint32_t nt_bits) {
@@ -1089,9 +1093,8 @@ __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t 
 }
 
 // Tile q of a transposed segment: batch index (outer dims), then block (ia, ib).
-// Deliberately not inlined: the block routines get a register allocation of
-// their own (inlined into the kernel's segment walk they spilled and cost the
-// other modes registers too), and forty kernel instantiations share the copies.
+// Inlined into the kernel of its MODE, which then reads its tables by scalar loads and has the registers of
+// that mode alone (see waves_of_kind), and into the kernel for any mode.
 // One copy per MODE: with the walk in strips and the choice of block routine in
 // the plain one's way, however predictable, 4 KiB blocks took 3 to 8 % longer.
 template <bool PACK, uint32_t MODE>
@@ -1402,10 +1405,11 @@ __device__ __forceinline__ void copy_tile_hinted(gbytes tensor, gbytes payload, 
 template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, uint32_t KIND>
 __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
                                             const AXR_CONST uint32_t* wave_seg, gbytes payload,
-                                            const KernelArgs& a, uint32_t wg, uint32_t lds_per_wave,
+                                            const KernelArgs& a, uint32_t wg, uint32_t lds_or_tail,
                                             uint32_t nt_bits) {
   constexpr bool runs = KIND == kKindRuns || KIND == kKindAny;   // runs, groups and fills may occur
-  // Where a payload that streams is packed in tiles of 1 KiB, `lds_per_wave` says how many MiB at its end are
+  // lds_or_tail: bytes of LDS per wavefront where tiles go through it.  Runs need none, and where a payload that
+  // streams is packed in tiles of 1 KiB it says how many MiB at the payload's end are
   // written with ordinary stores all the same (LaunchConfig::cached_tail; runs need no LDS).
   constexpr bool tail_stays = PACK && KIND == kKindRuns && ROWS == 1 && NTT && NTP;
   constexpr uint32_t kTile = ROWS * kRowBytes;
@@ -1435,7 +1439,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
     if constexpr (KIND == kKindAny) {
       copy_tile_hinted<PACK, ROWS>(ten, pay, left, lane, lane_off, nt_bits);
     } else if constexpr (tail_stays) {
-      if (a.ntiles - t <= lds_per_wave << 10) {   // (asm: as in copy_tile_hinted)
+      if (a.ntiles - t <= lds_or_tail << 10) {   // (asm: as in copy_tile_hinted)
         asm volatile("");
         copy_tile<PACK, ROWS, NTT, false>(ten, pay, left, lane, lane_off);
         asm volatile("");
@@ -1521,8 +1525,8 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         gbytes p = pay + static_cast<uint64_t>(run) * seg_run + boff;
         copy(ten, p, left);
       } else if constexpr (KIND != kKindRuns) {
-        extern __shared__ uint8_t lds_slices[];   // lds_per_wave bytes for each wavefront
-        lbytes lds = (lbytes)lds_slices + uniform(threadIdx.x >> 6) * lds_per_wave;
+        extern __shared__ uint8_t lds_slices[];   // lds_or_tail bytes for each wavefront
+        lbytes lds = (lbytes)lds_slices + uniform(threadIdx.x >> 6) * lds_or_tail;
         if (mode == kModeElements) element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
         else if (mode == kModeRows) rows_tile<PACK>(seg_ptr, static_cast<uint32_t>(seg_run), dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
@@ -1540,7 +1544,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
 // Tables in device memory (uploaded once per plan).
 // Scalar arguments (not one struct) so that the compiler can preload them into SGPRs at
 // dispatch instead of fetching the kernarg segment first.  Fourteen dwords are preloaded,
-// which is why the LDS bytes per wavefront (bits 0-16), the hints with the wavefronts per
+// which is why the LDS bytes per wavefront or the MiB of cached tail (bits 0-16), the hints with the wavefronts per
 // workgroup (bits 17-23, the argument bundle_body takes) and the tile-block shift (bits
 // 24-31) share one of them: the address delta then fits in as well, and no wavefront waits
 // for a kernel-argument load before it can form its first tensor address.
@@ -1551,7 +1555,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   segs_arg, dims_arg, wave_seg_arg, payload_arg, ntiles, tiles_per_wave, xcd_remap, geometry, tensor_delta
 template <bool PACK, uint32_t ROWS, bool NTT, bool NTP, uint32_t KIND>
 __device__ __forceinline__ void bundle_from_arguments(AXR_BUNDLE_PARAMETERS) {
-  const uint32_t lds_per_wave = geometry & 0x1ffffu;
+  const uint32_t lds_or_tail = geometry & 0x1ffffu;
   const uint32_t nt_bits = (geometry >> 17 & 3u) | (geometry >> 19 & 0x1fu) << 8;
   KernelArgs a;
   a.ntiles = ntiles;
@@ -1563,7 +1567,7 @@ __device__ __forceinline__ void bundle_from_arguments(AXR_BUNDLE_PARAMETERS) {
       reinterpret_cast<seg_table>(reinterpret_cast<uintptr_t>(segs_arg)),
       reinterpret_cast<dims_table>(reinterpret_cast<uintptr_t>(dims_arg)),
       reinterpret_cast<const AXR_CONST uint32_t*>(reinterpret_cast<uintptr_t>(wave_seg_arg)),
-      reinterpret_cast<gbytes>(reinterpret_cast<uintptr_t>(payload_arg)), a, blockIdx.x, lds_per_wave,
+      reinterpret_cast<gbytes>(reinterpret_cast<uintptr_t>(payload_arg)), a, blockIdx.x, lds_or_tail,
       nt_bits);
 }
 
@@ -1690,7 +1694,7 @@ __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThrea
 // nothing unless the first word carries the mark the host wrote.
 struct InlineScalars {   // mirrors the argument list of bundle_kernel_inline
   uint8_t* payload;
-  uint32_t ntiles, tiles_per_wave, xcd_remap, seg_shift, lds_per_wave, nt_bits, dims_at, wave_at;
+  uint32_t ntiles, tiles_per_wave, xcd_remap, seg_shift, lds_or_tail, nt_bits, dims_at, wave_at;
   InlineTables tables;
 };
 constexpr uint32_t kInlineTablesOffset = __builtin_offsetof(InlineScalars, tables);
@@ -1700,7 +1704,7 @@ template <bool PACK, uint32_t KIND, uint32_t ROWS, bool NTP>
 __global__ __attribute__((amdgpu_waves_per_eu(waves_of_kind(KIND, 2))))
 __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThreads) void bundle_kernel_inline(
     uint8_t* payload_arg, uint32_t ntiles, uint32_t tiles_per_wave, uint32_t xcd_remap,
-    uint32_t seg_shift, uint32_t lds_per_wave, uint32_t nt_bits, uint32_t dims_at, uint32_t wave_at,
+    uint32_t seg_shift, uint32_t lds_or_tail, uint32_t nt_bits, uint32_t dims_at, uint32_t wave_at,
     InlineTables tables) {
   (void)tables;
   const AXR_CONST uint8_t* base =
@@ -1717,7 +1721,7 @@ __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThrea
       reinterpret_cast<seg_table>(base + kInlineTablesHead),
       reinterpret_cast<dims_table>(base + kInlineTablesHead + dims_at),
       reinterpret_cast<const AXR_CONST uint32_t*>(base + kInlineTablesHead + wave_at),
-      reinterpret_cast<gbytes>(reinterpret_cast<uintptr_t>(payload_arg)), a, blockIdx.x, lds_per_wave,
+      reinterpret_cast<gbytes>(reinterpret_cast<uintptr_t>(payload_arg)), a, blockIdx.x, lds_or_tail,
       nt_bits);
 }
 

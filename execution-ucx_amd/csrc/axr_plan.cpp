@@ -977,8 +977,12 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   // evicts its own beginning.  Pack + unpack of the nine bf16 weights of a layer, three bundles in turn, all
   // streaming / 160 / 192 / 224 / 240 / 250 MiB kept: 405 MB 248.5 / 242 / 240 / 237 / 236 / 235 us, one bundle
   // over and over 247.5 / 242.5 / 240.6 / 237.7 / 236.5 / 246; 419 MB of cache blocks 268 / 264 / 262 / 259 / 258 /
-  // 279; 1 GiB of compact tensors 649 / - / 639 / 638 / 636 / -.  A pack whose payload nobody reads takes 129
-  // instead of 125 us at 405 MB: it writes back what an earlier one left.
+  // 279; 1 GiB of compact tensors 649 / - / 639 / 638 / 636 / -.  Chunks streamed on two streams, each with a tail of its
+  // own, gain as well: 6 of 320 MiB 1370 -> 1275 us, 4 of 512 MiB 1425 -> 1384, 2 of 1 GiB 1455 -> 1417.
+  // A pack whose payload nothing of this library reads: into one buffer over and over 94.1 -> 90.0 us at 306 MB, 124.3 ->
+  // 119.8 at 405; into three in turn, writing back what the earlier ones left, 93.8 -> 97.6 and 124.2 -> 128.0 (1 to 4 %
+  // whatever the length of the tail, and with its last 8 to 48 MiB streaming again); followed by a plain copy of the
+  // payload 215 -> 219 and 283.7 -> 286.3.  AXR_JOB_PAYLOAD_STREAMING declines it for a launch, "nontemporal" 3 for all.
   p->cfg.cached_tail = 0;
   if (rows == 1 && !p->cfg.elements && p->cfg.nontemporal == 3u && tn.nontemporal < 0)
     p->cfg.cached_tail = static_cast<uint32_t>(
@@ -2416,7 +2420,7 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       // every plan sized its workgroups for its own LDS need; the launch uses the largest
       const uint32_t fit = (64u * 1024u / cfg.lds_per_wave) * kWaveLanes;
       if (cfg.threads > fit)
-        return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs with transposed views of different block sizes");
+        return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs whose views need different amounts of LDS");
     }
     if (cfg.kind != kModeRows) cfg.kind = kKindAny;   // the kernels there are for several jobs
     int rc = launch_bundle_jobs(table, cfg, stream);

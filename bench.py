@@ -389,11 +389,11 @@ def _random_storage(torch, shape, dtype, seed):
 
 # Strided views: name -> (description, function(torch, seed) -> list of views of fresh storage)
 VIEW_WORKLOADS = {
-    "rows100": ("fp32 [2M, 64][:, :25]: rows of 100 B at a 256 B pitch (element mode, ragged 16-byte granules)",
+    "rows100": ("fp32 [2M, 64][:, :25]: rows of 100 B at a 256 B pitch (whole rows through LDS)",
                 lambda t, seed: [_random_storage(t, (1 << 21, 64), t.float32, seed)[:, :25]]),
-    "rows250": ("bf16 [1M, 512][:, :125]: rows of 250 B at a 1 KiB pitch (element mode, ragged 16-byte granules)",
+    "rows250": ("bf16 [1M, 512][:, :125]: rows of 250 B at a 1 KiB pitch (whole rows through LDS)",
                 lambda t, seed: [_random_storage(t, (1 << 20, 512), t.bfloat16, seed)[:, :125]]),
-    "rows512": ("bf16 [512K, 512][:, :256]: rows of 512 B at a 1 KiB pitch (element mode, 16-byte granules)",
+    "rows512": ("bf16 [512K, 512][:, :256]: rows of 512 B at a 1 KiB pitch (whole rows through LDS)",
                 lambda t, seed: [_random_storage(t, (1 << 19, 512), t.bfloat16, seed)[:, :256]]),
     "stepped": ("fp32 [16M, 8][:, ::2]: every second element (element mode, 4-byte granules)",
                 lambda t, seed: [_random_storage(t, (1 << 24, 8), t.float32, seed)[:, ::2]]),

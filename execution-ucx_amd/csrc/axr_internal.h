@@ -563,11 +563,11 @@ void table_block_release(TableBlock* block);
 // Events without timing for the current device, recycled: creating one costs more than a
 // microsecond, and every fresh plan that uploads tables needs one.  An event goes back
 // only once it has fired (or was never recorded).
-// device_scope: an event whose record releases what kernels wrote to the device, for streams of the same device
-// that wait for it (hipEventReleaseToDevice), and not to the host or other devices.  The kernel behind it starts
-// 2 us sooner (48 cache blocks of 32 runs, fresh, pack + unpack, 44.5 -> 40.8 us).  The host waits for no such event.
-int event_acquire(bool device_scope, void** event, int* device);
-void event_release(bool device_scope, void* event, int device);
+// They release to the system.  A kernel behind one that does not (hipEventDisableSystemFence) starts 1.6 us sooner
+// (140 views that all differ, fresh, pack + unpack, 56.1 -> 54.5 us), but nothing then promises that what is in
+// front of it is visible; with hipEventReleaseToDevice, which would be enough, it does not start sooner (56.3).
+int event_acquire(void** event, int* device);
+void event_release(void* event, int device);
 
 }  // namespace axr
 

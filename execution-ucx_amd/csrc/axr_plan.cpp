@@ -213,7 +213,6 @@ struct axr_plan {
   uint32_t last_launch = 0;          // axr_launch_info_t::last_launch
   hipEvent_t upload_event = nullptr;   // from event_acquire; behind the latest upload once `uploaded` is set
   int upload_event_device = -1;
-  bool upload_event_by_kernel = false;   // a device-scope event: a kernel wrote the tables
   hipStream_t upload_stream = nullptr;
   struct BusyStream {
     hipStream_t stream;
@@ -1011,16 +1010,11 @@ uint32_t rows_for_compact_bundle(const axr_plan* p) {
 // another stream waits for is recorded here, right behind the upload, on the default stream as on any
 // other: recorded later it would lie behind whatever the stream was given in between, and a launch
 // elsewhere would wait for work that is not its own.
-int note_upload(axr_plan* p, hipStream_t stream, bool by_kernel = true) {
+int note_upload(axr_plan* p, hipStream_t stream) {
   remember_stream(p, stream);
-  if (p->upload_event && p->upload_event_by_kernel != by_kernel) {   // (an earlier upload's, drained before its block was reused)
-    event_release(p->upload_event_by_kernel, p->upload_event, p->upload_event_device);
-    p->upload_event = nullptr;
-  }
   if (!p->upload_event) {
-    int rc = event_acquire(by_kernel, reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
+    int rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
     if (rc) return rc;
-    p->upload_event_by_kernel = by_kernel;
   }
   int rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
   if (rc) return rc;
@@ -1491,12 +1485,12 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
   if (!p->uploaded) {
     int rc = write_host_block(p);
     if (rc) return rc;
-    const bool by_kernel = p->table_bytes <= kKernelUploadBytes;
-    rc = by_kernel ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
-                   : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
-                               "hipMemcpyAsync(plan tables)");
+    rc = p->table_bytes <= kKernelUploadBytes
+             ? launch_upload_tables(p->block.host, p->block.device, p->table_bytes, stream)
+             : check_hip(hipMemcpyAsync(p->block.device, p->block.host, p->table_bytes, hipMemcpyHostToDevice, stream),
+                         "hipMemcpyAsync(plan tables)");
     if (rc) return rc;
-    return note_upload(p, stream, by_kernel);
+    return note_upload(p, stream);
   }
   if (stream != p->upload_stream)
     return check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
@@ -1891,7 +1885,7 @@ static int plan_free_body(axr_plan_t* plan) {
   if (!plan) return AXR_OK;
   quiesce(plan);
   table_block_release(&plan->block);
-  event_release(plan->upload_event_by_kernel, plan->upload_event, plan->upload_event_device);   // fired: the upload's stream has been drained
+  event_release(plan->upload_event, plan->upload_event_device);   // fired: the upload's stream has been drained
   plan->upload_event = nullptr;
   for (HostStage& st : plan->stage) {
     table_block_release(&st.block);
@@ -2467,9 +2461,7 @@ static int plan_prepare_body(axr_plan_t* plan, void* stream_) {
   if (plan->ntiles == 0 || plan->resident) return AXR_OK;
   rc = ensure_uploaded(plan, stream);
   if (rc) return rc;
-  // The upload or a wait for it is on `stream` now.  Later launches read the tables on any stream without
-  // waiting for anything, so the host waits for the stream itself and not for an event of device scope.
-  rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize(plan tables)");
+  rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
   if (rc) return rc;
   plan->resident = true;
   return AXR_OK;

@@ -101,17 +101,17 @@ size_t bucket_bytes(size_t bytes) {
 
 namespace {
 std::mutex g_event_mutex;
-std::map<std::pair<int, bool>, std::vector<hipEvent_t>> g_idle_events;   // per device and scope
+std::unordered_map<int, std::vector<hipEvent_t>> g_idle_events;   // per device
 constexpr size_t kMaxIdleEvents = 64;
 }  // namespace
 
-int event_acquire(bool device_scope, void** event, int* device) {
+int event_acquire(void** event, int* device) {
   int dev = -1;
   int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc) return rc;
   {
     std::lock_guard<std::mutex> lock(g_event_mutex);
-    std::vector<hipEvent_t>& idle = g_idle_events[{dev, device_scope}];
+    std::vector<hipEvent_t>& idle = g_idle_events[dev];
     if (!idle.empty()) {
       *event = idle.back();
       *device = dev;
@@ -120,18 +120,18 @@ int event_acquire(bool device_scope, void** event, int* device) {
     }
   }
   hipEvent_t e = nullptr;
-  rc = check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming | (device_scope ? hipEventReleaseToDevice : 0u)), "hipEventCreate");
+  rc = check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
   if (rc) return rc;
   *event = e;
   *device = dev;
   return AXR_OK;
 }
 
-void event_release(bool device_scope, void* event, int device) {
+void event_release(void* event, int device) {
   if (!event) return;
   {
     std::lock_guard<std::mutex> lock(g_event_mutex);
-    std::vector<hipEvent_t>& idle = g_idle_events[{device, device_scope}];
+    std::vector<hipEvent_t>& idle = g_idle_events[device];
     if (idle.size() < kMaxIdleEvents) {
       idle.push_back(static_cast<hipEvent_t>(event));
       return;

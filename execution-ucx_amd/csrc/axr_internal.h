@@ -439,9 +439,10 @@ struct Tunables {
   // Bundles of at least this many tensors, all of them contiguous device tensors, get their
   // tables in one pass over the tensors into pinned memory plus a kernel that brings them to
   // the device and writes the tile-block index (0: the general host path always).  Fresh bundles of 256 B
-  // to 64 KiB, pack + unpack, host / device tables: 256 tensors 49.1 / 49.7 us, 300 51.8 / 51.5, 360 55.9 / 53.9,
-  // 420 59.7 / 56.4; of 600 to 4000 bytes 300 49.2 / 51.4, 480 60.8 / 58.9.
-  std::atomic<int64_t> device_tables{320};
+  // to 64 KiB, pack + unpack, host tables read in place / device tables: 300 tensors 53.4 / 54.8 us, 340 55.6 / 56.2, 380
+  // 58.3 / 58.1, 420 61.1 / 59.7; of 600 to 4000 bytes 320 50.7 / 55.3, 480 61.6 / 63.4, 600 68.7 / 69.0; of 64 KiB 320
+  // 53.2 / 56.1, 440 61.8 / 63.3.
+  std::atomic<int64_t> device_tables{384};
   // axr_stream_synchronize may first poll, for up to this many microseconds, a word of pinned
   // memory that a one-wave kernel enqueued behind the stream's work writes, before it falls
   // back to the runtime's wait (0, the default: the runtime's wait only).  See the header.

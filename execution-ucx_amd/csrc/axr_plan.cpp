@@ -1145,9 +1145,10 @@ int device_build_tables(axr_plan* p, hipStream_t stream, bool* done) {
     }
     if (!all_device) return AXR_OK;   // before a block is taken: host tensors need no tables on the device
     if (small == n) {
-      // only from 1.6 times as many on: fresh, pack + unpack, groups from the host, read there / from the device,
-      // 330 tensors of 8 to 512 bytes 47.8 / 55.2 us, 500 57.0 / 62.7, 700 (more than 32 KiB) 76 / 72
-      return n * 5 >= static_cast<uint64_t>(least) * 8 ? device_build_groups(p, stream, done) : AXR_OK;
+      // only from a third more on: fresh, pack + unpack, groups from the host / from the device, 330 tensors of 8 to 512
+      // bytes 49.9 / 57.5 us, 420 54.4 / 62.1 (read in place up to here, uploaded beyond 32 KiB), 440 65.4 / 62.0, 512
+      // 70.1 / 65.9, 900 94.0 / 85.2; of 100 bytes 420 52.2 / 61.2, 512 57.0 / 65.2
+      return n * 3 >= static_cast<uint64_t>(least) * 4 ? device_build_groups(p, stream, done) : AXR_OK;
     }
     if (small * 4 >= n) return AXR_OK;
   }
@@ -1468,10 +1469,10 @@ int write_host_block(axr_plan* p) {
 
 // Whether a plan's first launch reads its host-built tables where the host has written them.  Every wavefront
 // then waits for the bus instead of for a cache, but the upload, the event behind it and the wait for both
-// go, about 5 us of a fresh bundle's round trip, pack + unpack, uploaded / read in place: 128 tensors of 256 B to
-// 64 KiB 47.0 / 42.1 us, 200 49.9 / 45.6, 300 56.2 / 51.7, 300 of 64 KiB 54.7 / 51.3, 256 cache blocks of 16 runs
-// 62.9 / 58.5.  Not where a wavefront reads a view's own record as well (140 views that all differ, 64 rows of 300
-// bytes each, 53.3 / 55.9; 100 rows of 2000 bytes 69.2 / 80.4), and with many wavefronts the reads add up (512
+// go, about 6 us of a fresh bundle's round trip, pack + unpack, uploaded / read in place: 128 tensors of 256 B to
+// 64 KiB 47.9 / 41.7 us, 200 52.3 / 46.2, 300 58.6 / 52.9, 300 of 64 KiB 57.0 / 51.6.  Not where a wavefront reads a
+// view's own record as well (140 views that all differ, 64 rows of 300 bytes each, level at 56; 100 rows of 2000
+// bytes 71 / 80), and with many wavefronts the reads add up (512
 // blocks of 64 runs, 1 GiB, 745 / 860).  A plan that is launched again is being reused and uploads then.
 constexpr size_t kHostTableBytes = 32u << 10;
 bool first_launch_reads_host_block(const axr_plan* p) {

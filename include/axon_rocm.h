@@ -469,8 +469,8 @@ AXR_API int axr_plan_segments(axr_plan_t* plan, axr_segment_info_t* out, size_t 
  * "device_tables" (a bundle of at least this many tensors, all contiguous device
  * tensors, takes a short path to its device tables: one pass over the tensors into
  * pinned memory and a kernel that brings the records to the device and writes the
- * tile-block index, instead of the general host build plus an upload; default 320,
- * 1.6 times as many where all are short; 0: never),
+ * tile-block index, instead of the general host build plus an upload; default 384,
+ * a third more where all are short; 0: never),
  * "loopback_copy_kernel" (1, default: the loopback context moves a device payload
  * to device memory with the library's copy kernel; 0: with hipMemcpyAsync),
  * "group_bytes" (contiguous device tensors of at most this many bytes that follow each

@@ -36,7 +36,7 @@ def expected(src, plan, gpu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("align", [1, 256])
-@pytest.mark.parametrize("kind, count", [("mixed", 112), ("mixed", 319), ("mixed", 320), ("short", 300), ("blocks", 110),
+@pytest.mark.parametrize("kind, count", [("mixed", 112), ("mixed", 319), ("mixed", 320), ("mixed", 383), ("mixed", 384), ("short", 300), ("blocks", 110),
                                          ("blocks", 400), ("views", 120)])
 def test_first_second_and_rebound_launches(pkg, gpu, kind, count, align):
     src = tensors(kind, count, gpu, 3)

@@ -42,10 +42,10 @@ def launches(pkg, tensors, count=2, align=256):
 @pytest.mark.parametrize("sizes,first,later", [
     ([64 * KIB] * 98, ARGUMENTS, UPLOADED),            # 3.5 KiB hold 99 records of 32 bytes, an index of as many blocks
     ([64 * KIB] * 99, PINNED, UPLOADED),               # and a mark, no more
-    ([64 * KIB] * 319, PINNED, UPLOADED),
-    ([64 * KIB] * 320, DEVICE_BUILT, DEVICE_BUILT),
+    ([64 * KIB] * 383, PINNED, UPLOADED),
+    ([64 * KIB] * 384, DEVICE_BUILT, DEVICE_BUILT),
     ([300] * 300, PINNED, UPLOADED),                   # blocks of groups: up to 32 KiB of them,
-    ([300] * 511, UPLOADED, UPLOADED),                 # from 1.6 times as many tensors on laid out by a kernel
+    ([300] * 511, UPLOADED, UPLOADED),                 # from a third more tensors on laid out by a kernel
     ([300] * 512, DEVICE_BUILT, DEVICE_BUILT),
     ([16384 * 2 * KIB], ARGUMENTS, UPLOADED),          # small bundles end at 16,384 tiles,
     ([16385 * 2 * KIB], ARGUMENTS, UPLOADED),          # a long tensor's index fits in wide blocks,
@@ -75,7 +75,7 @@ def test_switched_off(pkg, gpu):
         for n in (3, 200, 600):
             assert [r[0] for r in launches(pkg, carve(gpu, [64 * KIB] * n))] == [UPLOADED, UPLOADED]
     finally:
-        pkg.tune(inline_tables=16384, device_tables=320)
+        pkg.tune(inline_tables=16384, device_tables=384)
 
 
 VIEWS = {

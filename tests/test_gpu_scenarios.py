@@ -19,7 +19,7 @@ TUNABLES = {
     "nontemporal": [-1, -1, 0, 1, 2, 3], "max_waves": [1 << 20, 1 << 20, 96, 1024],
     "xcd_remap": [-1, 0, 1], "group_bytes": [512, 512, 0, 128], "group_slots": [64, 128],
     "payload_cache_bytes": [256 << 20, 256 << 20, 0], "head_align": [16, 0, 64],
-    "inline_tables": [16384, 0], "device_tables": [320, 0, 8], "transpose": [1, 1, 0],
+    "inline_tables": [16384, 0], "device_tables": [384, 0, 8], "transpose": [1, 1, 0],
     "ragged_runs": [1, 1, 0], "gather_run_bytes": [1280, 256, 4096], "submit_interleave": [1, 2, 0],
 }
 

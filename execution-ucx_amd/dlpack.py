@@ -276,16 +276,24 @@ def _plain_tensors(objs: Sequence[Any], exporter: tuple) -> Optional[tuple]:
     return None if direct is None else direct.describe(objs, exporter[2])
 
 
+_SAMPLED = 512    # objects from which on a list is asked in three places
+
+
 def _plain_sample(objs: Any) -> bool:
-    """Whether asking for plain tensors is worth the attempt: the first, the last and the middle one are.  (4095
-    tensors and an array behind them: the attempt is given up at the array, 190 of 2020 us.)"""
+    """Whether asking for plain tensors is worth the attempt: the first one is, and of many the last and the middle one.
+    (4095 tensors and an array behind them: the attempt is given up at the array, 190 of 2020 us.  Asking in three
+    places takes 0.2 us per plan, which shows in a fresh bundle of 300 tensors: pack + unpack 51.2 -> 51.6 us.)"""
     torch = sys.modules.get("torch")
     if torch is None:
         return False
     if not objs:
         return True
+    if type(objs[0]) is not torch.Tensor and type(objs[0]) is not torch.nn.Parameter:
+        return False
+    if len(objs) < _SAMPLED:
+        return True
     plain = (torch.Tensor, torch.nn.Parameter)
-    return type(objs[0]) in plain and type(objs[-1]) in plain and type(objs[len(objs) // 2]) in plain
+    return type(objs[-1]) in plain and type(objs[len(objs) // 2]) in plain
 
 
 _PLAN_MAKERS: dict = {}    # library -> addresses of axr_plan_create_from and axr_plan_bind_from

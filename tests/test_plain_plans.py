@@ -110,7 +110,8 @@ def test_null_sources_are_refused(pkg):
 
 
 def test_lists_with_other_arrays_are_not_tried(pkg, monkeypatch):
-    """An array in front, in the middle or at the end of tensors: no attempt that reads the tensors for nothing."""
+    """An array in front, in the middle or at the end of many tensors, or in front of a few: no attempt that reads the
+    tensors for nothing."""
     from execution_ucx_amd import dlpack
 
     class Native:
@@ -119,8 +120,8 @@ def test_lists_with_other_arrays_are_not_tried(pkg, monkeypatch):
 
     good, other = torch.zeros(3), np.zeros(3, np.float32)
     monkeypatch.setattr(dlpack, "_native_torch", lambda: Native())
-    for at in (0, 4, 8):
-        objs = [good] * 9
+    for count, at in ((512, 0), (512, 256), (512, 511), (9, 0)):
+        objs = [good] * count
         objs[at] = other
         assert dlpack.plain_plan(pkg._capi.load(), objs, 1) is None
         assert dlpack.plain_plan(pkg._capi.load(), tuple(objs), header=b"") is None

@@ -287,13 +287,11 @@ constexpr RowRule row_rule(uint64_t run_bytes, uint64_t pitch, uint32_t start, b
   const uint32_t lanes = per_lane * kWaveLanes;
   return {lanes / worst == lanes / whole ? worst : whole, per_lane};
 }
-// Whether bundles of these kinds may share a launch.  In the kernel for any mode the tiles of rows alone lose more
+// Whether bundles may share a launch that hold so many tiles of rows alone, and other kinds or not.  In the kernel for any mode the tiles of rows alone lose more
 // than a launch costs once there are a few thousand of them (rows of 300 bytes at 512 and 1 MiB of compact tensor, joined /
 // launched in turn: 640 tiles 5.2 / 6.9 us, 1280 7.5 / 7.7, 2560 11.7 / 10.9, 10240 34.5 / 28.6).
 constexpr uint32_t kRowTilesJoined = 2048;
-constexpr bool kinds_share_launch(uint32_t kind_x, uint32_t tiles_x, uint32_t kind_y, uint32_t tiles_y) {
-  return kind_x == kind_y || !((kind_x == kModeRows && tiles_x > kRowTilesJoined) || (kind_y == kModeRows && tiles_y > kRowTilesJoined));
-}
+constexpr bool rows_share_launch(uint64_t row_tiles, bool others) { return !others || row_tiles <= kRowTilesJoined; }
 constexpr uint32_t rows_lds_bytes(uint32_t rows, uint64_t run_bytes) {
   return static_cast<uint32_t>(rows * run_bytes) + kUnitBytes;
 }

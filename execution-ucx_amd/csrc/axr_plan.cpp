@@ -2338,7 +2338,6 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     const axr_plan *x = jx.plan, *y = jy.plan;
     return x->cfg.tile_rows == y->cfg.tile_rows && x->cfg.threads == y->cfg.threads &&
            effective_nontemporal(x, jx.flags) == effective_nontemporal(y, jy.flags) &&
-           kinds_share_launch(x->cfg.kind, x->ntiles, y->cfg.kind, y->ntiles) &&
            (!(x->cfg.elements || y->cfg.elements) || (x->cfg.tile_rows == 2 && x->cfg.threads <= kMaxElementThreads));
   };
   size_t i = 0;
@@ -2346,8 +2345,16 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     axr_plan* first = jobs[i].plan;
     size_t end = i + 1;
     if (batchable(first)) {
+      uint64_t row_tiles = 0;
+      bool others = false;
+      auto joins = [&](const axr_plan* p) {
+        if (p->cfg.kind == kModeRows) row_tiles += p->ntiles;
+        else others = true;
+        return rows_share_launch(row_tiles, others);
+      };
+      joins(first);
       while (end < n && end - i < kMaxJobs && batchable(jobs[end].plan) &&
-             same_geometry(jobs[i], jobs[end]))
+             same_geometry(jobs[i], jobs[end]) && joins(jobs[end].plan))
         ++end;
     }
     if (end - i == 1) {

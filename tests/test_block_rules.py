@@ -207,9 +207,8 @@ def test_rows_that_share_a_launch(tmp_path):
     source = r"""
 #include "axr_internal.h"
 using namespace axr;
-static_assert(kinds_share_launch(kModeRows, 1u << 20, kModeRows, 3) && kinds_share_launch(kModeRows, 2048, kKindAny, 1u << 20));
-static_assert(!kinds_share_launch(kModeRows, 2049, kKindAny, 3) && !kinds_share_launch(kModeTranspose, 3, kModeRows, 2049));
-static_assert(kinds_share_launch(kModeTranspose, 1u << 20, kKindAny, 1u << 20));
+static_assert(rows_share_launch(uint64_t(1) << 40, false) && rows_share_launch(0, true));
+static_assert(rows_share_launch(2048, true) && !rows_share_launch(2049, true));
 """
     src = str(tmp_path / "share.cpp")
     with open(src, "w") as f:

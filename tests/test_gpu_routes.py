@@ -105,11 +105,14 @@ def test_every_kind_has_its_kernel(pkg, gpu, kind):
 
 @pytest.mark.parametrize("kinds,want", [((ROWS, ROWS), (ROWS, ROWS)), ((ROWS, RUNS), (ANY, ANY)), ((BLOCKS, BLOCKS), (ANY, ANY)),
                                         ((RUNS, RUNS), (RUNS, RUNS)), (("many", RUNS), (ROWS, RUNS)), (("many", ROWS), (ROWS, ROWS)),
-                                        ((BLOCKS, "many"), (BLOCKS, ROWS))], ids=str)
+                                        ((BLOCKS, "many"), (BLOCKS, ROWS)), ((ROWS, "many", RUNS), (ROWS, ROWS, RUNS)),
+                                        ((ROWS, RUNS, "many"), (ANY, ANY, ROWS)), (("some", "some", RUNS), (ROWS, ROWS, RUNS)),
+                                        (("some", RUNS), (ANY, ANY))], ids=str)
 def test_kinds_in_one_submission(pkg, gpu, kinds, want):
     capi = pkg._capi
     store = torch.zeros(40000 * 131, dtype=torch.uint8, device=gpu)
-    plans = [pkg.BundlePlan.create([store.view(40000, 131)[:, :100]] if k == "many" else VIEWS[k](store), align=64).prepare() for k in kinds]
+    rows = {"many": 40000, "some": 20000}      # tiles of 16: 2500 and 1250 of them
+    plans = [pkg.BundlePlan.create([store.view(40000, 131)[:rows[k], :100]] if k in rows else VIEWS[k](store), align=64).prepare() for k in kinds]
     payloads = [torch.empty(p.payload_bytes, dtype=torch.uint8, device=gpu) for p in plans]
     jobs = (capi.Job * len(plans))()
     for j, p, y in zip(jobs, plans, payloads):

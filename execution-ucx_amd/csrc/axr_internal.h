@@ -482,6 +482,16 @@ struct HostCopyJob {
   size_t bytes;
 };
 void host_copy(const HostCopyJob* jobs, size_t count);
+// A staging block moved unit by unit from the front, by the caller and up to `helpers` short-lived threads in turn.
+struct HostUnits {
+  size_t span = 0, unit = 1, helpers = 0;   // the block's bytes [0, span), in units of `unit`
+  // Whether unit `u` may be moved; waits for it.  False (an error, known to the caller's thread) ends the thread's share.
+  virtual bool ready(size_t u, bool caller) = 0;
+  virtual void copy(size_t lo, size_t hi) = 0;   // moves bytes [lo, hi); from any of the threads
+  virtual int done(size_t u) = 0;                // units 0 .. u have been moved; in order, on the caller's thread
+  virtual ~HostUnits() = default;
+};
+int host_copy_units(HostUnits& units);   // what done() returned, or AXR_OK
 
 // True for a handle that axr_stream_destroy has destroyed (and no later
 // axr_stream_create has returned again).
@@ -541,6 +551,10 @@ int launch_expand_groups(const Member* members, const GroupStage* groups, uint32
 int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream);
 // dst[0, bytes) = src[0, bytes), both in device memory of the current device, no alignment needed.
 int launch_stream_copy(void* dst, const void* src, size_t bytes, bool nontemporal, void* stream);
+// dst[0, bytes) = src[0, bytes) from device memory to pinned host memory; flags[i] (pinned, cleared by the
+// caller) becomes 1 once bytes [i, i + 1) * kStagePieceBytes are there.
+constexpr uint32_t kStagePieceBytes = 16384, kStageGroups = 16;
+int launch_stage_out(void* dst, const void* src, size_t bytes, uint32_t* flags, void* stream);
 // Device address, on the current device, of the kStaticTableBytes bytes that hold the
 // tables of axr_pack_noalloc (a __device__ array of the code object: never allocated,
 // shared by every call on that device).

@@ -19,11 +19,13 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <mutex>
 #include <new>
+#include <thread>
 
 #include "axr_internal.h"
 #include "axr_source.h"
@@ -113,12 +115,27 @@ struct HostCopy {
 // Host tensors travel through pinned staging blocks: one device copy per chunk
 // of neighbouring pieces instead of one pageable copy per piece.
 constexpr size_t kStageBytes = 8u << 20;
+// How a block goes over the bus (fresh bundles of host arrays, pack + unpack, one transfer of the whole block each way
+// before / now: 64 KiB 44.6 / 33.8 us, 256 KiB 61 / 45, 512 KiB 83 / 63, 1 MiB 125 / 96, 4 MiB 357 / 270):
+//  - Threads take kStageUnit at a time.  A helper costs its starter 12 us, so there is one for every whole
+//    kStagePerThread behind the first (1 MiB with a helper 118 us).
+//  - To the payload goes a first piece of kStageSend or a sixteenth of the block, and then pieces of 5/16 of it, four
+//    in all: with eight or more the wait at the end takes 26 us instead of 4 (4 MiB 303 to 310).  A kernel's first
+//    bytes move sooner than the copy engine's, which moves more per second: kernels / engine 1 MiB 96 / 117, 4 MiB 276 / 268.
+//  - From the payload a kernel of kStageGroups workgroups brings the block and raises its flags in order (see
+//    stage_out_kernel; 4 MiB with 8 / 16 / 32 workgroups 307 / 276 / 300, one for every piece 320).  kStageSpins looks at a flag are some 200 us.
+constexpr size_t kStageUnit = 64u << 10, kStagePerThread = 1u << 20, kStageSend = 256u << 10, kStageEngine = 2u << 20;
+//  - With more than kStageChunksInPieces blocks the bus is busy all the time but for the first and the last of them: these go
+//    over it whole, by the engine (64 MiB 2945 us whole, 3100 in pieces; 16 MiB, two blocks, 983 / 827).
+constexpr size_t kStageChunksInPieces = 2;
+constexpr uint32_t kStageSpins = 20000;
 struct HostChunk {
   uint32_t first, count;     // range of host_copies
   uint64_t begin, end;       // payload byte range the chunk spans
 };
 struct HostStage {
   TableBlock block;
+  TableBlock flags;             // a word for every kStagePieceBytes of the block (unpacks in pieces)
   hipEvent_t ready = nullptr;   // recorded after the device copy that uses the block
   bool pending = false;
 };
@@ -1521,64 +1538,164 @@ int stage_acquire(HostStage* st, size_t bytes) {
   return stage_ready(st);
 }
 
-// kDLCPU tensors.  Pack: the pieces of a chunk are copied into a pinned block on
-// the calling thread (gaps zeroed: they are alignment padding or are rewritten by
-// the kernel that follows on the stream), then one asynchronous device copy moves
-// the chunk.  Unpack: one device copy per chunk into a pinned block; while the
-// next chunk is in flight the calling thread copies the previous one out, so the
-// call returns when the host tensors hold their data (as a copy into pageable
-// memory does).  Two blocks alternate.
+// In pieces go few blocks, and payloads that a kernel on `stream` reaches: memory of the current device, which is the
+// stream's (the copy engine takes any other, a payload in ordinary host memory included).
+bool stages_in_pieces(const axr_plan* p, const void* payload, hipStream_t stream) {
+  if (p->host_chunks.size() > kStageChunksInPieces) return false;
+  hipPointerAttribute_t attr;
+  int device = -1, stream_device = -1;
+  if (hipPointerGetAttributes(&attr, payload) != hipSuccess || hipGetDevice(&device) != hipSuccess ||
+      (stream && hipStreamGetDevice(stream, &stream_device) != hipSuccess)) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && attr.device == device && (!stream || stream_device == device);
+}
+
+// A staging block under way between host tensors and the payload.  The pieces of host memory that make up bytes
+// [lo, hi) of the block are found by their payload offset (the chunk's pieces ascend and do not overlap).
+struct StagedChunk : HostUnits {
+  const HostCopy *first, *last;   // the chunk's pieces
+  uint64_t begin;                 // payload offset of the block's first byte
+  uint8_t* staged;
+  uint8_t* payload;               // of that byte
+  hipStream_t stream;
+
+  bool in_pieces;                 // over the bus in pieces (see kStageUnit)
+
+  StagedChunk(const axr_plan* p, const HostChunk& c, uint8_t* block, uint8_t* whole_payload, hipStream_t s, bool pieces_)
+      : first(p->host_copies.data() + c.first), last(first + c.count), begin(c.begin), staged(block),
+        payload(whole_payload + c.begin), stream(s), in_pieces(pieces_) {
+    span = static_cast<size_t>(c.end - c.begin);
+    const size_t threads = std::max<size_t>(std::min(static_cast<size_t>(tunables().host_threads), span / kStagePerThread), 1);
+    helpers = threads - 1;
+    unit = in_pieces ? kStageUnit : ((span + threads - 1) / threads + 63) & ~static_cast<size_t>(63);
+  }
+  template <typename Move>
+  void pieces(size_t lo, size_t hi, Move&& move) const {
+    const HostCopy* hc = std::upper_bound(first, last, begin + lo, [](uint64_t at, const HostCopy& c) { return at < c.offset; });
+    if (hc != first) --hc;
+    for (; hc != last && hc->offset < begin + hi; ++hc) {
+      const uint64_t from = std::max(hc->offset, begin + lo), to = std::min(hc->offset + hc->bytes, begin + hi);
+      if (from < to) move(reinterpret_cast<uint8_t*>(hc->host) + (from - hc->offset), static_cast<size_t>(from - begin), static_cast<size_t>(to - from));
+    }
+  }
+};
+
+// Host tensors -> block -> payload.  Gaps between the pieces are zeroed: they are alignment padding or are
+// rewritten by the kernel that follows on the stream.
+struct ChunkIn : StagedChunk {
+  using StagedChunk::StagedChunk;
+  size_t sent = 0;
+  bool ready(size_t, bool) override { return true; }
+  void copy(size_t lo, size_t hi) override {
+    size_t at = lo;
+    pieces(lo, hi, [&](uint8_t* host, size_t to, size_t n) {
+      if (to > at) std::memset(staged + at, 0, to - at);
+      std::memcpy(staged + to, host, n);
+      at = to + n;
+    });
+    if (at < hi) std::memset(staged + at, 0, hi - at);
+  }
+  int done(size_t u) override {
+    const size_t upto = std::min((u + 1) * unit, span), piece = upto - sent;
+    if (upto < span && (!in_pieces || piece < std::max(kStageSend, sent ? span / 16 * 5 : span / 16))) return AXR_OK;
+    const int rc = in_pieces && span < kStageEngine
+                       ? launch_stream_copy(payload + sent, staged + sent, piece, true, stream)
+                       : check_hip(hipMemcpyAsync(payload + sent, staged + sent, piece, hipMemcpyDefault, stream),
+                                   "hipMemcpyAsync(host tensors -> payload)");
+    sent = upto;
+    return rc;
+  }
+};
+
+// Payload -> block -> host tensors.  stage_out_kernel raises a flag behind every piece of the block that has
+// arrived; a unit is emptied as soon as its flags are up, while the next ones are on the bus.  The flags are
+// polled for a while, then the caller's thread waits for the stream, behind which all of them are up, and the
+// helpers look again now and then.
+struct ChunkOut : StagedChunk {
+  const uint32_t* flags;
+  std::atomic<bool> failed{false};
+  int status = AXR_OK;
+  ChunkOut(const axr_plan* p, const HostChunk& c, uint8_t* block, const uint32_t* f, uint8_t* whole_payload, hipStream_t s,
+           bool in_pieces)
+      : StagedChunk(p, c, block, whole_payload, s, in_pieces), flags(f) {}
+  bool ready(size_t u, bool caller) override {
+    if (!in_pieces) return true;   // the block has been waited for
+    const size_t end = (std::min((u + 1) * unit, span) + kStagePieceBytes - 1) / kStagePieceBytes;
+    size_t i = u * unit / kStagePieceBytes;
+    for (uint32_t spins = 0; i < end; ++spins) {
+      if (__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) {
+        ++i;
+      } else if (spins < kStageSpins) {
+        __builtin_ia32_pause();
+      } else if (failed.load(std::memory_order_relaxed)) {
+        return false;
+      } else if (caller) {
+        if (!status) status = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize(staging)");
+        if (!status && !__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) status = fail(AXR_ERR_HIP, "a staging copy ended without its flags");
+        if (status) failed.store(true, std::memory_order_relaxed);
+      } else {
+        std::this_thread::sleep_for(std::chrono::microseconds(20));
+      }
+    }
+    return true;
+  }
+  void copy(size_t lo, size_t hi) override {
+    pieces(lo, hi, [&](uint8_t* host, size_t from, size_t n) { std::memcpy(host, staged + from, n); });
+  }
+  int done(size_t) override { return AXR_OK; }
+};
+
+// kDLCPU tensors.  Pack: the pieces of a chunk are copied into a pinned block, and what has been copied goes on
+// its way to the payload while the rest is still being copied.  Unpack: a kernel brings a chunk to a pinned block,
+// which is emptied from the front behind it, so the call returns when the host tensors hold their data (as a copy
+// into pageable memory does).  Two blocks alternate, so that the next chunk is on the bus meanwhile.
 int move_host_tensors(axr_plan* p, bool pack, uint8_t* payload, hipStream_t stream) {
   const size_t nchunks = p->host_chunks.size();
-  std::vector<HostCopyJob> jobs;
-  auto pieces_out = [p, &jobs](const HostChunk& c, const uint8_t* staged) {
-    jobs.clear();
-    for (uint32_t i = c.first; i < c.first + c.count; ++i) {
-      const HostCopy& hc = p->host_copies[i];
-      jobs.push_back({reinterpret_cast<void*>(hc.host), staged + (hc.offset - c.begin), hc.bytes});
-    }
-    host_copy(jobs.data(), jobs.size());
+  const bool in_pieces = stages_in_pieces(p, payload, stream);
+  auto block_of = [p](size_t k) { return static_cast<uint8_t*>(p->stage[k & 1].block.host); };
+  auto empty = [&](size_t k) {
+    HostStage* st = &p->stage[k & 1];
+    const HostChunk& c = p->host_chunks[k];
+    int rc = in_pieces ? AXR_OK : stage_ready(st);
+    if (rc) return rc;
+    ChunkOut out(p, c, block_of(k), static_cast<const uint32_t*>(st->flags.host), payload, stream, in_pieces);
+    rc = host_copy_units(out);
+    if (!rc) rc = out.status;
+    st->pending = rc != AXR_OK;   // with all flags up the device is done with the block
+    return rc;
   };
   for (size_t k = 0; k < nchunks; ++k) {
     const HostChunk& c = p->host_chunks[k];
     HostStage* st = &p->stage[k & 1];
-    if (!pack && k >= 2) {   // the block still holds chunk k - 2
-      int rc = stage_ready(st);
-      if (rc) return rc;
-      pieces_out(p->host_chunks[k - 2], static_cast<const uint8_t*>(st->block.host));
-    }
+    int rc = !pack && k >= 2 ? empty(k - 2) : AXR_OK;   // the block still holds chunk k - 2
+    if (rc) return rc;
     const size_t span = static_cast<size_t>(c.end - c.begin);
     // a block as long as the plan's longest chunk (8 MiB at most), not 8 MiB for all
-    int rc = stage_acquire(st, p->stage_bytes);
+    rc = stage_acquire(st, p->stage_bytes);
     if (rc) return rc;
-    uint8_t* staged = static_cast<uint8_t*>(st->block.host);
     if (pack) {
-      uint64_t at = c.begin;
-      jobs.clear();
-      for (uint32_t i = c.first; i < c.first + c.count; ++i) {
-        const HostCopy& hc = p->host_copies[i];
-        if (hc.offset > at) std::memset(staged + (at - c.begin), 0, hc.offset - at);
-        jobs.push_back({staged + (hc.offset - c.begin), reinterpret_cast<const void*>(hc.host), hc.bytes});
-        at = hc.offset + hc.bytes;
-      }
-      host_copy(jobs.data(), jobs.size());
-      rc = check_hip(hipMemcpyAsync(payload + c.begin, staged, span, hipMemcpyDefault, stream),
-                     "hipMemcpyAsync(host tensors -> payload)");
-    } else {
-      rc = check_hip(hipMemcpyAsync(staged, payload + c.begin, span, hipMemcpyDefault, stream),
+      ChunkIn in(p, c, block_of(k), payload, stream, in_pieces);
+      rc = host_copy_units(in);
+    } else if (!in_pieces) {
+      rc = check_hip(hipMemcpyAsync(block_of(k), payload + c.begin, span, hipMemcpyDefault, stream),
                      "hipMemcpyAsync(payload -> host tensors)");
+    } else {
+      constexpr size_t kFlagBytes = kStageBytes / kStagePieceBytes * sizeof(uint32_t);
+      if (!st->flags.host) rc = table_block_acquire(kFlagBytes, &st->flags);
+      if (rc) return rc;
+      std::memset(st->flags.host, 0, kFlagBytes);
+      rc = launch_stage_out(block_of(k), payload + c.begin, span, static_cast<uint32_t*>(st->flags.host), stream);
     }
-    if (rc) return rc;
-    rc = check_hip(hipEventRecord(st->ready, stream), "hipEventRecord(staging)");
-    if (rc) return rc;
-    st->pending = true;
+    const int recorded = check_hip(hipEventRecord(st->ready, stream), "hipEventRecord(staging)");
+    st->pending = recorded == AXR_OK;
+    if (rc || recorded) return rc ? rc : recorded;
   }
   if (!pack) {
     for (size_t k = nchunks >= 2 ? nchunks - 2 : 0; k < nchunks; ++k) {
-      HostStage* st = &p->stage[k & 1];
-      int rc = stage_ready(st);
+      int rc = empty(k);
       if (rc) return rc;
-      pieces_out(p->host_chunks[k], static_cast<const uint8_t*>(st->block.host));
     }
   }
   return AXR_OK;
@@ -1890,6 +2007,7 @@ static int plan_free_body(axr_plan_t* plan) {
   plan->upload_event = nullptr;
   for (HostStage& st : plan->stage) {
     table_block_release(&st.block);
+    table_block_release(&st.flags);
     if (st.ready) (void)hipEventDestroy(st.ready);
   }
   plan_delete(plan);

@@ -3,6 +3,8 @@
 // headers; host code above the C ABI never does.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
+#include <atomic>
 #include <chrono>
 
 #include <cstdlib>
@@ -232,6 +234,48 @@ void host_copy(const HostCopyJob* jobs, size_t count) {
   copy_share(jobs, count, 0, share < total ? share : total);
   if (begin < total) copy_share(jobs, count, begin, total);
   for (std::thread& t : helpers) t.join();
+}
+
+int host_copy_units(HostUnits& units) {
+  const size_t n = (units.span + units.unit - 1) / units.unit;
+  std::unique_ptr<std::atomic<uint8_t>[]> moved(new std::atomic<uint8_t>[n]());
+  std::atomic<size_t> next{0};
+  auto move_one = [&](size_t u, bool caller) {
+    if (!units.ready(u, caller)) return false;
+    units.copy(u * units.unit, std::min((u + 1) * units.unit, units.span));
+    moved[u].store(1, std::memory_order_release);
+    return true;
+  };
+  auto help = [&] {
+    for (size_t u; (u = next.fetch_add(1, std::memory_order_relaxed)) < n;)
+      if (!move_one(u, false)) return;
+  };
+  std::vector<std::thread> helpers;
+  try {
+    const size_t count = std::min(units.helpers, n - 1);
+    helpers.reserve(count);
+    for (size_t i = 0; i < count; ++i) helpers.emplace_back(help);
+  } catch (...) {
+    // no more threads to be had: fewer take part
+  }
+  int rc = AXR_OK;
+  size_t told = 0;   // units that done() has been called for
+  auto tell = [&] {
+    for (; !rc && told < n && moved[told].load(std::memory_order_acquire); ++told) rc = units.done(told);
+  };
+  bool ok = true;
+  for (size_t u; ok && (u = next.fetch_add(1, std::memory_order_relaxed)) < n;) {
+    ok = move_one(u, true);
+    tell();
+  }
+  // what the helpers still have in hand, in order
+  while (ok && !rc && told < n) {
+    if (moved[told].load(std::memory_order_acquire)) tell();
+    else if (!units.ready(told, true)) ok = false;
+    else __builtin_ia32_pause();
+  }
+  for (std::thread& t : helpers) t.join();
+  return rc;
 }
 }  // namespace axr
 

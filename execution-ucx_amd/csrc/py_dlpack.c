@@ -264,7 +264,56 @@ static PyObject* new_capsule(PyObject* self, PyObject* args) {
   return PyCapsule_New(managed, versioned ? "dltensor_versioned" : "dltensor", export_capsule_destructor);
 }
 
+/* geometry(address, count, host_type) -> (base, key): the address of the first of `count` descriptors' elements, and
+ * everything else about them as bytes, addresses relative to it.  Two arrays with equal keys differ by the distance
+ * of their bases alone.  When some tensor is of device type `host_type` the key holds the base itself as well. */
+static PyObject* geometry(PyObject* self, PyObject* args) {
+  (void)self;
+  PyObject* address = NULL;
+  Py_ssize_t n = 0;
+  int host_type = 0;
+  if (!PyArg_ParseTuple(args, "Oni", &address, &n, &host_type)) return NULL;
+  const axr_tensor_t* a = (const axr_tensor_t*)PyLong_AsVoidPtr(address);
+  if (!a && PyErr_Occurred()) return NULL;
+  if (!a || n < 1) {
+    PyErr_SetString(PyExc_ValueError, "geometry: no descriptors");
+    return NULL;
+  }
+  const uint64_t base = (uint64_t)(uintptr_t)a[0].data + a[0].byte_offset;
+  Py_ssize_t words = 2;
+  int host = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    if (a[i].ndim < 0) {
+      PyErr_SetString(PyExc_ValueError, "geometry: negative ndim");
+      return NULL;
+    }
+    words += 4 + (Py_ssize_t)a[i].ndim * (a[i].strides ? 2 : 1);
+    host = host || a[i].device_type == host_type;
+  }
+  PyObject* key = PyBytes_FromStringAndSize(NULL, words * 8);
+  if (!key) return NULL;
+  uint64_t* w = (uint64_t*)PyBytes_AS_STRING(key);
+  *w++ = host;
+  *w++ = host ? base : 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const axr_tensor_t* t = &a[i];
+    const size_t nd = (size_t)t->ndim;
+    *w++ = (uint64_t)(uintptr_t)t->data + t->byte_offset - base;
+    *w++ = (uint64_t)(uint32_t)t->device_type << 32 | (uint32_t)t->device_id;
+    *w++ = (uint64_t)nd << 1 | (t->strides != NULL);
+    *w++ = (uint64_t)t->dtype_code << 24 | (uint64_t)t->dtype_bits << 16 | t->dtype_lanes;
+    if (nd) memcpy(w, t->shape, 8 * nd);
+    w += nd;
+    if (t->strides) {
+      if (nd) memcpy(w, t->strides, 8 * nd);
+      w += nd;
+    }
+  }
+  return Py_BuildValue("KN", (unsigned long long)base, key);
+}
+
 static PyMethodDef methods[] = {
+    {"geometry", geometry, METH_VARARGS, "geometry(address, count, host_type) -> (base, key bytes)"},
     {"new_capsule", new_capsule, METH_VARARGS,
      "new_capsule(address[, versioned]) -> 'dltensor' (or 'dltensor_versioned') capsule that owns the "
      "managed tensor at address until consumed"},

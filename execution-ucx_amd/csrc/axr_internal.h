@@ -127,6 +127,14 @@ constexpr uint32_t transpose_skew_rows(uint32_t element_bytes) {
   const uint32_t per_access = kWaveLanes / (transpose_edge(element_bytes) * element_bytes / kVecBytes);
   return (transpose_edge(element_bytes) + kSkewBytes / element_bytes - 1 + per_access - 1) / per_access * per_access;
 }
+// The four wavefronts of a workgroup in the kernel of walked blocks alone take kSkewGroup skewed blocks that follow
+// each other along the written rows, and stage their rows together: the rows of the next block are staged once for
+// four blocks.  The rows, rounded up to what a round of the four covers.
+constexpr uint32_t kSkewGroup = 4;
+constexpr uint32_t transpose_group_rows(uint32_t element_bytes) {
+  const uint32_t round = kSkewGroup * (kWaveLanes / (transpose_edge(element_bytes) * element_bytes / kVecBytes));
+  return (kSkewGroup * transpose_edge(element_bytes) + kSkewBytes / element_bytes - 1 + round - 1) / round * round;
+}
 constexpr uint32_t kBlockStrip = 8;
 constexpr uint32_t kSkewPack = 16, kSkewUnpack = 32;   // Dims.nt_allowed bits 4, 5: blocks of that direction are skewed
 // How the blocks of a transposition are cut and walked when rows straddle lines: plain or skewed
@@ -301,7 +309,7 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t ndim;          // outer (non-run) dimensions after collapsing, <= kMaxOuterDims;
                           // transposed: batch dimensions (<= kMaxBatchDims)
   uint32_t tiles_per_run; // kModeRunTiles; kModeRows: runs per tile; kModeWalked: blocks per strip
-                          // (kBlockStrip or 1)
+                          // (kBlockStrip, or 1, or kSkewGroup in plain rows whose pack is skewed)
   uint32_t granule;       // kModeElements: bytes moved per lane access (1,2,4,8,16);
                           // kModeRunTiles: 1 + log2(tiles_per_run) when a power of two;
                           // transposed: element size
@@ -314,7 +322,8 @@ struct Dims {             // 176 bytes, one per strided segment
   int64_t stride_a;                // tensor byte stride of A
   uint64_t pstride_b;              // packed byte stride of B
   uint32_t ext_a, ext_b;
-  uint32_t tiles_a, tiles_b;
+  uint32_t tiles_a, tiles_b;       // kModeWalked alone: along a dimension in which blocks are skewed rounded up to
+                                   // kSkewGroup, and the segment's tiles likewise; those past the extents are empty
   uint32_t edge_a, edge_b;         // block extent along A and B (elements)
   uint32_t lanes_per_run;          // kModeRows: the lane slots a run occupies (pstride[0] holds the
                                    // number of runs, edge_a the slots per lane);
@@ -390,6 +399,7 @@ struct LaunchConfig {
   bool elements = false;   // some segment's mode is above kModeRunTiles
   uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (kModeRows and above)
+  uint32_t lds_walked = 0;     // and in the kernel of walked blocks alone
   uint32_t cached_tail = 0;    // MiB at the end of a streaming payload that a pack leaves in the cache (runs in
                            // 1 KiB tiles only; see finish_geometry)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a

@@ -641,6 +641,56 @@ __device__ __forceinline__ void transpose_full(gcbytes rd, int64_t rd_pitch, gby
   __builtin_amdgcn_wave_barrier();
 }
 
+// The written rows of skewed blocks, from the rows that have been staged for them.
+template <uint32_t E>
+struct SkewedRows {
+  static constexpr uint32_t PITCH = transpose_lds_pitch(E), EV = kVecBytes / E;
+  typedef typename unit_of<E>::type U;
+  typedef U __attribute__((aligned(E < 4 ? E : 4))) lds_unit;
+  gbytes wr;          // written row y from its element x = 0 on: wr + y * wr_pitch
+  int64_t wr_pitch;
+  uint32_t ext_x;     // elements of a written row
+  uint32_t w0;        // the first staged read row is element w0 of the written ones
+  lbytes lds;
+
+  // EV elements of written row y from element x on
+  __device__ __forceinline__ u32x4 gather(uint32_t x, uint32_t y) const {
+    U e[EV];
+#pragma unroll
+    for (uint32_t i = 0; i < EV; ++i)
+      e[i] = *reinterpret_cast<const AXR_LDS lds_unit*>(lds + (x - w0 + i) * PITCH + y * E);
+    u32x4 out;
+    __builtin_memcpy(&out, e, kVecBytes);
+    return out;
+  }
+  __device__ __forceinline__ uint32_t skew_of(uint32_t y) const {   // elements in front of row y's first 64-byte boundary
+    const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uint64_t>(wr)) + y * static_cast<uint32_t>(wr_pitch);
+    return ((0u - at) & (kSkewBytes - 1u)) / E;
+  }
+  // the vector of row y that lies `x` elements behind the row's first boundary, moved back where the row ends
+  __device__ __forceinline__ void write(uint32_t y, uint32_t x, bool nt_wr) const {
+    x += skew_of(y);
+    if (x < ext_x) {
+      if (x + EV > ext_x) x = ext_x - EV;   // overlaps its neighbour with identical data
+      gbytes to = wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E;
+      if (nt_wr) {   // (the empty asm statements keep the arms apart, see transpose_full)
+        asm volatile("");
+        store16<true>(to, gather(x, y));
+        asm volatile("");
+      } else {
+        store16<false>(to, gather(x, y));
+      }
+    }
+  }
+  // the elements in front of every row's first boundary, in whole vectors: rows of set `set`
+  static constexpr uint32_t kFrontVectors = kSkewBytes / kVecBytes, kFrontRows = kWaveLanes / kFrontVectors;
+  __device__ __forceinline__ void write_front(uint32_t set, uint32_t lane) const {
+    const uint32_t y = set * kFrontRows + lane / kFrontVectors, x = (lane % kFrontVectors) * EV;
+    if (y < transpose_edge(E) && x < skew_of(y))
+      store16<false>(wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E, gather(x, y));
+  }
+};
+
 // A block whose written rows do not start on 64-byte boundaries (where: block_rule).  Partly written
 // 64-byte pieces are what such a transposition loses its time on, not the reads: 128-byte row pieces at
 // any address read at the aligned rate, written they fall from 5.5 to 3.9 TB/s, and are back at 5.2 once
@@ -664,8 +714,6 @@ __device__ __forceinline__ void transpose_skewed(gcbytes rd, int64_t rd_pitch, g
   constexpr uint32_t NC = T * E / kVecBytes, RPI = kWaveLanes / NC;
   constexpr uint32_t W = transpose_skew_rows(E), NK = W / RPI;
   static_assert(W % RPI == 0 && W >= T + kSkewBytes / E - 1, "staged rows");
-  typedef typename unit_of<E>::type U;
-  typedef U __attribute__((aligned(E < 4 ? E : 4))) lds_unit;
   const uint32_t r = lane / NC, v = lane % NC;
   // staged rows w0 .. w0 + nrows - 1; at the end of the row the window moves back to end with it,
   // so that the last, moved back vectors find their elements
@@ -687,47 +735,63 @@ __device__ __forceinline__ void transpose_skewed(gcbytes rd, int64_t rd_pitch, g
     w[3] = q[k].w;
   }
   __builtin_amdgcn_wave_barrier();
-  // EV elements of written row y from element x on
-  auto gather = [&](uint32_t x, uint32_t y) {
-    U e[EV];
+  const SkewedRows<E> rows{wr, wr_pitch, ext_x, w0, lds};
 #pragma unroll
-    for (uint32_t i = 0; i < EV; ++i)
-      e[i] = *reinterpret_cast<const AXR_LDS lds_unit*>(lds + (x - w0 + i) * PITCH + y * E);
-    u32x4 out;
-    __builtin_memcpy(&out, e, kVecBytes);
-    return out;
-  };
-  auto skew_of = [&](uint32_t y) {   // elements in front of row y's first 64-byte boundary
-    const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uint64_t>(wr)) + y * static_cast<uint32_t>(wr_pitch);
-    return ((0u - at) & (kSkewBytes - 1u)) / E;
-  };
+  for (uint32_t k = 0; k < T / RPI; ++k) rows.write(k * RPI + r, x0 + v * EV, nt_wr);
+  if (x0 == 0) {
 #pragma unroll
-  for (uint32_t k = 0; k < T / RPI; ++k) {
-    const uint32_t y = k * RPI + r;
-    uint32_t x = x0 + skew_of(y) + v * EV;
-    if (x < ext_x) {
-      if (x + EV > ext_x) x = ext_x - EV;   // overlaps its neighbour with identical data
-      gbytes to = wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E;
-      if (nt_wr) {   // (the empty asm statements keep the arms apart, see transpose_full)
-        asm volatile("");
-        store16<true>(to, gather(x, y));
-        asm volatile("");
-      } else {
-        store16<false>(to, gather(x, y));
-      }
-    }
-  }
-  if (x0 == 0) {   // the elements in front of every row's first boundary, in whole vectors
-    constexpr uint32_t NV = kSkewBytes / kVecBytes, RPH = kWaveLanes / NV;
-    const uint32_t rh = lane / NV, x = (lane % NV) * EV;
-#pragma unroll
-    for (uint32_t k = 0; k < (T + RPH - 1) / RPH; ++k) {
-      const uint32_t y = k * RPH + rh;
-      if (y < T && x < skew_of(y))
-        store16<false>(wr + static_cast<int64_t>(y) * wr_pitch + static_cast<uint64_t>(x) * E, gather(x, y));
-    }
+    for (uint32_t set = 0; set < (T + rows.kFrontRows - 1) / rows.kFrontRows; ++set) rows.write_front(set, lane);
   }
   __builtin_amdgcn_wave_barrier();
+}
+
+// kSkewGroup such blocks by the wavefronts of a workgroup, `member` of them from element x0 + member * T on: rows of
+// the next block are staged once for all of them (2-byte elements 288 read rows for 256, 384 for four wavefronts
+// by themselves), and the LDS of a workgroup falls from 49.5 to 37.2 KiB, so that a compute unit holds 16 wavefronts of
+// them instead of 12.  Four odd bf16 matrices of 134 MB, pack + unpack, 108.8 us
+// with every wavefront by itself, 102.0 so; 537 MB of them 455 / 415, 4- and 8-byte elements 158.4 / 150.3 and 103.5 / 100.0.
+// Called by every wavefront of the workgroup with the same arguments but `member`; x0 < ext_x.
+template <uint32_t E>
+__device__ __forceinline__ void transpose_skewed_group(gcbytes rd, int64_t rd_pitch, gbytes wr, int64_t wr_pitch,
+                                                       uint32_t x0, uint32_t ext_x, lbytes lds, uint32_t member,
+                                                       uint32_t lane, bool nt_wr) {
+  constexpr uint32_t T = transpose_edge(E), PITCH = transpose_lds_pitch(E), EV = kVecBytes / E;
+  constexpr uint32_t NC = T * E / kVecBytes, RPI = kWaveLanes / NC;
+  constexpr uint32_t W = transpose_group_rows(E), NK = W / RPI / kSkewGroup;
+  static_assert(W == NK * RPI * kSkewGroup && W >= kSkewGroup * T + kSkewBytes / E - 1, "staged rows");
+  const uint32_t r = lane / NC, v = lane % NC;
+  // staged rows w0 .. w0 + nrows - 1; at the end of the row the window moves back to end with it,
+  // so that the last, moved back vectors find their elements
+  const uint32_t back = ext_x > W ? ext_x - W : 0u;
+  const uint32_t w0 = x0 < back ? x0 : back;
+  const uint32_t nrows = ext_x - w0 < W ? ext_x - w0 : W;
+  u32x4 q[NK];
+#pragma unroll
+  for (uint32_t k = 0; k < NK; ++k) {
+    const uint32_t row = (k * kSkewGroup + member) * RPI + r;
+    q[k] = load16<false>(rd + static_cast<int64_t>(w0 + (row < nrows ? row : nrows - 1u)) * rd_pitch + v * kVecBytes);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < NK; ++k) {
+    AXR_LDS uint32_t* w = reinterpret_cast<AXR_LDS uint32_t*>(lds + ((k * kSkewGroup + member) * RPI + r) * PITCH + v * kVecBytes);
+    w[0] = q[k].x;
+    w[1] = q[k].y;
+    w[2] = q[k].z;
+    w[3] = q[k].w;
+  }
+  __syncthreads();
+  const SkewedRows<E> rows{wr, wr_pitch, ext_x, w0, lds};
+  // Pieces of two blocks for 2-byte elements, of all four for wider ones, side by side: the 128-byte lines of a piece are
+  // written whole by one access, while the lanes' reads of LDS fall on more and more of the same banks (four bf16
+  // matrices above 104.4 / 102.0 / 104.0 us with one / two / four blocks to a piece, 4-byte ones 154.7 / 151.7 / 150.3).
+  constexpr uint32_t BLOCKS = E == 2 ? 2 : 4, LPR = BLOCKS * NC;   // lanes that take a row together
+  constexpr uint32_t ROWS = kWaveLanes / LPR, PARTS = kSkewGroup / BLOCKS;
+#pragma unroll
+  for (uint32_t k = 0; k < T / RPI; ++k) {
+    const uint32_t step = k * kSkewGroup + member;     // PARTS steps to a set of ROWS rows
+    rows.write(step / PARTS * ROWS + lane / LPR, x0 + (step % PARTS * LPR + lane % LPR) * EV, nt_wr);
+  }
+  if (x0 == 0) rows.write_front(member, lane);
 }
 
 // Quotient idx / d by multiplication, exact while idx * d < 2^32 (blocks hold at
@@ -1097,10 +1161,12 @@ __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t 
 // that mode alone (see waves_of_kind), and into the kernel for any mode.
 // One copy per MODE: with the walk in strips and the choice of block routine in
 // the plain one's way, however predictable, 4 KiB blocks took 3 to 8 % longer.
-template <bool PACK, uint32_t MODE>
+// GROUP: the wavefronts of a workgroup take kSkewGroup tiles that follow each other, and skewed blocks together;
+// `lds_group` is their LDS.
+template <bool PACK, uint32_t MODE, bool GROUP = false>
 __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, gbytes pay,
                                                uint32_t q, lbytes lds, uint32_t lane,
-                                               uint32_t nt_bits) {
+                                               uint32_t nt_bits, lbytes lds_group = nullptr) {
   const uint32_t E = dm->granule;
   const uint32_t es = static_cast<uint32_t>(__builtin_ctz(E));
   const uint32_t T = transpose_edge(E);
@@ -1115,12 +1181,21 @@ __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, 
   uint32_t ia, ib;
   if constexpr (MODE == kModeWalked) {
     // blocks in strips of `strip` along A, walked along B: with 8 of them 64 neighbouring tiles are a
-    // square of 8 x 8 blocks (1: plain rows of blocks)
-    const uint32_t strip = dm->tiles_per_run;
+    // square of 8 x 8 blocks (1: plain rows of blocks).  GROUP: kSkewGroup tiles that follow each other lie along the
+    // rows that are written where those are skewed, along A packing, where ta and strips are whole groups, along B
+    // unpacking, where tb is.  Single wavefronts keep to plain rows (two matrices of 2049 x 4099 4-byte elements next to a
+    // compact tensor 54.2 us in plain rows, 59.9 in strips of kSkewGroup).
+    const uint32_t strip = !GROUP && dm->tiles_per_run == kSkewGroup ? 1u : dm->tiles_per_run;
     const uint32_t is = rem / (strip * tb), in_strip = rem - is * strip * tb;
     const uint32_t strip_rows = ta - is * strip < strip ? ta - is * strip : strip;
-    ib = in_strip / strip_rows;
-    ia = is * strip + (in_strip - ib * strip_rows);
+    if (GROUP && !PACK && (allowed & kSkewUnpack) != 0) {
+      const uint32_t g = in_strip / (strip_rows * kSkewGroup), in_group = in_strip - g * strip_rows * kSkewGroup;
+      ia = is * strip + in_group / kSkewGroup;
+      ib = g * kSkewGroup + in_group % kSkewGroup;
+    } else {
+      ib = in_strip / strip_rows;
+      ia = is * strip + (in_strip - ib * strip_rows);
+    }
   } else {
     ia = rem / tb;
     ib = rem - ia * tb;
@@ -1128,6 +1203,7 @@ __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, 
   int64_t toff = 0;
   uint64_t poff = 0;
   const uint32_t nbatch = dm->ndim;
+  // (behind the loop `o` is 0, except for empty tiles past the last batch)
 #pragma unroll
   for (int d = static_cast<int>(kMaxBatchDims) - 1; d >= 0; --d) {
     if (static_cast<uint32_t>(d) + nbatch >= kMaxBatchDims) {
@@ -1140,6 +1216,17 @@ __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, 
     }
   }
   uint32_t a0 = ia * edge_a, b0 = ib * edge_b;
+  if constexpr (MODE == kModeWalked) {
+    // empty tiles past the extents (of a group, only where all of its tiles are empty)
+    constexpr uint32_t group = GROUP ? kSkewGroup - 1u : 0u;
+    const bool skewed = (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0;
+    const uint32_t first_a = skewed && PACK ? (ia & ~group) * edge_a : a0, first_b = skewed && !PACK ? (ib & ~group) * edge_b : b0;
+    if (first_a >= dm->ext_a || first_b >= dm->ext_b || o != 0) return;
+    if (skewed && GROUP) {
+      a0 = first_a;
+      b0 = first_b;
+    }
+  }
   if constexpr (MODE == kModePlanes) {
     // Few planes <-> interleaved: the short dimension is taken whole.  What is left of the long one
     // may be less than a vector: the block is then moved back to hold one.
@@ -1183,6 +1270,15 @@ __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, 
       ext_x = dm->ext_b;
     }
     const bool nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
+    if constexpr (GROUP) {
+      const uint32_t member = (PACK ? ia : ib) & (kSkewGroup - 1u);
+      switch (E) {
+        case 2: transpose_skewed_group<2>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds_group, member, lane, nt_wr); break;
+        case 4: transpose_skewed_group<4>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds_group, member, lane, nt_wr); break;
+        default: transpose_skewed_group<8>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds_group, member, lane, nt_wr); break;
+      }
+      return;
+    }
     switch (E) {
       case 2: transpose_skewed<2>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds, lane, nt_wr); break;
       case 4: transpose_skewed<4>(rd, rd_pitch, wr, wr_pitch, x0, ext_x, lds, lane, nt_wr); break;
@@ -1530,7 +1626,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         if (mode == kModeElements) element_tile<PACK, ROWS>(seg_ptr, seg_run, dm, pay, q, lane, nt_bits);
         else if (mode == kModeRows) rows_tile<PACK>(seg_ptr, static_cast<uint32_t>(seg_run), dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
-        else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
+        else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked, KIND == kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits, (lbytes)lds_slices);
         else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
       }
       if constexpr (PACK) {
@@ -2030,8 +2126,12 @@ uint32_t hint_argument(const LaunchConfig& cfg) {
 template <bool PACK, uint32_t ROWS>
 int launch_rows(const KernelArgs& args, const LaunchConfig& cfg, hipStream_t stream) {
   const dim3 grid(cfg.workgroups), block(cfg.threads);
-  const uint32_t lds_bytes = cfg.elements ? cfg.lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
-  const uint32_t low = cfg.elements ? cfg.lds_per_wave : cfg.cached_tail;
+  const bool walked = ROWS == 2 && cfg.elements && cfg.kind == kModeWalked;   // (that kernel's workgroups are groups)
+  if (walked && (cfg.threads != kSkewGroup * kWaveLanes || cfg.tiles_per_wave != 1))
+    return fail(AXR_ERR_INVALID, "walked blocks need workgroups of four wavefronts with a tile each");
+  const uint32_t lds_per_wave = walked ? cfg.lds_walked : cfg.lds_per_wave;
+  const uint32_t lds_bytes = cfg.elements ? lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
+  const uint32_t low = cfg.elements ? lds_per_wave : cfg.cached_tail;
   if (low > 0x1ffffu || args.seg_shift > 0xffu || cfg.threads / kWaveLanes > 0x1fu)
     return fail(AXR_ERR_INVALID, "launch geometry does not fit the kernel's geometry argument");
   // LDS bytes per wavefront, or MiB of cached tail | hints << 17 | wavefronts per workgroup << 19 | tile-block shift << 24
@@ -2098,7 +2198,8 @@ int launch_bundle_kernel(bool pack, const KernelArgs& args, const LaunchConfig& 
     return fail(AXR_ERR_INVALID, "die remapping needs a grid of whole rounds over the dies");
   if (cfg.elements && cfg.threads > kMaxElementThreads)
     return fail(AXR_ERR_INVALID, "bundles with short strided runs need workgroups of at most 256");
-  if (static_cast<uint64_t>(cfg.lds_per_wave) * (cfg.threads / kWaveLanes) > 64u * 1024u)
+  const uint32_t lds_per_wave = cfg.elements && cfg.kind == kModeWalked && cfg.tile_rows == 2 ? cfg.lds_walked : cfg.lds_per_wave;
+  if (static_cast<uint64_t>(lds_per_wave) * (cfg.threads / kWaveLanes) > 64u * 1024u)
     return fail(AXR_ERR_INVALID, "workgroup needs more than 64 KiB of LDS");
   const uint64_t covered = static_cast<uint64_t>(cfg.workgroups) * (cfg.threads / kWaveLanes) *
                            cfg.tiles_per_wave;

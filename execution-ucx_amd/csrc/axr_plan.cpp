@@ -216,6 +216,7 @@ struct axr_plan {
   uint32_t ntiles = 0;
   uint64_t shared_line_tiles = 0;    // tiles of transposed blocks whose rows straddle 128-byte lines
   uint64_t strip_tiles = 0;          // those of them that lie in strips of kBlockStrip blocks
+  bool whole_groups = false;         // walked blocks alone, in whole groups of kSkewGroup tiles
   LaunchConfig cfg;
   TableBlock block;
   size_t table_bytes = 0;
@@ -398,7 +399,8 @@ void invalidate_tables(axr_plan* p) {
   p->ntiles = 0;
   p->shared_line_tiles = 0;
   p->strip_tiles = 0;
-  p->cfg.lds_per_wave = 0;
+  p->whole_groups = false;
+  p->cfg.lds_per_wave = p->cfg.lds_walked = 0;
 }
 
 // Wait until the device no longer reads the plan's tables.  No event is
@@ -543,6 +545,7 @@ struct Builder {
   uint64_t tiles = 0;
   uint64_t shared_line_tiles = 0;   // transposed blocks whose rows straddle 128-byte lines
   uint64_t strip_tiles = 0;         // those of them that lie in strips of kBlockStrip blocks
+  bool whole_groups = false;        // see settle_walked
   bool rows = false, others = false;   // tensors moved in whole short rows, and any other way
   uint64_t group_bytes = 0;         // longest tensor that may share a wavefront (0: none)
   uint32_t slots_per_group = kGroupMaxSlots;
@@ -794,18 +797,23 @@ struct Builder {
         const bool square = edge_a == transpose_edge(e) && edge_b == edge_a;
         BlockRule rule = block_rule(e, dm.ext_a, dm.ext_b, square, p->payload_bytes, tensor_lines, payload_lines);
         if ((dm.ext_a | dm.ext_b) >= (1u << 31)) rule.skew_pack = rule.skew_unpack = false;
-        shared_line_tiles += ntile;
-        if (rule.strips || rule.skew_pack || rule.skew_unpack) dm.mode = kModeWalked;
-        if (rule.strips) {
-          dm.tiles_per_run = kBlockStrip;
-          strip_tiles += ntile;
+        if (rule.strips || rule.skew_pack || rule.skew_unpack) {
+          dm.mode = kModeWalked;
+          if (rule.strips) dm.tiles_per_run = kBlockStrip;
         }
+        shared_line_tiles += ntile;
+        if (rule.strips) strip_tiles += ntile;
         // The side that is written gets blocks that start on its own 64-byte boundaries.  Whole 64-byte
         // units may stream: streamed into the tensors they leave the last-level cache to the payload and
         // the next pass (134 MB of 2-byte elements, pack + unpack 143 -> 123 us).
         if (rule.skew_pack) dm.nt_allowed |= kSkewPack;
         if (rule.skew_unpack) dm.nt_allowed |= kSkewUnpack | 4u;
-        if (rule.skew_pack || rule.skew_unpack) lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
+        uint32_t walked = lds;
+        if (rule.skew_pack || rule.skew_unpack) {
+          lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
+          walked = std::max(walked, transpose_group_rows(e) * transpose_lds_pitch(e) / kSkewGroup + 1u);
+        }
+        p->cfg.lds_walked = std::max<uint32_t>(p->cfg.lds_walked, (walked + 15u) & ~15u);
       }
       p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
     } else if (run_bytes >= element_mode_limit(run_bytes)) {
@@ -884,6 +892,45 @@ struct Builder {
     }
   }
 
+  // Walked blocks alone have a kernel whose workgroups take kSkewGroup of them together: whole groups then, along the
+  // rows that are written.  (Next to other tensors the empty tiles behind the last group would only cost: a
+  // matrix of 4097 x 4099 2-byte elements and 1 MiB of compact tensor 32.5 -> 33.8 us.)
+  void settle_walked() {
+    if (p->segs.empty() || p->dims.empty()) return;
+    for (const Dims& dm : p->dims)
+      if (dm.mode != kModeWalked) return;
+    for (const Seg& sg : p->segs)
+      if ((sg.meta >> kSegDimsShift) == 0 || (sg.meta >> kSegDimsShift) >= kSegGroup) return;
+    auto groups = [](uint64_t blocks) { return (blocks + kSkewGroup - 1) / kSkewGroup * kSkewGroup; };
+    std::vector<uint64_t> tiles_of(p->dims.size());
+    uint64_t padded = 0;
+    for (size_t i = 0; i < p->dims.size(); ++i) {
+      const Dims& dm = p->dims[i];
+      const uint64_t a = dm.nt_allowed & kSkewPack ? groups(dm.tiles_a) : dm.tiles_a, b = dm.nt_allowed & kSkewUnpack ? groups(dm.tiles_b) : dm.tiles_b;
+      uint64_t batches = 1;
+      for (uint32_t d = kMaxOuterDims - kMaxBatchDims; d < kMaxOuterDims; ++d) batches *= dm.shape[d];
+      tiles_of[i] = groups(batches * a * b);
+    }
+    for (const Seg& sg : p->segs) padded += tiles_of[(sg.meta >> kSegDimsShift) - 1];
+    if (padded > 0x7fffffffull) return;
+    for (Dims& dm : p->dims) {
+      if (dm.nt_allowed & kSkewPack) {
+        dm.tiles_a = static_cast<uint32_t>(groups(dm.tiles_a));
+        if (dm.tiles_per_run == 1) dm.tiles_per_run = kSkewGroup;
+      }
+      if (dm.nt_allowed & kSkewUnpack) dm.tiles_b = static_cast<uint32_t>(groups(dm.tiles_b));
+    }
+    tiles = shared_line_tiles = strip_tiles = 0;
+    for (Seg& sg : p->segs) {
+      const size_t at = (sg.meta >> kSegDimsShift) - 1;
+      sg.tile_begin = static_cast<uint32_t>(tiles);
+      tiles += tiles_of[at];
+      if (p->dims[at].tiles_per_run == kBlockStrip) strip_tiles += tiles_of[at];
+    }
+    shared_line_tiles = tiles;
+    whole_groups = true;
+  }
+
   // Host (kDLCPU) tensors move with one async copy per contiguous run.
   int add_host(uint32_t tensor, uint64_t ptr, uint64_t off, const uint64_t* ext,
                const int64_t* str, size_t nd, uint64_t run_bytes) {
@@ -950,10 +997,13 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   const uint64_t max_waves = static_cast<uint64_t>(tn.max_waves) * (rows_alone ? 4 : 1);
   uint64_t tpw = (p->ntiles + max_waves - 1) / max_waves;
   if (tpw == 0) tpw = 1;
+  // the kernel of walked blocks alone works in groups of kSkewGroup wavefronts with a tile each
+  if (p->cfg.kind == kModeWalked && (!p->whole_groups || tpw != 1 || (tn.threads != 0 && tn.threads != kSkewGroup * kWaveLanes))) p->cfg.kind = kKindAny;
   p->cfg.threads = tn.threads ? static_cast<uint32_t>(tn.threads)
                               : (rows == 1 && tn.tile_rows == 0 ? kWaveLanes : (p->ntiles < 65536 ? 256u : 128u));
   if (p->cfg.elements) p->cfg.threads = std::min(p->cfg.threads, kMaxElementThreads);
-  if (p->cfg.lds_per_wave) {
+  if (p->cfg.kind == kModeWalked) p->cfg.threads = kSkewGroup * kWaveLanes;
+  if (p->cfg.lds_per_wave && p->cfg.kind != kModeWalked) {
     // transposed blocks: every wave of a workgroup owns a slice of at most 64 KiB of LDS
     const uint32_t fit = (64u * 1024u / p->cfg.lds_per_wave) * kWaveLanes;
     p->cfg.threads = std::min(p->cfg.threads, fit);
@@ -1363,6 +1413,8 @@ int build_tables(axr_plan* p) {
     if (rc) return rc;
   }
   b.settle_rows();
+  b.settle_walked();
+  p->whole_groups = b.whole_groups;
   // Group neighbouring host pieces (in payload order, at most an alignment gap
   // apart) into chunks that fit one staging block.
   for (uint32_t i = 0; i < p->host_copies.size(); ++i) {

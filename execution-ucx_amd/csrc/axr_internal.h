@@ -38,6 +38,7 @@ constexpr uint32_t kSegFillOnly = 0xfffffu;      // dims field value: segment on
 constexpr uint32_t kSegGroup = 0xffffeu;         // dims field value: one tile that holds several short tensors
 constexpr uint32_t kMaxAlign = 4096;
 constexpr uint32_t kDirectSegShift = 0xffu;      // seg_shift value: every segment is exactly one tile
+constexpr uint32_t kOneSegShift = 0xfdu;         // seg_shift value: one segment, a view moved otherwise than in runs
 constexpr uint32_t kGroupBlocksShift = 0xfeu;    // seg_shift value: every tile is a group block at a fixed stride
 // run_bytes of a contiguous (not strided) segment carries, in its top byte, the number
 // of leading bytes (< 128) that tile 0 moves in addition to its own range: with them

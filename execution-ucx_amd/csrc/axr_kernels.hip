@@ -1558,10 +1558,25 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   // blocks so that they rarely hold more than one segment); the loop below
   // walks forward from there to the segment of this wave's first tile.
   // (a bundle whose segments are one tile each needs no index: tile t is segment t)
-  uint32_t s = a.seg_shift == kDirectSegShift ? t : wave_seg[t >> a.seg_shift];
-  uint64_t seg_ptr = segs[s].ptr + delta, seg_off = segs[s].off, seg_run = segs[s].run_bytes;
+  // What a view's tile needs of the tables is three reads, each behind the other: the index, the segment, the view's
+  // own record.  A bundle of one view needs no index, and where every segment is a view of one mode the first record,
+  // which most of them share, is brought to the scalar cache meanwhile (pack + unpack of kept plans: 256 uint8 images of
+  // 224 x 224 x 3 29.4 -> 28.8 us, 64 of them 10.8 -> 10.3, 65,536 rows of 250 bytes at 1 KiB 18.2 -> 17.1).
+  constexpr bool one_mode = KIND != kKindRuns && KIND != kKindAny;
+  uint32_t warm[4] = {0, 0, 0, 0};
+  if constexpr (one_mode) {
+    const AXR_CONST uint32_t* record = reinterpret_cast<const AXR_CONST uint32_t*>(dims);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) warm[k] = record[k < 3 ? 16 * k : sizeof(Dims) / 4 - 1];
+  }
+  uint32_t s = a.seg_shift == kDirectSegShift ? t : KIND != kKindRuns && a.seg_shift == kOneSegShift ? 0u : wave_seg[t >> a.seg_shift];
+  uint64_t seg_ptr = segs[s].ptr, seg_off = segs[s].off, seg_run = segs[s].run_bytes;
   uint32_t seg_begin = segs[s].tile_begin, seg_meta = segs[s].meta;
   uint32_t seg_end = segs[s + 1].tile_begin;
+  if constexpr (one_mode)   // (waited for together)
+    asm volatile("" : "+s"(seg_ptr), "+s"(seg_off), "+s"(seg_run), "+s"(seg_begin), "+s"(seg_meta), "+s"(seg_end)
+                 : "s"(warm[0]), "s"(warm[1]), "s"(warm[2]), "s"(warm[3]));
+  seg_ptr += delta;
 
   while (t < t_end) {
     if (t >= seg_end) {   // wave-uniform: step to the next segment

@@ -1056,7 +1056,7 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
   uint32_t shift = 0;
   while (shift < 8 && (static_cast<uint64_t>(nseg) << (shift + 1)) <= p->ntiles) ++shift;
   // as many tiles as segments (none without a tile): tile t is segment t, no index to consult
-  p->cfg.seg_shift = may_be_direct && nseg == p->ntiles ? kDirectSegShift : shift;
+  p->cfg.seg_shift = may_be_direct && nseg == p->ntiles ? kDirectSegShift : nseg == 1 && p->cfg.elements ? kOneSegShift : shift;
 }
 
 // Tile rows of a bundle whose tensors are all compact: 2 KiB tiles, doubled while the bundle
@@ -1472,7 +1472,7 @@ int build_tables(axr_plan* p) {
   // a bundle of few large tensors gets a tiny index and a bundle of many small
   // ones one entry per few tiles; a wave walks at most a segment or two forward.
   const uint32_t shift = p->cfg.seg_shift;
-  const bool no_index = shift == kDirectSegShift || shift == kGroupBlocksShift;
+  const bool no_index = shift >= kOneSegShift;
   const size_t nblocks = no_index ? 1 : (static_cast<size_t>(p->ntiles) >> shift) + 1;
   p->wave_seg.assign(nblocks, 0);
   size_t s = 0;

@@ -2614,7 +2614,7 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       if (cfg.threads > fit)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs whose views need different amounts of LDS");
     }
-    if (cfg.kind != kModeRows) cfg.kind = kKindAny;   // the kernels there are for several jobs
+    if (cfg.kind != kModeRows && cfg.kind != kModePlanes) cfg.kind = kKindAny;   // the kernels there are for several jobs
     int rc = launch_bundle_jobs(table, cfg, stream);
     if (rc) return rc;
     for (size_t k = i; k < end; ++k) {

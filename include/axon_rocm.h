@@ -238,7 +238,8 @@ typedef struct axr_plan axr_plan_t;
  * ship the first nbytes of storage instead (dlpack_helpers.cpp:776-780).
  * Every tensor must be device-accessible (kDLROCM / kDLROCMHost) or kDLCPU;
  * kDLCPU tensors travel through pinned staging blocks of up to 8 MiB: neighbouring
- * pieces share one device copy per block; axr_pack returns once the host
+ * pieces share a block, and one or two blocks go over the bus in a few transfers
+ * while the rest is copied, more of them whole; axr_pack returns once the host
  * tensors have been read, axr_unpack once they hold their data (the device
  * tensors of the same bundle still complete asynchronously on the stream).
  * The plan copies shapes and strides; `tensors` may be freed on return.
@@ -379,7 +380,7 @@ typedef struct axr_launch_info {
   uint32_t segments;       /* device segment-table entries                    */
   uint32_t table_bytes;    /* device table size                               */
   uint32_t host_copies;    /* contiguous pieces of kDLCPU tensors              */
-  uint32_t host_chunks;    /* device copies that move them (pinned staging)    */
+  uint32_t host_chunks;    /* pinned staging blocks that they travel in         */
   uint32_t inline_tables;  /* 1: the next launch carries the tables inside the
                               kernel arguments, captured or not (small bundle,
                               first launch: no upload, no device block)        */

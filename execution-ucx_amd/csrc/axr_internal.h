@@ -214,13 +214,16 @@ constexpr uint32_t kRectBlockBytes = 8192;
 constexpr uint32_t kRectMaxEdge = 1024;
 constexpr uint32_t kMinBlockBytes = 1024;   // smaller blocks than this are left to element mode
 // Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
-// 16 bytes of every plane, a wavefront plane_rounds times that per lane.  One round where that gives a wavefront
-// 3 or 4 KiB: more wavefronts fit a compute unit's LDS and the last of them end closer together (pack + unpack, two
-// rounds, three of four-byte elements in three planes / one: 256 images of 224 x 224 x 3 bytes 28.6 / 27.3 us, 128 of 190 x 201 x 3
-// 16.8 / 13.8, 100 of 180 x 180 x 3 2-byte elements 17.3 / 15.8, 64 of 224 x 224 x 3 4-byte ones 31.1 / 27.1, 200 of 224 x 224 x 4
+// 16 bytes of every plane, a wavefront plane_rounds times that per lane.  Bytes and 2-byte elements: one round where
+// that gives a wavefront 3 or 4 KiB: more wavefronts fit a compute unit's LDS and the last of them end closer together
+// (pack + unpack, two rounds / one: 256 images of 224 x 224 x 3 bytes 28.6 / 27.3 us, 128 of 190 x 201 x 3
+// 16.8 / 13.8, 100 of 180 x 180 x 3 2-byte elements 17.3 / 15.8, 200 of 224 x 224 x 4
 // bytes 29.3 / 28.7).  Two where it would give it 2 KiB (300 of 210 x 200 x 2 bytes 18.8 / 19.5), and for four planes
-// of 2-byte elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6).
+// of 2-byte elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6).  4-byte elements take
+// as many as the 8 KiB rectangle of the other blocks with a short dimension has (1024, 680 and 512 elements of each of 2, 3 and
+// 4 planes); one round is faster for them as well, in blocks of another size (64 of 224 x 224 x 3 31.1 / 27.1).
 constexpr uint32_t plane_rounds(uint32_t element_bytes, uint32_t planes) {
+  if (element_bytes == 4) return planes == 4 ? 2u : planes == 3 ? 3u : 4u;
   return planes == 2 || (planes == 4 && element_bytes == 2) ? 2u : 1u;
 }
 constexpr uint32_t kMaxPlanes = 4;
@@ -230,7 +233,7 @@ constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes) {  
 }
 // Whether planes of `extent` elements are moved like this.  Whole vectors of 4-byte elements that one
 // access per lane holds are not: rectangles take no second round for them (38 MB in three planes of 200
-// elements 44 us for pack + unpack, 50 in rounds of the three there were then).
+// elements 44 us for pack + unpack, 50 in rounds).
 constexpr bool in_planes(uint32_t element_bytes, uint64_t extent) {
   return element_bytes <= 4 && extent * element_bytes >= kVecBytes &&
          !(element_bytes == 4 && extent <= kWaveLanes * kVecBytes / 4 && extent % 4 == 0);
@@ -238,7 +241,9 @@ constexpr bool in_planes(uint32_t element_bytes, uint64_t extent) {
 // Elements of every plane that a block takes of `extent` of them: whole vectors, as many as fit; the
 // block behind the last whole one takes what is left.
 constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t extent) {
-  const uint32_t vec = kVecBytes / element_bytes, block = plane_rounds(element_bytes, planes) * kWaveLanes * vec;
+  const uint32_t vec = kVecBytes / element_bytes, square = kRectBlockBytes / 4 / planes;
+  const uint32_t block = element_bytes < 4 ? plane_rounds(element_bytes, planes) * kWaveLanes * vec
+                                           : (square < kRectMaxEdge ? square : kRectMaxEdge) / vec * vec;
   return extent < block ? static_cast<uint32_t>((extent + vec - 1) / vec * vec) : block;
 }
 constexpr uint32_t kMaxBatchDims = 4;

@@ -974,7 +974,7 @@ __device__ __forceinline__ void interleaved_to_rows(gcbytes rd, gbytes wr, int64
 // pairs), 2 to 4 planes.  A lane owns 16 bytes of every plane: C vectors of the interleaved range,
 // regrouped in registers with byte permutes.  LDS only turns the lane's C neighbouring vectors
 // into wave-wide contiguous accesses.  Every access of the block to memory is in flight at once,
-// C KiB per round and one or two rounds (plane_rounds).  What it replaces gathered every element from LDS by
+// C KiB per round and one to four rounds (plane_rounds).  What it replaces gathered every element from LDS by
 // itself, 16 byte reads per vector, with one or two vectors in flight: 256 images of 224 x 224 x 3
 // bytes 47 -> 32 us for pack + unpack, 4 channels 55 -> 40, 64 such fp32 images 36 -> 32 (plain copy
 // of the bytes: 25.5 us).

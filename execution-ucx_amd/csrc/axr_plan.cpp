@@ -232,7 +232,6 @@ struct axr_plan {
   hipEvent_t upload_event = nullptr;   // from event_acquire; behind the latest upload once `uploaded` is set
   int upload_event_device = -1;
   hipStream_t upload_stream = nullptr;
-  bool upload_unrecorded = false;    // the event has not been recorded yet (never between two calls)
   struct BusyStream {
     hipStream_t stream;
     uint64_t mark;   // stream_mark_launch() of the plan's latest launch there
@@ -380,7 +379,7 @@ int check_align(uint32_t align) {
 void invalidate_tables(axr_plan* p) {
   p->tables_built = false;
   p->device_built = false;
-  p->uploaded = p->upload_unrecorded = false;
+  p->uploaded = false;
   p->tables_in_host_block = false;
   p->resident = false;
   p->inline_ready = false;
@@ -1074,28 +1073,20 @@ uint32_t rows_for_compact_bundle(const axr_plan* p) {
   return rows;
 }
 
-// Records the event that a launch on another stream waits for, once per upload.
-int record_upload(axr_plan* p) {
-  if (!p->upload_unrecorded) return AXR_OK;
-  p->upload_unrecorded = false;
-  return check_hip(hipEventRecord(p->upload_event, p->upload_stream), "hipEventRecord");
-}
-
-// Notes that the tables have just been put on their way on `stream`.  The event behind them is recorded by
-// record_upload before the call that uploads returns, on the default stream as on any other: recorded later it would lie
-// behind whatever the stream was given in between, and a launch elsewhere would wait for work that is not its
-// own.  The first launch of the plan itself is put in front of it (see run): it starts sooner without a
-// barrier for the event between the upload and itself, and a launch elsewhere waits for it as well (fresh pack + unpack,
-// event in front of / behind the first launch: 700 tensors of 256 B to 64 KiB 66.3 / 63.1 us, 1000 of 8 to 512 bytes 81.2 / 77.3).
+// Notes that the tables have just been put on their way on `stream`.  The event that a launch on
+// another stream waits for is recorded here, right behind the upload, on the default stream as on any
+// other: recorded later it would lie behind whatever the stream was given in between, and a launch
+// elsewhere would wait for work that is not its own.
 int note_upload(axr_plan* p, hipStream_t stream) {
   remember_stream(p, stream);
   if (!p->upload_event) {
     int rc = event_acquire(reinterpret_cast<void**>(&p->upload_event), &p->upload_event_device);
     if (rc) return rc;
   }
+  int rc = check_hip(hipEventRecord(p->upload_event, stream), "hipEventRecord");
+  if (rc) return rc;
   p->upload_stream = stream;
   p->uploaded = true;
-  p->upload_unrecorded = true;
   return AXR_OK;
 }
 
@@ -1571,11 +1562,8 @@ int ensure_uploaded(axr_plan* p, hipStream_t stream) {
     if (rc) return rc;
     return note_upload(p, stream);
   }
-  if (stream != p->upload_stream) {
-    const int rc = record_upload(p);   // (only where the call that uploaded has failed)
-    if (rc) return rc;
+  if (stream != p->upload_stream)
     return check_hip(hipStreamWaitEvent(stream, p->upload_event, 0), "hipStreamWaitEvent");
-  }
   return AXR_OK;
 }
 
@@ -1804,7 +1792,9 @@ uint32_t effective_nontemporal(const axr_plan* p, uint32_t job_flags) {
   return nt;
 }
 
-int launch_plan(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* stream_, int64_t delta, uint32_t job_flags) {
+int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* stream_, int64_t delta = 0,
+        uint32_t job_flags = 0) {
+  if (!p) return fail(AXR_ERR_INVALID, "null plan");
   if (!p->bound) return fail(AXR_ERR_INVALID, "plan has no tensor addresses bound");
   if (payload_bytes < p->payload_bytes)
     return fail(AXR_ERR_LENGTH, "payload buffer is smaller than the plan's payload");
@@ -1892,14 +1882,6 @@ int launch_plan(axr_plan* p, bool pack, void* payload, size_t payload_bytes, voi
   // for as long as the graph can run
   if (!capturing) remember_stream(p, stream);
   return AXR_OK;
-}
-
-int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* stream, int64_t delta = 0,
-        uint32_t job_flags = 0) {
-  if (!p) return fail(AXR_ERR_INVALID, "null plan");
-  const int rc = launch_plan(p, pack, payload, payload_bytes, stream, delta, job_flags);
-  const int recorded = record_upload(p);
-  return rc ? rc : recorded;
 }
 
 int store_tensor(RawVec<int64_t>& dims64, const axr_tensor_t& in, TensorRec* rec) {
@@ -2510,7 +2492,6 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     for (size_t k = 0; k < i; ++k)
       if (jobs[k].plan == p) return fail(AXR_ERR_INVALID, "axr_submit: one plan appears in two jobs");
     int rc = ensure_tables(p, stream, capturing);
-    if (!rc) rc = record_upload(p);
     if (rc) return rc;
     if (j.unpack && p->overlapping_dst)
       return fail(AXR_ERR_INVALID, "unpack destination has overlapping elements (zero stride)");
@@ -2574,7 +2555,6 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       axr_plan* p = j.plan;
       if (!p->resident) {
         int rc = ensure_uploaded(p, stream);
-        if (!rc) rc = record_upload(p);
         if (rc) return rc;
       }
       const uint8_t* d = static_cast<const uint8_t*>(p->block.device);
@@ -2658,7 +2638,6 @@ static int plan_prepare_body(axr_plan_t* plan, void* stream_) {
   if (rc) return rc;
   if (plan->ntiles == 0 || plan->resident) return AXR_OK;
   rc = ensure_uploaded(plan, stream);
-  if (!rc) rc = record_upload(plan);
   if (rc) return rc;
   rc = check_hip(hipEventSynchronize(plan->upload_event), "hipEventSynchronize(plan tables)");
   if (rc) return rc;

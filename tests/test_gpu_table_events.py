@@ -106,3 +106,26 @@ def test_prepared_plans_on_streams_that_wait_for_nothing(pkg, gpu, kind):
             assert all(torch.equal(out, expect) for out in outs)
     for s in streams:
         capi.check(lib.axr_stream_destroy(s))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tensors", [200, 700])    # tables of pitched views, by a kernel, and records laid out by one
+def test_tables_are_there_before_the_first_launch_is_done(pkg, gpu, tensors):
+    """What waits for a plan's tables (another stream, axr_plan_prepare on the host) does not wait for the launch
+    behind them: of the time that a pack of 6 GiB, some 2 ms, needs to end, a prepare takes the first few per cent."""
+    import time
+    parent = torch.zeros(tensors, (6 << 30) // tensors // 4096, 4096, dtype=torch.uint8, device=gpu)
+    ts = [t[1:, :4000] if tensors == 200 else t[1:] for t in parent]
+    payload = None
+    for _ in range(3):      # the first one loads kernels and allocates
+        with pkg.BundlePlan.create(ts, align=16) as plan:
+            payload = torch.empty(plan.payload_bytes, dtype=torch.uint8, device=gpu) if payload is None else payload
+            torch.cuda.synchronize()
+            plan.pack(payload.data_ptr(), payload.numel(), order=False)
+            start = time.perf_counter()
+            plan.prepare()
+            prepared = time.perf_counter()
+            torch.cuda.synchronize()
+            done = time.perf_counter()
+            assert plan.launch_info()["last_launch"] & 15 == (3 if tensors == 200 else 4)    # uploaded, device-built
+    assert prepared - start < (done - start) / 2

@@ -508,6 +508,20 @@ struct HostUnits {
   virtual int done(size_t u) = 0;                // units 0 .. u have been moved; in order, on the caller's thread
   virtual ~HostUnits() = default;
 };
+// Units of a block that the device fills from the front, raising a flag behind every `piece` bytes.  A flag is looked at
+// `looks` times in a row; then the caller's thread waits for the device and the others look again now and then.
+struct FlaggedUnits : HostUnits {
+  const uint32_t* flags = nullptr;
+  size_t piece = 1;
+  uint32_t looks = 0;
+  int status = AXR_OK;           // what ended the caller's share
+  virtual int arrive() = 0;      // returns once every flag has been raised (or with an error); on the caller's thread
+  bool ready(size_t u, bool caller) override;
+  void stop() { stopped_.store(true, std::memory_order_relaxed); }   // no ready() waits any longer
+
+ private:
+  std::atomic<bool> stopped_{false};
+};
 int host_copy_units(HostUnits& units);   // what done() returned, or AXR_OK
 
 // True for a handle that axr_stream_destroy has destroyed (and no later

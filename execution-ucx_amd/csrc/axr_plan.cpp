@@ -19,13 +19,11 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <thread>
 
 #include "axr_internal.h"
 #include "axr_source.h"
@@ -1606,22 +1604,23 @@ bool stages_in_pieces(const axr_plan* p, const void* payload, hipStream_t stream
 
 // A staging block under way between host tensors and the payload.  The pieces of host memory that make up bytes
 // [lo, hi) of the block are found by their payload offset (the chunk's pieces ascend and do not overlap).
-struct StagedChunk : HostUnits {
+template <typename Units>
+struct StagedChunk : Units {
   const HostCopy *first, *last;   // the chunk's pieces
   uint64_t begin;                 // payload offset of the block's first byte
   uint8_t* staged;
   uint8_t* payload;               // of that byte
   hipStream_t stream;
-
   bool in_pieces;                 // over the bus in pieces (see kStageUnit)
 
   StagedChunk(const axr_plan* p, const HostChunk& c, uint8_t* block, uint8_t* whole_payload, hipStream_t s, bool pieces_)
       : first(p->host_copies.data() + c.first), last(first + c.count), begin(c.begin), staged(block),
         payload(whole_payload + c.begin), stream(s), in_pieces(pieces_) {
-    span = static_cast<size_t>(c.end - c.begin);
+    const size_t span = static_cast<size_t>(c.end - c.begin);
     const size_t threads = std::max<size_t>(std::min(static_cast<size_t>(tunables().host_threads), span / kStagePerThread), 1);
-    helpers = threads - 1;
-    unit = in_pieces ? kStageUnit : ((span + threads - 1) / threads + 63) & ~static_cast<size_t>(63);
+    this->span = span;
+    this->helpers = threads - 1;
+    this->unit = in_pieces ? kStageUnit : ((span + threads - 1) / threads + 63) & ~static_cast<size_t>(63);
   }
   template <typename Move>
   void pieces(size_t lo, size_t hi, Move&& move) const {
@@ -1636,7 +1635,7 @@ struct StagedChunk : HostUnits {
 
 // Host tensors -> block -> payload.  Gaps between the pieces are zeroed: they are alignment padding or are
 // rewritten by the kernel that follows on the stream.
-struct ChunkIn : StagedChunk {
+struct ChunkIn : StagedChunk<HostUnits> {
   using StagedChunk::StagedChunk;
   size_t sent = 0;
   bool ready(size_t, bool) override { return true; }
@@ -1662,37 +1661,19 @@ struct ChunkIn : StagedChunk {
 };
 
 // Payload -> block -> host tensors.  stage_out_kernel raises a flag behind every piece of the block that has
-// arrived; a unit is emptied as soon as its flags are up, while the next ones are on the bus.  The flags are
-// polled for a while, then the caller's thread waits for the stream, behind which all of them are up, and the
-// helpers look again now and then.
-struct ChunkOut : StagedChunk {
-  const uint32_t* flags;
-  std::atomic<bool> failed{false};
-  int status = AXR_OK;
-  ChunkOut(const axr_plan* p, const HostChunk& c, uint8_t* block, const uint32_t* f, uint8_t* whole_payload, hipStream_t s,
-           bool in_pieces)
-      : StagedChunk(p, c, block, whole_payload, s, in_pieces), flags(f) {}
-  bool ready(size_t u, bool caller) override {
-    if (!in_pieces) return true;   // the block has been waited for
-    const size_t end = (std::min((u + 1) * unit, span) + kStagePieceBytes - 1) / kStagePieceBytes;
-    size_t i = u * unit / kStagePieceBytes;
-    for (uint32_t spins = 0; i < end; ++spins) {
-      if (__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) {
-        ++i;
-      } else if (spins < kStageSpins) {
-        __builtin_ia32_pause();
-      } else if (failed.load(std::memory_order_relaxed)) {
-        return false;
-      } else if (caller) {
-        if (!status) status = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize(staging)");
-        if (!status && !__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) status = fail(AXR_ERR_HIP, "a staging copy ended without its flags");
-        if (status) failed.store(true, std::memory_order_relaxed);
-      } else {
-        std::this_thread::sleep_for(std::chrono::microseconds(20));
-      }
-    }
-    return true;
+// arrived; a unit is emptied as soon as its flags are up, while the next ones are on the bus.  Behind work that takes longer
+// than the flags are polled for, the caller's thread waits for the block's own event: what others have put on the stream
+// since, which may wait for what this thread does next, is not waited for.
+struct ChunkOut : StagedChunk<FlaggedUnits> {
+  hipEvent_t arrived;   // behind the kernel
+  ChunkOut(const axr_plan* p, const HostChunk& c, const HostStage* st, uint8_t* whole_payload, hipStream_t s, bool pieces_)
+      : StagedChunk(p, c, static_cast<uint8_t*>(st->block.host), whole_payload, s, pieces_), arrived(st->ready) {
+    flags = static_cast<const uint32_t*>(st->flags.host);
+    piece = kStagePieceBytes;
+    looks = kStageSpins;
   }
+  bool ready(size_t u, bool caller) override { return !in_pieces || FlaggedUnits::ready(u, caller); }   // (whole: waited for before)
+  int arrive() override { return check_hip(hipEventSynchronize(arrived), "hipEventSynchronize(staging)"); }
   void copy(size_t lo, size_t hi) override {
     pieces(lo, hi, [&](uint8_t* host, size_t from, size_t n) { std::memcpy(host, staged + from, n); });
   }
@@ -1712,7 +1693,7 @@ int move_host_tensors(axr_plan* p, bool pack, uint8_t* payload, hipStream_t stre
     const HostChunk& c = p->host_chunks[k];
     int rc = in_pieces ? AXR_OK : stage_ready(st);
     if (rc) return rc;
-    ChunkOut out(p, c, block_of(k), static_cast<const uint32_t*>(st->flags.host), payload, stream, in_pieces);
+    ChunkOut out(p, c, st, payload, stream, in_pieces);
     rc = host_copy_units(out);
     if (!rc) rc = out.status;
     st->pending = rc != AXR_OK;   // with all flags up the device is done with the block

@@ -236,6 +236,27 @@ void host_copy(const HostCopyJob* jobs, size_t count) {
   for (std::thread& t : helpers) t.join();
 }
 
+bool FlaggedUnits::ready(size_t u, bool caller) {
+  const size_t end = (std::min((u + 1) * unit, span) + piece - 1) / piece;
+  size_t i = u * unit / piece;
+  for (uint32_t seen = 0; i < end; ++seen) {
+    if (__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) {
+      ++i;
+    } else if (seen < looks) {
+      __builtin_ia32_pause();
+    } else if (stopped_.load(std::memory_order_relaxed)) {
+      return false;
+    } else if (caller) {
+      status = arrive();
+      if (!status && !__atomic_load_n(flags + i, __ATOMIC_ACQUIRE)) status = fail(AXR_ERR_HIP, "a staging copy ended without its flags");
+      if (status) stop();
+    } else {
+      std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+  }
+  return true;
+}
+
 int host_copy_units(HostUnits& units) {
   const size_t n = (units.span + units.unit - 1) / units.unit;
   std::unique_ptr<std::atomic<uint8_t>[]> moved(new std::atomic<uint8_t>[n]());

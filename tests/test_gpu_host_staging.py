@@ -82,3 +82,54 @@ def test_behind_work_longer_than_the_flags_are_polled(pkg, gpu):
     assert np.array_equal(src[0], out[0])
     plan.close()
     recv.close()
+
+
+def test_later_work_on_the_stream_is_not_waited_for(pkg, gpu):
+    """An unpack that waits behind other work returns with its bytes while what another thread has put on the same
+    stream in the meantime is still running.  (Put there in the time in which flags are polled, which a thread may miss:
+    one of a few attempts has to show it.)"""
+    import threading
+    import time
+    import torch
+    rng = np.random.default_rng(4)
+    src = [rng.integers(0, 256, size=900000, dtype=np.uint8)]
+    out = [np.zeros_like(src[0])]
+    plan = pkg.BundlePlan.create(src)
+    n = plan.payload_bytes
+    recv = pkg.BundlePlan.from_header(plan.header).bind(out)
+    buf = torch.zeros(n, dtype=torch.uint8, device=gpu)
+    plan.pack(buf.data_ptr(), n)
+    recv.unpack(buf.data_ptr(), n)      # (its buffers are there from now on)
+    work = torch.zeros(1 << 28, dtype=torch.float32, device=gpu)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(1)
+    for _ in range(4):
+        out[0][...] = 0
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            for _ in range(30):
+                work += 1.0      # some 10 ms
+        started = threading.Event()
+
+        def unpack():
+            started.set()
+            recv.unpack(buf.data_ptr(), n, stream.cuda_stream, False)
+        moved = threading.Thread(target=unpack)
+        moved.start()
+        started.wait()
+        now = time.perf_counter()
+        while time.perf_counter() < now + 5e-5:
+            time.sleep(0)
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(1 << 27)      # some 50 ms
+        moved.join()
+        back = time.perf_counter()
+        assert np.array_equal(src[0], out[0])
+        torch.cuda.synchronize()
+        not_waited_for = time.perf_counter() - back > back - now
+        if not_waited_for:
+            break
+    assert not_waited_for
+    plan.close()
+    recv.close()

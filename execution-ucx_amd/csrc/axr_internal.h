@@ -506,6 +506,7 @@ struct HostUnits {
   virtual bool ready(size_t u, bool caller) = 0;
   virtual void copy(size_t lo, size_t hi) = 0;   // moves bytes [lo, hi); from any of the threads
   virtual int done(size_t u) = 0;                // units 0 .. u have been moved; in order, on the caller's thread
+  virtual void stop() {}                         // the caller gives up: no ready() may wait any longer
   virtual ~HostUnits() = default;
 };
 // Units of a block that the device fills from the front, raising a flag behind every `piece` bytes.  A flag is looked at
@@ -517,7 +518,7 @@ struct FlaggedUnits : HostUnits {
   int status = AXR_OK;           // what ended the caller's share
   virtual int arrive() = 0;      // returns once every flag has been raised (or with an error); on the caller's thread
   bool ready(size_t u, bool caller) override;
-  void stop() { stopped_.store(true, std::memory_order_relaxed); }   // no ready() waits any longer
+  void stop() override { stopped_.store(true, std::memory_order_relaxed); }
 
  private:
   std::atomic<bool> stopped_{false};

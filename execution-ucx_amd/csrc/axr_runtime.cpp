@@ -259,6 +259,7 @@ bool FlaggedUnits::ready(size_t u, bool caller) {
 
 int host_copy_units(HostUnits& units) {
   const size_t n = (units.span + units.unit - 1) / units.unit;
+  if (n == 0) return AXR_OK;
   std::unique_ptr<std::atomic<uint8_t>[]> moved(new std::atomic<uint8_t>[n]());
   std::atomic<size_t> next{0};
   auto move_one = [&](size_t u, bool caller) {
@@ -271,11 +272,20 @@ int host_copy_units(HostUnits& units) {
     for (size_t u; (u = next.fetch_add(1, std::memory_order_relaxed)) < n;)
       if (!move_one(u, false)) return;
   };
-  std::vector<std::thread> helpers;
+  // (joins on the way out of an exception as well, which a thread that is still joinable would turn into an abort)
+  struct Helpers {
+    HostUnits& units;
+    std::vector<std::thread> threads;
+    bool stop = true;
+    ~Helpers() {
+      if (stop) units.stop();
+      for (std::thread& t : threads) t.join();
+    }
+  } helpers{units, {}, true};
   try {
     const size_t count = std::min(units.helpers, n - 1);
-    helpers.reserve(count);
-    for (size_t i = 0; i < count; ++i) helpers.emplace_back(help);
+    helpers.threads.reserve(count);
+    for (size_t i = 0; i < count; ++i) helpers.threads.emplace_back(help);
   } catch (...) {
     // no more threads to be had: fewer take part
   }
@@ -285,7 +295,7 @@ int host_copy_units(HostUnits& units) {
     for (; !rc && told < n && moved[told].load(std::memory_order_acquire); ++told) rc = units.done(told);
   };
   bool ok = true;
-  for (size_t u; ok && (u = next.fetch_add(1, std::memory_order_relaxed)) < n;) {
+  for (size_t u; ok && !rc && (u = next.fetch_add(1, std::memory_order_relaxed)) < n;) {
     ok = move_one(u, true);
     tell();
   }
@@ -295,7 +305,7 @@ int host_copy_units(HostUnits& units) {
     else if (!units.ready(told, true)) ok = false;
     else __builtin_ia32_pause();
   }
-  for (std::thread& t : helpers) t.join();
+  helpers.stop = !ok || rc != AXR_OK;
   return rc;
 }
 }  // namespace axr

@@ -135,10 +135,11 @@ def test_loopback_context_under_thread_sanitizer(tmp_path):
     assert "loopback_stress ok 2500" in out.stdout      # 4 x 400, then 3 x 300 on a shared context
 
 
-def test_host_copy_helper_under_sanitizers(tmp_path):
-    """tests/cpp/host_copy_check.cpp: the threaded copy of the staging paths against plain
-    memcpy for random piece lists and 1 to 16 threads, with the runtime shim compiled with
-    AddressSanitizer and UBSan (host code only, no GPU)."""
+@pytest.mark.parametrize("sanitizers", [("address", "undefined"), ("thread",)], ids="+".join)
+def test_host_copy_helper_under_sanitizers(tmp_path, sanitizers):
+    """tests/cpp/host_copy_check.cpp: the threaded copies of the staging paths and of the runtime against plain
+    memcpy for random piece lists, units and 1 to 16 threads, errors and exceptions included, with the runtime
+    shim compiled with AddressSanitizer and UBSan, and with ThreadSanitizer (host code only, no GPU)."""
     pkgdir = os.path.join(ROOT, "execution-ucx_amd")
     objs = [os.path.join(pkgdir, "build", n) for n in
             ("axr_plan.cpp.o", "axr_loopback.cpp.o", "axr_kernels.hip.o")]
@@ -147,20 +148,21 @@ def test_host_copy_helper_under_sanitizers(tmp_path):
         pytest.skip("needs the library's object files (make -C execution-ucx_amd) and the ROCm compilers")
     inc = ["-I", os.path.join(ROOT, "include"), "-I", os.path.join(pkgdir, "csrc")]
     runtime_o, check_o, exe = (str(tmp_path / n) for n in ("axr_runtime.o", "host_copy_check.o", "host_copy_check"))
+    flags = ["-fsanitize=" + s for s in sanitizers]
     steps = [
         [hipcc, "--offload-arch=gfx950", "-O1", "-g", "-std=c++17", "-fPIC",
-         "-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=undefined",
+         *[a for f in flags for a in ("-Xarch_host", f)],
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option", *inc,
          "-x", "hip", "-c", os.path.join(pkgdir, "csrc", "axr_runtime.cpp"), "-o", runtime_o],
-        [clang, "-O1", "-g", "-std=c++17", "-fsanitize=address,undefined", *inc, "-c",
+        [clang, "-O1", "-g", "-std=c++17", *flags, *inc, "-c",
          os.path.join(ROOT, "tests", "cpp", "host_copy_check.cpp"), "-o", check_o],
-        [hipcc, "--offload-arch=gfx950", "-fsanitize=address", "-fsanitize=undefined", "-fno-gpu-sanitize",
+        [hipcc, "--offload-arch=gfx950", *flags, "-fno-gpu-sanitize",
          check_o, runtime_o, *objs, "-o", exe, "-lpthread"],
     ]
     for cmd in steps:
         out = subprocess.run(cmd, capture_output=True, text=True, timeout=600)
         assert out.returncode == 0, out.stderr[-3000:]
     out = subprocess.run([exe], capture_output=True, text=True, timeout=600)
-    assert out.returncode == 0, (out.stdout + out.stderr)[-3000:]
-    assert "host_copy_check ok" in out.stdout
+    assert out.returncode == 0 and "ThreadSanitizer" not in out.stderr, (out.stdout + out.stderr)[-3000:]
+    assert "host_copy_check ok" in out.stdout and "host_copy_units ok" in out.stdout

@@ -524,6 +524,13 @@ struct FlaggedUnits : HostUnits {
   std::atomic<bool> stopped_{false};
 };
 int host_copy_units(HostUnits& units);   // what done() returned, or AXR_OK
+// The least that goes to the payload at once of a staging block of `span` bytes, `sent` of which have gone (the rules of
+// staging blocks are in axr_plan.cpp).  Rounded up: four such pieces hold the block, whatever its length.
+constexpr size_t kStageUnit = 64u << 10, kStageSend = 256u << 10;
+constexpr size_t stage_piece(size_t span, size_t sent) {
+  const size_t part = ((sent ? 5 * span : span) + 15) / 16;
+  return part > kStageSend ? part : kStageSend;
+}
 
 // True for a handle that axr_stream_destroy has destroyed (and no later
 // axr_stream_create has returned again).

@@ -117,12 +117,12 @@ constexpr size_t kStageBytes = 8u << 20;
 // before / now: 64 KiB 44.6 / 33.8 us, 256 KiB 61 / 45, 512 KiB 83 / 63, 1 MiB 125 / 96, 4 MiB 357 / 270):
 //  - Threads take kStageUnit at a time.  A helper costs its starter 12 us, so there is one for every whole
 //    kStagePerThread behind the first (1 MiB with a helper 118 us).
-//  - To the payload goes a first piece of kStageSend or a sixteenth of the block, and then pieces of 5/16 of it, four
-//    in all: with eight or more the wait at the end takes 26 us instead of 4 (4 MiB 303 to 310).  A kernel's first
+//  - To the payload goes a first piece of kStageSend or a sixteenth of the block, and then pieces of 5/16 of it
+//    (stage_piece), at most four in all: with eight or more the wait at the end takes 26 us instead of 4 (4 MiB 303 to 310).  A kernel's first
 //    bytes move sooner than the copy engine's, which moves more per second: kernels / engine 1 MiB 96 / 117, 4 MiB 276 / 268.
 //  - From the payload a kernel of kStageGroups workgroups brings the block and raises its flags in order (see
 //    stage_out_kernel; 4 MiB with 8 / 16 / 32 workgroups 307 / 276 / 300, one for every piece 320).  kStageSpins looks at a flag are some 200 us.
-constexpr size_t kStageUnit = 64u << 10, kStagePerThread = 1u << 20, kStageSend = 256u << 10, kStageEngine = 2u << 20;
+constexpr size_t kStagePerThread = 1u << 20, kStageEngine = 2u << 20;
 //  - With more than kStageChunksInPieces blocks the bus is busy all the time but for the first and the last of them: these go
 //    over it whole, by the engine (64 MiB 2945 us whole, 3100 in pieces; 16 MiB, two blocks, 983 / 827).
 constexpr size_t kStageChunksInPieces = 2;
@@ -1650,7 +1650,7 @@ struct ChunkIn : StagedChunk<HostUnits> {
   }
   int done(size_t u) override {
     const size_t upto = std::min((u + 1) * unit, span), piece = upto - sent;
-    if (upto < span && (!in_pieces || piece < std::max(kStageSend, sent ? span / 16 * 5 : span / 16))) return AXR_OK;
+    if (upto < span && (!in_pieces || piece < stage_piece(span, sent))) return AXR_OK;
     const int rc = in_pieces && span < kStageEngine
                        ? launch_stream_copy(payload + sent, staged + sent, piece, true, stream)
                        : check_hip(hipMemcpyAsync(payload + sent, staged + sent, piece, hipMemcpyDefault, stream),

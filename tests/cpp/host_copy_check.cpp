@@ -100,6 +100,24 @@ int bad(const char* what, long at) {
   return 1;
 }
 
+// A block goes to the payload in at most four transfers, whatever its length.
+int check_pieces() {
+  std::mt19937_64 rng(13);
+  for (int i = 0; i < 20000; ++i) {
+    const size_t around = (size_t{1} << 18) * (1 + i % 32);
+    const size_t span = i < 200 ? around + i / 32 * 5 - 15 : 1 + rng() % (8u << 20);
+    size_t sent = 0, transfers = 0;
+    for (size_t at = 0; at < span;) {
+      at = std::min(at + axr::kStageUnit, span);
+      if (at < span && at - sent < axr::stage_piece(span, sent)) continue;
+      sent = at;
+      ++transfers;
+    }
+    if (transfers > 4 || (span <= axr::kStageSend && transfers != 1)) return bad("transfers of a block", static_cast<long>(span));
+  }
+  return 0;
+}
+
 int check_units() {
   std::mt19937_64 rng(12);
   auto pick = [&](uint64_t lo, uint64_t hi) { return lo + rng() % (hi - lo + 1); };
@@ -212,5 +230,5 @@ int main() {
     }
   }
   std::printf("host_copy_check ok %ld\n", cases);
-  return check_units();
+  return check_pieces() + check_units();
 }

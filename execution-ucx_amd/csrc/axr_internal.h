@@ -588,7 +588,7 @@ int launch_expand_groups(const Member* members, const GroupStage* groups, uint32
 // tables[0, bytes) = staged[0, bytes), rounded up to 16 bytes: a table block's pinned half into its
 // device half.
 int launch_upload_tables(const void* staged, void* tables, size_t bytes, void* stream);
-// dst[0, bytes) = src[0, bytes), both in device memory of the current device, no alignment needed.
+// dst[0, bytes) = src[0, bytes), no alignment needed; dst in memory of the current device, src there or in pinned host memory.
 int launch_stream_copy(void* dst, const void* src, size_t bytes, bool nontemporal, void* stream);
 // dst[0, bytes) = src[0, bytes) from device memory to pinned host memory; flags[i] (pinned, cleared by the
 // caller) becomes 1 once bytes [i, i + 1) * kStagePieceBytes are there.

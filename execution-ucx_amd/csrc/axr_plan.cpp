@@ -1588,8 +1588,9 @@ int stage_acquire(HostStage* st, size_t bytes) {
   return stage_ready(st);
 }
 
-// In pieces go few blocks, and payloads that a kernel on `stream` reaches: memory of the current device, which is the
-// stream's (the copy engine takes any other, a payload in ordinary host memory included).
+// In pieces go few blocks, and payloads in memory of the current device, which is the stream's.  The copy engine takes any
+// other that the device can access (pinned, managed, another device's).  Memory that it cannot access is none for a payload,
+// here as elsewhere: gaps between the pieces are written by the bundle kernel.
 bool stages_in_pieces(const axr_plan* p, const void* payload, hipStream_t stream) {
   if (p->host_chunks.size() > kStageChunksInPieces) return false;
   hipPointerAttribute_t attr;

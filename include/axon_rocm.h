@@ -295,7 +295,8 @@ AXR_API int axr_plan_split(const axr_plan_t* plan, void* payload, size_t payload
 
 /* Gather the bound tensors into payload[0, payload_bytes) / scatter payload
  * into the bound tensors, asynchronously on `stream`.  `payload` must be
- * device-accessible memory; payload_bytes must be >= axr_plan_payload_bytes
+ * device-accessible memory, for bundles of kDLCPU tensors as well (the kernel writes
+ * the gaps between them); payload_bytes must be >= axr_plan_payload_bytes
  * (AXR_ERR_LENGTH otherwise).  The first call uploads the plan's device
  * tables on the same stream.  A plan may be packed/unpacked any number of
  * times; concurrent calls on one plan from two threads are not allowed. */

@@ -15,6 +15,7 @@ VIEWS = {
     "walked": lambda s: s.view(torch.int16)[:1031 * 16001].view(1031, 16001).t(),
     "one_block": lambda s: s[:20 * 33].view(20, 33).t(),
 }
+JOINT = {"elements": 6, "blocks": 6, "walked": 6, "one_block": 6, "planes": 5, "rows": 2}    # kernels of joint launches: any mode, planes, rows
 
 
 @pytest.mark.gpu
@@ -44,7 +45,15 @@ def test_every_way(pkg, gpu, kind, align):
     packed()
     back = torch.zeros_like(store)
     out = VIEWS[kind](back)
-    recv = pkg.BundlePlan.from_header(send.header).bind([out])
+    if kind == "walked":           # (workgroups that are handed to the dies in turn share no launch)
+        send.close()
+        pkg.tune(xcd_remap=0)
+    try:
+        if kind == "walked":
+            send = pkg.BundlePlan.create([view], align=align).prepare()
+        recv = pkg.BundlePlan.from_header(send.header).bind([out]).prepare()
+    finally:
+        pkg.tune(xcd_remap=-1)
     jobs = (capi.Job * 2)()
     second = torch.zeros_like(payload)
     second[:want.numel()] = want
@@ -54,6 +63,8 @@ def test_every_way(pkg, gpu, kind, align):
         capi.check(lib.axr_submit(jobs, 2, None))
         packed()
         assert torch.equal(out, view)
+        if kind in JOINT:     # in one launch: alone each of them has a kernel of its own
+            assert [p.launch_info()["last_launch"] >> 4 & 15 for p in (send, recv)] == [JOINT[kind]] * 2
         back.zero_()
     recv.unpack(second.data_ptr(), n)
     assert torch.equal(out, view)

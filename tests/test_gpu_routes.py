@@ -104,6 +104,7 @@ def test_every_kind_has_its_kernel(pkg, gpu, kind):
 
 
 @pytest.mark.parametrize("kinds,want", [((ROWS, ROWS), (ROWS, ROWS)), ((ROWS, RUNS), (ANY, ANY)), ((BLOCKS, BLOCKS), (ANY, ANY)),
+                                        ((PLANES, PLANES), (PLANES, PLANES)), ((PLANES, ROWS), (ANY, ANY)),
                                         ((RUNS, RUNS), (RUNS, RUNS)), (("many", RUNS), (ROWS, RUNS)), (("many", ROWS), (ROWS, ROWS)),
                                         ((BLOCKS, "many"), (BLOCKS, ROWS)), ((ROWS, "many", RUNS), (ROWS, ROWS, RUNS)),
                                         ((ROWS, RUNS, "many"), (ANY, ANY, ROWS)), (("some", "some", RUNS), (ROWS, ROWS, RUNS)),

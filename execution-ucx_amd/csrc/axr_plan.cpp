@@ -121,7 +121,7 @@ constexpr size_t kStageBytes = 8u << 20;
 //    (stage_piece), at most four in all: with eight or more the wait at the end takes 26 us instead of 4 (4 MiB 303 to 310).  A kernel's first
 //    bytes move sooner than the copy engine's, which moves more per second: kernels / engine 1 MiB 96 / 117, 4 MiB 276 / 268.
 //  - From the payload a kernel of kStageGroups workgroups brings the block and raises its flags in order (see
-//    stage_out_kernel; 4 MiB with 8 / 16 / 32 workgroups 307 / 276 / 300, one for every piece 320).  kStageSpins looks at a flag are some 200 us.
+//    stage_out_kernel; 4 MiB with 8 / 16 / 32 workgroups 307 / 276 / 300, one for every piece 320).  kStageSpins looks at a flag are half a millisecond.
 constexpr size_t kStagePerThread = 1u << 20, kStageEngine = 2u << 20;
 //  - With more than kStageChunksInPieces blocks the bus is busy all the time but for the first and the last of them: these go
 //    over it whole, by the engine (64 MiB 2945 us whole, 3100 in pieces; 16 MiB, two blocks, 983 / 827).

@@ -214,22 +214,30 @@ constexpr uint32_t kRectBlockBytes = 8192;
 constexpr uint32_t kRectMaxEdge = 1024;
 constexpr uint32_t kMinBlockBytes = 1024;   // smaller blocks than this are left to element mode
 // Two to four planes of 1- to 4-byte elements against the same elements interleaved: a lane moves
-// 16 bytes of every plane, a wavefront plane_rounds times that per lane.  Bytes and 2-byte elements: one round where
-// that gives a wavefront 3 or 4 KiB: more wavefronts fit a compute unit's LDS and the last of them end closer together
-// (pack + unpack, two rounds / one: 256 images of 224 x 224 x 3 bytes 28.6 / 27.3 us, 128 of 190 x 201 x 3
-// 16.8 / 13.8, 100 of 180 x 180 x 3 2-byte elements 17.3 / 15.8, 200 of 224 x 224 x 4
-// bytes 29.3 / 28.7).  Two where it would give it 2 KiB (300 of 210 x 200 x 2 bytes 18.8 / 19.5), and for four planes
-// of 2-byte elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6).  4-byte elements take
-// as many as the 8 KiB rectangle of the other blocks with a short dimension has (1024, 680 and 512 elements of each of 2, 3 and
-// 4 planes); one round is faster for them as well, in blocks of another size (64 of 224 x 224 x 3 31.1 / 27.1).
+// 16 bytes of every plane, a wavefront up to plane_rounds times that per lane.  Bytes and 2-byte
+// elements take two rounds; 4-byte elements as many as the 8 KiB rectangle of the other blocks with
+// a short dimension has (1024, 680 and 512 elements of each of 2, 3 and 4 planes).
 constexpr uint32_t plane_rounds(uint32_t element_bytes, uint32_t planes) {
-  if (element_bytes == 4) return planes == 4 ? 2u : planes == 3 ? 3u : 4u;
-  return planes == 2 || (planes == 4 && element_bytes == 2) ? 2u : 1u;
+  return element_bytes < 4 || planes == 4 ? 2u : planes == 3 ? 3u : 4u;
 }
+// In the kernel of planes alone two wavefronts take a block together, a round each, where that leaves either of them 3 or
+// 4 KiB: more of them fit a compute unit's LDS and the last of them end closer together (pack + unpack, one wavefront to a
+// block / two: 256 images of 224 x 224 x 3 bytes 29.1 / 28.0 us, 128 of 190 x 201 x 3 20.1 / 17.1, 100 of 180 x 180 x 3 2-byte
+// elements 21.5 / 20.0, 200 of 224 x 224 x 4 bytes 30.0 / 29.2).  Not where it would leave them 2 KiB (300 of 210 x 200 x 2 bytes
+// 18.8 / 19.5), nor for four planes of 2-byte elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6), nor for
+// 4-byte elements, whose blocks are no whole rounds (in blocks of one round each 64 of 224 x 224 x 3 took 27.1 us instead of 31.1).
+// The kernel for any mode holds as many wavefronts either way and keeps whole blocks (next to 1 MiB of compact tensor, a
+// block to a wavefront / a round: 256 of 224 x 224 x 3 bytes 30.2 / 33.8, 150 of 180 x 180 x 3 2-byte elements 24.7 / 27.0).
+constexpr uint32_t plane_parts(uint32_t element_bytes, uint32_t planes) {
+  return element_bytes < 4 && (planes == 3 || (planes == 4 && element_bytes == 1)) ? 2u : 1u;
+}
+// The elements of every plane that lie in one round.
+constexpr uint32_t plane_round_elements(uint32_t element_bytes) { return kWaveLanes * kVecBytes / element_bytes; }
 constexpr uint32_t kMaxPlanes = 4;
 constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2;   // Dims.lanes_per_run of such a segment
-constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes) {   // one vector of padding behind every eight
-  return plane_rounds(element_bytes, planes) * kWaveLanes * planes * kVecBytes / 8 * 9;
+// LDS of a wavefront, one vector of padding behind every eight.
+constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes, uint32_t parts = 1) {
+  return plane_rounds(element_bytes, planes) / parts * kWaveLanes * planes * kVecBytes / 8 * 9;
 }
 // Whether planes of `extent` elements are moved like this.  Whole vectors of 4-byte elements that one
 // access per lane holds are not: rectangles take no second round for them (38 MB in three planes of 200
@@ -242,9 +250,28 @@ constexpr bool in_planes(uint32_t element_bytes, uint64_t extent) {
 // block behind the last whole one takes what is left.
 constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t extent) {
   const uint32_t vec = kVecBytes / element_bytes, square = kRectBlockBytes / 4 / planes;
-  const uint32_t block = element_bytes < 4 ? plane_rounds(element_bytes, planes) * kWaveLanes * vec
+  const uint32_t block = element_bytes < 4 ? plane_rounds(element_bytes, planes) * plane_round_elements(element_bytes)
                                            : (square < kRectMaxEdge ? square : kRectMaxEdge) / vec * vec;
   return extent < block ? static_cast<uint32_t>((extent + vec - 1) / vec * vec) : block;
+}
+// The elements (of 1 << element_shift bytes) of every plane that a wavefront moves: of the block of `edge` elements that begins at `at`, all or (part 0 or
+// 1) those of one round.  None where a part has nothing to move; otherwise a vector at least, moved back to end with
+// the planes where less is left of them.
+constexpr uint32_t kWholeBlock = 2;
+struct PlaneRange {
+  uint32_t at, count;
+};
+constexpr PlaneRange plane_range(uint32_t element_shift, uint32_t extent, uint32_t edge, uint32_t at, uint32_t part) {
+  uint32_t end = extent - at < edge ? extent : at + edge;
+  if (part != kWholeBlock) {
+    const uint32_t round = kWaveLanes * kVecBytes >> element_shift;
+    if (end - at <= part * round) return {at, 0};
+    at += part * round;
+    if (end - at > round) end = at + round;
+  }
+  const uint32_t least = kVecBytes >> element_shift;
+  if (extent - at < least) at = extent - least;
+  return {at, end - at};
 }
 constexpr uint32_t kMaxBatchDims = 4;
 constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (measured: 8 KiB beats 2, 4 and 16)
@@ -358,7 +385,7 @@ struct KernelArgs {
   uint8_t* payload;
   uint32_t nseg;
   uint32_t ntiles;
-  uint32_t tiles_per_wave;
+  uint32_t tiles_per_wave;    // or kHalfTile
   uint32_t xcd_remap;         // 0, or remap_code of the workgroup indices a die takes in a row
   uint32_t seg_shift;         // log2 of the tile-block size of wave_seg
   int64_t tensor_delta = 0;   // added to every tensor-side address of the tables
@@ -396,9 +423,12 @@ struct alignas(16) InlineTables {
   uint8_t bytes[kInlineTableBytes];
 };
 
+// tiles_per_wave value: two wavefronts take a tile together, the kernel of planes alone only (see plane_parts).
+constexpr uint32_t kHalfTile = 0;
+
 struct LaunchConfig {
   uint32_t workgroups = 0;
-  uint32_t tiles_per_wave = 0;
+  uint32_t tiles_per_wave = 0;   // or kHalfTile (whole_tiles gives the launch in which it is one)
   uint32_t tile_rows = 2;
   uint32_t threads = 128;   // per workgroup, a multiple of 64
   uint32_t seg_shift = 0;   // wave_seg has one entry per 2^seg_shift tiles
@@ -406,12 +436,20 @@ struct LaunchConfig {
   bool elements = false;   // some segment's mode is above kModeRunTiles
   uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (kModeRows and above)
-  uint32_t lds_walked = 0;     // and in the kernel of walked blocks alone
+  uint32_t lds_alone = 0;      // in the kernel of walked blocks alone, and in that of planes alone with kHalfTile
   uint32_t cached_tail = 0;    // MiB at the end of a streaming payload that a pack leaves in the cache (runs in
                            // 1 KiB tiles only; see finish_geometry)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
                            // multiple of 8 such runs)
 };
+// A launch of `ntiles` tiles in another kernel than the plan's own.
+inline LaunchConfig whole_tiles(LaunchConfig cfg, uint32_t ntiles) {
+  if (cfg.tiles_per_wave != kHalfTile) return cfg;
+  const uint32_t waves = cfg.threads / kWaveLanes;
+  cfg.tiles_per_wave = 1;
+  cfg.workgroups = ntiles / waves + (ntiles % waves != 0);
+  return cfg;
+}
 
 // ---------------------------------------------------------------- tunables
 

@@ -398,7 +398,7 @@ void invalidate_tables(axr_plan* p) {
   p->shared_line_tiles = 0;
   p->strip_tiles = 0;
   p->whole_groups = false;
-  p->cfg.lds_per_wave = p->cfg.lds_walked = 0;
+  p->cfg.lds_per_wave = p->cfg.lds_alone = 0;
 }
 
 // Wait until the device no longer reads the plan's tables.  No event is
@@ -534,6 +534,9 @@ uint64_t element_mode_limit(uint64_t run_bytes) {
   if (run_bytes >= kVecBytes && tunables().ragged_runs != 0) return std::min<uint64_t>(limit, kMaxRowBytes + 1);
   return (limit + 4) / 5;
 }
+
+// How many planes a segment of planes has.
+uint32_t planes_of(const Dims& dm) { return dm.lanes_per_run == kPlanesInPayload ? dm.edge_b : dm.edge_a; }
 
 struct Builder {
   axr_plan* p;
@@ -790,7 +793,9 @@ struct Builder {
       dm.tiles_per_run = 1;
       if (planes) {
         dm.mode = kModePlanes;
-        lds = planes_lds_bytes(e, planes == kPlanesInPayload ? edge_b : edge_a);
+        const uint32_t count = planes_of(dm);
+        lds = planes_lds_bytes(e, count);
+        p->cfg.lds_alone = std::max<uint32_t>(p->cfg.lds_alone, (planes_lds_bytes(e, count, plane_parts(e, count)) + 15u) & ~15u);
       } else if (!tensor_lines || !payload_lines) {
         const bool square = edge_a == transpose_edge(e) && edge_b == edge_a;
         BlockRule rule = block_rule(e, dm.ext_a, dm.ext_b, square, p->payload_bytes, tensor_lines, payload_lines);
@@ -811,7 +816,7 @@ struct Builder {
           lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
           walked = std::max(walked, transpose_group_rows(e) * transpose_lds_pitch(e) / kSkewGroup + 1u);
         }
-        p->cfg.lds_walked = std::max<uint32_t>(p->cfg.lds_walked, (walked + 15u) & ~15u);
+        p->cfg.lds_alone = std::max<uint32_t>(p->cfg.lds_alone, (walked + 15u) & ~15u);
       }
       p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
     } else if (run_bytes >= element_mode_limit(run_bytes)) {
@@ -969,6 +974,16 @@ bool streams_in_small_tiles(const axr_plan* p) {
          (p->payload_bytes >> 10) <= static_cast<uint64_t>(tn.max_tiles);
 }
 
+// Whether two wavefronts take every block of a bundle of planes alone: where all of them are better off so, and hold more
+// than the one round that a wavefront takes.
+bool in_halves(const axr_plan* p) {
+  for (const Dims& dm : p->dims) {
+    const uint32_t edge = dm.lanes_per_run == kPlanesInPayload ? dm.edge_a : dm.edge_b;
+    if (plane_parts(dm.granule, planes_of(dm)) != 2 || edge <= plane_round_elements(dm.granule)) return false;
+  }
+  return true;
+}
+
 // Launch geometry of a bundle of p->ntiles tiles in nseg segments: one tile per wave until
 // the grid would exceed max_waves, workgroup size, cache hints, and the size of the blocks of
 // the tile-block index (about one segment each, a power of two up to 256 tiles: a bundle of
@@ -1027,6 +1042,10 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
     while (2 * run * per_wg <= kBlockStrip * kBlockStrip) run *= 2;
   }
   p->cfg.xcd_remap = run ? remap_code(run, whole) : 0u;
+  if (p->cfg.kind == kModePlanes && tpw == 1 && !run && 2ull * p->ntiles <= max_waves && in_halves(p)) {
+    p->cfg.tiles_per_wave = kHalfTile;
+    p->cfg.workgroups = static_cast<uint32_t>((2ull * p->ntiles + waves_per_wg - 1) / waves_per_wg);
+  }
   if (run) p->cfg.workgroups = (p->cfg.workgroups + kXcds * run - 1) / (kXcds * run) * (kXcds * run);
   p->cfg.tile_rows = rows;
   if (tn.nontemporal < 0) {
@@ -1828,6 +1847,8 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
     // argument list (a 3.5 KiB argument costs 0.4 us per launch, the upload 4 us on the
     // host and 4 us on the device, once).
     if (!p->inline_ready) fill_inline_tables(p);
+    cfg = whole_tiles(cfg, p->ntiles);
+    a.tiles_per_wave = cfg.tiles_per_wave;
     rc = launch_bundle_kernel_inline(pack, a, cfg, *p->inline_tables,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
@@ -2377,7 +2398,9 @@ static int pack_noalloc_body(axr_plan_t* p, void* payload, size_t payload_bytes,
   };
   if (tables_fit_kernel_arguments(p)) {
     if (!p->inline_ready) fill_inline_tables(p);
-    rc = launch_bundle_kernel_inline(true, a, p->cfg, *p->inline_tables,
+    const LaunchConfig cfg = whole_tiles(p->cfg, p->ntiles);
+    a.tiles_per_wave = cfg.tiles_per_wave;
+    rc = launch_bundle_kernel_inline(true, a, cfg, *p->inline_tables,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
     if (rc) return rc;
@@ -2520,6 +2543,13 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     std::memset(&table, 0, sizeof(table));
     LaunchConfig cfg = first->cfg;
     cfg.nontemporal = effective_nontemporal(first, jobs[i].flags);
+    for (size_t k = i; k < end; ++k) {
+      cfg.elements = cfg.elements || jobs[k].plan->cfg.elements;
+      if (jobs[k].plan->cfg.kind != cfg.kind) cfg.kind = kKindAny;   // (also the kind of a plan without such views)
+    }
+    if (cfg.kind != kModeRows && cfg.kind != kModePlanes) cfg.kind = kKindAny;   // the kernels there are for several jobs
+    auto launched = [&](const axr_plan* p) { return cfg.kind == kModePlanes ? p->cfg : whole_tiles(p->cfg, p->ntiles); };
+    cfg.lds_per_wave = 0;
     uint32_t wg = 0;
     // The jobs of a call do not depend on each other, so their order inside the launch is free:
     // gathers take the first workgroups, scatters follow.  A scatter then mostly runs while the
@@ -2546,23 +2576,22 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       jd.wave_seg = reinterpret_cast<uint64_t>(d + p->wave_at);
       jd.payload = reinterpret_cast<uint64_t>(j.payload);
       jd.tensor_delta = j.tensor_delta;
+      const LaunchConfig own = launched(p);
       jd.ntiles = p->ntiles;
-      jd.tiles_per_wave = p->cfg.tiles_per_wave;
+      jd.tiles_per_wave = own.tiles_per_wave;
       jd.seg_shift = p->cfg.seg_shift;
       jd.wg_begin = wg;
       jd.unpack = j.unpack ? 1u : 0u;
-      if (static_cast<uint64_t>(wg) + p->cfg.workgroups > 0x7fffffffull)
+      if (static_cast<uint64_t>(wg) + own.workgroups > 0x7fffffffull)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: the jobs' grids exceed one launch");
-      wg += p->cfg.workgroups;
-      cfg.elements = cfg.elements || p->cfg.elements;
-      if (p->cfg.kind != cfg.kind) cfg.kind = kKindAny;   // (also the kind of a plan without such views)
-      cfg.lds_per_wave = std::max(cfg.lds_per_wave, p->cfg.lds_per_wave);
+      wg += own.workgroups;
+      cfg.lds_per_wave = std::max(cfg.lds_per_wave, own.tiles_per_wave == kHalfTile ? own.lds_alone : own.lds_per_wave);
     }
     table.count = static_cast<uint32_t>(end - i);
     for (uint32_t k = 0; k < kMaxJobs; ++k) table.begins[k] = k < table.count ? table.job[k].wg_begin : kNoJobBegin;
     const int64_t interleave = tunables().submit_interleave;
     if (interleave != 0 && (cfg.nontemporal & 2u) != 0 && end - i == 2 &&   // the streaming instantiations carry the code
-        jobs[i + 1].plan->cfg.workgroups == first->cfg.workgroups) {
+        launched(jobs[i + 1].plan).workgroups == launched(first).workgroups) {
       const uint64_t cache = static_cast<uint64_t>(tunables().payload_cache_bytes);
       const bool beyond_cache = first->payload_bytes > cache && jobs[i + 1].plan->payload_bytes > cache;
       table.interleaved = (beyond_cache || interleave > 1) ? 1u : 0u;
@@ -2576,7 +2605,6 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       if (cfg.threads > fit)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs whose views need different amounts of LDS");
     }
-    if (cfg.kind != kModeRows && cfg.kind != kModePlanes) cfg.kind = kKindAny;   // the kernels there are for several jobs
     int rc = launch_bundle_jobs(table, cfg, stream);
     if (rc) return rc;
     for (size_t k = i; k < end; ++k) {

@@ -109,6 +109,47 @@ static_assert(in_planes(1, 16) && !in_planes(1, 15) && in_planes(4, 201) && !in_
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
 
 
+def test_halves_of_plane_blocks_cover_them(tmp_path):
+    """Two wavefronts of a block move what one does: whole vectors from the front, in order, the last ones moved back to end
+    with the planes, a round each at most."""
+    source = r"""
+#include "axr_internal.h"
+using namespace axr;
+constexpr bool covered(uint32_t shift, uint32_t planes) {
+  const uint32_t e = 1u << shift, vec = kVecBytes / e, round = plane_round_elements(e);
+  if (plane_parts(e, planes) != 2 || plane_rounds(e, planes) != 2) return false;
+  for (uint32_t extent = vec; extent < 5 * round; ++extent) {
+    const uint32_t edge = plane_edge(e, planes, extent);
+    uint32_t end = 0;
+    for (uint32_t at = 0; at < extent; at += edge) {
+      const PlaneRange all = plane_range(shift, extent, edge, at, kWholeBlock);
+      if (all.count < vec || all.at > end || all.at + all.count < at + (extent - at < edge ? extent - at : edge)) return false;
+      for (uint32_t part = 0; part < 2; ++part) {
+        const PlaneRange r = plane_range(shift, extent, edge, at, part);
+        if (r.count == 0) {
+          if (part == 0 || all.at + all.count > at + round) return false;
+          continue;
+        }
+        if (r.count < vec || r.count > round || r.at > end || end - r.at >= vec) return false;
+        end = r.at + r.count;
+      }
+      if (end != all.at + all.count) return false;
+    }
+    if (end != extent) return false;
+  }
+  return true;
+}
+static_assert(covered(0, 3), "three planes of bytes");
+static_assert(covered(0, 4), "four planes of bytes");
+static_assert(covered(1, 3), "three planes of 2-byte elements");
+"""
+    src = str(tmp_path / "halves.cpp")
+    with open(src, "w") as f:
+        f.write(source)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=100000000", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
+
+
 def test_chunks_in_line(tmp_path):
     """On the side that was measured to be faster, for sizes where the two differ by more than 4 %."""
     turn = [(2, 2, 136), (2, 2, 148), (3, 3, 94), (3, 3, 105), (4, 4, 68), (4, 4, 84), (4, 2, 136), (6, 3, 84), (2, 2, 269),

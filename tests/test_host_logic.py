@@ -383,6 +383,27 @@ def test_wavefronts_of_a_launch(pkg):
         pkg.tune(max_waves=old.value)
 
 
+@pytest.mark.parametrize("code,bits,planes,block", [(1, 8, 3, 2048), (1, 8, 4, 2048), (4, 16, 3, 1024), (1, 8, 2, 2048), (4, 16, 4, 1024)])
+def test_blocks_of_planes_do_not_depend_on_their_neighbours(pkg, code, bits, planes, block):
+    """A bundle of planes alone gives two wavefronts to a block where that is faster (three planes, four of bytes; not below
+    a round of 16 bytes per lane); next to other tensors such a block is one wavefront's."""
+    images, item = 6, bits // 8
+    compact = tv(pkg, 0x10000000, [3000])
+
+    def shape(pixels, *others):
+        view = tv(pkg, 0x10000, [images, planes, pixels], strides=[planes * pixels, 1, planes], dtype=(code, bits, 1))
+        with pkg.BundlePlan.create([view, *others]) as plan:
+            info = plan.launch_info()
+            return plan.segments()[0]["tiles"], info["tiles"], info["workgroups"], info["threads_per_workgroup"] // 64
+    for pixels in (block // 4, block // 2, block // 2 + 1, 5 * block + 3, 50176):
+        want = images * -(-pixels // block)
+        tiles, alone, workgroups, waves = shape(pixels)
+        halves = planes != 2 and (planes, item) != (4, 2) and pixels > block // 2
+        assert (tiles, alone, workgroups) == (want, want, -(-want * (2 if halves else 1) // waves))
+        tiles, among, workgroups, waves = shape(pixels, compact)
+        assert (tiles, workgroups) == (want, -(-among // waves))
+
+
 def test_transposed_views_use_square_blocks(pkg):
     # fp16 [300, 200] transposed: B (contiguous in the tensor) = 300, A (packed inner) = 200
     segs, info = seg_of(pkg, tv(pkg, 0x10000, [300, 200], strides=[1, 300], dtype=(4, 16, 1)))

@@ -220,24 +220,47 @@ constexpr uint32_t kMinBlockBytes = 1024;   // smaller blocks than this are left
 constexpr uint32_t plane_rounds(uint32_t element_bytes, uint32_t planes) {
   return element_bytes < 4 || planes == 4 ? 2u : planes == 3 ? 3u : 4u;
 }
-// In the kernel of planes alone two wavefronts take a block together, a round each, where that leaves either of them 3 or
-// 4 KiB: more of them fit a compute unit's LDS and the last of them end closer together (pack + unpack, one wavefront to a
-// block / two: 256 images of 224 x 224 x 3 bytes 29.1 / 28.0 us, 128 of 190 x 201 x 3 20.1 / 17.1, 100 of 180 x 180 x 3 2-byte
-// elements 21.5 / 20.0, 200 of 224 x 224 x 4 bytes 30.0 / 29.2).  Not where it would leave them 2 KiB (300 of 210 x 200 x 2 bytes
-// 18.8 / 19.5), nor for four planes of 2-byte elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6), nor for
-// 4-byte elements, whose blocks are no whole rounds (in blocks of one round each 64 of 224 x 224 x 3 took 27.1 us instead of 31.1).
-// The kernel for any mode holds as many wavefronts either way and keeps whole blocks (next to 1 MiB of compact tensor, a
-// block to a wavefront / a round: 256 of 224 x 224 x 3 bytes 30.2 / 33.8, 150 of 180 x 180 x 3 2-byte elements 24.7 / 27.0).
-constexpr uint32_t plane_parts(uint32_t element_bytes, uint32_t planes) {
-  return element_bytes < 4 && (planes == 3 || (planes == 4 && element_bytes == 1)) ? 2u : 1u;
-}
 // The elements of every plane that lie in one round.
 constexpr uint32_t plane_round_elements(uint32_t element_bytes) { return kWaveLanes * kVecBytes / element_bytes; }
+// Planes whose blocks have a routine of one round as well, for blocks that hold no more.
+constexpr bool plane_single_round(uint32_t element_bytes, uint32_t planes) {
+  return element_bytes < 4 && (planes == 3 || (planes == 4 && element_bytes == 1));
+}
+// Whether planes are moved in blocks of one round: a wavefront has less to do and needs less LDS, more of them run at once and the
+// last of them end closer together, but there are twice as many, and twice as many ends of blocks that share a line (pack +
+// unpack, blocks of two rounds / of one, unless said otherwise as a share of the time with two).
+//  - Three planes of bytes alone, up to kShortBlocksMaxPayload: 256 images of 224 x 224 28.8 / 27.4 us, 3 MB 0.92 to 0.98,
+//    24 MB 0.92 to 1.02, 40 MB 0.96 to 1.04, four planes 0.88 to 0.97, 0.92 to 1.05, 0.96 to 1.03.  Beyond that planes of whole
+//    rounds only (300 MB of 50,176 x 3 204.6 / 199.4): 180 MB of 7501 x 3 151.1 / 157.9, 300 MB of 7501 x 4 222.9 / 252.9.
+//  - Three planes of 2-byte elements alone likewise (24 MB of 3563 26.0 / 24.9), and beyond that those of kShortBlocksLongPlane
+//    elements and more (180 MB of 7501 159.0 / 135.3, of 50,176 124.8 / 122.8, but 300 MB of 3000 227.0 / 234.2, of 809 packed and
+//    unpacked in one launch 201.6 / 243.5).
+//  - Next to other tensors, in the kernel for any mode, which holds 5 wavefronts on a SIMD whatever their LDS, where (nearly)
+//    all of them run at once: with 1 MiB of compact tensor 1 MB 0.84 to 0.97, 3 MB 0.85 to 0.96, 10 MB 0.89 to 1.03,
+//    16 MB of three planes 0.92 to 1.11, 256 images of 224 x 224 x 3 bytes 31.2 / 33.5.  Such long planes of 2-byte elements beyond
+//    kShortBlocksMinMixed again: 36 MB 0.89 to 0.97, 64 MB 0.90 to 0.99, 130 MB 0.92 to 0.98 (28 MB of 32,400 x 3 25.0 / 26.4).
+//  - Not where a round gives a wavefront 2 KiB (two planes: 300 of 210 x 200 bytes 18.8 / 19.5), nor for four planes of 2-byte
+//    elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6).  4-byte elements keep the 8 KiB of the other
+//    blocks with a short dimension (in one round 64 of 224 x 224 x 3 took 27.1 us instead of 31.1).
+constexpr uint64_t kShortBlocksMaxPayload = 48u << 20, kShortBlocksMixedRounds = 4096, kShortBlocksMinMixed = 28u << 20, kShortBlocksLongPlane = 4096;
+constexpr bool plane_short_blocks(uint32_t element_bytes, uint32_t planes, uint64_t extent, uint64_t payload_bytes, bool alone) {
+  if (!plane_single_round(element_bytes, planes)) return false;
+  const bool long_planes = element_bytes == 2 && extent >= kShortBlocksLongPlane;
+  if (!alone) return payload_bytes <= kShortBlocksMixedRounds * planes * kRowBytes || (long_planes && payload_bytes > kShortBlocksMinMixed);
+  return long_planes || payload_bytes <= kShortBlocksMaxPayload || extent % plane_round_elements(element_bytes) == 0;
+}
 constexpr uint32_t kMaxPlanes = 4;
-constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2;   // Dims.lanes_per_run of such a segment
+// Dims.lanes_per_run of such a segment: which side holds the planes, and above that the routine that moves its blocks.
+constexpr uint32_t kPlanesInPayload = 1, kPlanesInTensor = 2, kPlaneRoutineShift = 2;
+constexpr uint32_t plane_routine(uint32_t element_bytes, uint32_t planes, bool one_round) {
+  const uint32_t all = (element_bytes >> 1) * 3 + planes - 2;   // 0 to 8
+  return one_round ? 9 + (element_bytes == 2 ? 2 : planes - 3) : all;
+}
+static_assert(plane_routine(1, 2, false) == 0 && plane_routine(4, 4, false) == 8 && plane_routine(1, 3, true) == 9 &&
+                  plane_routine(2, 3, true) == 11, "one after the other");
 // LDS of a wavefront, one vector of padding behind every eight.
-constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes, uint32_t parts = 1) {
-  return plane_rounds(element_bytes, planes) / parts * kWaveLanes * planes * kVecBytes / 8 * 9;
+constexpr uint32_t planes_lds_bytes(uint32_t element_bytes, uint32_t planes, bool single) {
+  return (single ? 1u : plane_rounds(element_bytes, planes)) * kWaveLanes * planes * kVecBytes / 8 * 9;
 }
 // Whether planes of `extent` elements are moved like this.  Whole vectors of 4-byte elements that one
 // access per lane holds are not: rectangles take no second round for them (38 MB in three planes of 200
@@ -253,25 +276,6 @@ constexpr uint32_t plane_edge(uint32_t element_bytes, uint32_t planes, uint64_t 
   const uint32_t block = element_bytes < 4 ? plane_rounds(element_bytes, planes) * plane_round_elements(element_bytes)
                                            : (square < kRectMaxEdge ? square : kRectMaxEdge) / vec * vec;
   return extent < block ? static_cast<uint32_t>((extent + vec - 1) / vec * vec) : block;
-}
-// The elements (of 1 << element_shift bytes) of every plane that a wavefront moves: of the block of `edge` elements that begins at `at`, all or (part 0 or
-// 1) those of one round.  None where a part has nothing to move; otherwise a vector at least, moved back to end with
-// the planes where less is left of them.
-constexpr uint32_t kWholeBlock = 2;
-struct PlaneRange {
-  uint32_t at, count;
-};
-constexpr PlaneRange plane_range(uint32_t element_shift, uint32_t extent, uint32_t edge, uint32_t at, uint32_t part) {
-  uint32_t end = extent - at < edge ? extent : at + edge;
-  if (part != kWholeBlock) {
-    const uint32_t round = kWaveLanes * kVecBytes >> element_shift;
-    if (end - at <= part * round) return {at, 0};
-    at += part * round;
-    if (end - at > round) end = at + round;
-  }
-  const uint32_t least = kVecBytes >> element_shift;
-  if (extent - at < least) at = extent - least;
-  return {at, end - at};
 }
 constexpr uint32_t kMaxBatchDims = 4;
 constexpr uint32_t kMinElementTileBytes = 8192;   // element-mode work unit (measured: 8 KiB beats 2, 4 and 16)
@@ -362,7 +366,7 @@ struct Dims {             // 176 bytes, one per strided segment
   uint32_t lanes_per_run;          // kModeRows: the lane slots a run occupies (pstride[0] holds the
                                    // number of runs, edge_a the slots per lane);
                                    // kModePlanes: which side holds the planes (kPlanesInPayload,
-                                   // kPlanesInTensor)
+                                   // kPlanesInTensor), and plane_routine << kPlaneRoutineShift
   uint32_t nt_allowed;             // kModeElements, transposed: sides that may keep the launch's
                                    // non-temporal hint when packing (bit 0 tensor, bit 1 payload) and when
                                    // unpacking (bits 2, 3).  Transposed block rows that straddle 128-byte
@@ -385,7 +389,7 @@ struct KernelArgs {
   uint8_t* payload;
   uint32_t nseg;
   uint32_t ntiles;
-  uint32_t tiles_per_wave;    // or kHalfTile
+  uint32_t tiles_per_wave;
   uint32_t xcd_remap;         // 0, or remap_code of the workgroup indices a die takes in a row
   uint32_t seg_shift;         // log2 of the tile-block size of wave_seg
   int64_t tensor_delta = 0;   // added to every tensor-side address of the tables
@@ -423,12 +427,9 @@ struct alignas(16) InlineTables {
   uint8_t bytes[kInlineTableBytes];
 };
 
-// tiles_per_wave value: two wavefronts take a tile together, the kernel of planes alone only (see plane_parts).
-constexpr uint32_t kHalfTile = 0;
-
 struct LaunchConfig {
   uint32_t workgroups = 0;
-  uint32_t tiles_per_wave = 0;   // or kHalfTile (whole_tiles gives the launch in which it is one)
+  uint32_t tiles_per_wave = 0;
   uint32_t tile_rows = 2;
   uint32_t threads = 128;   // per workgroup, a multiple of 64
   uint32_t seg_shift = 0;   // wave_seg has one entry per 2^seg_shift tiles
@@ -436,20 +437,12 @@ struct LaunchConfig {
   bool elements = false;   // some segment's mode is above kModeRunTiles
   uint32_t kind = kKindAny;   // the mode of every segment where all have the same and one kernel is built for it
   uint32_t lds_per_wave = 0;   // bytes of LDS each wavefront needs (kModeRows and above)
-  uint32_t lds_alone = 0;      // in the kernel of walked blocks alone, and in that of planes alone with kHalfTile
+  uint32_t lds_walked = 0;     // and in the kernel of walked blocks alone
   uint32_t cached_tail = 0;    // MiB at the end of a streaming payload that a pack leaves in the cache (runs in
                            // 1 KiB tiles only; see finish_geometry)
   uint32_t xcd_remap = 0;  // 0, or remap_code of the workgroup indices each die takes in a row (the grid is a
                            // multiple of 8 such runs)
 };
-// A launch of `ntiles` tiles in another kernel than the plan's own.
-inline LaunchConfig whole_tiles(LaunchConfig cfg, uint32_t ntiles) {
-  if (cfg.tiles_per_wave != kHalfTile) return cfg;
-  const uint32_t waves = cfg.threads / kWaveLanes;
-  cfg.tiles_per_wave = 1;
-  cfg.workgroups = ntiles / waves + (ntiles % waves != 0);
-  return cfg;
-}
 
 // ---------------------------------------------------------------- tunables
 

@@ -974,7 +974,7 @@ __device__ __forceinline__ void interleaved_to_rows(gcbytes rd, gbytes wr, int64
 // pairs), 2 to 4 planes.  A lane owns 16 bytes of every plane: C vectors of the interleaved range,
 // regrouped in registers with byte permutes.  LDS only turns the lane's C neighbouring vectors
 // into wave-wide contiguous accesses.  Every access of the block to memory is in flight at once,
-// C KiB per round and R rounds (one, or plane_rounds).  What it replaces gathered every element from LDS by
+// C KiB per round and R rounds (one to plane_rounds).  What it replaces gathered every element from LDS by
 // itself, 16 byte reads per vector, with one or two vectors in flight: 256 images of 224 x 224 x 3
 // bytes 47 -> 32 us for pack + unpack, 4 channels 55 -> 40, 64 such fp32 images 36 -> 32 (plain copy
 // of the bytes: 25.5 us).
@@ -1100,32 +1100,29 @@ __device__ __forceinline__ void planes_block(gbytes inter, gbytes plane, int64_t
   __builtin_amdgcn_wave_barrier();
 }
 
-// `whole`: a block, otherwise a round of one that plane_parts wavefronts take together.
 template <bool TO_PLANES>
-__device__ __forceinline__ void planes_of(uint32_t E, uint32_t C, gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t count,
-                                          bool whole, lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
-#define AXR_ROUNDS(e, c, r) planes_block<e, c, TO_PLANES, r>(inter, plane, plane_pitch, count, lds, lane, nt_rd, nt_wr)
-#define AXR_PLANES(e, c) AXR_ROUNDS(e, c, plane_rounds(e, c))
-  if (!whole) {
-    static_assert(plane_parts(1, 3) == 2 && plane_parts(1, 4) == 2 && plane_parts(2, 3) == 2, "blocks in two parts");
-    if (E == 2) AXR_ROUNDS(2, 3, 1);
-    else if (C == 3) AXR_ROUNDS(1, 3, 1);
-    else AXR_ROUNDS(1, 4, 1);
-    return;
-  }
-  switch (E << 4 | C) {
-    case 0x12: AXR_PLANES(1, 2); break;
-    case 0x13: AXR_PLANES(1, 3); break;
-    case 0x14: AXR_PLANES(1, 4); break;
-    case 0x22: AXR_PLANES(2, 2); break;
-    case 0x23: AXR_PLANES(2, 3); break;
-    case 0x24: AXR_PLANES(2, 4); break;
-    case 0x42: AXR_PLANES(4, 2); break;
-    case 0x43: AXR_PLANES(4, 3); break;
-    default: AXR_PLANES(4, 4); break;
+__device__ __forceinline__ void planes_of(uint32_t routine, gbytes inter, gbytes plane, int64_t plane_pitch, uint32_t count,
+                                          lbytes lds, uint32_t lane, bool nt_rd, bool nt_wr) {
+#define AXR_PLANES(e, c) \
+  case plane_routine(e, c, false): planes_block<e, c, TO_PLANES, plane_rounds(e, c)>(inter, plane, plane_pitch, count, lds, lane, nt_rd, nt_wr); break
+#define AXR_ONE_ROUND(e, c) \
+  case plane_routine(e, c, true): planes_block<e, c, TO_PLANES, 1>(inter, plane, plane_pitch, count, lds, lane, nt_rd, nt_wr); break
+  switch (routine) {
+    AXR_PLANES(1, 2);
+    AXR_PLANES(1, 3);
+    AXR_PLANES(1, 4);
+    AXR_PLANES(2, 2);
+    AXR_PLANES(2, 3);
+    AXR_PLANES(2, 4);
+    AXR_PLANES(4, 2);
+    AXR_PLANES(4, 3);
+    AXR_PLANES(4, 4);
+    AXR_ONE_ROUND(1, 3);
+    AXR_ONE_ROUND(1, 4);
+    AXR_ONE_ROUND(2, 3);
   }
 #undef AXR_PLANES
-#undef AXR_ROUNDS
+#undef AXR_ONE_ROUND
 }
 
 // Reads nr rows of nc elements (rows rd_pitch bytes apart) and writes nc rows of
@@ -1171,12 +1168,11 @@ __device__ __forceinline__ void transpose_block(uint32_t E, gcbytes rd, int64_t 
 // One copy per MODE: with the walk in strips and the choice of block routine in
 // the plain one's way, however predictable, 4 KiB blocks took 3 to 8 % longer.
 // GROUP: the wavefronts of a workgroup take kSkewGroup tiles that follow each other, and skewed blocks together;
-// `lds_group` is their LDS.  `part`: of a block of planes, see plane_range.
+// `lds_group` is their LDS.
 template <bool PACK, uint32_t MODE, bool GROUP = false>
 __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, gbytes pay,
                                                uint32_t q, lbytes lds, uint32_t lane,
-                                               uint32_t nt_bits, lbytes lds_group = nullptr,
-                                               uint32_t part = kWholeBlock) {
+                                               uint32_t nt_bits, lbytes lds_group = nullptr) {
   const uint32_t E = dm->granule;
   const uint32_t es = static_cast<uint32_t>(__builtin_ctz(E));
   const uint32_t T = transpose_edge(E);
@@ -1238,20 +1234,23 @@ __device__ __forceinline__ void transpose_tile(uint64_t seg_ptr, dims_table dm, 
     }
   }
   if constexpr (MODE == kModePlanes) {
-    // Few planes <-> interleaved: the short dimension is taken whole.
-    const bool payload_planes = dm->lanes_per_run == kPlanesInPayload;   // the long dimension is A, else B
+    // Few planes <-> interleaved: the short dimension is taken whole.  What is left of the long one
+    // may be less than a vector: the block is then moved back to hold one.
+    const uint32_t planes = dm->lanes_per_run;
+    const bool payload_planes = (planes & kPlanesInPayload) != 0;   // the long dimension is A, else B
     const uint32_t ext = payload_planes ? dm->ext_a : dm->ext_b, edge = payload_planes ? edge_a : edge_b;
-    const PlaneRange range = plane_range(es, ext, edge, payload_planes ? a0 : b0, part);
-    const uint32_t n0 = range.at, count = range.count;
-    if (count == 0) return;
+    const uint32_t least = kVecBytes / E;
+    uint32_t n0 = payload_planes ? a0 : b0;
+    n0 = ext - n0 < least ? ext - least : n0;
+    const uint32_t count = ext - n0 < edge ? ext - n0 : edge;
     const uint32_t C = payload_planes ? edge_b : edge_a;
     const uint64_t inter_at = static_cast<uint64_t>(n0) * C << es, plane_at = static_cast<uint64_t>(n0) << es;
     gbytes ten = as_global(seg_ptr) + toff, pp = pay + poff;
     const bool nt_rd = (nt_bits & (PACK ? 1u : 2u)) != 0, nt_wr = (nt_bits & (PACK ? 2u : 1u)) != 0;
     if (payload_planes)
-      planes_of<PACK>(E, C, ten + inter_at, pp + plane_at, static_cast<int64_t>(dm->pstride_b), count, part == kWholeBlock, lds, lane, nt_rd, nt_wr);
+      planes_of<PACK>(planes >> kPlaneRoutineShift, ten + inter_at, pp + plane_at, static_cast<int64_t>(dm->pstride_b), count, lds, lane, nt_rd, nt_wr);
     else
-      planes_of<!PACK>(E, C, pp + inter_at, ten + plane_at, dm->stride_a, count, part == kWholeBlock, lds, lane, nt_rd, nt_wr);
+      planes_of<!PACK>(planes >> kPlaneRoutineShift, pp + inter_at, ten + plane_at, dm->stride_a, count, lds, lane, nt_rd, nt_wr);
     return;
   }
   if (MODE == kModeWalked && (allowed & (PACK ? kSkewPack : kSkewUnpack)) != 0) {
@@ -1533,12 +1532,10 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
   const uint32_t waves_per_wg = nt_bits >> 8;
   nt_bits &= 3u;
   const uint32_t wave = uniform(wg * waves_per_wg + (threadIdx.x >> 6));
-  const bool halves = KIND == kModePlanes && a.tiles_per_wave == kHalfTile;
-  const uint32_t tiles_per_wave = halves ? 1u : a.tiles_per_wave, part = halves ? wave & 1u : kWholeBlock;
-  uint32_t t = halves ? wave >> 1 : wave * tiles_per_wave;
+  uint32_t t = wave * a.tiles_per_wave;
   if (t >= a.ntiles) return;
   const uint32_t t_end =
-      (a.ntiles - t > tiles_per_wave) ? t + tiles_per_wave : a.ntiles;
+      (a.ntiles - t > a.tiles_per_wave) ? t + a.tiles_per_wave : a.ntiles;
   const uint64_t delta = static_cast<uint64_t>(a.tensor_delta);
   // a whole tile or what is left of a run, at `ten` in the tensor and at `pay` in the payload
   auto copy = [&](gbytes ten, gbytes pay, uint64_t left) {
@@ -1652,7 +1649,7 @@ __device__ __forceinline__ void bundle_body(seg_table segs, dims_table dims,
         else if (mode == kModeRows) rows_tile<PACK>(seg_ptr, static_cast<uint32_t>(seg_run), dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeTranspose) transpose_tile<PACK, kModeTranspose>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
         else if (mode == kModeWalked) transpose_tile<PACK, kModeWalked, KIND == kModeWalked>(seg_ptr, dm, pay, q, lds, lane, nt_bits, (lbytes)lds_slices);
-        else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits, nullptr, part);
+        else transpose_tile<PACK, kModePlanes>(seg_ptr, dm, pay, q, lds, lane, nt_bits);
       }
       if constexpr (PACK) {
         if (last && pad) wave_zero(pay + dm->nbytes, pad, lane);
@@ -1731,7 +1728,7 @@ __device__ __forceinline__ uint32_t at_or_beyond(uint32_t wg, uint32_t begin) {
 // the job table: leading scalar arguments are preloaded into scalar registers when a wavefront
 // starts, a struct passed by value is not (and the kernel-argument segment is slow memory).
 // `head` = job count (bits 0-7), the in-turn flag (bit 8), the directions of jobs 0 and 1 (bits
-// 9, 10: 1 = unpack), "jobs 0 and 1 give every wavefront one tile, or half of one" (bit 11; bits 12, 13: half) and their tile-block
+// 9, 10: 1 = unpack), "jobs 0 and 1 give every wavefront one tile" (bit 11) and their tile-block
 // shifts (bits 16-23, 24-31); then the hints, the first workgroup of job 1 and, for jobs 0 and 1,
 // the tile count and the addresses of the tile-block index and of the segment records.  A
 // workgroup of a launch of one or two jobs (a pack and an unpack handed over together) finds its
@@ -1775,7 +1772,7 @@ __launch_bounds__(KIND == kKindRuns ? kMaxThreadsPerWorkgroup : kMaxElementThrea
     wave_seg = reinterpret_cast<const AXR_CONST uint32_t*>(j ? index1 : index0);
     segs = reinterpret_cast<seg_table>(j ? segs1 : segs0);
     a.ntiles = j ? ntiles1 : ntiles0;
-    a.tiles_per_wave = KIND == kModePlanes && ((head >> (12u + j)) & 1u) != 0 ? kHalfTile : 1u;
+    a.tiles_per_wave = 1;
     a.seg_shift = (head >> (16u + 8u * j)) & 0xffu;
     unpack = (head >> (9u + j)) & 1u;
     begin = j ? b1 : 0u;
@@ -2154,7 +2151,7 @@ int launch_rows(const KernelArgs& args, const LaunchConfig& cfg, hipStream_t str
   const bool walked = ROWS == 2 && cfg.elements && cfg.kind == kModeWalked;   // (that kernel's workgroups are groups)
   if (walked && (cfg.threads != kSkewGroup * kWaveLanes || cfg.tiles_per_wave != 1))
     return fail(AXR_ERR_INVALID, "walked blocks need workgroups of four wavefronts with a tile each");
-  const uint32_t lds_per_wave = walked || cfg.tiles_per_wave == kHalfTile ? cfg.lds_alone : cfg.lds_per_wave;
+  const uint32_t lds_per_wave = walked ? cfg.lds_walked : cfg.lds_per_wave;
   const uint32_t lds_bytes = cfg.elements ? lds_per_wave * (cfg.threads / kWaveLanes) : 0u;
   const uint32_t low = cfg.elements ? lds_per_wave : cfg.cached_tail;
   if (low > 0x1ffffu || args.seg_shift > 0xffu || cfg.threads / kWaveLanes > 0x1fu)
@@ -2223,15 +2220,11 @@ int launch_bundle_kernel(bool pack, const KernelArgs& args, const LaunchConfig& 
     return fail(AXR_ERR_INVALID, "die remapping needs a grid of whole rounds over the dies");
   if (cfg.elements && cfg.threads > kMaxElementThreads)
     return fail(AXR_ERR_INVALID, "bundles with short strided runs need workgroups of at most 256");
-  const bool halves = cfg.tiles_per_wave == kHalfTile;
-  if (halves && (!cfg.elements || cfg.kind != kModePlanes || cfg.tile_rows != 2))
-    return fail(AXR_ERR_INVALID, "half a tile to a wavefront goes with planes alone");
-  const bool alone = halves || (cfg.elements && cfg.kind == kModeWalked && cfg.tile_rows == 2);
-  const uint32_t lds_per_wave = alone ? cfg.lds_alone : cfg.lds_per_wave;
+  const uint32_t lds_per_wave = cfg.elements && cfg.kind == kModeWalked && cfg.tile_rows == 2 ? cfg.lds_walked : cfg.lds_per_wave;
   if (static_cast<uint64_t>(lds_per_wave) * (cfg.threads / kWaveLanes) > 64u * 1024u)
     return fail(AXR_ERR_INVALID, "workgroup needs more than 64 KiB of LDS");
-  const uint64_t waves = static_cast<uint64_t>(cfg.workgroups) * (cfg.threads / kWaveLanes);
-  const uint64_t covered = halves ? waves / 2 : waves * cfg.tiles_per_wave;
+  const uint64_t covered = static_cast<uint64_t>(cfg.workgroups) * (cfg.threads / kWaveLanes) *
+                           cfg.tiles_per_wave;
   if (covered < args.ntiles || args.tiles_per_wave != cfg.tiles_per_wave) {
     return fail(AXR_ERR_INVALID, "launch geometry does not cover the tile range");
   }
@@ -2253,11 +2246,7 @@ int launch_bundle_jobs(const JobTable& jobs, const LaunchConfig& cfg, void* stre
     const uint32_t end = k + 1 < jobs.count ? jobs.job[k + 1].wg_begin : cfg.workgroups;
     if (d.wg_begin > end || (k == 0 && d.wg_begin != 0))
       return fail(AXR_ERR_INVALID, "job workgroup ranges are not consecutive");
-    const bool halves = d.tiles_per_wave == kHalfTile;
-    if (halves && (!cfg.elements || cfg.kind != kModePlanes))
-      return fail(AXR_ERR_INVALID, "half a tile to a wavefront goes with planes alone");
-    const uint64_t waves = static_cast<uint64_t>(end - d.wg_begin) * waves_per_wg;
-    const uint64_t covered = halves ? waves / 2 : waves * d.tiles_per_wave;
+    const uint64_t covered = static_cast<uint64_t>(end - d.wg_begin) * waves_per_wg * d.tiles_per_wave;
     if (covered < d.ntiles) return fail(AXR_ERR_INVALID, "launch geometry does not cover a job's tiles");
   }
   const dim3 grid(cfg.workgroups), block(cfg.threads);
@@ -2265,12 +2254,11 @@ int launch_bundle_jobs(const JobTable& jobs, const LaunchConfig& cfg, void* stre
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (uint32_t k = 0; k < 2 && k < jobs.count; ++k)
     if (jobs.job[k].seg_shift > 0xffu) return fail(AXR_ERR_INVALID, "tile-block shift does not fit the job head");
-  // count, in-turn flag, directions, one tile or half of one per wavefront and tile-block shifts of jobs 0 and 1
-  const bool one_tile_each = jobs.job[0].tiles_per_wave <= 1 && (jobs.count < 2 || jobs.job[1].tiles_per_wave <= 1);
+  // count, in-turn flag, directions, one tile per wavefront and tile-block shifts of jobs 0 and 1
+  const bool one_tile_each = jobs.job[0].tiles_per_wave == 1 && (jobs.count < 2 || jobs.job[1].tiles_per_wave == 1);
   const uint32_t head = (jobs.count & 0xffu) | (jobs.interleaved ? 0x100u : 0u) |
                         (jobs.job[0].unpack ? 0x200u : 0u) | (jobs.count > 1 && jobs.job[1].unpack ? 0x400u : 0u) |
-                        (one_tile_each ? 0x800u : 0u) | (jobs.job[0].tiles_per_wave == kHalfTile ? 0x1000u : 0u) |
-                        (jobs.count > 1 && jobs.job[1].tiles_per_wave == kHalfTile ? 0x2000u : 0u) |
+                        (one_tile_each ? 0x800u : 0u) |
                         (jobs.job[0].seg_shift & 0xffu) << 16 | (jobs.count > 1 ? jobs.job[1].seg_shift & 0xffu : 0u) << 24;
 #define AXR_JOBS(ROWS, NTT, NTP, KIND) \
   hipLaunchKernelGGL((bundle_jobs_kernel<ROWS, NTT, NTP, KIND>), grid, block, lds_bytes, s, head, jobs.nt_bits, \
@@ -2310,7 +2298,6 @@ int launch_bundle_kernel_inline(bool pack, const KernelArgs& args, const LaunchC
                                 const InlineTables& tables, uint32_t dims_at, uint32_t wave_at,
                                 void* stream) {
   if (args.ntiles == 0 || cfg.workgroups == 0) return AXR_OK;
-  if (cfg.tiles_per_wave == kHalfTile) return fail(AXR_ERR_INVALID, "half a tile to a wavefront goes with planes alone");
   const bool streaming = cfg.tile_rows == 1 && (cfg.nontemporal & 3u) == 3u && !cfg.elements;
   if ((!streaming && (cfg.tile_rows != 2 || (cfg.nontemporal & 3u) != 1u)) || args.xcd_remap)
     return fail(AXR_ERR_INVALID, "inline tables go with two launch geometries only");

@@ -398,7 +398,7 @@ void invalidate_tables(axr_plan* p) {
   p->shared_line_tiles = 0;
   p->strip_tiles = 0;
   p->whole_groups = false;
-  p->cfg.lds_per_wave = p->cfg.lds_alone = 0;
+  p->cfg.lds_per_wave = p->cfg.lds_walked = 0;
 }
 
 // Wait until the device no longer reads the plan's tables.  No event is
@@ -535,8 +535,9 @@ uint64_t element_mode_limit(uint64_t run_bytes) {
   return (limit + 4) / 5;
 }
 
-// How many planes a segment of planes has.
-uint32_t planes_of(const Dims& dm) { return dm.lanes_per_run == kPlanesInPayload ? dm.edge_b : dm.edge_a; }
+// How many planes a segment of planes has, and their elements.
+uint32_t planes_of(const Dims& dm) { return dm.lanes_per_run & kPlanesInPayload ? dm.edge_b : dm.edge_a; }
+uint32_t plane_extent(const Dims& dm) { return dm.lanes_per_run & kPlanesInPayload ? dm.ext_a : dm.ext_b; }
 
 struct Builder {
   axr_plan* p;
@@ -793,9 +794,9 @@ struct Builder {
       dm.tiles_per_run = 1;
       if (planes) {
         dm.mode = kModePlanes;
-        const uint32_t count = planes_of(dm);
-        lds = planes_lds_bytes(e, count);
-        p->cfg.lds_alone = std::max<uint32_t>(p->cfg.lds_alone, (planes_lds_bytes(e, count, plane_parts(e, count)) + 15u) & ~15u);
+        const bool single = plane_single_round(e, planes_of(dm)) && plane_extent(dm) <= plane_round_elements(e);
+        dm.lanes_per_run |= plane_routine(e, planes_of(dm), single) << kPlaneRoutineShift;
+        lds = planes_lds_bytes(e, planes_of(dm), single);
       } else if (!tensor_lines || !payload_lines) {
         const bool square = edge_a == transpose_edge(e) && edge_b == edge_a;
         BlockRule rule = block_rule(e, dm.ext_a, dm.ext_b, square, p->payload_bytes, tensor_lines, payload_lines);
@@ -816,7 +817,7 @@ struct Builder {
           lds = std::max(lds, transpose_skew_rows(e) * transpose_lds_pitch(e));
           walked = std::max(walked, transpose_group_rows(e) * transpose_lds_pitch(e) / kSkewGroup + 1u);
         }
-        p->cfg.lds_alone = std::max<uint32_t>(p->cfg.lds_alone, (walked + 15u) & ~15u);
+        p->cfg.lds_walked = std::max<uint32_t>(p->cfg.lds_walked, (walked + 15u) & ~15u);
       }
       p->cfg.lds_per_wave = std::max<uint32_t>(p->cfg.lds_per_wave, (lds + 15u) & ~15u);
     } else if (run_bytes >= element_mode_limit(run_bytes)) {
@@ -892,6 +893,52 @@ struct Builder {
       }
       sg.tile_begin = static_cast<uint32_t>(tiles);
       tiles += ntile;
+    }
+  }
+
+  // Blocks of planes that are better off with one round than with two: which depends on the bundle, and is known once every
+  // tensor has been seen.
+  void settle_planes() {
+    bool alone = tile_bytes == 2 * kRowBytes, any = false;
+    for (const Dims& dm : p->dims) (dm.mode == kModePlanes ? any : alone) = dm.mode == kModePlanes;
+    if (!any) return;
+    for (const Seg& sg : p->segs) alone = alone && (sg.meta >> kSegDimsShift) != 0 && (sg.meta >> kSegDimsShift) < kSegGroup;
+    std::vector<uint64_t> tiles_of(p->dims.size(), 0);   // of the segments whose blocks become shorter
+    uint32_t lds = 0;
+    for (size_t i = 0; i < p->dims.size(); ++i) {
+      const Dims& dm = p->dims[i];
+      if (dm.mode != kModePlanes) continue;
+      const uint32_t round = plane_round_elements(dm.granule), edge = dm.lanes_per_run & kPlanesInPayload ? dm.edge_a : dm.edge_b;
+      const bool one = plane_short_blocks(dm.granule, planes_of(dm), plane_extent(dm), p->payload_bytes, alone);
+      if (one && edge > round) {
+        tiles_of[i] = (plane_extent(dm) + round - 1) / round;
+        for (uint32_t d = kMaxOuterDims - kMaxBatchDims; d < kMaxOuterDims; ++d) tiles_of[i] *= dm.shape[d];
+      }
+      lds = std::max(lds, planes_lds_bytes(dm.granule, planes_of(dm), one || (plane_single_round(dm.granule, planes_of(dm)) && edge <= round)));
+    }
+    const uint64_t end = tiles;
+    uint64_t at = 0;
+    std::vector<uint32_t> begins(p->segs.size());
+    for (size_t i = 0; i < p->segs.size(); ++i) {
+      const Seg& sg = p->segs[i];
+      const uint32_t dsel = sg.meta >> kSegDimsShift;
+      const uint64_t shorter = dsel != 0 && dsel < kSegGroup ? tiles_of[dsel - 1] : 0;
+      begins[i] = static_cast<uint32_t>(at);
+      at += shorter ? shorter : (i + 1 < p->segs.size() ? p->segs[i + 1].tile_begin : end) - sg.tile_begin;
+    }
+    if (at > 0xffffffffull) return;
+    tiles = at;
+    for (size_t i = 0; i < p->segs.size(); ++i) p->segs[i].tile_begin = begins[i];
+    if (alone) p->cfg.lds_per_wave = (lds + 15u) & ~15u;
+    for (size_t i = 0; i < p->dims.size(); ++i) {
+      if (tiles_of[i] == 0) continue;
+      Dims& dm = p->dims[i];
+      const bool along_a = (dm.lanes_per_run & kPlanesInPayload) != 0;
+      const uint32_t edge = plane_round_elements(dm.granule);
+      (along_a ? dm.edge_a : dm.edge_b) = edge;
+      (along_a ? dm.tiles_a : dm.tiles_b) = (plane_extent(dm) + edge - 1) / edge;
+      const uint32_t side = dm.lanes_per_run & (kPlanesInPayload | kPlanesInTensor);
+      dm.lanes_per_run = side | plane_routine(dm.granule, planes_of(dm), true) << kPlaneRoutineShift;
     }
   }
 
@@ -974,16 +1021,6 @@ bool streams_in_small_tiles(const axr_plan* p) {
          (p->payload_bytes >> 10) <= static_cast<uint64_t>(tn.max_tiles);
 }
 
-// Whether two wavefronts take every block of a bundle of planes alone: where all of them are better off so, and hold more
-// than the one round that a wavefront takes.
-bool in_halves(const axr_plan* p) {
-  for (const Dims& dm : p->dims) {
-    const uint32_t edge = dm.lanes_per_run == kPlanesInPayload ? dm.edge_a : dm.edge_b;
-    if (plane_parts(dm.granule, planes_of(dm)) != 2 || edge <= plane_round_elements(dm.granule)) return false;
-  }
-  return true;
-}
-
 // Launch geometry of a bundle of p->ntiles tiles in nseg segments: one tile per wave until
 // the grid would exceed max_waves, workgroup size, cache hints, and the size of the blocks of
 // the tile-block index (about one segment each, a power of two up to 256 tiles: a bundle of
@@ -1042,10 +1079,6 @@ void finish_geometry(axr_plan* p, uint32_t rows, size_t nseg, bool may_be_direct
     while (2 * run * per_wg <= kBlockStrip * kBlockStrip) run *= 2;
   }
   p->cfg.xcd_remap = run ? remap_code(run, whole) : 0u;
-  if (p->cfg.kind == kModePlanes && tpw == 1 && !run && 2ull * p->ntiles <= max_waves && in_halves(p)) {
-    p->cfg.tiles_per_wave = kHalfTile;
-    p->cfg.workgroups = static_cast<uint32_t>((2ull * p->ntiles + waves_per_wg - 1) / waves_per_wg);
-  }
   if (run) p->cfg.workgroups = (p->cfg.workgroups + kXcds * run - 1) / (kXcds * run) * (kXcds * run);
   p->cfg.tile_rows = rows;
   if (tn.nontemporal < 0) {
@@ -1430,6 +1463,7 @@ int build_tables(axr_plan* p) {
     if (rc) return rc;
   }
   b.settle_rows();
+  b.settle_planes();
   b.settle_walked();
   p->whole_groups = b.whole_groups;
   // Group neighbouring host pieces (in payload order, at most an alignment gap
@@ -1847,8 +1881,6 @@ int run(axr_plan* p, bool pack, void* payload, size_t payload_bytes, void* strea
     // argument list (a 3.5 KiB argument costs 0.4 us per launch, the upload 4 us on the
     // host and 4 us on the device, once).
     if (!p->inline_ready) fill_inline_tables(p);
-    cfg = whole_tiles(cfg, p->ntiles);
-    a.tiles_per_wave = cfg.tiles_per_wave;
     rc = launch_bundle_kernel_inline(pack, a, cfg, *p->inline_tables,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
@@ -2398,9 +2430,7 @@ static int pack_noalloc_body(axr_plan_t* p, void* payload, size_t payload_bytes,
   };
   if (tables_fit_kernel_arguments(p)) {
     if (!p->inline_ready) fill_inline_tables(p);
-    const LaunchConfig cfg = whole_tiles(p->cfg, p->ntiles);
-    a.tiles_per_wave = cfg.tiles_per_wave;
-    rc = launch_bundle_kernel_inline(true, a, cfg, *p->inline_tables,
+    rc = launch_bundle_kernel_inline(true, a, p->cfg, *p->inline_tables,
                                      static_cast<uint32_t>(dims_arg_at(p)),
                                      static_cast<uint32_t>(p->wave_at), stream);
     if (rc) return rc;
@@ -2543,13 +2573,6 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
     std::memset(&table, 0, sizeof(table));
     LaunchConfig cfg = first->cfg;
     cfg.nontemporal = effective_nontemporal(first, jobs[i].flags);
-    for (size_t k = i; k < end; ++k) {
-      cfg.elements = cfg.elements || jobs[k].plan->cfg.elements;
-      if (jobs[k].plan->cfg.kind != cfg.kind) cfg.kind = kKindAny;   // (also the kind of a plan without such views)
-    }
-    if (cfg.kind != kModeRows && cfg.kind != kModePlanes) cfg.kind = kKindAny;   // the kernels there are for several jobs
-    auto launched = [&](const axr_plan* p) { return cfg.kind == kModePlanes ? p->cfg : whole_tiles(p->cfg, p->ntiles); };
-    cfg.lds_per_wave = 0;
     uint32_t wg = 0;
     // The jobs of a call do not depend on each other, so their order inside the launch is free:
     // gathers take the first workgroups, scatters follow.  A scatter then mostly runs while the
@@ -2576,22 +2599,23 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       jd.wave_seg = reinterpret_cast<uint64_t>(d + p->wave_at);
       jd.payload = reinterpret_cast<uint64_t>(j.payload);
       jd.tensor_delta = j.tensor_delta;
-      const LaunchConfig own = launched(p);
       jd.ntiles = p->ntiles;
-      jd.tiles_per_wave = own.tiles_per_wave;
+      jd.tiles_per_wave = p->cfg.tiles_per_wave;
       jd.seg_shift = p->cfg.seg_shift;
       jd.wg_begin = wg;
       jd.unpack = j.unpack ? 1u : 0u;
-      if (static_cast<uint64_t>(wg) + own.workgroups > 0x7fffffffull)
+      if (static_cast<uint64_t>(wg) + p->cfg.workgroups > 0x7fffffffull)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: the jobs' grids exceed one launch");
-      wg += own.workgroups;
-      cfg.lds_per_wave = std::max(cfg.lds_per_wave, own.tiles_per_wave == kHalfTile ? own.lds_alone : own.lds_per_wave);
+      wg += p->cfg.workgroups;
+      cfg.elements = cfg.elements || p->cfg.elements;
+      if (p->cfg.kind != cfg.kind) cfg.kind = kKindAny;   // (also the kind of a plan without such views)
+      cfg.lds_per_wave = std::max(cfg.lds_per_wave, p->cfg.lds_per_wave);
     }
     table.count = static_cast<uint32_t>(end - i);
     for (uint32_t k = 0; k < kMaxJobs; ++k) table.begins[k] = k < table.count ? table.job[k].wg_begin : kNoJobBegin;
     const int64_t interleave = tunables().submit_interleave;
     if (interleave != 0 && (cfg.nontemporal & 2u) != 0 && end - i == 2 &&   // the streaming instantiations carry the code
-        launched(jobs[i + 1].plan).workgroups == launched(first).workgroups) {
+        jobs[i + 1].plan->cfg.workgroups == first->cfg.workgroups) {
       const uint64_t cache = static_cast<uint64_t>(tunables().payload_cache_bytes);
       const bool beyond_cache = first->payload_bytes > cache && jobs[i + 1].plan->payload_bytes > cache;
       table.interleaved = (beyond_cache || interleave > 1) ? 1u : 0u;
@@ -2605,6 +2629,7 @@ static int submit_body(const axr_job_t* jobs, size_t n, void* stream_) {
       if (cfg.threads > fit)
         return fail(AXR_ERR_UNSUPPORTED, "axr_submit: jobs whose views need different amounts of LDS");
     }
+    if (cfg.kind != kModeRows && cfg.kind != kModePlanes) cfg.kind = kKindAny;   // the kernels there are for several jobs
     int rc = launch_bundle_jobs(table, cfg, stream);
     if (rc) return rc;
     for (size_t k = i; k < end; ++k) {

@@ -109,44 +109,19 @@ static_assert(in_planes(1, 16) && !in_planes(1, 15) && in_planes(4, 201) && !in_
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
 
 
-def test_halves_of_plane_blocks_cover_them(tmp_path):
-    """Two wavefronts of a block move what one does: whole vectors from the front, in order, the last ones moved back to end
-    with the planes, a round each at most."""
-    source = r"""
-#include "axr_internal.h"
-using namespace axr;
-constexpr bool covered(uint32_t shift, uint32_t planes) {
-  const uint32_t e = 1u << shift, vec = kVecBytes / e, round = plane_round_elements(e);
-  if (plane_parts(e, planes) != 2 || plane_rounds(e, planes) != 2) return false;
-  for (uint32_t extent = vec; extent < 5 * round; ++extent) {
-    const uint32_t edge = plane_edge(e, planes, extent);
-    uint32_t end = 0;
-    for (uint32_t at = 0; at < extent; at += edge) {
-      const PlaneRange all = plane_range(shift, extent, edge, at, kWholeBlock);
-      if (all.count < vec || all.at > end || all.at + all.count < at + (extent - at < edge ? extent - at : edge)) return false;
-      for (uint32_t part = 0; part < 2; ++part) {
-        const PlaneRange r = plane_range(shift, extent, edge, at, part);
-        if (r.count == 0) {
-          if (part == 0 || all.at + all.count > at + round) return false;
-          continue;
-        }
-        if (r.count < vec || r.count > round || r.at > end || end - r.at >= vec) return false;
-        end = r.at + r.count;
-      }
-      if (end != all.at + all.count) return false;
-    }
-    if (end != extent) return false;
-  }
-  return true;
-}
-static_assert(covered(0, 3), "three planes of bytes");
-static_assert(covered(0, 4), "four planes of bytes");
-static_assert(covered(1, 3), "three planes of 2-byte elements");
-"""
-    src = str(tmp_path / "halves.cpp")
+def test_short_blocks_of_planes(tmp_path):
+    """In blocks of one round on the side that was measured to be faster: (element bytes, planes, elements of a plane, MB, alone)."""
+    short = [(1, 3, 50176, 37, 1), (1, 3, 7501, 24, 1), (1, 4, 30011, 40, 1), (1, 4, 3072, 256, 1), (1, 3, 50176, 300, 1), (2, 3, 7501, 180, 1),
+             (2, 3, 3563, 24, 1), (1, 3, 50176, 9, 0), (1, 4, 7501, 10, 0), (2, 3, 32400, 4, 0), (2, 3, 7501, 36, 0), (2, 3, 7501, 130, 0)]
+    two = [(1, 3, 7501, 180, 1), (1, 4, 7501, 300, 1), (1, 4, 50000, 64, 1), (1, 2, 42000, 25, 1), (2, 4, 16256, 17, 1), (2, 2, 40000, 10, 1),
+           (4, 3, 50176, 38, 1), (1, 3, 50176, 38, 0), (1, 3, 38190, 15, 0), (1, 4, 50176, 40, 0), (2, 3, 32400, 19, 0), (2, 3, 32400, 28, 0), (2, 2, 3000, 2, 0),
+           (2, 3, 3000, 300, 1), (2, 3, 809, 298, 1), (2, 3, 3000, 36, 0)]
+    checks = "".join(f"static_assert({no}plane_short_blocks({e}, {c}, {n}, {mb}000000ull, {alone}), \"{e} {c} {n} {mb} {alone}\");\n"
+                     for cases, no in ((short, ""), (two, "!")) for e, c, n, mb, alone in cases)
+    src = str(tmp_path / "short.cpp")
     with open(src, "w") as f:
-        f.write(source)
-    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-ops-limit=100000000", "-I", os.path.join(ROOT, "include"),
+        f.write('#include "axr_internal.h"\nusing namespace axr;\n' + checks)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "execution-ucx_amd", "csrc"), src], check=True, timeout=120)
 
 

@@ -1,5 +1,5 @@
-"""Few planes against the same elements interleaved, in bundles of their own, where two wavefronts take a block together, and
-wherever else such a plan is launched: every byte against the tensors, and the kernel that moved it."""
+"""Few planes against the same elements interleaved, in blocks of one round or of two, in bundles of their own and wherever
+else such a plan is launched: every byte against the tensors, and the kernel that moved it."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -68,8 +68,8 @@ def together(pkg, movers, kernel):
         m.check(kernel)
 
 
-# a round is 1024 bytes of every plane, a block two: less than one, one and a bit, just below and above two, a
-# block and one round, a block and more than one, ends that are no whole vector
+# a round is 1024 bytes of every plane, a block one or two: less than one, one and a bit, just below and above two, more
+# of them, ends that are no whole vector
 @pytest.mark.gpu
 @pytest.mark.parametrize("item,planes", [(1, 3), (1, 4), (2, 3), (1, 2), (2, 4), (4, 3)])
 @pytest.mark.parametrize("interleaved", [True, False])
@@ -89,18 +89,20 @@ def test_ends_of_blocks(pkg, gpu, item, planes, interleaved):
 
 @pytest.mark.gpu
 def test_neighbours(pkg, gpu):
-    """Planes with halves next to planes without, to runs and to rows, in one bundle and in one launch."""
+    """Planes in blocks of one round and of two, next to each other and to runs, in one bundle and in one launch."""
     three = views(gpu, 1, 3, 5003, 9, True, 1)
     four = views(gpu, 1, 4, 3001, 7, False, 0)
     wide = views(gpu, 4, 3, 2005, 5, True, 0)
     compact = torch.randint(0, 256, (70001,), dtype=torch.uint8, device=gpu)
-    for ts, kernel in (([three, four], PLANES), ([three, wide], PLANES), ([three, compact], ANY), ([compact, four, wide], ANY)):
+    large = views(gpu, 1, 3, 50177, 100, True, 0)      # two rounds next to others
+    for ts, kernel in (([three, four], PLANES), ([three, wide], PLANES), ([three, compact], ANY), ([compact, four, wide], ANY),
+                       ([large, compact], ANY), ([large, three, wide], PLANES)):
         m = Mover(pkg, ts, 256)
         m.alone(kernel)
         m.alone(kernel)
         m.close()
     for lists, kernel in (([[three], [four]], PLANES), ([[wide], [three]], PLANES), ([[three], [wide], [four]], PLANES),
-                          ([[three], [compact]], ANY), ([[compact], [four], [three]], ANY), ([[three, compact], [four]], ANY)):
+                          ([[three], [compact]], ANY), ([[large], [three, compact]], ANY), ([[large], [three]], PLANES), ([[compact], [four], [three]], ANY), ([[three, compact], [four]], ANY)):
         movers = [Mover(pkg, ts, 256) for ts in lists]
         for _ in range(2):
             together(pkg, movers, kernel)

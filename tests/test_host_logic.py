@@ -383,25 +383,34 @@ def test_wavefronts_of_a_launch(pkg):
         pkg.tune(max_waves=old.value)
 
 
-@pytest.mark.parametrize("code,bits,planes,block", [(1, 8, 3, 2048), (1, 8, 4, 2048), (4, 16, 3, 1024), (1, 8, 2, 2048), (4, 16, 4, 1024)])
-def test_blocks_of_planes_do_not_depend_on_their_neighbours(pkg, code, bits, planes, block):
-    """A bundle of planes alone gives two wavefronts to a block where that is faster (three planes, four of bytes; not below
-    a round of 16 bytes per lane); next to other tensors such a block is one wavefront's."""
-    images, item = 6, bits // 8
-    compact = tv(pkg, 0x10000000, [3000])
+@pytest.mark.parametrize("code,bits,planes", [(1, 8, 2), (1, 8, 3), (1, 8, 4), (4, 16, 2), (4, 16, 3), (4, 16, 4)])
+def test_blocks_of_planes_next_to_other_tensors(pkg, code, bits, planes):
+    """One or two rounds of 16 bytes of every plane per lane, 1 or 2 KiB of a plane: three planes, and four of bytes, in blocks of
+    one by themselves and in small bundles, of two next to others in larger ones, whatever the order of the tensors."""
+    item, mib = bits // 8, 1 << 20
+    single = planes == 3 or (planes, item) == (4, 1)
+    compact = tv(pkg, 0x7000000000, [3000])
+    rows = tv(pkg, 0x7100000000, [300, 100], strides=[131, 1])
+    host = tv(pkg, 0x7200000000, [1000], device_type=1)
+    two, one = 2048 // item, 1024 // item
 
-    def shape(pixels, *others):
+    def tiles(tensors):
+        with pkg.BundlePlan.create(tensors) as plan:
+            segs = [s for s in plan.segments() if s["mode"] == 5]
+            assert len(segs) == 1
+            return segs[0]["tiles"], plan.launch_info()["tiles"]
+    for pixels, images in ((one // 2, 6), (one, 6), (one + 1, 6), (5 * two + 3, 6), (50176, 6), (50176, 120), (50177, 120), (50176, 900), (50177, 900), (809, 60000)):
         view = tv(pkg, 0x10000, [images, planes, pixels], strides=[planes * pixels, 1, planes], dtype=(code, bits, 1))
-        with pkg.BundlePlan.create([view, *others]) as plan:
-            info = plan.launch_info()
-            return plan.segments()[0]["tiles"], info["tiles"], info["workgroups"], info["threads_per_workgroup"] // 64
-    for pixels in (block // 4, block // 2, block // 2 + 1, 5 * block + 3, 50176):
-        want = images * -(-pixels // block)
-        tiles, alone, workgroups, waves = shape(pixels)
-        halves = planes != 2 and (planes, item) != (4, 2) and pixels > block // 2
-        assert (tiles, alone, workgroups) == (want, want, -(-want * (2 if halves else 1) // waves))
-        tiles, among, workgroups, waves = shape(pixels, compact)
-        assert (tiles, workgroups) == (want, -(-among // waves))
+        payload = images * planes * pixels * item
+        long, short = images * -(-pixels // two), images * -(-pixels // one)
+        mixed = single and (payload + 100000 <= planes * 4 * mib or (item == 2 and pixels >= 4096 and payload > 28 * mib))
+        for others in ([compact], [rows], [compact, rows], [host, compact]):
+            want = short if mixed else long
+            found = {tiles([view] + others), tiles(others + [view])}
+            assert {f[0] for f in found} == {want} and all(f[1] > want for f in found)
+        alone = single and ((item == 2 and pixels >= 4096) or payload <= 48 * mib or pixels % one == 0)
+        want = short if alone else long
+        assert tiles([view]) == (want, want)
 
 
 def test_transposed_views_use_square_blocks(pkg):

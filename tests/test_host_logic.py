@@ -383,6 +383,25 @@ def test_wavefronts_of_a_launch(pkg):
         pkg.tune(max_waves=old.value)
 
 
+def test_whole_groups_leave_a_tile_to_each_wavefront(pkg):
+    """Skewed blocks alone are rounded up to whole groups of four along the rows that are written (65 x 65 blocks to 68 x 68),
+    unless the empty ones would exceed max_waves: then the bundle keeps its tiles, and each of them its wavefront."""
+    matrix = tv(pkg, 0x10000, [4099, 4097], strides=[1, 4099], dtype=(4, 16, 1))
+    old = C.c_int64()
+    pkg._capi.check(pkg._capi.load().axr_tune_get(b"max_waves", C.byref(old)))
+    try:
+        for most, tiles, each in ((old.value, 68 * 68, 1), (68 * 68, 68 * 68, 1), (68 * 68 - 1, 65 * 65, 1), (65 * 65, 65 * 65, 1),
+                                  (65 * 65 - 1, 65 * 65, 2)):
+            pkg.tune(max_waves=most)
+            with pkg.BundlePlan.create([matrix]) as plan:
+                info = plan.launch_info()
+                assert info["tiles"] == tiles, most
+                waves = info["workgroups"] * info["threads_per_workgroup"] // 64
+                assert (waves >= tiles) == (each == 1), most
+    finally:
+        pkg.tune(max_waves=old.value)
+
+
 @pytest.mark.parametrize("code,bits,planes", [(1, 8, 2), (1, 8, 3), (1, 8, 4), (4, 16, 2), (4, 16, 3), (4, 16, 4)])
 def test_blocks_of_planes_next_to_other_tensors(pkg, code, bits, planes):
     """One or two rounds of 16 bytes of every plane per lane, 1 or 2 KiB of a plane: three planes, and four of bytes, in blocks of

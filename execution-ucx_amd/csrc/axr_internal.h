@@ -239,15 +239,21 @@ constexpr bool plane_single_round(uint32_t element_bytes, uint32_t planes) {
 //    all of them run at once: with 1 MiB of compact tensor 1 MB 0.84 to 0.97, 3 MB 0.85 to 0.96, 10 MB 0.89 to 1.03,
 //    16 MB of three planes 0.92 to 1.11, 256 images of 224 x 224 x 3 bytes 31.2 / 33.5.  Such long planes of 2-byte elements beyond
 //    kShortBlocksMinMixed again: 36 MB 0.89 to 0.97, 64 MB 0.90 to 0.99, 130 MB 0.92 to 0.98 (28 MB of 32,400 x 3 25.0 / 26.4).
+//  - Beyond kShortBlocksMaxLong, where the default tile ends and with it the kernel of planes alone, long planes of whole rounds
+//    only (3.5 GB of 50,176 2300 / 2273, of 50,177 2650 / 2873, of 5000 2730 / 2895, 2.3 GB of 20,001 1720 / 1820, 6 GB 4570 /
+//    4920; slower for one length in eight, whose blocks of two rounds leave the short last ones to the same die, up to
+//    3 GB: 2.3 GB of 7501 1890 / 1820).
 //  - Not where a round gives a wavefront 2 KiB (two planes: 300 of 210 x 200 bytes 18.8 / 19.5), nor for four planes of 2-byte
 //    elements (128 of 128 x 127 14.3 / 15.0, 150 of 200 x 200 33.1 / 33.6).  4-byte elements keep the 8 KiB of the other
 //    blocks with a short dimension (in one round 64 of 224 x 224 x 3 took 27.1 us instead of 31.1).
-constexpr uint64_t kShortBlocksMaxPayload = 48u << 20, kShortBlocksMixedRounds = 4096, kShortBlocksMinMixed = 28u << 20, kShortBlocksLongPlane = 4096;
+constexpr uint64_t kShortBlocksMaxPayload = 48u << 20, kShortBlocksMixedRounds = 4096, kShortBlocksMinMixed = 28u << 20, kShortBlocksMaxLong = 2ull << 30;
+constexpr uint64_t kShortBlocksLongPlane = 4096;
 constexpr bool plane_short_blocks(uint32_t element_bytes, uint32_t planes, uint64_t extent, uint64_t payload_bytes, bool alone) {
   if (!plane_single_round(element_bytes, planes)) return false;
-  const bool long_planes = element_bytes == 2 && extent >= kShortBlocksLongPlane;
+  const bool whole = extent % plane_round_elements(element_bytes) == 0;
+  const bool long_planes = element_bytes == 2 && extent >= kShortBlocksLongPlane && (whole || payload_bytes <= kShortBlocksMaxLong);
   if (!alone) return payload_bytes <= kShortBlocksMixedRounds * planes * kRowBytes || (long_planes && payload_bytes > kShortBlocksMinMixed);
-  return long_planes || payload_bytes <= kShortBlocksMaxPayload || extent % plane_round_elements(element_bytes) == 0;
+  return long_planes || payload_bytes <= kShortBlocksMaxPayload || whole;
 }
 constexpr uint32_t kMaxPlanes = 4;
 // Dims.lanes_per_run of such a segment: which side holds the planes, and above that the routine that moves its blocks.

@@ -112,10 +112,12 @@ static_assert(in_planes(1, 16) && !in_planes(1, 15) && in_planes(4, 201) && !in_
 def test_short_blocks_of_planes(tmp_path):
     """In blocks of one round on the side that was measured to be faster: (element bytes, planes, elements of a plane, MB, alone)."""
     short = [(1, 3, 50176, 37, 1), (1, 3, 7501, 24, 1), (1, 4, 30011, 40, 1), (1, 4, 3072, 256, 1), (1, 3, 50176, 300, 1), (2, 3, 7501, 180, 1),
-             (2, 3, 3563, 24, 1), (1, 3, 50176, 9, 0), (1, 4, 7501, 10, 0), (2, 3, 32400, 4, 0), (2, 3, 7501, 36, 0), (2, 3, 7501, 130, 0)]
+             (2, 3, 3563, 24, 1), (1, 3, 50176, 9, 0), (1, 4, 7501, 10, 0), (2, 3, 32400, 4, 0), (2, 3, 7501, 36, 0), (2, 3, 7501, 130, 0),
+             (2, 3, 50176, 3500, 0)]
     two = [(1, 3, 7501, 180, 1), (1, 4, 7501, 300, 1), (1, 4, 50000, 64, 1), (1, 2, 42000, 25, 1), (2, 4, 16256, 17, 1), (2, 2, 40000, 10, 1),
            (4, 3, 50176, 38, 1), (1, 3, 50176, 38, 0), (1, 3, 38190, 15, 0), (1, 4, 50176, 40, 0), (2, 3, 32400, 19, 0), (2, 3, 32400, 28, 0), (2, 2, 3000, 2, 0),
-           (2, 3, 3000, 300, 1), (2, 3, 809, 298, 1), (2, 3, 3000, 36, 0)]
+           (2, 3, 3000, 300, 1), (2, 3, 809, 298, 1), (2, 3, 3000, 36, 0),
+           (2, 3, 50177, 3500, 0), (2, 3, 5000, 3500, 0), (2, 3, 20001, 2300, 0), (2, 3, 20001, 6000, 0)]
     checks = "".join(f"static_assert({no}plane_short_blocks({e}, {c}, {n}, {mb}000000ull, {alone}), \"{e} {c} {n} {mb} {alone}\");\n"
                      for cases, no in ((short, ""), (two, "!")) for e, c, n, mb, alone in cases)
     src = str(tmp_path / "short.cpp")
